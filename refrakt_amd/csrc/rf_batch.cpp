@@ -24,7 +24,7 @@ struct rf_batch {
   size_t total_bins = 0;
   DevBuf blocks, palettes, frames, hist, images, perms;
   DevBuf drawn, remaining, done_ts, items, tiles_done, de_done_ts, t0;
-  DevBuf de_rad, de_wt;            // density estimation: radius per bin (largest frame), weight table
+  DevBuf de_rad, de_tab;           // density estimation: radius per bin (largest frame), chord table
   // A replay runs in slices: ranges of work items in frame order, each one
   // chaos-game launch (plus, with RF_HIST_SORT, its record passes), followed
   // by the density estimation of the frames it completes on a second stream.
@@ -380,14 +380,11 @@ int capture(rf_batch* b) {
       g.H = b->H[f];
       g.R = std::max(0, std::min(d.estimator_radius, 100));  // src/main.cpp:502
       g.rmin = std::max(0, std::min(d.estimator_min, 100));
-      g.rad = (signed char*)b->de_rad.p;
-      g.wt = (float*)b->de_wt.p;
+      g.rad = (uint8_t*)b->de_rad.p;
+      g.tab = (const rfk::DETable*)b->de_tab.p;
       g.curve = d.estimator_curve;
       g.do_tonemap = 1;
-      g.gamma = d.gamma;
-      g.brightness = d.brightness;
-      g.vibrancy = d.vibrancy;
-      g.k = 1.0f / 10000.0f;                                   // src/main.cpp:228
+      g.tone = rfk::tone_args(d.gamma, d.brightness, d.vibrancy, 1.0f / 10000.0f);  // src/main.cpp:228
       g.tiles_done = (uint32_t*)b->tiles_done.p + f;
       g.done_ts = (unsigned long long*)b->de_done_ts.p + f;
       e = rfk::launch_de_tonemap(g, b->de_stream);
@@ -490,15 +487,12 @@ int rf_batch_create(rf_ctx* ctx, const rf_frame_desc* frames, uint32_t n, rf_bat
   if (e == hipSuccess) e = b->de_done_ts.alloc(8ull * n);
   if (e == hipSuccess) e = b->t0.alloc(8);
   size_t max_bins = 0;
-  int span = 0;
-  for (uint32_t f = 0; f < n; ++f) {
-    max_bins = std::max(max_bins, (size_t)b->W[f] * b->H[f]);
-    span = std::max(span, std::max(0, std::min(std::max(b->desc[f].estimator_radius, b->desc[f].estimator_min), 100)));
-  }
+  for (uint32_t f = 0; f < n; ++f) max_bins = std::max(max_bins, (size_t)b->W[f] * b->H[f]);
   // frames' DE launches run one after another on the batch's stream, so they
   // share one radius buffer
   if (e == hipSuccess) e = b->de_rad.alloc(max_bins);
-  if (e == hipSuccess) e = b->de_wt.alloc(rfk::de_weight_bytes(span));
+  if (e == hipSuccess) e = b->de_tab.alloc(sizeof(rfk::DETable));
+  if (e == hipSuccess) e = rfk::launch_de_chords((rfk::DETable*)b->de_tab.p, b->stream);
   if (e == hipSuccess) e = hipMemcpy(b->blocks.p, blk.data(), sizeof(Block) * n, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(b->palettes.p, pal.data(), pal.size() * sizeof(float), hipMemcpyHostToDevice);
   if (e != hipSuccess) {

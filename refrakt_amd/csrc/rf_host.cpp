@@ -861,8 +861,9 @@ static int do_draw(rf_ctx* ctx, rf_flame* f, rf_hist* h, uint32_t num_iter, cons
   return RF_OK;
 }
 
-// DE arguments for histogram h; grows the histogram's radius buffer and the
-// context's weight table to what the launch needs.
+// DE arguments for histogram h; grows the histogram's radius buffer to
+// what the launch needs and fills the context's chord table (constants) on
+// its first use.
 static int de_args(rf_ctx* ctx, rf_hist* h, const rf_de_params* de, rfk::DEArgs& a) {
   a = rfk::DEArgs{};
   a.hist = (const float4*)h->ptr;
@@ -872,11 +873,14 @@ static int de_args(rf_ctx* ctx, rf_hist* h, const rf_de_params* de, rfk::DEArgs&
     a.rmin = std::max(0, std::min(de->estimator_min, 100));
     a.curve = de->estimator_curve;
   }
-  const size_t nb = (size_t)h->w * h->h, wb = rfk::de_weight_bytes(std::max(a.R, a.rmin));
+  const size_t nb = (size_t)h->w * h->h;
   if (h->de_rad.bytes < nb) HIPCHK(ctx, h->de_rad.alloc(nb));
-  if (ctx->de_wt.bytes < wb) HIPCHK(ctx, ctx->de_wt.alloc(wb));
-  a.rad = (signed char*)h->de_rad.p;
-  a.wt = (float*)ctx->de_wt.p;
+  if (!ctx->de_tab.p) {
+    HIPCHK(ctx, ctx->de_tab.alloc(sizeof(rfk::DETable)));
+    HIPCHK(ctx, rfk::launch_de_chords((rfk::DETable*)ctx->de_tab.p, ctx->stream));
+  }
+  a.rad = (uint8_t*)h->de_rad.p;
+  a.tab = (const rfk::DETable*)ctx->de_tab.p;
   return RF_OK;
 }
 
@@ -1313,8 +1317,9 @@ int rf_density_estimate(rf_ctx* ctx, rf_hist* h, const rf_de_params* de, void* o
 
 int rf_tonemap(rf_ctx* ctx, const void* in, void* out, uint32_t w, uint32_t h, const rf_tonemap_params* tm) {
   if (!ctx || !in || !out || !tm) return set_err(ctx, RF_ERR_ARG, "null argument");
-  HIPCHK(ctx, rfk::launch_tonemap((const float4*)in, (float4*)out, w * h, tm->gamma, tm->brightness, tm->vibrancy,
-                                  tm->scale_constant, ctx->stream));
+  HIPCHK(ctx, rfk::launch_tonemap((const float4*)in, (float4*)out, w * h,
+                                  rfk::tone_args(tm->gamma, tm->brightness, tm->vibrancy, tm->scale_constant),
+                                  ctx->stream));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   return RF_OK;
 }
@@ -1327,7 +1332,7 @@ int rf_density_tonemap(rf_ctx* ctx, rf_hist* h, const rf_de_params* de, const rf
   if (rc) return rc;
   a.img_out = (float4*)out;
   a.do_tonemap = 1;
-  a.gamma = tm->gamma; a.brightness = tm->brightness; a.vibrancy = tm->vibrancy; a.k = tm->scale_constant;
+  a.tone = rfk::tone_args(tm->gamma, tm->brightness, tm->vibrancy, tm->scale_constant);
   HIPCHK(ctx, rfk::launch_de_tonemap(a, ctx->stream));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   return RF_OK;
@@ -1370,8 +1375,10 @@ int rf_render(rf_ctx* ctx, rf_flame* f, const rf_render_params* rp, float* hist_
   HIPCHK(ctx, rfk::launch_de_tonemap(da, ctx->stream));
   HIPCHK(ctx, hipEventRecord(ctx->ev[1], ctx->stream));
   HIPCHK(ctx, rfk::launch_tonemap((const float4*)ctx->render_img.p, (float4*)ctx->render_img.p,
-                                  rp->width * rp->height, rp->tm.gamma, rp->tm.brightness, rp->tm.vibrancy,
-                                  rp->tm.scale_constant, ctx->stream));
+                                  rp->width * rp->height,
+                                  rfk::tone_args(rp->tm.gamma, rp->tm.brightness, rp->tm.vibrancy,
+                                                 rp->tm.scale_constant),
+                                  ctx->stream));
   if (!ctx->ev[2]) { HIPCHK(ctx, hipEventCreate(&ctx->ev[2])); HIPCHK(ctx, hipEventCreate(&ctx->ev[3])); }
   HIPCHK(ctx, hipEventRecord(ctx->ev[2], ctx->stream));
   HIPCHK(ctx, hipEventSynchronize(ctx->ev[2]));

@@ -112,7 +112,7 @@ struct rf_ctx {
   rfh::DevBuf probe;           // atomic probe scratch
   rf_hist* render_hist = nullptr;
   rfh::DevBuf render_img;
-  rfh::DevBuf de_wt;           // density estimation: splat weight table
+  rfh::DevBuf de_tab;          // density estimation: chord table
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   double last_draw_ms = 0.0;   // device time of the last draw_to_bins' chaos-game launches
   bool programs = true;        // fast engine: run flame programs (rf_jit.cpp)

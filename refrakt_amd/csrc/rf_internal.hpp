@@ -48,6 +48,29 @@ struct FastArgs {
   SortArgs sort;                 // RF_HIST_SORT only
 };
 
+// The splat's shape: see k_de_chords.
+constexpr int DE_MAX_R = 100;          // largest splat radius
+constexpr int DE_CHORD_STRIDE = 128;   // radii per table row
+constexpr int DE_C_ROW0 = 108, DE_C_ROWS = 216;
+struct DEChord {
+  int hl;
+  float nx, step, pad;
+};
+struct DETable {
+  DEChord rows[2 * DE_MAX_R + 1][DE_CHORD_STRIDE];
+  float c[DE_MAX_R + 1][DE_C_ROWS];
+};
+
+// Tonemap parameters; ig = 1 / gamma, rounded once.
+struct ToneArgs {
+  float ig, brightness, vibrancy, k;
+};
+#ifndef __HIPCC_RTC__
+inline ToneArgs tone_args(float gamma, float brightness, float vibrancy, float k) {
+  return ToneArgs{(float)(1.0 / (double)gamma), brightness, vibrancy, k};
+}
+#endif
+
 struct DEArgs {
   const float4* hist;            // W*H bins (rows bottom-up)
   float4* de_out;                // may be null
@@ -56,19 +79,16 @@ struct DEArgs {
   int32_t R, rmin;
   float curve;
   int32_t do_tonemap;
-  float gamma, brightness, vibrancy, k;
+  ToneArgs tone;
   // Optional completion stamp (batched rendering): the last workgroup to
   // finish writes the wall clock to *done_ts; *tiles_done counts workgroups.
   uint32_t* tiles_done;
   unsigned long long* done_ts;
-  // Work buffers: every bin's splat radius (W*H bytes, -1 empty) and the
-  // splat weights of radii 0..max(R, rmin) (de_weight_bytes).
-  signed char* rad;
-  float* wt;
+  // Work buffer: every bin's splat radius (W*H bytes, see k_de_radius).
+  uint8_t* rad;
+  // Chord table (launch_de_chords).
+  const DETable* tab;
 };
-
-// Bytes of the splat-weight table of radii 0..R (sum over r of (2r+1)^2 floats).
-inline size_t de_weight_bytes(int R) { return (size_t)(4 * (R + 1) * (R + 1) * (R + 1) - (R + 1)) / 3 * 4; }
 
 constexpr int NPERM = 8;          // permutation rows of the fast engine (held in LDS)
 // Draw counters: COUNTER_SLOTS slots of COUNTER_STRIDE u64 (one 128-byte
@@ -86,12 +106,12 @@ hipError_t launch_fast(const FastArgs& a, uint64_t n_particles, int waves, int h
 // Fills n u64 with zero (a kernel, not a memset: safe under graph capture).
 hipError_t launch_zero_u64(unsigned long long* p, uint32_t n, hipStream_t s);
 hipError_t launch_animate(rfd::Block* blocks, uint32_t T, float tss_width, const float* rot, hipStream_t s);
-// Density estimation (+ tonemap): a.rad (W*H bytes) and a.wt
-// (de_weight_bytes(max(a.R, a.rmin))) must be device buffers the launch may
-// overwrite; R and rmin in [0, 100].
+// Fills the chord table.
+hipError_t launch_de_chords(DETable* tab, hipStream_t s);
+// Density estimation (+ tonemap): a.rad (W*H bytes) is a device buffer the
+// launch may overwrite, a.tab the chord table; R and rmin in [0, DE_MAX_R].
 hipError_t launch_de_tonemap(const DEArgs& a, hipStream_t s);
-hipError_t launch_tonemap(const float4* in, float4* out, uint32_t n, float gamma, float brightness,
-                          float vibrancy, float k, hipStream_t s);
+hipError_t launch_tonemap(const float4* in, float4* out, uint32_t n, const ToneArgs& t, hipStream_t s);
 hipError_t launch_rgba8(const float4* in, uchar4* out, uint32_t n, hipStream_t s);
 hipError_t launch_eval_xform(const rfd::Block* blk, const float* pts, const float* rands, float* out,
                              uint32_t n, hipStream_t s);

@@ -2,6 +2,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "rf_kern_common.hpp"
 
 using namespace rfd;
@@ -65,55 +67,39 @@ __global__ __launch_bounds__(256) void k_animate(Block* blocks, uint32_t T, floa
 // r = max(rmin, min(R, int(R / a^curve))).
 // A splat reaches span = max(R, rmin) texels from its centre.
 
-struct DESrc { float r, e, nrm, pad; };
-
-__device__ __forceinline__ void de_source(const DEArgs& g, int cx, int cy, float4& col, DESrc& m) {
-  col = make_float4(0.f, 0.f, 0.f, 0.f);
-  m.r = -1.0f; m.e = 0.0f; m.nrm = 0.0f; m.pad = 0.0f;
-  const int px = cx + 1, py = (int)g.H - 1 - cy;
-  if (cx < 0 || px >= (int)g.W || cy < 0 || cy >= (int)g.H) return;
-  const float4 b = g.hist[(size_t)py * g.W + px];
-  if (!(b.w != 0.0f)) return;  // color.a == 0.0 -> point moved out of the view volume
-  const float q = rf_div_rn((float)g.R, powf(b.w, g.curve));
-  int ri = (q >= (float)g.R) ? g.R : (int)q;
-  if (!(q == q)) ri = g.R;
-  int r = ri > g.rmin ? ri : g.rmin;
-  if (r < 0) r = 0;
-  col = b;
-  m.r = (float)r;
-  const int S = 2 * r + 1;
-  m.e = rf_div_rn(1.0f, (float)S);
-  m.nrm = (r > 0) ? rf_div_rn(0.63661977236f, (float)(r * r)) : 1.0f;
-}
-
-__device__ __forceinline__ float de_weight(const DESrc& m, int i, int j) {
-  const int r = (int)m.r;
-  if (r < 0) return 0.0f;
-  if (r == 0) return (i == 0 && j == 0) ? 1.0f : 0.0f;
-  if (i > r || i < -r || j > r || j < -r) return 0.0f;
-  const float nx = (2.0f * (float)j + m.e) * m.e;
-  const float ny = (2.0f * (float)i + m.e) * m.e;
-  const float d = nx * nx + ny * ny;
-  if (d > 1.0f) return 0.0f;
-  return (1.0f - d) * m.nrm;
-}
+// x^y for x >= 0: the library's powf without its sign and integer-exponent
+// cases, the same bits.
+extern "C" __device__ float __ocml_powr_f32(float, float);
 
 // shaders/tonemap.glsl:18-39 with scale_constant k; an empty texel (a = 0,
-// where the shader divides 0/0) maps to black.
-__device__ __forceinline__ float4 tonemap_px(float4 c, float gamma, float brightness, float vib, float k) {
+// where the shader divides 0/0) maps to black.  Bound by VALU issue: four
+// powers of about 160 instructions each; powr in their place takes 3840x2160
+// with 8-bit conversion from 117 to 110 us, and at vibrancy 1 one power is
+// left.
+__device__ __forceinline__ float4 tonemap_px(float4 c, const ToneArgs& t) {
   if (!(c.w > 0.0f)) return make_float4(0.f, 0.f, 0.f, 1.0f);
   // log(1 + a k) through log1pf: the shader's float log(1.0 + a*k) loses most
   // digits when a*k is small (k = 1e-4 makes that every sparse texel).
-  const float ls = rf_div_rn(((0.5f * brightness) * log1pf(c.w * k)) * LOG10E, c.w);
+  const float ls = rf_div_rn(((0.5f * t.brightness) * log1pf(c.w * t.k)) * LOG10E, c.w);
   c.x *= ls; c.y *= ls; c.z *= ls; c.w *= ls;
-  const float ig = rf_div_rn(1.0f, gamma);
-  const float z = powf(c.w, ig);
-  const float gf = rf_div_rn(z, c.w);
   float o[3] = {c.x, c.y, c.z};
+  const float lo = fminf(fminf(c.x, c.y), fminf(c.z, c.w)), hi = fmaxf(c.x, fmaxf(c.y, c.z));
+  if (t.ig > 0.0f && t.ig <= 1.0f && lo >= 0.0f && hi < __builtin_inff()) {
+    const float gf = rf_div_rn(__ocml_powr_f32(c.w, t.ig), c.w);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const float g = gf * o[q];
+      // at vibrancy 1 the power has weight 0 (and is finite: 0 <= o < inf, ig <= 1)
+      o[q] = t.vibrancy == 1.0f ? g : rf_mix(__ocml_powr_f32(o[q], t.ig), g, t.vibrancy);
+    }
+  } else {
+    const float gf = rf_div_rn(powf(c.w, t.ig), c.w);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) o[q] = rf_mix(powf(o[q], t.ig), gf * o[q], t.vibrancy);
+  }
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
-    float v = rf_mix(powf(o[q], ig), gf * o[q], vib);
-    v = fminf(fmaxf(v, 0.0f), 1.0f);
+    float v = fminf(fmaxf(o[q], 0.0f), 1.0f);
     if (!(v == v)) v = 0.0f;
     o[q] = v;
   }
@@ -135,190 +121,316 @@ __device__ __forceinline__ void de_stamp(const DEArgs& g) {
   }
 }
 
-// Splat weights of every radius 0..R with de_weight's arithmetic: entry
-// (i + r) * (2r + 1) + (r - j) of radius r (each row's columns in descending
-// order, the order in which the gather walks a chord) starts at
-// de_wt_off(r) = sum over q < r of (2q + 1)^2.
-__device__ __forceinline__ int de_wt_off(int r) { return (4 * r * r * r - r) / 3; }
+// Chord table, constants of the splat's shape.  rows[i + DE_MAX_R][r]
+// describes the row of the radius-r splat that lies i texels from its centre:
+// the columns j with a positive weight form the interval [hi - len, hi]
+// (hl = hi & 0xff | len << 8, -1 where the splat has no such row), and the
+// weight of column hi - b is c - (nx - b * step)^2, the reference's
+// (1 - nx^2 - ny^2) * norm with sqrt(norm) folded into nx and step and the
+// row's share into c = c[r][i + DE_C_ROW0], which is negative outside the splat.
+__device__ __forceinline__ float de_chord_weight(float nx, float c) { return fmaf(-nx, nx, c); }
 
-__global__ __launch_bounds__(256) void k_de_weights(float* __restrict__ wt, int R) {
-  for (int r = 0; r <= R; ++r) {
-    const int S = 2 * r + 1;
-    DESrc m;
-    m.r = (float)r;
-    m.e = rf_div_rn(1.0f, (float)S);
-    m.nrm = (r > 0) ? rf_div_rn(0.63661977236f, (float)(r * r)) : 1.0f;
-    for (int q = threadIdx.x; q < S * S; q += blockDim.x) wt[de_wt_off(r) + q] = de_weight(m, q / S - r, r - q % S);
+__global__ __launch_bounds__(DE_CHORD_STRIDE) void k_de_chords(DETable* __restrict__ tab) {
+  const int r = (int)threadIdx.x, i = (int)blockIdx.x - DE_C_ROW0;
+  DEChord e;
+  e.hl = -1; e.nx = 0.0f; e.step = 0.0f; e.pad = 0.0f;
+  float c = -1.0f;
+  if (r == 0 && i == 0) {
+    e.hl = 0; c = 1.0f;
+  } else if (r <= DE_MAX_R && i >= -r && i <= r) {
+    // the weight's terms in double, rounded once
+    const double inv = 1.0 / (double)(2 * r + 1), sn = sqrt((double)M_2_PI_F) / (double)r;
+    const double ny = (2.0 * i + inv) * inv;
+    e.step = (float)(2.0 * inv * sn);
+    c = (float)((1.0 - ny * ny) * sn * sn);
+    // the chord's ends in real arithmetic, then inwards to the first positive
+    // weight as it is evaluated
+    const double half = 0.5 * (double)(2 * r + 1) * sqrt(1.0 - ny * ny);
+    auto positive = [&](int j) { return de_chord_weight((float)((2.0 * j + inv) * inv * sn), c) > 0.0f; };
+    int hi = min(r, (int)ceil(half)), lo = max(-r, (int)floor(-half) - 1);
+    while (hi >= lo && !positive(hi)) --hi;
+    while (hi >= lo && !positive(lo)) ++lo;
+    e.nx = (float)((2.0 * hi + inv) * inv * sn);
+    if (hi >= lo) e.hl = (int)((uint32_t)(hi & 0xff) | ((uint32_t)(hi - lo) << 8));
   }
+  if (r <= DE_MAX_R) tab->c[r][blockIdx.x] = c;
+  if (i >= -DE_MAX_R && i <= DE_MAX_R) tab->rows[i + DE_MAX_R][r] = e;
 }
 
-// Every bin's splat radius (de_source's arithmetic), -1 for an empty bin.
+// Every bin's splat radius: DE_EMPTY for an empty bin, DE_ODD added where the
+// bin holds an infinity or NaN.
+constexpr uint32_t DE_EMPTY = 255u, DE_ODD = 128u;
+
 __global__ __launch_bounds__(256) void k_de_radius(DEArgs g) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (size_t)g.W * g.H) return;
-  const float a = g.hist[i].w;
-  int r = -1;
-  if (a != 0.0f) {
-    const float q = rf_div_rn((float)g.R, powf(a, g.curve));
+  const float4 c = g.hist[i];
+  uint32_t v = DE_EMPTY;
+  if (c.w != 0.0f) {
+    const float q = rf_div_rn((float)g.R, powf(c.w, g.curve));
     int ri = (q >= (float)g.R) ? g.R : (int)q;
     if (!(q == q)) ri = g.R;
-    r = ri > g.rmin ? ri : g.rmin;
-    if (r < 0) r = 0;
+    const int r = max(max(ri, g.rmin), 0);
+    // one infinity or NaN makes the sum of the products one
+    const float z = fmaf(c.x, 0.0f, fmaf(c.y, 0.0f, fmaf(c.z, 0.0f, c.w * 0.0f)));
+    v = (uint32_t)r + (z != 0.0f ? DE_ODD : 0u);
   }
-  g.rad[i] = (signed char)r;
+  g.rad[i] = (uint8_t)v;
 }
 
-// A TW x TH tile of texels per workgroup of 256 threads (TH / 8 texels per
-// thread) from an LDS copy of the (TW + 2R) x (TH + 2R) sources around it.
-// Per source row the tile keeps one 64-bit column mask per radius r (the
-// sources whose radius is exactly r) and a mask of the radii present, so a
-// texel visits, for row offset i, only the radii r >= |i| present in that
-// row and, per radius, only the columns within r of its own: every source
-// it reads contributes (up to the disc test inside the square).
-constexpr int DE_TW = 32;
-// Row strides of the per-radius tables, powers of two so that indexing by
-// radius is a shift (a multiply by 2R + 1 or by the tile height is a
-// quarter-rate integer instruction in the innermost (row, radius) loop):
-// s_e rows of DE_ES >= TH + 2R entries, s_jx rows of DE_JS >= 2R + 1.
-constexpr int DE_ES_SHIFT = 6, DE_JS_SHIFT = 5;
-constexpr int DE_ES = 1 << DE_ES_SHIFT, DE_JS = 1 << DE_JS_SHIFT;
+// Density estimation of a 64 x (8 V) tile of texels per workgroup of eight
+// waves, for any radius up to 100 (bound: VALU issue).  A wave owns V adjacent
+// texel rows of 64 columns, so the source row, the radius and the splat rows
+// it visits are uniform over the wave: the loop over them runs on the scalar
+// unit and the chord table is read with scalar loads.  LDS holds, per source
+// row, one column mask per radius (the sources whose radius is exactly r) and
+// the radii present, for K source rows at a time.  For a radius present in a
+// row a lane shifts the mask to its own column, keeps the bits of the widest
+// chord of its V rows (32 columns at a time) and adds the sources they name
+// to all V texels: the bit scan, the colour's load and the horizontal part of
+// the weight are paid once per source and V texels (27 VALU per source and
+// four texels; the same gather texel by texel took 10 to 11 per source), and
+// the vertical part is one clamped fma per texel, 0 outside the row's own
+// chord.  The colours are read straight from the histogram, where the waves
+// of a tile find them in L1 or L2: staged in LDS they limited the tile to
+// strips of 16 source rows, between which waves waited (7680x4320 radius 9:
+// 1637 us against 1525).  Two sources a round, so that two loads are in
+// flight: 1525 -> 1416 us.  Tiles are numbered down their columns: neighbours
+// in flight share source rows (2048x2048 radius 9: 286 -> 258 us).
+constexpr int DR_W = 64, DR_WAVES = 8;
 
-template <int TH, int NTH>
-__global__ __launch_bounds__(NTH) void k_de_tiled(DEArgs g) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int R = max(g.R, g.rmin);  // span
-  const int SW = DE_TW + 2 * R, SH = TH + 2 * R;
-  float4* s_col = reinterpret_cast<float4*>(smem);
-  unsigned long long* s_e = reinterpret_cast<unsigned long long*>(smem + sizeof(float4) * SW * SH);  // [r][row]
-  uint32_t* s_rp = reinterpret_cast<uint32_t*>(s_e + (R + 1) * DE_ES);                                 // [row]
-  float* s_wt = reinterpret_cast<float*>(s_rp + SH);
-  // s_jx[r * DE_JS + i + R]: the columns j with a non-zero weight in row
-  // offset i of radius r form the interval [lo, hi] (the disc's chord);
-  // .x = (R - hi) | (index of w(i, hi) in s_wt) << 8 (the mask shift
-  // relative to the texel's column, then the weights), .y = the chord's bit
-  // mask (2 << (hi - lo)) - 1, 0 when the row has none.  One 8-byte entry,
-  // read beside the source mask it applies to, so neither read waits on the
-  // other; 8 bytes keep three workgroups per CU at R = 9.
-  const size_t jx_off = ((size_t)(reinterpret_cast<unsigned char*>(s_wt + de_wt_off(R + 1)) - smem) + 7) & ~(size_t)7;
-  uint2* s_jx = reinterpret_cast<uint2*>(smem + jx_off);
-  __shared__ int s_rmax;
-  const int tx0 = blockIdx.x * DE_TW, ty0 = blockIdx.y * TH;
-  const int tid = threadIdx.x;
-  if (tid == 0) s_rmax = 0;
-  for (int q = tid; q < de_wt_off(R + 1); q += NTH) s_wt[q] = g.wt[q];
-  for (int q = tid; q < (R + 1) * DE_ES; q += NTH) s_e[q] = 0ull;
-  for (int q = tid; q < SH; q += NTH) s_rp[q] = 0u;
-  for (int q = tid; q < (R + 1) * DE_JS; q += NTH) {
-    const int r = q >> DE_JS_SHIFT, i = (q & (DE_JS - 1)) - R;
-    uint2 v = make_uint2(0u, 0u);
-    if (i >= -r && i <= r) {
-      const float* w = g.wt + de_wt_off(r) + (i + r) * (2 * r + 1);
-      int lo = r + 1, hi = -r - 1;
-      for (int j = -r; j <= r; ++j)
-        if (w[r - j] != 0.0f) { lo = min(lo, j); hi = max(hi, j); }
-      // a chord is at most 2r + 1 <= 31 columns wide: its mask fits 32 bits
-      if (lo <= hi)
-        v = make_uint2((uint32_t)(R - hi) | ((uint32_t)(de_wt_off(r) + (i + r) * (2 * r + 1) + r - hi) << 8),
-                       (2u << (hi - lo)) - 1u);
+typedef const __attribute__((address_space(4))) DETable CDETable;
+typedef int int4_t __attribute__((ext_vector_type(4)));
+
+// One visit's uniform values: the widest chord and the V rows' shares.
+template <int V>
+struct DEVisit {
+  int hl;
+  float nx, step, c[V];
+};
+
+// Rows i .. i + V - 1 of radius r, the widest of them row iw.
+template <int V>
+__device__ __forceinline__ DEVisit<V> de_visit(CDETable* tab, int r, int i, int iw) {
+  const int4_t q = *reinterpret_cast<const __attribute__((address_space(4))) int4_t*>(&tab->rows[iw + DE_MAX_R][r]);
+  DEVisit<V> v;
+  v.hl = q.x;
+  v.nx = __int_as_float(q.y);
+  v.step = __int_as_float(q.z);
+#pragma unroll
+  for (int k = 0; k < V; ++k) v.c[k] = tab->c[r][i + DE_C_ROW0 + k];
+  return v;
+}
+
+// LDS words per source row of the tile: colours, masks, radii present.
+__host__ __device__ inline int dr_mask_words(int R) { return ((DR_W - 1 + 2 * R) >> 5) + 2; }
+inline uint64_t dr_tiles(uint32_t W, uint32_t H, int V) {
+  return ((uint64_t)W + DR_W - 1) / DR_W * (((uint64_t)H + DR_WAVES * V - 1) / (DR_WAVES * V));
+}
+inline size_t dr_row_bytes(int R) {
+  return (size_t)(R + 1) * dr_mask_words(R) * 4 + (R < 32 ? 4u : 16u);
+}
+
+__device__ __forceinline__ float4 de_source(const float4* row, int x) {
+  return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(row) + (uint32_t)(x << 4));
+}
+
+// Adds a source of weight v (none where v <= 0).
+template <bool ALL>
+__device__ __forceinline__ void de_add(float4& acc, const float4& c, float v) {
+  const float w = __builtin_amdgcn_fmed3f(v, 0.0f, 1.0f);
+  const bool in = ALL || w > 0.0f;  // a select, not a branch: the sums stay in their registers
+  acc.x = fmaf(in ? c.x : 0.0f, w, acc.x);
+  acc.y = fmaf(in ? c.y : 0.0f, w, acc.y);
+  acc.z = fmaf(in ? c.z : 0.0f, w, acc.z);
+  acc.w = fmaf(in ? c.w : 0.0f, w, acc.w);
+}
+
+// Adds the sources of one visit to the V texels of this lane.  With ALL the
+// sources are finite and a texel outside its row's chord adds 0 of them;
+// otherwise it must leave them out (0 * inf).
+template <int V, bool ALL, bool SHORT>
+__device__ __forceinline__ void de_taps(float4 (&acc)[V], const DEVisit<V>& v, int col0, const uint32_t* em,
+                                        const float4* cr) {
+  const int len = v.hl >> 8;  // the row is within the radius: never empty
+  for (int b0 = 0; SHORT ? b0 == 0 : b0 <= len; b0 += 32) {
+    const int col = col0 + b0;
+    const uint32_t* const ew = em + (col >> 5);
+    uint32_t m = __builtin_amdgcn_alignbit(ew[1], ew[0], col & 31);
+    if (SHORT || len - b0 < 31) m &= (2u << (len - b0)) - 1u;
+    const float nx0 = fmaf(-(float)b0, v.step, v.nx);
+    // two sources a round, so that two loads are in flight
+    while (m) {
+      const int b = __builtin_ctz(m);
+      m &= m - 1u;
+      const float4 c = de_source(cr, col + b);
+      const bool two = m != 0u;
+      const int b2 = two ? __builtin_ctz(m) : b;
+      m &= m - 1u;
+      const float4 c2 = de_source(cr, col + b2);
+      const float nx = fmaf(-(float)b, v.step, nx0);
+      // a missing second source lies outside every chord
+      const float nx2 = two ? fmaf(-(float)b2, v.step, nx0) : 2.0f;
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        de_add<ALL>(acc[k], c, de_chord_weight(nx, v.c[k]));
+        de_add<ALL>(acc[k], c2, de_chord_weight(nx2, v.c[k]));
+      }
     }
-    s_jx[q] = v;
   }
-  __syncthreads();
-  int rloc = 0;
-  for (int k = tid; k < SW * SH; k += NTH) {
-    const int ly = k / SW, lx = k % SW;
-    const int cx = tx0 - R + lx, cy = ty0 - R + ly;
-    const int px = cx + 1, py = (int)g.H - 1 - cy;
-    if (cx < 0 || px >= (int)g.W || cy < 0 || cy >= (int)g.H) continue;
-    const size_t b = (size_t)py * g.W + px;
-    const int r = g.rad[b];
-    if (r < 0) continue;
-    s_col[k] = g.hist[b];
-    atomicOr(&s_e[(r << DE_ES_SHIFT) + ly], 1ull << lx);
-    atomicOr(&s_rp[ly], 1u << r);
-    rloc = max(rloc, r);
-  }
-  rloc = max(rloc, __shfl_xor(rloc, 32));
-  rloc = max(rloc, __shfl_xor(rloc, 16));
-  rloc = max(rloc, __shfl_xor(rloc, 8));
-  rloc = max(rloc, __shfl_xor(rloc, 4));
-  rloc = max(rloc, __shfl_xor(rloc, 2));
-  rloc = max(rloc, __shfl_xor(rloc, 1));
-  if ((tid & 63) == 0) atomicMax(&s_rmax, rloc);
-  __syncthreads();
-  const int RM = min(R, s_rmax);
-  const int lx = tid % DE_TW;
-#pragma unroll 1
-  for (int ly = tid / DE_TW; ly < TH; ly += NTH / DE_TW) {
-    const int tx = tx0 + lx, ty = ty0 + ly;
-    if (tx >= (int)g.W || ty >= (int)g.H) continue;
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    // source (row ly + R - i, column lx + R - j) adds weight w_r(i, j)
-    for (int i = -RM; i <= RM; ++i) {
-      const int rowi = ly + R - i;
-      const int ai = i < 0 ? -i : i;
-      uint32_t radii = s_rp[rowi] >> ai;
-      while (radii) {
-        const int r = ai + __builtin_ctz(radii);
+}
+
+// Adds a strip's sources to the wave's V texel rows.
+template <int V, int NRW, bool ALL, bool SHORT>
+__device__ __forceinline__ void de_strip(float4 (&acc)[V], CDETable* tab, const float4* src, int W, const uint32_t* s_e,
+                                         const uint32_t* s_rp, int R, int K, int s0, int rows) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int nwd = dr_mask_words(R), mrow = (R + 1) * nwd;
+  // this wave's texel rows lie i0 - k .. i0 - k + V - 1 rows from source row k
+  const int i0 = wave * V + R - s0;
+  const int k0 = max(0, i0 - R), k1 = min(rows, i0 + V + R);
+#pragma unroll
+  for (int w = 0; w < NRW; ++w) {
+    if (32 * w > R) break;
+    // lane k holds the radii present in source row k of the strip
+    const int rpv = (int)s_rp[w * K + (lane < rows ? lane : 0)];
+    for (int k = k0; k < k1; ++k) {
+      const int i = i0 - k;
+      const int iw = i > 0 ? i : (i + V - 1 < 0 ? i + V - 1 : 0);  // the row nearest the centre
+      const int low = (iw < 0 ? -iw : iw) - 32 * w;
+      uint32_t radii = (uint32_t)__builtin_amdgcn_readlane(rpv, k);
+      if constexpr (NRW == 1) radii &= ~0u << low;
+      else radii = low <= 0 ? radii : (low < 32 ? radii & (~0u << low) : 0u);
+      if (!radii) continue;
+      const uint32_t* const er = s_e + k * mrow;
+      const float4* const cr = src - (ptrdiff_t)(s0 + k) * W;  // bins run bottom-up
+      int r = 32 * w + __builtin_ctz(radii);
+      DEVisit<V> next = de_visit<V>(tab, r, i, iw);
+      for (;;) {
+        // the next radius' values are on their way while this one's are used
+        const DEVisit<V> v = next;
+        const uint32_t* const em = er + r * nwd;
         radii &= radii - 1u;
-        const uint2 jx = s_jx[(r << DE_JS_SHIFT) + i + R];
-        const unsigned long long e = s_e[(r << DE_ES_SHIFT) + rowi];
-        const int c0 = lx + (int)(jx.x & 0xffu);  // columns c0 .. c0 + hi - lo: j = hi .. lo
-        uint32_t m = (uint32_t)(e >> c0) & jx.y;
-        const float* w = s_wt + (jx.x >> 8);  // w[b]: j = hi - b
-        const int base = rowi * SW + c0;
-        while (m) {
-          const int b = __builtin_ctz(m);
-          m &= m - 1u;
-          const float wgt = w[b];
-          const float4 c = s_col[base + b];
-          acc.x = fmaf(c.x, wgt, acc.x);
-          acc.y = fmaf(c.y, wgt, acc.y);
-          acc.z = fmaf(c.z, wgt, acc.z);
-          acc.w = fmaf(c.w, wgt, acc.w);
+        r = radii ? 32 * w + __builtin_ctz(radii) : r;
+        next = de_visit<V>(tab, r, i, iw);
+        const int col0 = lane + R - (int)(signed char)(v.hl & 0xff);  // column of j = hi
+        de_taps<V, ALL, SHORT>(acc, v, col0, em, cr);
+        if (!radii) break;
+      }
+    }
+  }
+}
+
+// SHORT: chords of at most 31 columns (radius below 16).  NRW words of 32
+// radii each.
+template <int V, int NRW, bool SHORT>
+__global__ __launch_bounds__(64 * DR_WAVES) __attribute__((amdgpu_waves_per_eu(8))) void k_de_rows(DEArgs g, int K) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ int s_odd;  // the strip holds a source that is not finite
+  const int R = max(g.R, g.rmin);  // span
+  const int SW = DR_W + 2 * R, nwd = dr_mask_words(R);
+  const int mrow = (R + 1) * nwd;  // mask words per source row
+  uint32_t* s_e = reinterpret_cast<uint32_t*>(smem);  // [row][radius][word]
+  uint32_t* s_rp = s_e + K * mrow;                    // [word][row]
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int W = (int)g.W, H = (int)g.H;
+  const uint32_t ny = (uint32_t)(H + DR_WAVES * V - 1) / (DR_WAVES * V);
+  const uint32_t tile = blockIdx.x;  // down the columns of tiles: neighbours share source rows in L2
+  const int tx0 = (int)(tile / ny) * DR_W, ty0 = (int)(tile % ny) * (DR_WAVES * V);
+  CDETable* const tab = (CDETable*)g.tab;
+  float4 acc[V];
+#pragma unroll
+  for (int q = 0; q < V; ++q) acc[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (threadIdx.x == 0) s_odd = 0;
+  // the bin of source row 0, window column 0 (read only where a mask bit is set)
+  const float4* const src = g.hist + ((ptrdiff_t)(H - 1 - ty0 + R) * W + tx0 - R + 1);
+  // source row s of the tile is texel row ty0 - R + s of the image
+  const int s_begin = max(0, R - ty0), s_end = min(DR_WAVES * V + 2 * R, H - ty0 + R);
+  for (int s0 = s_begin; s0 < s_end; s0 += K) {  // workgroup-uniform
+    const int rows = min(K, s_end - s0);
+    __syncthreads();  // the previous strip is read
+    // radius of window column x of strip row k, DE_EMPTY outside the image
+    // (bins of column 0 have no texel)
+    auto radius_at = [&](int k, int x) -> uint32_t {
+      const int px = tx0 - R + x + 1;
+      if (k >= rows || x >= SW || px < 1 || px >= W) return DE_EMPTY;
+      return g.rad[(size_t)(H - 1 - (ty0 - R + s0 + k)) * W + px];
+    };
+    uint32_t v0 = radius_at(wave, lane), v1 = radius_at(wave, WAVE + lane);
+    for (int k = wave; k < rows; k += DR_WAVES) {
+      uint32_t* const er = s_e + k * mrow;
+      for (int q = lane; q < mrow; q += WAVE) er[q] = 0u;
+      uint32_t rp[NRW];
+#pragma unroll
+      for (int w = 0; w < NRW; ++w) rp[w] = 0u;
+      bool odd = false;
+      for (int x0 = 0; x0 < SW; x0 += WAVE) {
+        // this row's first 128 columns were loaded during the previous row
+        const uint32_t v = x0 == 0 ? v0 : (x0 == WAVE ? v1 : radius_at(k, x0 + lane));
+        if (x0 == 0) v0 = radius_at(k + DR_WAVES, lane);
+        if (x0 == WAVE) v1 = radius_at(k + DR_WAVES, WAVE + lane);
+        const int r = v == DE_EMPTY ? -1 : (int)(v & (DE_ODD - 1u));
+        odd = odd || (v != DE_EMPTY && v >= DE_ODD);
+        uint64_t left = __builtin_amdgcn_ballot_w64(r >= 0);
+        uint32_t* const ex = er + (x0 >> 5);
+        const bool put = lane < 2 && (x0 >> 5) + lane < nwd;
+        while (left) {  // one round per radius among these 64 columns
+          const int rr = __builtin_amdgcn_readlane(r, __builtin_ctzll(left));
+          const uint64_t m = __builtin_amdgcn_ballot_w64(r == rr);
+          left &= ~m;
+          if (put) ex[rr * nwd + lane] = (uint32_t)(m >> (32 * lane));
+          if constexpr (NRW == 1) {
+            rp[0] |= 1u << rr;
+          } else {
+#pragma unroll
+            for (int w = 0; w < NRW; ++w) rp[w] |= (rr >> 5) == w ? 1u << (rr & 31) : 0u;
+          }
         }
       }
+      if (odd) s_odd = 1;
+#pragma unroll
+      for (int w = 0; w < NRW; ++w)
+        if (lane == 0) s_rp[w * K + k] = rp[w];
     }
-    const size_t o = (size_t)ty * g.W + tx;
-    if (g.de_out) g.de_out[o] = acc;
-    if (g.img_out && g.do_tonemap) g.img_out[o] = tonemap_px(acc, g.gamma, g.brightness, g.vibrancy, g.k);
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(s_odd) == 0) de_strip<V, NRW, true, SHORT>(acc, tab, src, W, s_e, s_rp, R, K, s0, rows);
+    else de_strip<V, NRW, false, SHORT>(acc, tab, src, W, s_e, s_rp, R, K, s0, rows);
+  }
+  const int tx = tx0 + lane;
+#pragma unroll
+  for (int q = 0; q < V; ++q) {
+    __builtin_amdgcn_sched_barrier(0);  // one tonemap's registers at a time
+    const int ty = ty0 + wave * V + q;
+    if (tx < W && ty < H) {
+      const size_t o = (size_t)ty * W + tx;
+      if (g.de_out) g.de_out[o] = acc[q];
+      if (g.img_out && g.do_tonemap) g.img_out[o] = tonemap_px(acc[q], g.tone);
+    }
   }
   de_stamp(g);
 }
 
-template <int TH>
-size_t de_tiled_lds(int R) {
-  const size_t SW = DE_TW + 2 * R, SH = TH + 2 * R;
-  return SW * SH * sizeof(float4) + (size_t)(R + 1) * DE_ES * 8 + SH * 4 + de_weight_bytes(R) + 8 +
-         (size_t)(R + 1) * DE_JS * 8;
-}
-
-// Radii beyond the LDS tile: the same gather straight from memory.
-__global__ __launch_bounds__(256) void k_de_global(DEArgs g) {
-  const int tx = blockIdx.x * 16 + (threadIdx.x % 16);
-  const int ty = blockIdx.y * 16 + (threadIdx.x / 16);
-  if (tx < (int)g.W && ty < (int)g.H) {
-    const int R = max(g.R, g.rmin);
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int i = -R; i <= R; ++i) {
-      for (int j = -R; j <= R; ++j) {
-        float4 c; DESrc m;
-        de_source(g, tx - j, ty - i, c, m);
-        const float wgt = de_weight(m, i, j);
-        if (wgt != 0.0f) { acc.x += c.x * wgt; acc.y += c.y * wgt; acc.z += c.z * wgt; acc.w += c.w * wgt; }
-      }
+// Radius 0 everywhere: every bin is its own texel.
+__global__ __launch_bounds__(256) void k_de_copy(DEArgs g) {
+  const uint32_t tx = blockIdx.x * 64 + (threadIdx.x & 63u), ty = blockIdx.y * 4 + threadIdx.x / 64;
+  if (tx < g.W && ty < g.H) {
+    float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (tx + 1 < g.W) {
+      const float4 b = g.hist[(size_t)(g.H - 1 - ty) * g.W + tx + 1];
+      if (b.w != 0.0f) c = b;
     }
     const size_t o = (size_t)ty * g.W + tx;
-    if (g.de_out) g.de_out[o] = acc;
-    if (g.img_out && g.do_tonemap) g.img_out[o] = tonemap_px(acc, g.gamma, g.brightness, g.vibrancy, g.k);
+    if (g.de_out) g.de_out[o] = c;
+    if (g.img_out && g.do_tonemap) g.img_out[o] = tonemap_px(c, g.tone);
   }
   de_stamp(g);
 }
 
-__global__ void k_tonemap(const float4* __restrict__ in, float4* __restrict__ out, uint32_t n,
-                          float gamma, float brightness, float vib, float k) {
+__global__ void k_tonemap(const float4* __restrict__ in, float4* __restrict__ out, uint32_t n, ToneArgs t) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = tonemap_px(in[i], gamma, brightness, vib, k);
+  if (i < n) out[i] = tonemap_px(in[i], t);
 }
 
 // RGBA float -> RGBA8: clamp to [0, 1], x255, round to nearest (NaN -> 0);
@@ -387,40 +499,49 @@ hipError_t launch_animate(Block* blocks, uint32_t T, float tss_width, const floa
   return hipGetLastError();
 }
 
-hipError_t launch_de_tonemap(const DEArgs& a, hipStream_t s) {
-  if (!a.rad || !a.wt) return hipErrorInvalidValue;
-  const uint64_t n = (uint64_t)a.W * a.H;
-  // Tiles of 32 x 32 texels while they fit the 64 KiB of LDS one launch gets
-  // by default (R <= 11), 32 x 8 up to R = 14 (64-column masks need
-  // 32 + 2R <= 64 as well), the global-memory gather beyond.
-  const int span = a.R > a.rmin ? a.R : a.rmin;
-  // (chords of at most 31 columns keep the tap masks in 32 bits)
-  // span <= 15 keeps 2 span + 1 <= DE_JS and TH + 2 span <= DE_ES
-  const bool tall = de_tiled_lds<32>(span) <= 65536 && span <= 15;
-  const bool flat = de_tiled_lds<8>(span) <= 65536 && 32 + 2 * span <= 64 && span <= 15;
-  if (tall || flat) {
-    hipLaunchKernelGGL(k_de_weights, dim3(1), dim3(256), 0, s, a.wt, span);
-    if (n) hipLaunchKernelGGL(k_de_radius, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
-  }
-  if (tall) {
-    dim3 grid((a.W + DE_TW - 1) / DE_TW, (a.H + 31) / 32);
-    // eight waves per 32 x 32 tile: the LDS allows three tiles per CU, so
-    // 24 waves per CU hide the gather's LDS latency (12 with four waves)
-    hipLaunchKernelGGL((k_de_tiled<32, 512>), grid, dim3(512), de_tiled_lds<32>(span), s, a);
-  } else if (flat) {
-    dim3 grid((a.W + DE_TW - 1) / DE_TW, (a.H + 7) / 8);
-    hipLaunchKernelGGL((k_de_tiled<8, 256>), grid, dim3(256), de_tiled_lds<8>(span), s, a);
-  } else {
-    dim3 grid((a.W + 15) / 16, (a.H + 15) / 16);
-    hipLaunchKernelGGL(k_de_global, grid, dim3(256), 0, s, a);
-  }
+hipError_t launch_de_chords(DETable* tab, hipStream_t s) {
+  hipLaunchKernelGGL(k_de_chords, dim3(DE_C_ROWS), dim3(DE_CHORD_STRIDE), 0, s, tab);
   return hipGetLastError();
 }
 
-hipError_t launch_tonemap(const float4* in, float4* out, uint32_t n, float gamma, float brightness,
-                          float vibrancy, float k, hipStream_t s) {
-  hipLaunchKernelGGL(k_tonemap, dim3((n + 255) / 256), dim3(256), 0, s, in, out, n, gamma, brightness,
-                     vibrancy, k);
+template <int V>
+static void launch_de_rows(const DEArgs& a, int R, hipStream_t s) {
+  // all source rows of the tile at once while their masks fit 32 KiB (four
+  // workgroups per CU, as many as its waves allow)
+  const size_t row = dr_row_bytes(R);
+  const int K = (int)std::min<size_t>({(size_t)(DR_WAVES * V + 2 * R), (size_t)WAVE, (size_t)32768 / row});
+  const dim3 grid((unsigned)dr_tiles(a.W, a.H, V));
+  if (R < 16) hipLaunchKernelGGL((k_de_rows<V, 1, true>), grid, dim3(64 * DR_WAVES), K * row, s, a, K);
+  else if (R < 32) hipLaunchKernelGGL((k_de_rows<V, 1, false>), grid, dim3(64 * DR_WAVES), K * row, s, a, K);
+  else hipLaunchKernelGGL((k_de_rows<V, 4, false>), grid, dim3(64 * DR_WAVES), K * row, s, a, K);
+}
+
+hipError_t launch_de_tonemap(const DEArgs& a, hipStream_t s) {
+  const int R = a.R > a.rmin ? a.R : a.rmin;
+  const uint64_t n = (uint64_t)a.W * a.H;
+  if (!a.rad || !a.tab || R < 0 || R > DE_MAX_R) return hipErrorInvalidValue;
+  if (n == 0) return hipSuccess;
+  if (R == 0) {
+    hipLaunchKernelGGL(k_de_copy, dim3((a.W + 63) / 64, (a.H + 3) / 4), dim3(256), 0, s, a);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL(k_de_radius, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
+  // Texel rows per wave.  Four share the most work per source but need many
+  // tiles to fill the chip and to even out its last round; the wider the
+  // splat, the sooner that pays.  Measured (us, 4 / 2 / 1 rows; the 32 x 32
+  // tiles in LDS they replace, and the global gather beyond radius 15):
+  // 7680x4320 radius 9: 1365 / 1720 / 2760 (1780); 2048x2048 radius 9: 240 /
+  // 236 / 329 (268), radius 24: 789 / 811 / 1252 (22258); 1920x1080 radius 9:
+  // 161 / 149 / 210 (178), radius 24: 585 / 553 / 879 (13743); 512x512 radius
+  // 9: 88 / 64 / 70 (85); 320x240 radius 9: 65 / 51 / 45 (57).
+  if (dr_tiles(a.W, a.H, 4) * (uint64_t)(R + 16) >= 65536) launch_de_rows<4>(a, R, s);
+  else if (dr_tiles(a.W, a.H, 2) >= 128) launch_de_rows<2>(a, R, s);
+  else launch_de_rows<1>(a, R, s);
+  return hipGetLastError();
+}
+
+hipError_t launch_tonemap(const float4* in, float4* out, uint32_t n, const ToneArgs& t, hipStream_t s) {
+  hipLaunchKernelGGL(k_tonemap, dim3((n + 255) / 256), dim3(256), 0, s, in, out, n, t);
   return hipGetLastError();
 }
 

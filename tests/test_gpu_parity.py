@@ -354,6 +354,45 @@ def test_density_estimation_vs_oracle(rf, orc, gpu_available, R, rmin, curve):
     assert np.abs(g - ref).max() <= tol
 
 
+# Tiles of 64 x 8, 64 x 16 and 64 x 32 texels (by image size and radius), one
+# to four words of radii, chords beyond 32 columns, ragged edges, an image
+# smaller than one tile and smaller than the splat.
+@pytest.mark.parametrize("W,H,R,rmin,curve,density", [
+    (1, 1, 9, 0, 0.4, 1.0), (5, 3, 40, 0, 0.4, 1.0), (65, 9, 15, 0, 0.45, 0.5), (63, 70, 16, 1, 0.5, 0.3),
+    (130, 41, 31, 0, 0.3, 0.2), (129, 33, 32, 0, 0.3, 0.2), (200, 150, 100, 2, 0.25, 0.05), (90, 61, 5, 70, 0.4, 0.02),
+    (1030, 129, 9, 0, 0.4, 0.3), (1025, 130, 33, 0, 0.35, 0.05), (2501, 2150, 9, 0, 0.4, 0.05),
+    (1537, 769, 100, 0, 0.3, 0.002)])
+def test_density_estimation_tiles_vs_oracle(rf, orc, gpu_available, W, H, R, rmin, curve, density):
+    import torch
+    h = _sparse_hist(np.random.default_rng(1000 * R + W), W, H, density)
+    ctx = _ctx(rf, 1 << 10, 1, rf.RF_ENGINE_FAST)
+    hist = ctx.histogram(W, H)
+    hist.upload(h)
+    out = torch.zeros((H, W, 4), dtype=torch.float32, device="cuda")
+    ctx.density_estimate(hist, rf.DEParams(R, rmin, curve), out.data_ptr())
+    ref = orc.density(h, R, rmin, curve, fp32=True)
+    assert np.abs(out.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("W,H,R", [(97, 75, 9), (1030, 129, 20)])
+def test_density_estimation_keeps_an_infinity_in_its_splat(rf, orc, gpu_available, W, H, R):
+    """A bin with an infinite colour reaches the texels of its own splat only."""
+    import torch
+    h = _sparse_hist(np.random.default_rng(R), W, H)
+    h[H // 2, W // 2] = [np.inf, 0.5, 0.5, 1.0]
+    ctx = _ctx(rf, 1 << 10, 1, rf.RF_ENGINE_FAST)
+    hist = ctx.histogram(W, H)
+    hist.upload(h)
+    out = torch.zeros((H, W, 4), dtype=torch.float32, device="cuda")
+    ctx.density_estimate(hist, rf.DEParams(R, 0, 0.4), out.data_ptr())
+    g = out.cpu().numpy()
+    ref = orc.density(h, R, 0, 0.4, fp32=True)
+    fin = np.isfinite(ref)
+    assert (~fin).sum() > R * R and not np.isnan(ref).any()
+    assert np.array_equal(np.isfinite(g), fin)
+    assert np.abs(g[fin] - ref[fin]).max() <= 2e-5 * np.abs(ref[fin]).max()
+
+
 def test_density_identity_layout(rf, orc, gpu_available):
     """R = 0: each bin lands on texel (px - 1, H - 1 - py); column 0 is clipped."""
     import torch
