@@ -90,13 +90,19 @@ inline const float* bias_of(rf_denoiser* d, int l) { return (const float*)d->p.p
 inline const bf16* w_of(rf_denoiser* d, int l) { return (const bf16*)d->pb.p + d->L[l].w_off; }
 inline const bf16* wt_of(rf_denoiser* d, int l) { return (const bf16*)d->wt.p + d->wt_off[l]; }
 
+int flip_all(rf_denoiser* d) {
+  rfn::FlipLayers f{};
+  for (int l = 0; l < kLayers; ++l)
+    f.layer[l] = {d->L[l].cin, d->L[l].cout, (int)d->L[l].w_off, (int)d->wt_off[l]};
+  HIPCHK(d->ctx, rfn::flip_weights_all(f, kLayers, (const bf16*)d->pb.p, (bf16*)d->wt.p, d->ctx->stream));
+  return RF_OK;
+}
+
 int refresh_weights(rf_denoiser* d) {
   rf_ctx* ctx = d->ctx;
   hipStream_t s = ctx->stream;
   HIPCHK(ctx, rfn::to_bf16((const float*)d->p.p, (bf16*)d->pb.p, (int)d->n_params, s));
-  for (int l = 0; l < kLayers; ++l)
-    HIPCHK(ctx, rfn::flip_weights(w_of(d, l), (bf16*)wt_of(d, l), d->L[l].cin, d->L[l].cout, s));
-  return RF_OK;
+  return flip_all(d);
 }
 
 int check_shape(rf_denoiser* d, int N, int H, int W) {
@@ -176,63 +182,54 @@ int backward(rf_denoiser* d, const bf16* x, int N, int H, int W) {
   rf_ctx* ctx = d->ctx;
   hipStream_t s = ctx->stream;
   const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4, H3 = H / 8, W3 = W / 8;
-  const size_t P0 = (size_t)N * H * W, P1 = P0 / 4, P2 = P0 / 16, P3 = P0 / 64;
   float* g = (float*)d->g.p;
   HIPCHK(ctx, rfn::zero_f32(g, d->n_params, s));
   auto wgrad = [&](int l, View xin, View dy, int h, int w) {
     return rfn::conv3x3_wgrad(xin, dy, g + d->L[l].w_off, g + d->L[l].b_off, N, h, w, d->L[l].cin, d->L[l].cout,
                               (float*)d->wg_work.p, d->wg_work.bytes / sizeof(float), s);
   };
-  auto dgrad = [&](int l, View dy, View dx, int h, int w) {
-    return rfn::conv3x3(dy, wt_of(d, l), nullptr, dx, N, h, w, d->L[l].cout, d->L[l].cin, 0, s);
+  // with y, the gradient of the layer's input y is masked by y > 0
+  auto dgrad = [&](int l, View dy, View dx, int h, int w, View y = View{nullptr, 0, 0}) {
+    rfn::ConvFuse f;
+    f.mask = y;
+    return rfn::conv3x3(dy, wt_of(d, l), nullptr, dx, N, h, w, d->L[l].cout, d->L[l].cin, 0, s, f);
   };
   const View vx{(bf16*)x, 16, 0};
   // out and dec0
   HIPCHK(ctx, wgrad(11, V(d->d0b, 32), V(d->g_o, 16), H, W));
-  HIPCHK(ctx, dgrad(11, V(d->g_o, 16), V(d->g_d0b, 32), H, W));
-  HIPCHK(ctx, rfn::relu_mask(V(d->g_d0b, 32), V(d->d0b, 32), (int)P0, 32, s));
+  HIPCHK(ctx, dgrad(11, V(d->g_o, 16), V(d->g_d0b, 32), H, W, V(d->d0b, 32)));
   HIPCHK(ctx, wgrad(10, V(d->d0a, 32), V(d->g_d0b, 32), H, W));
-  HIPCHK(ctx, dgrad(10, V(d->g_d0b, 32), V(d->g_d0a, 32), H, W));
-  HIPCHK(ctx, rfn::relu_mask(V(d->g_d0a, 32), V(d->d0a, 32), (int)P0, 32, s));
+  HIPCHK(ctx, dgrad(10, V(d->g_d0b, 32), V(d->g_d0a, 32), H, W, V(d->d0a, 32)));
   HIPCHK(ctx, wgrad(9, V(d->cat0, 96), V(d->g_d0a, 32), H, W));
   HIPCHK(ctx, dgrad(9, V(d->g_d0a, 32), V(d->g_cat0, 96), H, W));
   // dec1
-  HIPCHK(ctx, rfn::upsample2_bwd(V(d->g_cat0, 96, 0), V(d->g_d1, 64), N, H1, W1, 64, s));
-  HIPCHK(ctx, rfn::relu_mask(V(d->g_d1, 64), V(d->d1, 64), (int)P1, 64, s));
+  HIPCHK(ctx, rfn::upsample2_bwd(V(d->g_cat0, 96, 0), V(d->g_d1, 64), V(d->d1, 64), N, H1, W1, 64, s));
   HIPCHK(ctx, wgrad(8, V(d->cat1, 192), V(d->g_d1, 64), H1, W1));
   HIPCHK(ctx, dgrad(8, V(d->g_d1, 64), V(d->g_cat1, 192), H1, W1));
   // dec2
-  HIPCHK(ctx, rfn::upsample2_bwd(V(d->g_cat1, 192, 0), V(d->g_d2, 128), N, H2, W2, 128, s));
-  HIPCHK(ctx, rfn::relu_mask(V(d->g_d2, 128), V(d->d2, 128), (int)P2, 128, s));
+  HIPCHK(ctx, rfn::upsample2_bwd(V(d->g_cat1, 192, 0), V(d->g_d2, 128), V(d->d2, 128), N, H2, W2, 128, s));
   HIPCHK(ctx, wgrad(7, V(d->cat2, 384), V(d->g_d2, 128), H2, W2));
   HIPCHK(ctx, dgrad(7, V(d->g_d2, 128), V(d->g_cat2, 384), H2, W2));
   // bottleneck
-  HIPCHK(ctx, rfn::upsample2_bwd(V(d->g_cat2, 384, 0), V(d->g_b, 256), N, H3, W3, 256, s));
-  HIPCHK(ctx, rfn::relu_mask(V(d->g_b, 256), V(d->b, 256), (int)P3, 256, s));
+  HIPCHK(ctx, rfn::upsample2_bwd(V(d->g_cat2, 384, 0), V(d->g_b, 256), V(d->b, 256), N, H3, W3, 256, s));
   HIPCHK(ctx, wgrad(6, V(d->p2, 128), V(d->g_b, 256), H3, W3));
   HIPCHK(ctx, dgrad(6, V(d->g_b, 256), V(d->g_p2, 128), H3, W3));
   // enc2: skip2 gradient = concat part + pooled path
-  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p2, 128), V(d->g_cat2, 384, 256), N, H2, W2, 128, 1, s));
-  HIPCHK(ctx, rfn::relu_mask(V(d->g_cat2, 384, 256), V(d->cat2, 384, 256), (int)P2, 128, s));
+  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p2, 128), V(d->g_cat2, 384, 256), V(d->cat2, 384, 256), N, H2, W2, 128, s));
   HIPCHK(ctx, wgrad(5, V(d->e2a, 128), V(d->g_cat2, 384, 256), H2, W2));
-  HIPCHK(ctx, dgrad(5, V(d->g_cat2, 384, 256), V(d->g_e2a, 128), H2, W2));
-  HIPCHK(ctx, rfn::relu_mask(V(d->g_e2a, 128), V(d->e2a, 128), (int)P2, 128, s));
+  HIPCHK(ctx, dgrad(5, V(d->g_cat2, 384, 256), V(d->g_e2a, 128), H2, W2, V(d->e2a, 128)));
   HIPCHK(ctx, wgrad(4, V(d->p1, 64), V(d->g_e2a, 128), H2, W2));
   HIPCHK(ctx, dgrad(4, V(d->g_e2a, 128), V(d->g_p1, 64), H2, W2));
   // enc1
-  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p1, 64), V(d->g_cat1, 192, 128), N, H1, W1, 64, 1, s));
-  HIPCHK(ctx, rfn::relu_mask(V(d->g_cat1, 192, 128), V(d->cat1, 192, 128), (int)P1, 64, s));
+  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p1, 64), V(d->g_cat1, 192, 128), V(d->cat1, 192, 128), N, H1, W1, 64, s));
   HIPCHK(ctx, wgrad(3, V(d->e1a, 64), V(d->g_cat1, 192, 128), H1, W1));
-  HIPCHK(ctx, dgrad(3, V(d->g_cat1, 192, 128), V(d->g_e1a, 64), H1, W1));
-  HIPCHK(ctx, rfn::relu_mask(V(d->g_e1a, 64), V(d->e1a, 64), (int)P1, 64, s));
+  HIPCHK(ctx, dgrad(3, V(d->g_cat1, 192, 128), V(d->g_e1a, 64), H1, W1, V(d->e1a, 64)));
   HIPCHK(ctx, wgrad(2, V(d->p0, 32), V(d->g_e1a, 64), H1, W1));
   HIPCHK(ctx, dgrad(2, V(d->g_e1a, 64), V(d->g_p0, 32), H1, W1));
   // enc0
-  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p0, 32), V(d->g_cat0, 96, 64), N, H, W, 32, 1, s));
-  HIPCHK(ctx, rfn::relu_mask(V(d->g_cat0, 96, 64), V(d->cat0, 96, 64), (int)P0, 32, s));
+  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p0, 32), V(d->g_cat0, 96, 64), V(d->cat0, 96, 64), N, H, W, 32, s));
   HIPCHK(ctx, wgrad(1, V(d->e0a, 32), V(d->g_cat0, 96, 64), H, W));
-  HIPCHK(ctx, dgrad(1, V(d->g_cat0, 96, 64), V(d->g_e0a, 32), H, W));
-  HIPCHK(ctx, rfn::relu_mask(V(d->g_e0a, 32), V(d->e0a, 32), (int)P0, 32, s));
+  HIPCHK(ctx, dgrad(1, V(d->g_cat0, 96, 64), V(d->g_e0a, 32), H, W, V(d->e0a, 32)));
   HIPCHK(ctx, wgrad(0, vx, V(d->g_e0a, 32), H, W));
   return RF_OK;
 }
@@ -328,8 +325,7 @@ int rf_denoiser_train_step(rf_denoiser* d, const void* x, const void* target, in
   const float c1 = 1.0f - std::pow(b1, (float)d->step), c2 = 1.0f - std::pow(b2, (float)d->step);
   HIPCHK(ctx, rfn::adam((float*)d->p.p, (const float*)d->g.p, (float*)d->m.p, (float*)d->v.p, (bf16*)d->pb.p,
                         (int)d->n_params, lr, b1, b2, 1e-8f, c1, c2, s));
-  for (int l = 0; l < kLayers; ++l)
-    HIPCHK(ctx, rfn::flip_weights(w_of(d, l), (bf16*)wt_of(d, l), d->L[l].cin, d->L[l].cout, s));
+  if ((rc = flip_all(d))) return rc;
   if (loss_out) {
     float ls = 0.0f;
     HIPCHK(ctx, hipMemcpyAsync(&ls, d->loss.p, 4, hipMemcpyDeviceToHost, s));

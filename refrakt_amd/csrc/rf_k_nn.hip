@@ -174,6 +174,16 @@ struct ConvFrag<32> {
   }
 };
 
+// Two bf16 values, each kept where the other word's value in its place is
+// positive (ReLU's backward).
+__device__ __forceinline__ uint32_t relu_keep(uint32_t v, uint32_t y) {
+  const uint32_t lo = bf_lo(y) > 0.0f ? 0xffffu : 0u, hi = bf_hi(y) > 0.0f ? 0xffff0000u : 0u;
+  return v & (lo | hi);
+}
+__device__ __forceinline__ uint4 relu_keep(const uint4& v, const uint4& y) {
+  return make_uint4(relu_keep(v.x, y.x), relu_keep(v.y, y.y), relu_keep(v.z, y.z), relu_keep(v.w, y.w));
+}
+
 // Output of one tile: bias, ReLU and bf16 in LDS (tile row RW * wave + rr is
 // image row y0 + RW * wave + rr), then 16-byte stores per pixel, the fused
 // 2x2 averages or the fused fp32 residual.  The output tile reuses the
@@ -227,9 +237,13 @@ __device__ __forceinline__ void conv_store_lds(const float4_t (&acc)[RW][4][NT],
 #pragma unroll
         for (int q = lane; q < CT_W * PQ; q += 64) {
           const int px = q / PQ, piece = q % PQ;
-          if (x0 + px < W)
-            *reinterpret_cast<uint4*>(out.p + ((size_t)(n * H + y) * W + x0 + px) * out.cs + out.co + co0 +
-                                      8 * piece) = *reinterpret_cast<const uint4*>(s_o + px * OS + 8 * piece);
+          if (x0 + px < W) {
+            const size_t p = (size_t)(n * H + y) * W + x0 + px;
+            uint4 v = *reinterpret_cast<const uint4*>(s_o + px * OS + 8 * piece);
+            if (fz.mask.p)  // workgroup-uniform
+              v = relu_keep(v, *reinterpret_cast<const uint4*>(fz.mask.p + p * fz.mask.cs + fz.mask.co + co0 + 8 * piece));
+            *reinterpret_cast<uint4*>(out.p + p * out.cs + out.co + co0 + 8 * piece) = v;
+          }
         }
       }
     }
@@ -663,22 +677,24 @@ __global__ __launch_bounds__(1024) void k_wgrad_reduce(const float* __restrict__
   }
 }
 
-__global__ void k_flip(const bf16* __restrict__ w, bf16* __restrict__ wt, int Cin, int Cout) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int n = 9 * Cin * Cout;
-  if (i >= n) return;
-  // wt index: [r][s][c][k] with k fastest
+__device__ __forceinline__ bf16 flipped(const bf16* __restrict__ w, int i, int Cin, int Cout) {
+  // index i: [r][s][c][k] with k fastest
   const int k = i % Cout, c = (i / Cout) % Cin, rs = i / (Cout * Cin);
-  const int r = rs / 3, s = rs % 3;
-  wt[i] = w[((size_t)((2 - r) * 3 + (2 - s)) * Cout + k) * Cin + c];
+  return w[((size_t)(8 - rs) * Cout + k) * Cin + c];
 }
 
-__global__ void k_relu_mask(View dy, View y, int npix, int C) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)npix * C) return;
-  const size_t p = i / C, c = i % C;
-  bf16* d = dy.p + p * dy.cs + dy.co + c;
-  if (!(bf2f(y.p[p * y.cs + y.co + c]) > 0.0f)) *d = 0;
+__global__ void k_flip(const bf16* __restrict__ w, bf16* __restrict__ wt, int Cin, int Cout) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < 9 * Cin * Cout) wt[i] = flipped(w, i, Cin, Cout);
+}
+
+// Every layer's weights in one launch (one launch per layer took 58 us of
+// the 2.17 ms of an 8 x 256^2 training step): blockIdx.y is the layer.
+__global__ void k_flip_all(FlipLayers L, const bf16* __restrict__ w, bf16* __restrict__ wt) {
+  const FlipLayers::Layer y = L.layer[blockIdx.y];
+  const int n = 9 * y.cin * y.cout;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    wt[y.wt_off + i] = flipped(w + y.w_off, i, y.cin, y.cout);
 }
 
 __global__ void k_avgpool2(View in, View out, int N, int H, int W, int C) {
@@ -694,17 +710,6 @@ __global__ void k_avgpool2(View in, View out, int N, int H, int W, int C) {
 #pragma unroll
     for (int b = 0; b < 2; ++b) s += bf2f(in.p[((size_t)(n * H + 2 * yo + a) * W + 2 * xo + b) * in.cs + in.co + c]);
   out.p[po * out.cs + out.co + c] = f2bf(0.25f * s);
-}
-
-__global__ void k_avgpool2_bwd(View dout, View din, int N, int H, int W, int C, int acc) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)N * H * W * C) return;
-  const int c = (int)(i % C);
-  const size_t p = i / C;
-  const int x = (int)(p % W), y = (int)((p / W) % H), n = (int)(p / ((size_t)W * H));
-  const float g = 0.25f * bf2f(dout.p[((size_t)(n * (H / 2) + y / 2) * (W / 2) + x / 2) * dout.cs + dout.co + c]);
-  bf16* d = din.p + p * din.cs + din.co + c;
-  *d = f2bf(acc ? bf2f(*d) + g : g);
 }
 
 __global__ void k_upsample2(View in, View out, int N, int H, int W, int C) {
@@ -756,50 +761,114 @@ __global__ void k_upsample2_v8(View in, View out, int N, int H, int W, int C) {
       *reinterpret_cast<const uint4*>(in.p + ((size_t)(n * H + yo / 2) * W + xo / 2) * in.cs + in.co + 8 * g);
 }
 
+// Gradient of the 2x2 average added to din (8 channels per thread), then
+// ReLU's mask of y.
+__global__ void k_avgpool2_bwd_v8(View dout, View din, View y, int N, int H, int W, int C) {
+  const int G = C / 8;
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (size_t)N * H * W * G) return;
+  const int g = (int)(i % G);
+  const size_t p = i / G;
+  const int x = (int)(p % W), yy = (int)((p / W) % H), n = (int)(p / ((size_t)W * H));
+  const uint4 v = *reinterpret_cast<const uint4*>(
+      dout.p + ((size_t)(n * (H / 2) + yy / 2) * (W / 2) + x / 2) * dout.cs + dout.co + 8 * g);
+  uint4* const d = reinterpret_cast<uint4*>(din.p + p * din.cs + din.co + 8 * g);
+  const uint4 o = *d;
+  const uint32_t q[4] = {v.x, v.y, v.z, v.w}, a[4] = {o.x, o.y, o.z, o.w};
+  uint32_t r[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    r[k] = (uint32_t)f2bf(bf_lo(a[k]) + 0.25f * bf_lo(q[k])) |
+           ((uint32_t)f2bf(bf_hi(a[k]) + 0.25f * bf_hi(q[k])) << 16);
+  *d = relu_keep(make_uint4(r[0], r[1], r[2], r[3]), *reinterpret_cast<const uint4*>(y.p + p * y.cs + y.co + 8 * g));
+}
+
+// Gradient of the 2x upsampling (8 channels per thread), then ReLU's mask of y.
+__global__ void k_upsample2_bwd_v8(View dout, View din, View y, int N, int H, int W, int C) {
+  const int G = C / 8;
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (size_t)N * H * W * G) return;
+  const int g = (int)(i % G);
+  const size_t p = i / G;
+  const int x = (int)(p % W), yy = (int)((p / W) % H), n = (int)(p / ((size_t)W * H));
+  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const uint4 v = *reinterpret_cast<const uint4*>(
+          dout.p + ((size_t)(n * 2 * H + 2 * yy + a) * (2 * W) + 2 * x + b) * dout.cs + dout.co + 8 * g);
+      const uint32_t q[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) { s[2 * k] += bf_lo(q[k]); s[2 * k + 1] += bf_hi(q[k]); }
+    }
+  uint32_t r[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) r[k] = (uint32_t)f2bf(s[2 * k]) | ((uint32_t)f2bf(s[2 * k + 1]) << 16);
+  *reinterpret_cast<uint4*>(din.p + p * din.cs + din.co + 8 * g) =
+      relu_keep(make_uint4(r[0], r[1], r[2], r[3]), *reinterpret_cast<const uint4*>(y.p + p * y.cs + y.co + 8 * g));
+}
+
 inline bool v8_ok(const View& a, const View& b, int C) {
   return C % 8 == 0 && a.cs % 8 == 0 && a.co % 8 == 0 && b.cs % 8 == 0 && b.co % 8 == 0 &&
          ((uintptr_t)a.p & 15u) == 0 && ((uintptr_t)b.p & 15u) == 0;
 }
 
-__global__ void k_upsample2_bwd(View dout, View din, int N, int H, int W, int C) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)N * H * W * C) return;
-  const int c = (int)(i % C);
-  const size_t p = i / C;
-  const int x = (int)(p % W), y = (int)((p / W) % H), n = (int)(p / ((size_t)W * H));
-  float s = 0.0f;
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-      s += bf2f(dout.p[((size_t)(n * 2 * H + 2 * y + a) * (2 * W) + 2 * x + b) * dout.cs + dout.co + c]);
-  din.p[p * din.cs + din.co + c] = f2bf(s);
-}
+// One pixel per thread and round.  The loss goes out as one atomic per
+// workgroup: one per wave (8192 to one address at 8 x 256^2) held the kernel
+// for 125 us.  VEC: 16-byte aligned buffers, 8- and 16-byte accesses.
+constexpr int RES_GRID = 1024;
 
-__global__ void k_residual_loss(View x, View o, const bf16* __restrict__ t, float* __restrict__ y_out,
-                                float* __restrict__ loss_sum, bf16* __restrict__ dO, int npix, float inv_count) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+template <bool VEC>
+__global__ __launch_bounds__(256) void k_residual_loss(View x, View o, const bf16* __restrict__ t,
+                                                       float* __restrict__ y_out, float* __restrict__ loss_sum,
+                                                       bf16* __restrict__ dO, int npix, float inv_count) {
+  __shared__ float s_l[4];
+  auto load4 = [](const bf16* p, float (&v)[4]) {
+    if constexpr (VEC) {
+      const uint2 q = *reinterpret_cast<const uint2*>(p);
+      v[0] = bf_lo(q.x); v[1] = bf_hi(q.x); v[2] = bf_lo(q.y); v[3] = bf_hi(q.y);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[c] = bf2f(p[c]);
+    }
+  };
   float l = 0.0f;
-  if (p < npix) {
+  for (int p = blockIdx.x * 256 + threadIdx.x; p < npix; p += gridDim.x * 256) {
+    float y[4], ov[4];
+    load4(x.p + (size_t)p * x.cs + x.co, y);
+    load4(o.p + (size_t)p * o.cs + o.co, ov);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      const float y = bf2f(x.p[(size_t)p * x.cs + x.co + c]) + bf2f(o.p[(size_t)p * o.cs + o.co + c]);
-      if (y_out) y_out[(size_t)p * 4 + c] = y;
-      if (t) {
-        const float d = y - bf2f(t[(size_t)p * 16 + c]);
-        l += d * d;
-        dO[(size_t)p * 16 + c] = f2bf(2.0f * d * inv_count);
-      }
+      y[c] = y[c] + ov[c];
+      if (y_out) y_out[(size_t)p * 4 + c] = y[c];
     }
     if (t) {
+      float tv[4];
+      bf16 g[4];
+      load4(t + (size_t)p * 16, tv);
 #pragma unroll
-      for (int c = 4; c < 16; ++c) dO[(size_t)p * 16 + c] = 0;
+      for (int c = 0; c < 4; ++c) {
+        const float d = y[c] - tv[c];
+        l += d * d;
+        g[c] = f2bf(2.0f * d * inv_count);
+      }
+      if constexpr (VEC) {
+        uint4* q = reinterpret_cast<uint4*>(dO + (size_t)p * 16);
+        q[0] = make_uint4((uint32_t)g[0] | ((uint32_t)g[1] << 16), (uint32_t)g[2] | ((uint32_t)g[3] << 16), 0u, 0u);
+        q[1] = make_uint4(0u, 0u, 0u, 0u);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) dO[(size_t)p * 16 + c] = c < 4 ? g[c] : (bf16)0;
+      }
     }
   }
   if (t) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) l += __shfl_xor(l, off);
-    if ((threadIdx.x & 63) == 0) atomicAdd(loss_sum, l);
+    if ((threadIdx.x & 63) == 0) s_l[threadIdx.x >> 6] = l;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(loss_sum, (s_l[0] + s_l[1]) + (s_l[2] + s_l[3]));
   }
 }
 
@@ -904,6 +973,10 @@ hipError_t conv3x3(View in, const bf16* w, const float* bias, View out, int N, i
     // otherwise the output is written and the residual computed afterwards
     const bool fuse_res = fuse.y && vec_out && Cout == 16 && fuse.res.cs % 4 == 0 && fuse.res.co % 4 == 0 &&
                           ((uintptr_t)fuse.res.p & 7u) == 0 && ((uintptr_t)fuse.y & 15u) == 0 && !pool.p;
+    // so does the mask of a gradient
+    if (fuse.mask.p && (!vec_out || fuse.y || fuse.mask.cs % 8 || fuse.mask.co % 8 ||
+                        ((uintptr_t)fuse.mask.p & 15u) != 0))
+      return hipErrorInvalidValue;
     ConvFuse fz = fuse;
     if (!fuse_pool) fz.pool = View{nullptr, 0, 0};
     if (!fuse_res) { fz.res = View{nullptr, 0, 0}; fz.y = nullptr; }
@@ -930,6 +1003,7 @@ hipError_t conv3x3(View in, const bf16* w, const float* bias, View out, int N, i
       e = residual_loss(fuse.res, out, nullptr, fuse.y, nullptr, nullptr, N * H * W, 0.0f, s);
     return e;
   }
+  if (fuse.mask.p) return hipErrorInvalidValue;
   const dim3 grid((W + 63) / 64, N * H, Cout / (16 * nt));
   switch (nt) {
     case 4: hipLaunchKernelGGL(k_conv3x3<4>, grid, dim3(256), 0, s, in, w, bias, out, H, W, Cin, Cout, relu); break;
@@ -1000,8 +1074,9 @@ hipError_t flip_weights(const bf16* w, bf16* wt, int Cin, int Cout, hipStream_t 
   return hipGetLastError();
 }
 
-hipError_t relu_mask(View dy, View y, int npix, int C, hipStream_t s) {
-  hipLaunchKernelGGL(k_relu_mask, grid1((size_t)npix * C), dim3(256), 0, s, dy, y, npix, C);
+hipError_t flip_weights_all(const FlipLayers& L, int n_layers, const bf16* w, bf16* wt, hipStream_t s) {
+  if (n_layers < 1 || n_layers > FlipLayers::kMax) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_flip_all, dim3(128, (unsigned)n_layers), dim3(256), 0, s, L, w, wt);
   return hipGetLastError();
 }
 
@@ -1014,8 +1089,9 @@ hipError_t avgpool2(View in, View out, int N, int H, int W, int C, hipStream_t s
   return hipGetLastError();
 }
 
-hipError_t avgpool2_bwd(View dout, View din, int N, int H, int W, int C, int acc, hipStream_t s) {
-  hipLaunchKernelGGL(k_avgpool2_bwd, grid1((size_t)N * H * W * C), dim3(256), 0, s, dout, din, N, H, W, C, acc);
+hipError_t avgpool2_bwd(View dout, View din, View y, int N, int H, int W, int C, hipStream_t s) {
+  if (!v8_ok(dout, din, C) || !v8_ok(y, y, C)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_avgpool2_bwd_v8, grid1((size_t)N * H * W * (C / 8)), dim3(256), 0, s, dout, din, y, N, H, W, C);
   return hipGetLastError();
 }
 
@@ -1027,15 +1103,21 @@ hipError_t upsample2(View in, View out, int N, int H, int W, int C, hipStream_t 
   return hipGetLastError();
 }
 
-hipError_t upsample2_bwd(View dout, View din, int N, int H, int W, int C, hipStream_t s) {
-  hipLaunchKernelGGL(k_upsample2_bwd, grid1((size_t)N * H * W * C), dim3(256), 0, s, dout, din, N, H, W, C);
+hipError_t upsample2_bwd(View dout, View din, View y, int N, int H, int W, int C, hipStream_t s) {
+  if (!v8_ok(dout, din, C) || !v8_ok(y, y, C)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_upsample2_bwd_v8, grid1((size_t)N * H * W * (C / 8)), dim3(256), 0, s, dout, din, y, N, H, W, C);
   return hipGetLastError();
 }
 
 hipError_t residual_loss(View x, View o, const bf16* t, float* y_out, float* loss_sum, bf16* dO, int npix,
                          float inv_count, hipStream_t s) {
-  hipLaunchKernelGGL(k_residual_loss, grid1((size_t)npix), dim3(256), 0, s, x, o, t, y_out, loss_sum, dO, npix,
-                     inv_count);
+  const dim3 grid((unsigned)std::min((npix + 255) / 256, RES_GRID));
+  const bool vec = (((uintptr_t)x.p | (uintptr_t)o.p | (uintptr_t)t | (uintptr_t)dO) & 15u) == 0 && x.cs % 4 == 0 &&
+                   x.co % 4 == 0 && o.cs % 4 == 0 && o.co % 4 == 0;
+  if (vec)
+    hipLaunchKernelGGL(k_residual_loss<true>, grid, dim3(256), 0, s, x, o, t, y_out, loss_sum, dO, npix, inv_count);
+  else
+    hipLaunchKernelGGL(k_residual_loss<false>, grid, dim3(256), 0, s, x, o, t, y_out, loss_sum, dO, npix, inv_count);
   return hipGetLastError();
 }
 

@@ -37,6 +37,10 @@ struct ConvFuse {
   // residual_loss computes it).
   View res{nullptr, 0, 0};
   float* y = nullptr;
+  // mask.p set: the output is kept where mask > 0 and 0 elsewhere (ReLU's
+  // backward; mask has the output's Cout channels, 16-byte aligned runs as
+  // in the input and the output).
+  View mask{nullptr, 0, 0};
 };
 hipError_t conv3x3(View in, const bf16* w, const float* bias, View out, int N, int H, int W, int Cin, int Cout,
                    int relu, hipStream_t s, const ConvFuse& fuse = ConvFuse{});
@@ -51,14 +55,22 @@ hipError_t conv3x3_wgrad(View x, View dy, float* dw, float* db, int N, int H, in
 // w_t[r][s][c][k] = w[2-r][2-s][k][c]: the weights of the input-gradient
 // convolution (dx = conv3x3(dy, w_t) with Cin' = Cout, Cout' = Cin).
 hipError_t flip_weights(const bf16* w, bf16* wt, int Cin, int Cout, hipStream_t s);
-// dy *= (y > 0) on a C-channel view pair.
-hipError_t relu_mask(View dy, View y, int npix, int C, hipStream_t s);
-// 2x2 average pooling and its gradient (accumulated into dx when acc).
+// The same for several layers in one launch; the offsets are into w and wt.
+struct FlipLayers {
+  static constexpr int kMax = 16;
+  struct Layer {
+    int cin, cout, w_off, wt_off;
+  } layer[kMax];
+};
+hipError_t flip_weights_all(const FlipLayers& L, int n_layers, const bf16* w, bf16* wt, hipStream_t s);
+// 2x2 average pooling; its gradient is added to din, and din is kept where
+// y > 0 (channel runs 16-byte aligned, C a multiple of 8).
 hipError_t avgpool2(View in, View out, int N, int H, int W, int C, hipStream_t s);
-hipError_t avgpool2_bwd(View dout, View din, int N, int H, int W, int C, int acc, hipStream_t s);
-// Nearest 2x upsampling (H, W are the input size) and its gradient.
+hipError_t avgpool2_bwd(View dout, View din, View y, int N, int H, int W, int C, hipStream_t s);
+// Nearest 2x upsampling (H, W are the input size) and its gradient, kept
+// where y > 0 (channel runs 16-byte aligned, C a multiple of 8).
 hipError_t upsample2(View in, View out, int N, int H, int W, int C, hipStream_t s);
-hipError_t upsample2_bwd(View dout, View din, int N, int H, int W, int C, hipStream_t s);
+hipError_t upsample2_bwd(View dout, View din, View y, int N, int H, int W, int C, hipStream_t s);
 // y = x[:, :4] + o[:, :4] (fp32, 4 channels, when y_out != null); when t != null: loss_sum += sum (y - t)^2 and
 // do = 2 (y - t) / count in channels 0..3, 0 in the rest (16-channel do).
 hipError_t residual_loss(View x, View o, const bf16* t, float* y_out, float* loss_sum, bf16* dO, int npix,

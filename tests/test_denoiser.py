@@ -238,6 +238,34 @@ def test_unet_gradients_match_torch(rf, gpu_available):
         assert cos > 0.99 and rel < 0.1, (i, cos, rel)
 
 
+# The smallest image (a bottleneck of one pixel), ragged tiles and strips, a
+# batch: pooling, upsampling and ReLU backward run fused in 16-byte pieces.
+@pytest.mark.parametrize("N,H,W", [(1, 8, 8), (3, 24, 72), (2, 8, 136)])
+def test_unet_gradients_at_tile_edges(rf, gpu_available, N, H, W):
+    import torch
+    ctx = rf.Context(1 << 12, 1, 16)
+    dn = ctx.denoiser(seed=4)
+    p = dn.params()
+    p[-(9 * 32 * 16 + 16):] *= 10.0
+    dn.set_params(p)
+    x, t = _inputs(N + W, N, H, W)
+    xd = x.permute(0, 2, 3, 1).contiguous().cuda()
+    td = t.permute(0, 2, 3, 1).contiguous().cuda()
+    g, loss = dn.grads(xd.data_ptr(), td.data_ptr(), N, H, W)
+    pt = torch.from_numpy(p.copy()).requires_grad_(True)
+    ref_loss = ((_unet_ref_autograd(pt, x.float()) - t.float()[:, :4]) ** 2).mean()
+    ref_loss.backward()
+    assert abs(loss - float(ref_loss)) <= 0.02 * float(ref_loss)
+    gr, off = pt.grad.numpy(), 0
+    for i, (cin, cout, _) in enumerate(SPEC):
+        n = 9 * cin * cout + cout
+        a, b = g[off:off + n], gr[off:off + n]
+        off += n
+        cos = float(np.dot(a, b) / (np.linalg.norm(a) * np.linalg.norm(b) + 1e-30))
+        rel = float(np.linalg.norm(a - b) / (np.linalg.norm(b) + 1e-30))
+        assert cos > 0.99 and rel < 0.1, (i, cos, rel)
+
+
 def _unet_ref_autograd(pt, x):
     import torch
     import torch.nn.functional as F
