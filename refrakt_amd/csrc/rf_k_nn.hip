@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "rf_nn.hpp"
 
@@ -413,128 +414,62 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RW == 2 ? (
 //   dw[r][s][k][c] = sum_p dy[p][k] x[p + (r - 1, s - 1)][c].
 // A workgroup owns a TCO x TCI channel tile, all nine taps, and a run of
 // "units" (one 64-pixel strip of one dy row; units are strip-major, so a
-// run walks down the rows of a strip).  The three input rows around the
-// current dy row live in a ring of LDS slots (image row yy in slot yy % 3):
-// moving one row down loads one new input row, a new image or strip two.
-// Staging is transposed to channel-major ([channel][pixel]) so a lane's eight
-// consecutive pixels are one 16-byte fragment read, and each input row is
-// stored at the three column shifts s = 0, 1, 2 so every tap reads aligned
-// fragments.  The next unit's rows are loaded into registers while the
-// current unit's MFMAs run (v_mfma_f32_16x16x32_bf16: lane l holds
-// A[l % 16][8 (l / 16) + e], B[8 (l / 16) + e][l % 16], D[4 (l / 16) + e][l % 16]).
-// Waves own SPW 16-channel output blocks x one 16-channel input block; when
-// the tile has fewer such groups than waves, WK = 2 waves split each strip's
-// two 32-pixel K steps and add in LDS at the end.  The bias gradient is the
-// product with an all-ones B.  Each run's sums go to its own slice of `part`
-// (no atomics); k_wgrad_reduce adds the slices to dw and db in a fixed order.
-constexpr int WG_SEG = 64, WG_XS = WG_SEG + 8;  // strip width, LDS row stride (bf16)
+// run walks down the rows of a strip).  LDS holds pixels as they lie in
+// memory (all channels of a pixel together), two input rows of 66 pixels and
+// two dy rows, one of each being filled while the other is read.  The matrix
+// operands need eight consecutive pixels of one channel per lane; gfx950's
+// transposing LDS read delivers them from that layout, so staging is one
+// 16-byte store per eight channels and a column shift is a pixel offset.
+// (Stored channel-major at three column shifts, staging took 24 two-byte
+// stores per eight channels and most of the kernel's time.)  An input row's
+// fragments stay in registers for the three dy rows they serve: one row down
+// reads three shifts of one input row.  v_mfma_f32_16x16x32_bf16: lane l
+// holds A[l % 16][8 (l / 16) + e], B[8 (l / 16) + e][l % 16], D[4 (l / 16) +
+// e][l % 16].  Waves own SPW 16-channel output blocks x one 16-channel input
+// block; when the tile has fewer such groups than waves, WK = 2 waves split
+// each strip's two 32-pixel K steps and add in LDS at the end.  The bias
+// gradient is the product with an all-ones B.  Each run's sums go to its own
+// slice of `part` (no atomics); k_wgrad_reduce adds the slices to dw and db
+// in a fixed order.  Per 8 x 256^2 training step the twelve layers take 0.38 ms
+// (0.62 ms before), the 192 -> 64 and 384 -> 128 layers at 640 TFLOP/s.
+constexpr int WG_SEG = 64;  // strip width
 
 template <int TCO, int TCI, int SPW>
 struct WgradCfg {
-  static constexpr int GROUPS = (TCO / (16 * SPW)) * (TCI / 16);  // wave groups of the tile
-  static constexpr int WK = GROUPS >= 4 ? 1 : 2;                  // waves per group (K split)
+  static constexpr int NCI = TCI / 16, GROUPS = NCI * (TCO / (16 * SPW));  // wave groups of the tile
+  static constexpr int WK = GROUPS >= 4 ? 1 : 2;                          // waves per group (K split)
+  static constexpr int KS = 2 / WK;                                       // K steps of a strip per wave
   static_assert(GROUPS * WK <= 4 && (GROUPS == 4 || WK == 2), "four waves cover the tile");
-  static constexpr int PQO = TCO / 8, PQI = TCI / 8;               // 16-byte pieces per pixel
+  static constexpr int PQO = TCO / 8, PQI = TCI / 8;                      // 16-byte pieces per pixel
   static constexpr int DY_Q = WG_SEG * PQO, XROW_Q = (WG_SEG + 2) * PQI;
-  static constexpr int NPER = (DY_Q + 3 * XROW_Q + 255) / 256;    // pieces per thread, at most 3 rows
-  static constexpr int LDS_X = 3 * 3 * TCI * WG_XS, LDS_DY = TCO * WG_XS;  // bf16 elements
-  static constexpr int RED = 10 * SPW * 4 * 64;                   // floats of the K-split reduction
-  static_assert(WK == 1 || GROUPS * RED * 4 <= LDS_X * 2, "the reduction fits the input ring");
+  static constexpr int DY_PER = (DY_Q + 255) / 256, X_PER = (XROW_Q + 255) / 256;  // pieces per thread
+  // LDS pixel strides: 16 bytes of padding spread the transposing reads' rows
+  // over the banks and keep the stores aligned
+  static constexpr int OS = TCO + 8, IS = TCI + 8;
+  static constexpr int X_ROW = (WG_SEG + 2) * IS, DY_ROW = WG_SEG * OS;
+  static constexpr int LDS = 2 * X_ROW + 2 * DY_ROW;  // bf16 elements
+  static constexpr int RED_Q = 5;                     // taps per round of the K-split reduction
+  static_assert(WK == 1 || GROUPS * RED_Q * SPW * 4 * 64 * 4 <= LDS * 2, "the reduction fits the staging buffers");
 };
 
-// What one stage loads: dy row y of image n in strip xs and the nr (at most
-// three) consecutive input rows y0 .. y0 + nr - 1 of the same image and strip.
-struct WgradStage {
-  int n, y, xs, y0, nr;
-};
-
-__device__ __forceinline__ WgradStage wgrad_stage(int u, int H, int rows, bool fresh) {
-  WgradStage st;
-  const int strip = u / rows, row = u % rows;
-  st.n = row / H;
-  st.y = row % H;
-  st.xs = strip * WG_SEG;
-  // a run's first unit, a new image or a new strip: rows y - 1 .. y + 1;
-  // otherwise only y + 1 is new
-  const int lo = (fresh || st.y == 0) ? st.y - 1 : st.y + 1;
-  st.y0 = max(lo, 0);
-  st.nr = max(0, min(st.y + 1, H - 1) - st.y0 + 1);
-  return st;
+// A lane's eight consecutive pixels of one channel from pixel-major LDS: p
+// points at the lane's piece (pixel 8 (l / 16) + (l % 16) / 4 of the K step,
+// channels 4 (l % 4) .. + 3 of the block).
+typedef __attribute__((address_space(3))) short4_t* lds_short4_p;
+template <int STRIDE>
+__device__ __forceinline__ bf16x8_t wgrad_frag(const bf16* p) {
+  const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_p)p);
+  const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_p)(p + 4 * STRIDE));
+  return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
 template <int TCO, int TCI, int SPW>
-__device__ __forceinline__ void wgrad_load(uint4* v, const WgradStage& st,
-                                           const View& x, const View& dy, int H, int W, int ci0, int co0) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TCO == 64 ? 2 : 3))) void k_wgrad_mfma(
+    View x, View dy, float* __restrict__ part, int N, int H, int W, int Cin, int Cout, int runs, int with_bias) {
   using C = WgradCfg<TCO, TCI, SPW>;
-  const int tid = threadIdx.x;
-  const int total = C::DY_Q + st.nr * C::XROW_Q;
-#pragma unroll
-  for (int k = 0; k < C::NPER; ++k) {
-    const int q = tid + 256 * k;
-    uint4 r = make_uint4(0u, 0u, 0u, 0u);
-    if (q < C::DY_Q) {
-      const int p = q / C::PQO, pc = q % C::PQO;
-      if (st.xs + p < W)
-        r = *reinterpret_cast<const uint4*>(dy.p + ((size_t)(st.n * H + st.y) * W + st.xs + p) * dy.cs + dy.co +
-                                            co0 + 8 * pc);
-    } else if (q < total) {
-      const int qq = q - C::DY_Q;
-      const int ri = qq / C::XROW_Q, rem = qq % C::XROW_Q;
-      const int p = rem / C::PQI, pc = rem % C::PQI;
-      const int gx = st.xs + p - 1;
-      if (gx >= 0 && gx < W)
-        r = *reinterpret_cast<const uint4*>(x.p + ((size_t)(st.n * H + st.y0 + ri) * W + gx) * x.cs + x.co + ci0 +
-                                            8 * pc);
-    }
-    v[k] = r;
-  }
-}
-
-template <int TCO, int TCI, int SPW>
-__device__ __forceinline__ void wgrad_store(const uint4* v, const WgradStage& st,
-                                            bf16* s_x, bf16* s_dy) {
-  using C = WgradCfg<TCO, TCI, SPW>;
-  const int tid = threadIdx.x;
-  const int total = C::DY_Q + st.nr * C::XROW_Q;
-#pragma unroll
-  for (int k = 0; k < C::NPER; ++k) {
-    const int q = tid + 256 * k;
-    const uint32_t w4[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-    if (q < C::DY_Q) {
-      const int p = q / C::PQO, pc = q % C::PQO;
-      bf16* d = s_dy + (8 * pc) * WG_XS + p;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        d[(2 * e) * WG_XS] = (bf16)(w4[e] & 0xffffu);
-        d[(2 * e + 1) * WG_XS] = (bf16)(w4[e] >> 16);
-      }
-    } else if (q < total) {
-      const int qq = q - C::DY_Q;
-      const int ri = qq / C::XROW_Q, rem = qq % C::XROW_Q;
-      const int p = rem / C::PQI, pc = rem % C::PQI;
-      const int slot = (st.y0 + ri) % 3;
-#pragma unroll
-      for (int sh = 0; sh < 3; ++sh) {
-        // copy sh holds x[xs + j + sh - 1] at column j; staged pixel p is x[xs + p - 1]
-        const int j = p - sh;
-        if (j < 0 || j >= WG_SEG) continue;
-        bf16* d = s_x + ((slot * 3 + sh) * TCI + 8 * pc) * WG_XS + j;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          d[(2 * e) * WG_XS] = (bf16)(w4[e] & 0xffffu);
-          d[(2 * e + 1) * WG_XS] = (bf16)(w4[e] >> 16);
-        }
-      }
-    }
-  }
-}
-
-template <int TCO, int TCI, int SPW>
-__global__ __launch_bounds__(256) void k_wgrad_mfma(View x, View dy, float* __restrict__ part, int N, int H, int W,
-                                                    int Cin, int Cout, int runs, int with_bias) {
-  using C = WgradCfg<TCO, TCI, SPW>;
-  __shared__ __attribute__((aligned(16))) bf16 s_x[C::LDS_X];   // [slot][shift][ci][px]
-  __shared__ __attribute__((aligned(16))) bf16 s_dy[C::LDS_DY]; // [co][px]
+  __shared__ __attribute__((aligned(16))) bf16 s_buf[C::LDS];
+  bf16* const s_x = s_buf;                  // [row & 1][pixel][ci]
+  bf16* const s_dy = s_buf + 2 * C::X_ROW;  // [row & 1][pixel][co]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i = lane & 15, kq = lane >> 4;
   const int run = blockIdx.x, cb = blockIdx.y, kb = blockIdx.z;
@@ -544,8 +479,12 @@ __global__ __launch_bounds__(256) void k_wgrad_mfma(View x, View dy, float* __re
   // this wave's group: output blocks sco0 .. sco0 + SPW - 1, input block sci, K steps kw, kw + WK, ...
   const int kw = wave % C::WK, grp = wave / C::WK;
   const bool active = grp < C::GROUPS;
-  const int sci = grp % (TCI / 16), sco0 = (grp / (TCI / 16)) * SPW;
+  const int sci = grp % C::NCI, sco0 = (grp / C::NCI) * SPW;
   const bool bias = with_bias && cb == 0 && sci == 0 && active;
+  // this lane's piece within a K step (see wgrad_frag)
+  const int fpx = 32 * kw + 8 * kq + (i >> 2), fch = 4 * (i & 3);
+  const bf16* const fdy = s_dy + fpx * C::OS + 16 * (active ? sco0 : 0) + fch;
+  const bf16* const fx = s_x + fpx * C::IS + 16 * sci + fch;
   float4_t acc[9][SPW], accb[SPW];
 #pragma unroll
   for (int q = 0; q < 9; ++q)
@@ -555,78 +494,152 @@ __global__ __launch_bounds__(256) void k_wgrad_mfma(View x, View dy, float* __re
   for (int t = 0; t < SPW; ++t) accb[t] = float4_t{0.f, 0.f, 0.f, 0.f};
   const uint4 one4 = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
   const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, one4);
-  uint4 v[C::NPER];
-  if (u0 < u1) {
-    WgradStage st = wgrad_stage(u0, H, rows, true);
-    wgrad_load<TCO, TCI, SPW>(v, st, x, dy, H, W, ci0, co0);
-    wgrad_store<TCO, TCI, SPW>(v, st, s_x, s_dy);
-    __syncthreads();
-    for (int u = u0; u < u1; ++u) {
-      const WgradStage cur = st;
-      const bool more = u + 1 < u1;
-      if (more) {
-        st = wgrad_stage(u + 1, H, rows, false);
-        wgrad_load<TCO, TCI, SPW>(v, st, x, dy, H, W, ci0, co0);
-      }
-      if (active) {
+  uint4 vd[C::DY_PER], vx[C::X_PER];
+  // dy row y and input row yy of image n, strip at xs
+  auto load_dy = [&](int n, int y, int xs) {
 #pragma unroll
-        for (int ks = kw; ks < WG_SEG / 32; ks += C::WK) {
-          const int px = 32 * ks + 8 * kq;
-          bf16x8_t a[SPW];
+    for (int k = 0; k < C::DY_PER; ++k) {
+      const int q = tid + 256 * k, p = q / C::PQO, pc = q % C::PQO;
+      vd[k] = make_uint4(0u, 0u, 0u, 0u);
+      if (q < C::DY_Q && xs + p < W)
+        vd[k] = *reinterpret_cast<const uint4*>(dy.p + ((size_t)(n * H + y) * W + xs + p) * dy.cs + dy.co + co0 +
+                                                8 * pc);
+    }
+  };
+  auto store_dy = [&](int y) {
+#pragma unroll
+    for (int k = 0; k < C::DY_PER; ++k) {
+      const int q = tid + 256 * k, p = q / C::PQO, pc = q % C::PQO;
+      if (q < C::DY_Q) *reinterpret_cast<uint4*>(s_dy + (y & 1) * C::DY_ROW + p * C::OS + 8 * pc) = vd[k];
+    }
+  };
+  auto load_x = [&](int n, int yy, int xs) {
+#pragma unroll
+    for (int k = 0; k < C::X_PER; ++k) {
+      const int q = tid + 256 * k, p = q / C::PQI, pc = q % C::PQI, gx = xs + p - 1;
+      vx[k] = make_uint4(0u, 0u, 0u, 0u);
+      if (q < C::XROW_Q && gx >= 0 && gx < W)
+        vx[k] = *reinterpret_cast<const uint4*>(x.p + ((size_t)(n * H + yy) * W + gx) * x.cs + x.co + ci0 + 8 * pc);
+    }
+  };
+  auto store_x = [&](int yy) {
+#pragma unroll
+    for (int k = 0; k < C::X_PER; ++k) {
+      const int q = tid + 256 * k, p = q / C::PQI, pc = q % C::PQI;
+      if (q < C::XROW_Q) *reinterpret_cast<uint4*>(s_x + (yy & 1) * C::X_ROW + p * C::IS + 8 * pc) = vx[k];
+    }
+  };
+  // fragments of the input rows around the current dy row: [row][shift][K step]
+  bf16x8_t xf[3][3][C::KS];
+  auto read_x = [&](bf16x8_t (&f)[3][C::KS], int yy) {
+    const bf16* const fr = fx + (yy & 1) * C::X_ROW;
+#pragma unroll
+    for (int sh = 0; sh < 3; ++sh)
+#pragma unroll
+      for (int ks = 0; ks < C::KS; ++ks) f[sh][ks] = wgrad_frag<C::IS>(fr + (sh + 32 * ks) * C::IS);
+  };
+  // One dy row; xf[R] holds input row y - 1, xf[R + 1] row y, and row y + 1
+  // is read into xf[R + 2] (indices modulo 3).  Ends with the next dy row
+  // and input row y + 2 in LDS when the strip goes on.
+  auto unit = [&](auto rot, int n, int y, int xs, bool more) {
+    constexpr int R = decltype(rot)::value;
+    const bool more_x = more && y + 2 < H;
+    if (more) load_dy(n, y + 1, xs);
+    if (more_x) load_x(n, y + 2, xs);
+    if (active) {
+      if (y + 1 < H) read_x(xf[(R + 2) % 3], y + 1);
+#pragma unroll
+      for (int ks = 0; ks < C::KS; ++ks) {
+        bf16x8_t a[SPW];
+#pragma unroll
+        for (int t = 0; t < SPW; ++t)
+          a[t] = wgrad_frag<C::OS>(fdy + (y & 1) * C::DY_ROW + 32 * ks * C::OS + 16 * t);
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+          if (y + r < 1 || y + r > H) continue;  // zero padding: no products
+#pragma unroll
+          for (int sh = 0; sh < 3; ++sh)
+#pragma unroll
+            for (int t = 0; t < SPW; ++t)
+              acc[r * 3 + sh][t] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], xf[(R + r) % 3][sh][ks], acc[r * 3 + sh][t], 0, 0, 0);
+        }
+        if (bias) {
 #pragma unroll
           for (int t = 0; t < SPW; ++t)
-            a[t] = *reinterpret_cast<const bf16x8_t*>(s_dy + (16 * (sco0 + t) + i) * WG_XS + px);
-#pragma unroll
-          for (int r = 0; r < 3; ++r) {
-            const int yy = cur.y + r - 1;
-            if (yy < 0 || yy >= H) continue;  // zero padding: no products
-            const int slot = yy % 3;
-#pragma unroll
-            for (int sh = 0; sh < 3; ++sh) {
-              const bf16x8_t b =
-                  *reinterpret_cast<const bf16x8_t*>(s_x + ((slot * 3 + sh) * TCI + 16 * sci + i) * WG_XS + px);
-#pragma unroll
-              for (int t = 0; t < SPW; ++t)
-                acc[r * 3 + sh][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b, acc[r * 3 + sh][t], 0, 0, 0);
-            }
-          }
-          if (bias) {
-#pragma unroll
-            for (int t = 0; t < SPW; ++t) accb[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], ones, accb[t], 0, 0, 0);
-          }
+            accb[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], ones, accb[t], 0, 0, 0);
         }
       }
-      __syncthreads();  // the ring slot and dy buffer the next stage overwrites are read
-      if (more) {
-        wgrad_store<TCO, TCI, SPW>(v, st, s_x, s_dy);
-        __syncthreads();
-      }
     }
-  }
-  // K-split groups: the second wave of each group adds its sums to the first's
-  if (C::WK == 2) {
-    float* s_red = reinterpret_cast<float*>(s_x);  // free: the last unit's reads ended at a barrier
-    if (active && kw == 1) {
-#pragma unroll
-      for (int q = 0; q < 10; ++q)
-#pragma unroll
-        for (int t = 0; t < SPW; ++t)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            s_red[((grp * 10 + q) * SPW + t) * 4 * 64 + e * 64 + lane] = q < 9 ? acc[q][t][e] : accb[t][e];
+    if (more) {
+      store_dy(y + 1);
+      if (more_x) store_x(y + 2);
+      __syncthreads();
+    }
+  };
+  for (int u = u0; u < u1;) {
+    // a new strip or image
+    const int row = u % rows, n = row / H, y0 = row % H, xs = (u / rows) * WG_SEG;
+    const int y1 = min(H, y0 + (u1 - u));  // this run's dy rows of it: y0 .. y1 - 1
+    __syncthreads();  // the previous rows are read
+    load_dy(n, y0, xs);
+    store_dy(y0);
+    if (y0 > 0) {
+      load_x(n, y0 - 1, xs);
+      store_x(y0 - 1);
+    }
+    load_x(n, y0, xs);
+    store_x(y0);
+    __syncthreads();
+    if (active) {
+      if (y0 > 0) read_x(xf[0], y0 - 1);
+      read_x(xf[1], y0);
+    }
+    __syncthreads();  // row y0 - 1 makes room for row y0 + 1
+    if (y0 + 1 < H) {
+      load_x(n, y0 + 1, xs);
+      store_x(y0 + 1);
     }
     __syncthreads();
-    if (active && kw == 0) {
+    for (int y = y0; y < y1;) {
+      unit(std::integral_constant<int, 0>(), n, y, xs, y + 1 < y1);
+      if (++y >= y1) break;
+      unit(std::integral_constant<int, 1>(), n, y, xs, y + 1 < y1);
+      if (++y >= y1) break;
+      unit(std::integral_constant<int, 2>(), n, y, xs, y + 1 < y1);
+      ++y;
+    }
+    u += y1 - y0;
+  }
+  // K-split groups: the second wave of each group adds its sums to the first's
+  if constexpr (C::WK == 2) {
+    float* const s_red = reinterpret_cast<float*>(s_buf);
 #pragma unroll
-      for (int q = 0; q < 10; ++q)
+    for (int q0 = 0; q0 < 10; q0 += C::RED_Q) {  // taps 0..8, then the bias
+      __syncthreads();
+      if (active && kw == 1) {
 #pragma unroll
-        for (int t = 0; t < SPW; ++t)
+        for (int q = q0; q < q0 + C::RED_Q; ++q)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float o = s_red[((grp * 10 + q) * SPW + t) * 4 * 64 + e * 64 + lane];
-            if (q < 9) acc[q][t][e] += o;
-            else accb[t][e] += o;
-          }
+          for (int t = 0; t < SPW; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              s_red[(((grp * C::RED_Q + q - q0) * SPW + t) * 4 + e) * 64 + lane] =
+                  q < 9 ? acc[q < 9 ? q : 0][t][e] : accb[t][e];
+      }
+      __syncthreads();
+      if (active && kw == 0) {
+#pragma unroll
+        for (int q = q0; q < q0 + C::RED_Q; ++q)
+#pragma unroll
+          for (int t = 0; t < SPW; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float o = s_red[(((grp * C::RED_Q + q - q0) * SPW + t) * 4 + e) * 64 + lane];
+              if (q < 9) acc[q < 9 ? q : 0][t][e] += o;
+              else accb[t][e] += o;
+            }
+      }
     }
   }
   if (!active || kw != 0) return;
@@ -654,17 +667,28 @@ __global__ __launch_bounds__(256) void k_wgrad_mfma(View x, View dy, float* __re
 
 // dw[i] += sum over runs of part (bias entries after the weights): 64
 // outputs per workgroup, 16 lanes per output summing every 16th run, the 16
-// sums added in a fixed order (deterministic).
+// sums added in a fixed order (deterministic).  Four loads in flight per lane
+// (17.6 -> 11.0 us a layer); eight, or 16 outputs per workgroup for the small
+// layers, took 13 us.
 __global__ __launch_bounds__(1024) void k_wgrad_reduce(const float* __restrict__ part, float* __restrict__ dw,
                                                        float* __restrict__ db, int runs, int n_w, int n_b) {
   __shared__ float s_sum[16][65];
   const int o = threadIdx.x & 63, g = threadIdx.x >> 6;
   const int idx = blockIdx.x * 64 + o;
   float acc = 0.0f;
-  if (idx < n_w) {
-    for (int k = g; k < runs; k += 16) acc += part[(size_t)k * n_w + idx];
-  } else if (idx < n_w + n_b) {
-    for (int k = g; k < runs; k += 16) acc += part[(size_t)runs * n_w + (size_t)k * n_b + (idx - n_w)];
+  if (idx < n_w + n_b) {
+    const float* const src = idx < n_w ? part + idx : part + (size_t)runs * n_w + (idx - n_w);
+    const size_t step = idx < n_w ? (size_t)n_w : (size_t)n_b;
+    int k = g;
+    for (; k + 48 < runs; k += 64) {
+      const float v0 = src[(size_t)k * step], v1 = src[(size_t)(k + 16) * step], v2 = src[(size_t)(k + 32) * step],
+                  v3 = src[(size_t)(k + 48) * step];
+      acc += v0;
+      acc += v1;
+      acc += v2;
+      acc += v3;
+    }
+    for (; k < runs; k += 16) acc += src[(size_t)k * step];
   }
   s_sum[g][o] = acc;
   __syncthreads();

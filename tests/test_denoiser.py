@@ -128,6 +128,31 @@ def test_conv3x3_gradients_match_torch(rf, gpu_available, Cin, Cout, W, H):
     assert (err <= 2.0 ** -8 * ref_dx.abs() + 1e-4).all(), float(err.max())
 
 
+# One row, two rows, a strip of exactly 64 pixels and one more, runs that
+# start inside a strip, several images: every channel tile.
+@pytest.mark.parametrize("Cin,Cout,N,H,W", [(64, 64, 1, 1, 64), (32, 32, 2, 2, 65), (16, 32, 1, 3, 1),
+                                            (32, 16, 5, 7, 64), (16, 16, 3, 1, 129), (64, 128, 1, 70, 64),
+                                            (32, 64, 2, 37, 200)])
+def test_conv3x3_wgrad_at_strip_edges(rf, gpu_available, Cin, Cout, N, H, W):
+    import torch
+    import torch.nn.functional as F
+    ctx = rf.Context(1 << 12, 1, 16)
+    g = torch.Generator().manual_seed(Cin + 7 * Cout + H)
+    x = _bf16(torch.randn(N, H, W, Cin, generator=g))
+    dy = _bf16(torch.randn(N, H, W, Cout, generator=g))
+    wr = torch.zeros(Cout, Cin, 3, 3, requires_grad=True)
+    br = torch.zeros(Cout, requires_grad=True)
+    F.conv2d(x.float().permute(0, 3, 1, 2), wr, br, padding=1).backward(dy.float().permute(0, 3, 1, 2))
+    dw = torch.zeros(3, 3, Cout, Cin, device="cuda")
+    db = torch.zeros(Cout, device="cuda")
+    xd, dyd = x.cuda(), dy.cuda()
+    ctx.check(ctx.L.rf_nn_conv3x3_wgrad(ctx.h, xd.data_ptr(), Cin, 0, dyd.data_ptr(), Cout, 0, dw.data_ptr(),
+                                        db.data_ptr(), N, H, W, Cin, Cout))
+    # fp32 sums of N H W products of unit variance: their rounding stays far below 1e-3
+    torch.testing.assert_close(dw.cpu(), wr.grad.permute(2, 3, 0, 1), rtol=1e-4, atol=1e-3)
+    torch.testing.assert_close(db.cpu(), br.grad, rtol=1e-4, atol=1e-3)
+
+
 @pytest.mark.parametrize("npix", [1, 257, 4096 + 3])
 def test_log_density_input_matches_formula(rf, gpu_available, npix):
     """bf16(log10(1 + v scale)) in channels 0..3, the noise level
