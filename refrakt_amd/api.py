@@ -511,12 +511,12 @@ class Context:
 
     def shuffle_rows(self) -> np.ndarray:
         ppt = self.total_particles // self.temporal_samples
-        out = np.zeros((self.shuffle_count, ppt), np.uint32)
+        out = np.empty((self.shuffle_count, ppt), np.uint32)
         self.check(self.L.rf_shuffle_download(self.h, _uptr(out)))
         return out
 
     def rng_states(self) -> np.ndarray:
-        out = np.zeros((self.total_particles, 4), np.uint32)
+        out = np.empty((self.total_particles, 4), np.uint32)
         self.check(self.L.rf_rng_download(self.h, _uptr(out)))
         return out
 
@@ -572,8 +572,8 @@ class Context:
 
     def render(self, fh: "FlameHandle", params: RenderParams, want_hist=True, want_image=True):
         W, H = params.width, params.height
-        hist = np.zeros((H, W, 4), np.float32) if want_hist else None
-        img = np.zeros((H, W, 4), np.float32) if want_image else None
+        hist = np.empty((H, W, 4), np.float32) if want_hist else None
+        img = np.empty((H, W, 4), np.float32) if want_image else None
         st = Stats()
         self.check(self.L.rf_render(self.h, fh.h, C.byref(params), _fptr(hist) if want_hist else None,
                                     _fptr(img) if want_image else None, C.byref(st)))
@@ -634,7 +634,7 @@ class FlameHandle:
         return drawn.value
 
     def particles(self) -> np.ndarray:
-        out = np.zeros((self.ctx.total_particles, 4), np.float32)
+        out = np.empty((self.ctx.total_particles, 4), np.float32)
         self.ctx.check(self.ctx.L.rf_particles_download(self.ctx.h, self.h, _fptr(out)))
         return out
 
@@ -692,7 +692,7 @@ class Histogram:
         self.ctx.check(self.ctx.L.rf_hist_zero(self.h))
 
     def download(self) -> np.ndarray:
-        out = np.zeros((self.height, self.width, 4), np.float32)
+        out = np.empty((self.height, self.width, 4), np.float32)
         self.ctx.check(self.ctx.L.rf_hist_download(self.h, _fptr(out)))
         return out
 
@@ -782,7 +782,7 @@ class Batch:
 
     def _download(self, i: int, which: int) -> np.ndarray:
         w, h = self.sizes[i]
-        out = np.zeros((h, w, 4), np.float32)
+        out = np.empty((h, w, 4), np.float32)
         self.ctx.check(self.ctx.L.rf_batch_download(self.h, i, which, out.ctypes.data))
         return out
 
@@ -821,7 +821,7 @@ class Denoiser:
             pass
 
     def params(self) -> np.ndarray:
-        out = np.zeros(self.n_params, np.float32)
+        out = np.empty(self.n_params, np.float32)
         self.ctx.check(self.ctx.L.rf_denoiser_get_params(self.h, out.ctypes.data, self.n_params))
         return out
 
@@ -839,7 +839,7 @@ class Denoiser:
         self.ctx.check(self.ctx.L.rf_denoiser_infer(self.h, C.c_void_p(x_ptr), C.c_void_p(y_ptr), N, H, W))
 
     def grads(self, x_ptr: int, t_ptr: int, N: int, H: int, W: int):
-        g = np.zeros(self.n_params, np.float32)
+        g = np.empty(self.n_params, np.float32)
         loss = C.c_float(0.0)
         self.ctx.check(self.ctx.L.rf_denoiser_grads(self.h, C.c_void_p(x_ptr), C.c_void_p(t_ptr), N, H, W,
                                                     g.ctypes.data, C.byref(loss)))

@@ -11,7 +11,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "librefrakt_amd.so")
-SOURCES = ["rf_k_compat.hip", "rf_k_fast.hip", "rf_k_misc.hip", "rf_host.cpp", "rf_flam3.cpp", "rf_output.cpp",
+SOURCES = ["rf_k_compat.hip", "rf_k_fast.hip", "rf_k_misc.hip", "rf_host.cpp", "rf_stage.cpp", "rf_flam3.cpp", "rf_output.cpp",
            "rf_k_batch.hip", "rf_batch.cpp", "rf_k_nn.hip", "rf_denoiser.cpp", "rf_k_sort.hip", "rf_jit.cpp"]
 # Device headers of the fast engine's kernel body, embedded in the library so
 # that flame programs (rf_jit.cpp) can be compiled at run time with hiprtc;

@@ -611,7 +611,7 @@ int rf_batch_download(rf_batch* b, uint32_t i, int32_t which, float* host) {
   if (!b || !host) return RF_ERR_ARG;
   if (i >= b->n || (which != 0 && which != 1)) return rfh::set_err(b->ctx, RF_ERR_ARG, "batch: bad frame or buffer");
   const void* src = which == 0 ? rf_batch_hist_ptr(b, i) : rf_batch_image_ptr(b, i);
-  HIPCHK(b->ctx, hipMemcpy(host, src, (size_t)b->W[i] * b->H[i] * 16, hipMemcpyDeviceToHost));
+  HIPCHK(b->ctx, rfh::download(host, src, (size_t)b->W[i] * b->H[i] * 16, b->ctx->stream));
   return RF_OK;
 }
 

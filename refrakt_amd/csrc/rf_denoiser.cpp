@@ -290,8 +290,7 @@ size_t rf_denoiser_num_params(const rf_denoiser* d) { return d ? d->n_params : 0
 int rf_denoiser_get_params(rf_denoiser* d, float* host, size_t n) {
   if (!d || !host) return RF_ERR_ARG;
   if (n != d->n_params) return rfh::set_err(d->ctx, RF_ERR_ARG, "denoiser: parameter count mismatch");
-  HIPCHK(d->ctx, hipStreamSynchronize(d->ctx->stream));
-  HIPCHK(d->ctx, hipMemcpy(host, d->p.p, n * 4, hipMemcpyDeviceToHost));
+  HIPCHK(d->ctx, rfh::download(host, d->p.p, n * 4, d->ctx->stream));
   return RF_OK;
 }
 
@@ -359,8 +358,7 @@ int rf_denoiser_grads(rf_denoiser* d, const void* x, const void* target, int32_t
   HIPCHK(ctx, rfn::residual_loss(View{(bf16*)x, 16, 0}, V(d->o, 16), (const bf16*)target, nullptr,
                                  (float*)d->loss.p, (bf16*)d->g_o.p, npix, 1.0f / (4.0f * (float)npix), s));
   if ((rc = backward(d, (const bf16*)x, N, H, W))) return rc;
-  HIPCHK(ctx, hipStreamSynchronize(s));
-  HIPCHK(ctx, hipMemcpy(grads_host, d->g.p, d->n_params * 4, hipMemcpyDeviceToHost));
+  HIPCHK(ctx, rfh::download(grads_host, d->g.p, d->n_params * 4, s));
   if (loss_out) {
     float ls = 0.0f;
     HIPCHK(ctx, hipMemcpy(&ls, d->loss.p, 4, hipMemcpyDeviceToHost));

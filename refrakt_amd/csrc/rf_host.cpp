@@ -988,6 +988,8 @@ int rf_create(const rf_sim_params* p, rf_ctx** out) {
   ctx->ppt = p->total_particles / p->temporal_samples;
   ctx->shuffle_count = ctx->sp.shuffle_count;
   ctx->row_state = p->seed ^ 0x0123456789ABCDEFull;
+  stage_hold();
+  ctx->holds_stage = true;
   *out = ctx;
   return RF_OK;
 }
@@ -997,6 +999,7 @@ void rf_destroy(rf_ctx* ctx) {
   if (ctx->render_hist) rf_hist_destroy(ctx->render_hist);
   if (ctx->stream) { (void)hipStreamSynchronize(ctx->stream); (void)hipStreamDestroy(ctx->stream); }
   for (auto& e : ctx->ev) if (e) (void)hipEventDestroy(e);
+  if (ctx->holds_stage) stage_release();
   delete ctx;
 }
 
@@ -1225,8 +1228,7 @@ int rf_hist_zero(rf_hist* h) {
 
 int rf_hist_download(rf_hist* h, float* host) {
   if (!h || !host) return RF_ERR_ARG;
-  HIPCHK(h->ctx, hipMemcpyAsync(host, h->ptr, (size_t)h->w * h->h * 16, hipMemcpyDeviceToHost, h->ctx->stream));
-  HIPCHK(h->ctx, hipStreamSynchronize(h->ctx->stream));
+  HIPCHK(h->ctx, download(host, h->ptr, (size_t)h->w * h->h * 16, h->ctx->stream));
   return RF_OK;
 }
 
@@ -1387,7 +1389,7 @@ int rf_render(rf_ctx* ctx, rf_flame* f, const rf_render_params* rp, float* hist_
   HIPCHK(ctx, hipEventElapsedTime(&tm_ms, ctx->ev[1], ctx->ev[2]));
   if (hist_out) if ((rc = rf_hist_download(h, hist_out))) return rc;
   if (image_out) {
-    HIPCHK(ctx, hipMemcpy(image_out, ctx->render_img.p, (size_t)rp->width * rp->height * 16, hipMemcpyDeviceToHost));
+    HIPCHK(ctx, download(image_out, ctx->render_img.p, (size_t)rp->width * rp->height * 16, ctx->stream));
   }
   s.iterations = ctx->sp.total_particles * ((uint64_t)rp->warmup_passes + 1 + (uint64_t)rp->draw_passes * rp->draw_calls);
   s.ms_warmup = ms(t0, t1);
@@ -1400,21 +1402,21 @@ int rf_render(rf_ctx* ctx, rf_flame* f, const rf_render_params* rp, float* hist_
 
 int rf_particles_download(rf_ctx* ctx, rf_flame* f, float* host) {
   if (!ctx || !f || !host || !f->local.p) return set_err(ctx, RF_ERR_ARG, "no particles");
-  HIPCHK(ctx, hipMemcpy(host, f->local.p, ctx->sp.total_particles * 16, hipMemcpyDeviceToHost));
+  HIPCHK(ctx, download(host, f->local.p, ctx->sp.total_particles * 16, ctx->stream));
   return RF_OK;
 }
 int rf_rng_download(rf_ctx* ctx, uint32_t* host) {
   if (!ctx || !host) return RF_ERR_ARG;
   int rc = ensure_compat(ctx);
   if (rc) return rc;
-  HIPCHK(ctx, hipMemcpy(host, ctx->rs.p, ctx->sp.total_particles * 16, hipMemcpyDeviceToHost));
+  HIPCHK(ctx, download(host, ctx->rs.p, ctx->sp.total_particles * 16, ctx->stream));
   return RF_OK;
 }
 int rf_shuffle_download(rf_ctx* ctx, uint32_t* host) {
   if (!ctx || !host) return RF_ERR_ARG;
   int rc = ensure_compat(ctx);
   if (rc) return rc;
-  HIPCHK(ctx, hipMemcpy(host, ctx->shuf.p, ctx->shuf.bytes, hipMemcpyDeviceToHost));
+  HIPCHK(ctx, download(host, ctx->shuf.p, ctx->shuf.bytes, ctx->stream));
   return RF_OK;
 }
 int rf_sample_points_download(rf_ctx* ctx, float* host) {

@@ -8,6 +8,7 @@
 
 #include "../../include/refrakt_amd.h"
 #include "rf_device.hpp"
+#include "rf_stage.hpp"
 
 struct rf_ctx;
 namespace rfj {
@@ -116,6 +117,7 @@ struct rf_ctx {
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   double last_draw_ms = 0.0;   // device time of the last draw_to_bins' chaos-game launches
   bool programs = true;        // fast engine: run flame programs (rf_jit.cpp)
+  bool holds_stage = false;    // counted by stage_hold
 };
 
 struct rf_flame {
