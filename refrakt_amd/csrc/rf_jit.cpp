@@ -238,7 +238,7 @@ const Program* get_program(const rfd::Block& b, const std::vector<std::pair<int,
     hipFunction_t fn = nullptr;
     e = hipModuleGetFunction(&fn, mod, entry_name(k.first, k.second).c_str());
     if (e != hipSuccess) { err = std::string("hipModuleGetFunction: ") + hipGetErrorString(e); return nullptr; }
-    if (k.second == 4 || k.second >= kBatchKernel) {
+    if (k.second == 4 || k.second == 5 || k.second >= kBatchKernel) {
       int per_cu = 0, cus = 0;
       e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64 * k.first, 0);
       if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -293,6 +293,9 @@ hipError_t launch_fast(const Program* p, const rfk::FastArgs& a0, uint64_t n, in
   a.n_batches = (uint32_t)(n / (64u * (uint32_t)waves));
   uint32_t grid = a.n_batches;
   if (hist_mode == 4) grid = std::min<uint32_t>(grid, (uint32_t)p->resident.at({waves, hist_mode}));
+  if (hist_mode == 5 && a.do_draw)
+    grid = rfk::sort_grid(a.n_batches, a.n_iter, a.sort.n_buckets, rfk::SORT_STAGE_SLOTS / (64u * (uint32_t)waves),
+                          (uint32_t)p->resident.at({waves, hist_mode}));
   const rfd::Block* blocks = a.blocks;
   void* args[] = {&a, &blocks};
   return hipModuleLaunchKernel(it->second, grid, 1, 1, 64u * (uint32_t)waves, 1, 1, 0, s, args, nullptr);

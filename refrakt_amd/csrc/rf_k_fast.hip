@@ -25,9 +25,10 @@ static hipError_t launch_fast_k(const FastArgs& a0, uint64_t n, hipStream_t s) {
   FastArgs a = a0;
   a.n_batches = (uint32_t)(n / (64u * W));
   uint32_t grid = a.n_batches;
-  if (HM == 4) {
-    // one workgroup per resident slot (cached per instantiation and device),
-    // so that each LDS table spans many batches before it is flushed
+  if (HM == 4 || (HM == 5 && a.do_draw)) {
+    // resident workgroups (cached per instantiation and device): for the LDS
+    // table the grid, so that each table spans many batches before it is
+    // flushed
     constexpr int kMaxDev = 64;
     static int resident[kMaxDev] = {0};
     int dev = 0;
@@ -44,7 +45,8 @@ static hipError_t launch_fast_k(const FastArgs& a0, uint64_t n, hipStream_t s) {
       res = cus * (per_cu > 0 ? per_cu : 1);
       if (dev < kMaxDev) resident[dev] = res;
     }
-    grid = std::min<uint32_t>(grid, (uint32_t)res);
+    grid = HM == 4 ? std::min<uint32_t>(grid, (uint32_t)res)
+                   : sort_grid(grid, a.n_iter, a.sort.n_buckets, SORT_STAGE_SLOTS / (64u * W), (uint32_t)res);
   }
   hipLaunchKernelGGL((k_fast<W, HM, LOGK>), dim3(grid), dim3(64 * W), 0, s, a, a.blocks);
   return hipGetLastError();

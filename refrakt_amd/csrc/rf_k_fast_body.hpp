@@ -25,9 +25,10 @@ using namespace rfd;
 // streams are keyed by particle, wave-of-batch and batch index, never by the
 // workgroup, so the results do not depend on the grid size.
 //
-// HM 1/2/3/5 launch one workgroup per batch; HM 4 (LDS bin cache) launches
-// one workgroup per resident slot so that each workgroup's LDS table spans
-// many batches before it is flushed.
+// HM 1/2/3 launch one workgroup per batch; HM 4 (LDS bin cache) launches one
+// workgroup per resident slot so that each workgroup's LDS table spans many
+// batches before it is flushed; HM 5 (sort) lets a workgroup's stage fill over
+// up to four batches (sort_grid).
 // HIST_SORT staging: the samples of SI = sort_stage_iters<N>() iterations
 // wait in LDS (one fixed slot per lane and iteration, no append atomics).  A
 // flush ranks them within their buckets (each lane loads its staged bins
@@ -137,6 +138,17 @@ __device__ __forceinline__ void sort_flush(SortStage<N, true>& st, uint32_t n_st
   }
 }
 
+// The kernel's arguments (its first parameter is a FastArgs) read anew from
+// the kernarg segment: what only a batch's start and end need is loaded there
+// instead of being kept in scalar registers over the iterations, which need
+// all of them.
+typedef const __attribute__((address_space(4))) FastArgs CFastArgs;
+__device__ __forceinline__ CFastArgs* fast_args() {
+  CFastArgs* p = (CFastArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
 template <int WAVES, int HM, int LOGK, class Prog>
 __device__ __forceinline__ void k_fast_body(const FastArgs& g, const Block* __restrict__ blocks) {
   constexpr int N = 64 * WAVES;
@@ -153,6 +165,7 @@ __device__ __forceinline__ void k_fast_body(const FastArgs& g, const Block* __re
   __shared__ __attribute__((aligned(16))) uint16_t s_perm[NPERM * N];
   __shared__ LdsBins<LOGK> s_bins;
   __shared__ SortStage<N, HM == 5> s_sort;
+  __shared__ uint4 s_seed[WAVES + 1];  // the streams of a batch's waves, then the batch's own
   const uint32_t tid = threadIdx.x;
   if constexpr (HM != 5)
     for (uint32_t i = tid; i < 256u; i += N) s_pal[i] = g.palette[i];
@@ -173,28 +186,60 @@ __device__ __forceinline__ void k_fast_body(const FastArgs& g, const Block* __re
       }
     }
   }
-  __syncthreads();
+  // (the barrier behind the first batch's seeds orders these writes too)
 
   unsigned long long drawn = 0;
   uint32_t hits = 0;
+  uint32_t staged = 0;  // iterations waiting in the sort stage
   for (uint32_t batch = blockIdx.x; batch < g.n_batches; batch += gridDim.x) {
+    CFastArgs* a = fast_args();
     const uint32_t base = batch * (uint32_t)N;
     const uint32_t pid = base + tid;
+    const bool first_run = a->first_run != 0u;
+    float4 start = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (!first_run) start = a->pos[pid];
     // Integer division runs on the VALU, so the quotient is not known to be
     // uniform; without readfirstlane every Block access would be a vector load.
-    const uint32_t t = __builtin_amdgcn_readfirstlane(base / g.ppt);
-    CBlock* blk = as_constant(blocks + (size_t)t * g.block_stride);
+    const uint32_t t = __builtin_amdgcn_readfirstlane(base / a->ppt);
+    CBlock* blk = as_constant(blocks + (size_t)t * a->block_stride);
 
-    Jsf32 lrng = jsf_from_philox(g.seed, pid, g.launch, 0u);
-    const uint32_t wid = __builtin_amdgcn_readfirstlane(batch * WAVES + (tid >> 6));
-    Jsf32 wrng = jsf_from_philox(g.seed, wid, g.launch, 1u);
-    Jsf32 grng = jsf_from_philox(g.seed, batch, g.launch, 2u);
+    // The streams of the batch's waves and of the batch itself.  A workgroup
+    // of several batches has one wave (the next one for the next batch, so
+    // that the SIMDs share this) seed them all, a lane each; the others read
+    // the states from LDS.  With one batch each wave seeds its own on the
+    // scalar unit, beside the lanes' seeding: no wave waits for another's, but
+    // the 450 scalar instructions a wave cost as much as the lanes' vector
+    // ones where many batches start at once.  (One pass over 4 Mi particles:
+    // 115 us a draw with four batches a workgroup, 126 with the scalar seeds;
+    // eight passes and one batch: 405 us with shared seeds, 394 with scalar.)
+    Jsf32 lrng = jsf_from_philox(a->seed, pid, a->launch, 0u), wrng, grng;
+    if (gridDim.x < g.n_batches) {
+      if (tid / WAVE == batch % WAVES) {
+        uint32_t lane = tid % WAVE;
+        asm volatile("" : "+v"(lane));  // computed here, not held over the batches
+        const bool of_wave = lane < WAVES;
+        const Jsf32 r = jsf_from_philox(a->seed, of_wave ? batch * WAVES + lane : batch, a->launch, of_wave ? 1u : 2u);
+        if (lane <= WAVES) s_seed[lane] = make_uint4(r.a, r.b, r.c, r.d);
+      }
+      lds_barrier();
+      auto stream = [&](uint32_t i) {
+        const uint4 v = s_seed[i];
+        return Jsf32{(uint32_t)__builtin_amdgcn_readfirstlane(v.x), (uint32_t)__builtin_amdgcn_readfirstlane(v.y),
+                     (uint32_t)__builtin_amdgcn_readfirstlane(v.z), (uint32_t)__builtin_amdgcn_readfirstlane(v.w)};
+      };
+      wrng = stream(tid / WAVE);
+      grng = stream(WAVES);
+    } else {
+      wrng = jsf_from_philox(a->seed, __builtin_amdgcn_readfirstlane(batch * WAVES + tid / WAVE), a->launch, 1u);
+      grng = jsf_from_philox(a->seed, batch, a->launch, 2u);
+      lds_barrier();
+    }
 
     float x, y, c;
-    if (g.first_run) {
+    if (first_run) {
       // Hammersley point (src/hammersley.cpp:29-48) of index pid mod ppt, jittered
       // like the first run of shaders/flame.glsl:63-66.
-      const uint32_t cnt = g.ppt;
+      const uint32_t cnt = a->ppt;
       const uint32_t mx = (cnt % 2u == 0u) ? cnt : (1u << (32 - __clz(cnt - 1u)));
       const float inv_max = rf_div_rn(1.0f, (float)mx);
       const uint32_t rbits = 31u - __clz(mx);
@@ -211,8 +256,7 @@ __device__ __forceinline__ void k_fast_body(const FastArgs& g, const Block* __re
       x = x + s * sn;
       y = y + s * cs;
     } else {
-      const float4 p = g.pos[pid];
-      x = p.x; y = p.y; c = p.z;
+      x = start.x; y = start.y; c = start.z;
     }
 
     for (uint32_t it = 0; it < g.n_iter; ++it) {
@@ -220,7 +264,7 @@ __device__ __forceinline__ void k_fast_body(const FastArgs& g, const Block* __re
       // (float compares would run on the VALU, make xid look divergent and turn
       // every xform/term access into vector loads behind the atomics).
       const int xid = Prog::select(blk, wrng.next_a());
-      XOut o = Prog::apply(blk, xid, x, y, c, g.first_run && it == 0, lrng);
+      XOut o = Prog::apply(blk, xid, x, y, c, first_run && it == 0, lrng);
       if (rf_badval(o.x) || rf_badval(o.y)) {
         // A particle that left the finite plane restarts at a random point and
         // is not drawn this iteration (the reference leaves it NaN forever,
@@ -235,7 +279,7 @@ __device__ __forceinline__ void k_fast_body(const FastArgs& g, const Block* __re
         if constexpr (HM == 4) {
           bin_lds(s_bins, g.bins, L.bidx, L.valid, L.pidx, L.w, s_pal, hits);
         } else if constexpr (HM == 5) {
-          const uint32_t slot = (it % sort_stage_iters<N>()) * N + tid;
+          const uint32_t slot = staged * N + tid;
           s_sort.bin[slot] = L.valid ? L.bidx : SORT_NONE;
           s_sort.pid[slot] = (uint8_t)L.pidx;
         } else {
@@ -251,15 +295,18 @@ __device__ __forceinline__ void k_fast_body(const FastArgs& g, const Block* __re
       x = s_x[b][tid]; y = s_y[b][tid]; c = s_c[b][tid];
       if constexpr (HM == 5) {
         // the exchange barrier above also orders the staging writes before the flush
-        constexpr uint32_t SI = sort_stage_iters<N>();
-        if (g.do_draw && ((it % SI) == SI - 1 || it + 1 == g.n_iter))
-          sort_flush(s_sort, (it % SI) + 1, g.sort, g.bins, g.palette);
+        if (g.do_draw && (++staged == (uint32_t)sort_stage_iters<N>() ||
+                          (it + 1 == g.n_iter && batch + gridDim.x >= g.n_batches))) {
+          sort_flush(s_sort, staged, g.sort, g.bins, g.palette);
+          staged = 0;
+        }
       }
     }
-    g.pos[pid] = make_float4(x, y, c, 0.0f);
-    // The next batch's first exchange writes buffer 0, which slower waves may
-    // still be reading from this batch's last iteration.
-    lds_barrier();
+    // The next batch's first exchange comes after the barrier behind its
+    // seeds, and so after every wave's last reads of this batch; its seeds are
+    // written after the barrier of this batch's last iteration, and so after
+    // every wave has read this batch's.
+    fast_args()->pos[batch * (uint32_t)N + tid] = make_float4(x, y, c, 0.0f);
   }
   if (g.do_draw) {
     count_drawn(g.counter, drawn);

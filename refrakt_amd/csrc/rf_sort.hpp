@@ -53,6 +53,35 @@ struct SortArgs {
 };
 
 #ifndef __HIPCC_RTC__
+// Workgroups of a draw of n_batches batches of n_iter iterations each, when a
+// flush takes `stage` iterations and `resident` workgroups run at once.  A
+// flush of any size reserves its runs with one atomic per bucket on the same
+// few cache lines (about 9 ns per workgroup and line, one after another), so
+// draws of few iterations are bound by their flushes, and a workgroup takes up
+// to four batches if that makes the stages fuller.  One draw of 4 Mi
+// particles, one batch against this rule (us):
+//   iterations              1          2          3          5          10
+//   8 buckets (2048^2)   164 / 116  180 / 154  206 / 198  275 / 279* 493 / 502*
+//   32 buckets (4096^2)  197 / 141  214 / 180  229 / 214  294 / 289* 466 / 472*
+//   64 buckets           277 / 171  308 / 205  334 / 254  384 / 326  605 / 500
+// Where more than half a stage is filled anyway, up to 32 buckets (one line of
+// cursors) hide the flushes behind the other workgroups' iterations and the
+// coarser grid costs more than it saves (*: not done).  More batches than four
+// fill no stage better than 7/8 of what four do, and a grid below the resident
+// workgroups leaves compute units idle: 262144 particles, 5 iterations, 68 us
+// with one batch, 79 with three.
+inline uint32_t sort_grid(uint32_t n_batches, uint32_t n_iter, uint32_t n_buckets, uint32_t stage,
+                          uint32_t resident) {
+  if (n_iter == 0 || (n_buckets <= 32 && n_iter > stage / 2)) return n_batches;
+  auto flushes = [&](uint64_t m) { return (m * n_iter + stage - 1) / stage; };
+  uint64_t per = 1;
+  for (uint64_t m = 2; m <= 4; ++m)
+    if (flushes(m) * per < flushes(per) * m) per = m;
+  const uint32_t grid = (uint32_t)((n_batches + per - 1) / per);
+  const uint32_t least = n_batches < resident ? n_batches : resident;
+  return grid > least ? grid : least;
+}
+
 // Clears the cursors and, when counter is given, counter_words words of it.
 hipError_t launch_sort_reset(const SortArgs& a, hipStream_t s, unsigned long long* counter = nullptr,
                              uint32_t counter_words = 0);

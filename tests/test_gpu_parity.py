@@ -160,6 +160,40 @@ def test_fast_sort_long_draw_runs_as_subdraws(rf, orc, gpu_available):
     assert fh.sort_overflow() == 0.0
 
 
+@pytest.mark.parametrize("waves,batches,passes,W,H,programs", [
+    (8, 4101, 1, 192, 160, True),      # four batches a workgroup, the last ones three: half a stage
+    (8, 1027, 1, 192, 160, True),      # fewer batches than two per resident workgroup
+    (8, 2053, 3, 192, 160, False),     # two batches, six of eight iterations; interpreted
+    (8, 2051, 5, 5120, 4097, True),    # 41 buckets: stages that end inside a batch
+    (4, 4099, 3, 192, 160, True),      # stages of sixteen iterations
+])
+def test_fast_sort_stage_over_batches(rf, orc, gpu_available, waves, batches, passes, W, H, programs):
+    """A sort draw of few passes fills a workgroup's stage over several batches
+    and seeds their streams together: positions, bins and counts as the replica,
+    which knows no workgroups."""
+    P, seed = 64 * waves * batches, 31
+    fl = _linear_flame(rf, 41, W=W, H=H)
+    print(f"stage over batches: waves={waves} batches={batches} passes={passes} {W}x{H}", flush=True)
+    ctx = _ctx(rf, P, 1, rf.RF_ENGINE_FAST, hist_mode=rf.RF_HIST_SORT, seed=seed, waves=waves)
+    ctx.set_flame_programs(programs)
+    fh = ctx.flame(fl)
+    hist = ctx.histogram(W, H)
+    fh.warmup(0)
+    drawn = fh.draw_to_bins(hist, passes)
+    g_hist = hist.download()
+    g_pos = fh.particles()
+    fc = orc.flame_to_c(fl)
+    ss = orc.screen_affine(fl, W, H)
+    perms = ctx.fast_perms(waves)
+    pos = np.zeros((P, 4), np.float32)
+    orc.fast_run(fc, P, P, waves, perms, seed, 0, 1, True, False, W, H, ss, pos)
+    hits = np.zeros((H, W), np.uint32)
+    o_drawn = orc.fast_run(fc, P, P, waves, perms, seed, 1, passes, False, True, W, H, ss, pos, None, hits)
+    assert drawn == o_drawn > 0
+    assert np.array_equal(g_pos.view(np.uint32), pos.view(np.uint32))
+    assert np.array_equal(g_hist[..., 3].astype(np.uint32), hits)
+
+
 # ------------------------------------------------- non-finite particle policy
 def _nan_xform(rf, kind):
     """An xform whose output is never finite: a NaN variation weight, or an
