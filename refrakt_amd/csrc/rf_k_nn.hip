@@ -16,11 +16,22 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float bf2f(bf16 h) { return __uint_as_float((uint32_t)h << 16); }
 
-// Round to nearest even; NaN stays NaN.
-__device__ __forceinline__ bf16 f2bf(float f) {
-  const uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (bf16)0x7fc0u;
-  return (bf16)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+// Round to nearest even; NaN stays NaN.  (v_cvt_pk_bf16_f32; the same bits as
+// rounding by integer arithmetic for every value but NaN.)
+typedef float float2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t f2bf2(float lo, float hi) {
+  const float2_t v = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+}
+__device__ __forceinline__ bf16 f2bf(float f) { return (bf16)f2bf2(f, 0.0f); }
+
+// Workgroup barrier that orders LDS only: __syncthreads() would also wait for
+// every global load and store under way.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // ------------------------------------------------------------ convolution
@@ -181,6 +192,9 @@ __device__ __forceinline__ uint32_t relu_keep(uint32_t v, uint32_t y) {
   const uint32_t lo = bf_lo(y) > 0.0f ? 0xffffu : 0u, hi = bf_hi(y) > 0.0f ? 0xffff0000u : 0u;
   return v & (lo | hi);
 }
+__device__ __forceinline__ uint2 relu_keep(const uint2& v, const uint2& y) {
+  return make_uint2(relu_keep(v.x, y.x), relu_keep(v.y, y.y));
+}
 __device__ __forceinline__ uint4 relu_keep(const uint4& v, const uint4& y) {
   return make_uint4(relu_keep(v.x, y.x), relu_keep(v.y, y.y), relu_keep(v.z, y.z), relu_keep(v.w, y.w));
 }
@@ -269,7 +283,7 @@ __device__ __forceinline__ void conv_store_lds(const float4_t (&acc)[RW][4][NT],
           uint32_t r[4];
 #pragma unroll
           for (int k = 0; k < 4; ++k)
-            r[k] = (uint32_t)f2bf(0.25f * sum[2 * k]) | ((uint32_t)f2bf(0.25f * sum[2 * k + 1]) << 16);
+            r[k] = f2bf2(0.25f * sum[2 * k], 0.25f * sum[2 * k + 1]);
           *reinterpret_cast<uint4*>(pool.p + ((size_t)(n * (H >> 1) + yo) * (W >> 1) + xo) * pool.cs + pool.co +
                                     co0 + 8 * piece) = make_uint4(r[0], r[1], r[2], r[3]);
         }
@@ -408,6 +422,259 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RW == 2 ? (
   }
 }
 
+// Persistent convolution of the narrow layers (Cin 16 or 32, at most 32
+// output channels per block), which memory bounds (a 32 -> 32 layer at 2048^2
+// moves 537 MB for 77 GFLOP).  A workgroup of 4 waves keeps its 9 x Cin x
+// 16 NT weights in registers and walks tiles of 8 rows x 64 pixels, first
+// tile blockIdx / nbz, step gridDim / nbz; the next tile's input (halo
+// included) is loaded into registers while the MFMAs of the current one run,
+// so loads are in flight all the time, and only the input goes through LDS.
+// The weights are the A operand: a lane's four (NT = 1) or eight consecutive
+// output channels of one pixel leave as one store, without LDS; for NT = 2
+// fragment t's row m is channel 8 (m / 4) + 4 t + m % 4, which makes the
+// eight consecutive.
+//
+// Every output sums 16-channel products in k_conv3x3_lds<NT, 16, 2>'s order
+// (input channel halves, then tap columns, then tap rows) and has its bits:
+// v_mfma_f32_16x16x32_bf16 adds its first sixteen products, then the others,
+// exactly as two chained 16x16x16 instructions do, so two successive taps
+// share one instruction at twice the rate.  Lanes 0..31 hold the first tap's
+// eight channels each, lanes 32..63 the second's: in a pair of successive
+// taps the second lies one of three distances behind the first, and with one
+// base address for each all fragment offsets are constants.
+//
+// One tile a workgroup (k_conv3x3_lds) exposes each tile's first load and its
+// store: at 2048^2 the 16 -> 32, 32 -> 32 and 32 -> 16 layers took 132, 206
+// and 116 us there and take 98, 144 and 98 us here (3.7 to 4.1 TB/s).
+constexpr int CF_PIX = ct_in_pix(2);
+
+template <int NT>
+constexpr int conv_few_waves() { return NT == 2 ? 2 : 3; }  // workgroups per CU, by registers
+
+template <int CIN, int NT, bool RELU>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_few_waves<NT>()))) void k_conv3x3_few(
+    View in, const bf16* __restrict__ w, const float* __restrict__ bias, View out, int H, int W, int Cout,
+    ConvFuse fz, int nbx, int nbz, int n_tiles) {
+  constexpr int PQ = CIN / 8, PS = CIN + 8, PW = CT_W + 2;
+  constexpr int IN_Q = CF_PIX * PQ, IN_PER = (IN_Q + 255) / 256;
+  constexpr int NP = 9 * CIN / 16, NQ = NP / 2;  // products of 16 channels and pairs of them per output
+  __shared__ __attribute__((aligned(16))) bf16 s_in[CF_PIX * PS];
+  __shared__ __attribute__((aligned(16))) float s_bias[16 * NT];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i = lane & 15, kq = lane >> 4;
+  const int nrb = (H + 7) / 8;
+  const int bz = blockIdx.x % nbz, step = gridDim.x / nbz;
+  const int co0 = bz * 16 * NT;
+  const bool hi = kq >= 2;
+  // product p: channel half, tap column, tap row
+  auto half = [](int p) { return p / 9; };
+  auto tap = [](int p) { return (p % 3) * 3 + (p % 9) / 3; };
+  auto at = [&](int p) { return ((p % 3) * PW + (p % 9) / 3) * PS + 16 * half(p); };
+
+  bf16x8_t wf[NQ][NT];
+  short4_t wl[NT];  // the odd product's weights
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int co = co0 + (NT == 2 ? 8 * (i >> 2) + 4 * t + (i & 3) : i);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const bf16* const wa = w + ((size_t)tap(2 * q) * Cout + co) * CIN + 16 * half(2 * q);
+      const bf16* const wb = w + ((size_t)tap(2 * q + 1) * Cout + co) * CIN + 16 * half(2 * q + 1);
+      wf[q][t] = *reinterpret_cast<const bf16x8_t*>((hi ? wb : wa) + 8 * (kq & 1));
+    }
+    if constexpr (NP % 2)
+      wl[t] = *reinterpret_cast<const short4_t*>(w + ((size_t)tap(NP - 1) * Cout + co) * CIN + 4 * kq);
+  }
+  if (tid < 16 * NT) s_bias[tid] = bias ? bias[co0 + tid] : 0.0f;
+  // four outputs of one pixel: bias, ReLU, bf16
+  auto out4 = [&](const float4_t& a, const float4_t& b) {
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = a[e] + b[e];
+      if (RELU) v[e] = fmaxf(v[e], 0.0f);
+    }
+    return make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
+  };
+  uint4 st[IN_PER];
+  auto load = [&](int tile) {
+    const int bx = tile % nbx, by = tile / nbx;
+    const int n = by / nrb, y0 = (by % nrb) * 8, x0 = bx * CT_W;
+    // the patch's first pixel (outside the image for a tile at its edge) and
+    // the pieces' offsets from it (conv3x3 takes this kernel if 31 bits hold
+    // ten rows)
+    const bf16* const src = in.p + ((ptrdiff_t)(n * H + y0 - 1) * W + (x0 - 1)) * in.cs + in.co;
+    int q0 = tid;
+    asm volatile("" : "+v"(q0));  // the pieces' places computed here, not held over the tiles
+    if (y0 > 0 && y0 + 9 <= H && x0 > 0 && x0 + CT_W + 1 <= W) {  // workgroup-uniform: no pixel outside
+#pragma unroll
+      for (int k = 0; k < IN_PER; ++k) {
+        // (the last round's spare threads read the patch's last piece again)
+        const int q = k + 1 < IN_PER ? q0 + 256 * k : min(q0 + 256 * k, IN_Q - 1);
+        const int piece = q % PQ, pix = q / PQ;
+        st[k] = *reinterpret_cast<const uint4*>(src + (uint32_t)((pix / PW * W + pix % PW) * in.cs + 8 * piece));
+      }
+      return;
+    }
+#pragma unroll
+    for (int k = 0; k < IN_PER; ++k) {
+      const int q = q0 + 256 * k;
+      const int piece = q % PQ, pix = q / PQ;
+      const int yy = y0 + pix / PW - 1, gx = x0 + pix % PW - 1;
+      uint4 v = make_uint4(0u, 0u, 0u, 0u);
+      if (q < IN_Q && yy >= 0 && yy < H && gx >= 0 && gx < W)
+        v = *reinterpret_cast<const uint4*>(src + (uint32_t)((pix / PW * W + pix % PW) * in.cs + 8 * piece));
+      st[k] = v;
+    }
+  };
+  int tile = blockIdx.x / nbz;
+  if (tile < n_tiles) load(tile);
+  for (; tile < n_tiles; tile += step) {  // workgroup-uniform
+    int q0 = tid;
+    asm volatile("" : "+v"(q0));  // as in load
+    lds_barrier();                // the last tile's fragment reads are done
+#pragma unroll
+    for (int k = 0; k < IN_PER; ++k) {
+      const int q = q0 + 256 * k;
+      if (q < IN_Q) *reinterpret_cast<uint4*>(s_in + (q / PQ) * PS + 8 * (q % PQ)) = st[k];
+    }
+    lds_barrier();
+    if (tile + step < n_tiles) load(tile + step);
+    const int bx = tile % nbx, by = tile / nbx;
+    const int n = by / nrb, y0 = (by % nrb) * 8 + 2 * wave, x0 = bx * CT_W;
+    // a pixel's place in a view: that of the wave's first pixel, and an offset
+    auto row = [&](const View& v) { return v.p + ((size_t)(n * H + y0) * W + x0) * v.cs + v.co; };
+    uint2 xv[2] = {make_uint2(0u, 0u), make_uint2(0u, 0u)};  // the residual's input, under way during the MFMAs
+    if (NT == 1 && fz.y) {
+#pragma unroll
+      for (int rr = 0; rr < 2; ++rr)
+        if (y0 + rr < H && x0 + lane < W)
+          xv[rr] = *reinterpret_cast<const uint2*>(row(fz.res) + (ptrdiff_t)rr * W * fz.res.cs + lane * fz.res.cs);
+    }
+
+    float4_t acc[2][4][NT];
+#pragma unroll
+    for (int rr = 0; rr < 2; ++rr)
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[rr][f][t] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const bf16* const base = s_in + (2 * wave * PW + i) * PS + 8 * (kq & 1);
+    const bf16* const base_r = base + (hi ? PW * PS : 0);                  // the next tap row
+    const bf16* const base_s = base + (hi ? PS - 2 * PW * PS : 0);         // the next tap column's first row
+    const bf16* const base_h = base + (hi ? 16 - (2 * PW + 2) * PS : 0);   // the next channel half's first tap
+    // group g = (pair q, output row rr): its four fragments are read while
+    // the group before runs
+    auto frags = [&](int g, bf16x8_t (&b)[4]) {
+      const int q = g / 2, d = at(2 * q + 1) - at(2 * q);
+      const bf16* const bp = (d == PW * PS ? base_r : d == PS - 2 * PW * PS ? base_s : base_h) + at(2 * q) + (g % 2) * PW * PS;
+#pragma unroll
+      for (int f = 0; f < 4; ++f) b[f] = *reinterpret_cast<const bf16x8_t*>(bp + 16 * f * PS);
+    };
+    bf16x8_t b[2][4];
+    frags(0, b[0]);
+#pragma unroll
+    for (int g = 0; g < 2 * NQ; ++g) {
+      if (g + 1 < 2 * NQ) frags(g + 1, b[(g + 1) & 1]);
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          acc[g % 2][f][t] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[g / 2][t], b[g & 1][f], acc[g % 2][f][t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);  // no fragments read further ahead: they would spill
+    }
+    if constexpr (NP % 2) {
+      const bf16* const bp = s_in + (2 * wave * PW + i) * PS + 4 * kq + at(NP - 1);
+#pragma unroll
+      for (int rr = 0; rr < 2; ++rr)
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+          const short4_t bl = *reinterpret_cast<const short4_t*>(bp + (rr * PW + 16 * f) * PS);
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+            acc[rr][f][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wl[t], bl, acc[rr][f][t], 0, 0, 0);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+
+    float4_t bv[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) bv[t] = *reinterpret_cast<const float4_t*>(s_bias + 4 * NT * kq + 4 * t);
+    if (NT == 1 && fz.y) {  // workgroup-uniform: the residual output replaces `out`
+      // channels 0..3 are lanes 0..15's; lane l takes pixel l of the row
+#pragma unroll
+      for (int rr = 0; rr < 2; ++rr) {
+        uint2 o = make_uint2(0u, 0u);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+          const uint2 v = out4(acc[rr][f][0], bv[0]);
+          const uint32_t vx = (uint32_t)__shfl((int)v.x, i), vy = (uint32_t)__shfl((int)v.y, i);
+          if (kq == f) o = make_uint2(vx, vy);
+        }
+        if (y0 + rr < H && x0 + lane < W)
+          *reinterpret_cast<float4*>(fz.y + ((size_t)(n * H + y0 + rr) * W + x0 + lane) * 4) =
+              make_float4(bf_lo(xv[rr].x) + bf_lo(o.x), bf_hi(xv[rr].x) + bf_hi(o.x), bf_lo(xv[rr].y) + bf_lo(o.y),
+                          bf_hi(xv[rr].y) + bf_hi(o.y));
+      }
+      continue;
+    }
+    typedef typename std::conditional<NT == 2, uint4, uint2>::type Out;
+    // (uniform) row and fragment, this lane's pixel and channels in it
+    const bf16* const mrow = row(fz.mask);
+    bf16* const orow = row(out);
+    const uint32_t mlane = (uint32_t)(i * fz.mask.cs + co0 + 4 * NT * kq), olane = (uint32_t)(i * out.cs + co0 + 4 * NT * kq);
+    auto inside = [&](int f, int rr) { return y0 + rr < H && x0 + 16 * f + i < W; };
+    // the mask of this fragment and, where registers allow, the next
+    constexpr int MD = conv_few_waves<NT>() == 2 ? 2 : 1;
+    Out m[MD][2];
+    auto mask = [&](int f) {
+#pragma unroll
+      for (int rr = 0; rr < 2; ++rr)
+        if (inside(f, rr))
+          m[f % MD][rr] = *reinterpret_cast<const Out*>(mrow + (ptrdiff_t)(rr * W + 16 * f) * fz.mask.cs + mlane);
+    };
+    if (MD == 2 && fz.mask.p) mask(0);  // workgroup-uniform
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (fz.mask.p && f + MD - 1 < 4) mask(f + MD - 1);
+      Out o[2];
+#pragma unroll
+      for (int rr = 0; rr < 2; ++rr) {
+        if constexpr (NT == 2) {
+          const uint2 a = out4(acc[rr][f][0], bv[0]), c = out4(acc[rr][f][1], bv[1]);
+          o[rr] = make_uint4(a.x, a.y, c.x, c.y);
+        } else {
+          o[rr] = out4(acc[rr][f][0], bv[0]);
+        }
+        if (!inside(f, rr)) continue;
+        Out v = o[rr];
+        if (fz.mask.p) v = relu_keep(v, m[f % MD][rr]);
+        *reinterpret_cast<Out*>(orow + (ptrdiff_t)(rr * W + 16 * f) * out.cs + olane) = v;
+      }
+      if (fz.pool.p) {  // workgroup-uniform: the 2x2 averages, summed in k_avgpool2_v8's order
+        const uint32_t* const r0 = reinterpret_cast<const uint32_t*>(&o[0]);
+        const uint32_t* const r1 = reinterpret_cast<const uint32_t*>(&o[1]);
+        Out pv;
+        uint32_t* const r = reinterpret_cast<uint32_t*>(&pv);
+#pragma unroll
+        for (int h = 0; h < 2 * NT; ++h) {
+          // the neighbouring pixel's values, from the neighbouring lane
+          const uint32_t a1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)r0[h], 0xB1, 0xf, 0xf, true);
+          const uint32_t b1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)r1[h], 0xB1, 0xf, 0xf, true);
+          const float lo = (((0.0f + bf_lo(r0[h])) + bf_lo(a1)) + bf_lo(r1[h])) + bf_lo(b1);
+          const float hi2 = (((0.0f + bf_hi(r0[h])) + bf_hi(a1)) + bf_hi(r1[h])) + bf_hi(b1);
+          r[h] = f2bf2(0.25f * lo, 0.25f * hi2);
+        }
+        const int yo = y0 >> 1, xo = (x0 + 16 * f + i) >> 1;
+        if ((i & 1) == 0 && yo < (H >> 1) && xo < (W >> 1))
+          *reinterpret_cast<Out*>(fz.pool.p + ((size_t)(n * (H >> 1) + yo) * (W >> 1) + xo) * fz.pool.cs + fz.pool.co +
+                                  co0 + 4 * NT * kq) = pv;
+      }
+    }
+  }
+}
 
 // Weight gradient on MFMA: an implicit GEMM per tap (r, s) with M = output
 // channels, N = input channels, K = pixels:
@@ -770,7 +1037,7 @@ __global__ void k_avgpool2_v8(View in, View out, int N, int H, int W, int C) {
   uint32_t r[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k)
-    r[k] = (uint32_t)f2bf(0.25f * s[2 * k]) | ((uint32_t)f2bf(0.25f * s[2 * k + 1]) << 16);
+    r[k] = f2bf2(0.25f * s[2 * k], 0.25f * s[2 * k + 1]);
   *reinterpret_cast<uint4*>(out.p + po * out.cs + out.co + 8 * g) = make_uint4(r[0], r[1], r[2], r[3]);
 }
 
@@ -828,7 +1095,7 @@ __global__ void k_upsample2_bwd_v8(View dout, View din, View y, int N, int H, in
     }
   uint32_t r[4];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) r[k] = (uint32_t)f2bf(s[2 * k]) | ((uint32_t)f2bf(s[2 * k + 1]) << 16);
+  for (int k = 0; k < 4; ++k) r[k] = f2bf2(s[2 * k], s[2 * k + 1]);
   *reinterpret_cast<uint4*>(din.p + p * din.cs + din.co + 8 * g) =
       relu_keep(make_uint4(r[0], r[1], r[2], r[3]), *reinterpret_cast<const uint4*>(y.p + p * y.cs + y.co + 8 * g));
 }
@@ -935,8 +1202,8 @@ __global__ void k_log_density_v(const float4* __restrict__ hist, uint4* __restri
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= npix) return;
   const float4 h = hist[p];
-  const uint32_t lo = (uint32_t)f2bf(log10f(1.0f + h.x * scale)) | ((uint32_t)f2bf(log10f(1.0f + h.y * scale)) << 16);
-  const uint32_t hi = (uint32_t)f2bf(log10f(1.0f + h.z * scale)) | ((uint32_t)f2bf(log10f(1.0f + h.w * scale)) << 16);
+  const uint32_t lo = f2bf2(log10f(1.0f + h.x * scale), log10f(1.0f + h.y * scale));
+  const uint32_t hi = f2bf2(log10f(1.0f + h.z * scale), log10f(1.0f + h.w * scale));
   const uint32_t nl = (uint32_t)f2bf(log10f(1.0f + scale));
   out[2 * (size_t)p] = make_uint4(lo, hi, nl, 0u);
   out[2 * (size_t)p + 1] = make_uint4(0u, 0u, 0u, 0u);
@@ -977,12 +1244,11 @@ hipError_t conv3x3(View in, const bf16* w, const float* bias, View out, int N, i
     // instruction) pay off where each staged step feeds 64 output channels or
     // the input has 64 channels or more: the 96 -> 32 decoder layer at full
     // resolution takes 320 us at 2048^2 with them, 389 us without.  The
-    // narrow layers with 16 or 32 input channels keep the smaller K = 16
+    // narrow layers with 16, 32 or 48 input channels keep the smaller K = 16
     // tiles, whose LDS and registers fit three workgroups per CU instead of
-    // two (K = 32 there measured 203 -> 205 and 167 -> 175 us for the 32 ->
-    // 32 layers, 118 -> 144 us for the 32 -> 16 output layer).  The narrow
-    // layers give each wave two rows (RW = 2), whose shared input rows halve
-    // the B and cut the A fragment reads per output by a third.
+    // two.  The narrow layers give each wave two rows (RW = 2), whose shared
+    // input rows halve the B and cut the A fragment reads per output by a
+    // third.
     const bool k32 = Cin % 32 == 0 && (nt == 4 || Cin >= 64);
     const int rw = nt <= 2 ? 2 : 1;
     const int nbx = (W + CT_W - 1) / CT_W, nbz = Cout / (16 * nt);
@@ -1004,6 +1270,30 @@ hipError_t conv3x3(View in, const bf16* w, const float* bias, View out, int N, i
     ConvFuse fz = fuse;
     if (!fuse_pool) fz.pool = View{nullptr, 0, 0};
     if (!fuse_res) { fz.res = View{nullptr, 0, 0}; fz.y = nullptr; }
+    // Weights that fit the registers (Cin 16 or 32) and no part that needs
+    // another path: the persistent kernel, faster at every size (32 -> 32,
+    // with the call's 17 us: 2048^2 223 -> 162 us, 8 x 256^2 43 -> 33, 517 x
+    // 333 28 -> 23; 16 -> 32 at 64^2 20.6 -> 17.3).
+    const bool few = (long long)10 * W * in.cs < (1ll << 31) && !k32 && nt <= 2 && Cin <= 32 && !Cup && vec_out && (!pool.p || fuse_pool) && (!fuse.y || fuse_res);
+    if (few) {
+      int dev = 0, cus = 0;
+      hipError_t e = hipGetDevice(&dev);
+      if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+      if (e != hipSuccess) return e;
+#define RF_CONV_FEW(CIN_, NT_, RELU_)                                                                             \
+  hipLaunchKernelGGL((k_conv3x3_few<CIN_, NT_, RELU_>),                                                           \
+                     dim3((unsigned)(std::min(n_tiles / nbz, std::max(1, conv_few_waves<NT_>() * cus / nbz)) * nbz)), \
+                     dim3(256), 0, s, in, w, bias, out, H, W, Cout, fz, nbx, nbz, n_tiles / nbz)
+      if (relu) {
+        if (Cin == 32) { if (nt == 2) RF_CONV_FEW(32, 2, true); else RF_CONV_FEW(32, 1, true); }
+        else { if (nt == 2) RF_CONV_FEW(16, 2, true); else RF_CONV_FEW(16, 1, true); }
+      } else {
+        if (Cin == 32) { if (nt == 2) RF_CONV_FEW(32, 2, false); else RF_CONV_FEW(32, 1, false); }
+        else { if (nt == 2) RF_CONV_FEW(16, 2, false); else RF_CONV_FEW(16, 1, false); }
+      }
+#undef RF_CONV_FEW
+      return hipGetLastError();
+    }
 #define RF_CONV_LDS(NT_, KC_, RW_)                                                                            \
   hipLaunchKernelGGL((k_conv3x3_lds<NT_, KC_, RW_>), dim3((unsigned)n_tiles), dim3(256), 0, s, in, w, bias, out, H, \
                      W, Cin, Cout, relu, vec_out, fz, nbx, nbz, n_tiles)

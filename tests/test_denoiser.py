@@ -128,6 +128,38 @@ def test_conv3x3_gradients_match_torch(rf, gpu_available, Cin, Cout, W, H):
     assert (err <= 2.0 ** -8 * ref_dx.abs() + 1e-4).all(), float(err.max())
 
 
+# One pixel, tiles of exactly 8 rows x 64 pixels and one more of each, images
+# that end inside a tile, more tiles than workgroups, three channel blocks.
+@pytest.mark.parametrize("Cin,Cout,N,H,W", [(16, 32, 1, 1, 1), (32, 32, 1, 8, 64), (32, 16, 2, 9, 65),
+                                            (16, 16, 1, 17, 63), (32, 96, 2, 25, 130), (32, 32, 3, 100, 1000),
+                                            (16, 32, 5, 50, 900), (32, 16, 5, 70, 1100)])
+@pytest.mark.parametrize("relu", [0, 1])
+def test_conv3x3_narrow_layers_have_the_general_kernels_bits(rf, gpu_available, Cin, Cout, N, H, W, relu):
+    """The persistent kernel of the narrow layers sums in the general kernel's
+    order: the same bits.  (An output 8 bytes off a 16-byte run takes the
+    general kernel.)"""
+    import torch
+    import torch.nn.functional as F
+    print(f"narrow conv {Cin}->{Cout} {N}x{H}x{W} relu={relu}", flush=True)
+    ctx = rf.Context(1 << 12, 1, 16)
+    g = torch.Generator().manual_seed(Cin + 3 * Cout + H)
+    x = _bf16(torch.randn(N, H, W, Cin + 8, generator=g)).cuda()
+    w = _bf16(0.1 * torch.randn(3, 3, Cout, Cin, generator=g)).cuda()
+    b = torch.randn(Cout, generator=g).cuda()
+    out = {}
+    for cs, co in ((Cout + 16, 8), (Cout + 8, 4)):
+        o = torch.zeros(N, H, W, cs, dtype=torch.bfloat16, device="cuda")
+        ctx.check(ctx.L.rf_nn_conv3x3(ctx.h, x.data_ptr(), Cin + 8, 8, w.data_ptr(), b.data_ptr(), o.data_ptr(), cs, co,
+                                      N, H, W, Cin, Cout, relu))
+        assert not o[..., :co].any() and not o[..., co + Cout:].any()
+        out[co] = o[..., co:co + Cout].cpu()
+    assert torch.equal(out[8].view(torch.int16), out[4].view(torch.int16))
+    ref = F.conv2d(x[..., 8:].float().cpu().permute(0, 3, 1, 2), w.float().cpu().permute(2, 3, 0, 1), b.cpu(), padding=1)
+    ref = (torch.relu(ref) if relu else ref).permute(0, 2, 3, 1)
+    # half a bf16 ulp, and fp32 sums of 9 Cin products
+    assert ((out[8].float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4).all()
+
+
 # One row, two rows, a strip of exactly 64 pixels and one more, runs that
 # start inside a strip, several images: every channel tile.
 @pytest.mark.parametrize("Cin,Cout,N,H,W", [(64, 64, 1, 1, 64), (32, 32, 2, 2, 65), (16, 32, 1, 3, 1),
