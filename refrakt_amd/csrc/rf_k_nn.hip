@@ -99,15 +99,17 @@ __device__ __forceinline__ float bf_hi(uint32_t u) { return __uint_as_float(u & 
 // 16*NT output channels.  Per KC-channel step of Cin (KC = 32 with gfx950's
 // v_mfma_f32_16x16x32_bf16 for the wide layers, else 16 with the 16x16x16 form)
 // it stages the (4 RW + 2) x (CT_W + 2) input patch (zero halo) and the
-// step's 3x3 x 16*NT x KC weights in LDS, KC + 8 channels per pixel / weight
-// row (the pad spreads 16 consecutive rows over distinct banks and keeps
-// 16-byte stores aligned); every A fragment then feeds NT MFMAs and every B
+// step's 3x3 x 16*NT x KC weights in LDS (strides: ConvStage); every A fragment then feeds NT MFMAs and every B
 // fragment four per output row it reaches.  With RW = 2 a wave's four input
 // rows serve six (row, tap row) pairs, so each A fragment read from LDS feeds
 // up to 2 NT MFMAs: the narrow layers, whose NT is small, read a third fewer
 // A fragments and half the B fragments per output.  The next step's operands
-// are loaded into registers while the MFMAs of the current one run.  Needs 16-byte aligned channel runs (Cin,
-// channel strides and offsets multiples of 8).
+// are loaded into registers while the MFMAs of the current one run.  Needs
+// 16-byte aligned channel runs (Cin, channel strides and offsets multiples of
+// 8).  At 1024^2 the 192 -> 64 layer takes 269 us and the 384 -> 128 layer at
+// 512^2 207 us (860 and 1120 TFLOP/s, the latter near a large matrix
+// product's rate on this card); with places and bounds recomputed every step,
+// LDS rows of 80 bytes and fragments read as they were needed 287 and 232.
 // Operand layouts (wave64, i = lane % 16, kq = lane / 16): 16x16x16 lane
 // holds A[i][4 kq + e], B[4 kq + e][i] (e < 4); 16x16x32 lane holds
 // A[i][8 kq + e], B[8 kq + e][i] (e < 8); both give D[4 kq + e][i] (e < 4).
@@ -119,7 +121,17 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
 template <int NT, int KC, int RW>
 struct ConvStage {
-  static constexpr int PS = KC + 8;             // LDS row stride (bf16)
+  // LDS strides (bf16) of a pixel and of a weight row.  A 16-byte LDS read of
+  // a wave takes four cycles when each of its groups of 16 lanes (lanes 0..3,
+  // 12..15 and 20..27, and so on) covers all banks, else eight or more: the
+  // 16 lanes of a fragment and the four 16-byte pieces of their rows do so at
+  // 96 bytes a row, or at 64 with the pieces swizzled (w_piece) where rows
+  // start at multiples of 16.  80 bytes, the smallest odd multiple of 16,
+  // take eight.
+  static constexpr int PS = KC == 32 ? 48 : 24, WS = KC == 32 ? 32 : 24;
+  static __device__ __forceinline__ int w_piece(int row, int piece) {
+    return KC == 32 ? piece ^ (-(row >> 2) & 3) : piece;
+  }
   static constexpr int PQ = KC / 8;             // 16-byte pieces per pixel / weight row
   static constexpr int IN_Q = ct_in_pix(RW) * PQ;
   static constexpr int W_Q = 9 * 16 * NT * PQ;
@@ -127,44 +139,79 @@ struct ConvStage {
   static constexpr int W_PER = (W_Q + 255) / 256;
   uint4 vin[IN_PER];
   uint4 vw[W_PER];
+  uint32_t place[IN_PER];  // see conv_places
 };
 
-// Channels [0, Cup) come from the half-resolution `up` (nearest-neighbour
-// upsampling read in place), the rest from `in`; a KC step never straddles
-// the two (Cup is a multiple of 32).
-template <int NT, int KC, int RW>
-__device__ __forceinline__ void conv_load(ConvStage<NT, KC, RW>& st, const View& in, const View& up, int Cup,
-                                          const bf16* __restrict__ w, int n, int y0, int x0, int co0, int c0, int H,
-                                          int W, int Cin, int Cout) {
+// Buffer loads: an offset at or beyond BUF_RANGE reads zeros, which is how the
+// halo outside the image is filled without branches.
+constexpr uint32_t BUF_RANGE = 0x7fffffffu, BUF_NONE = 0x80000000u;
+typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_at(const bf16* p) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(p), 0, (int)BUF_RANGE, 0x00020000);
+}
+__device__ __forceinline__ uint4 buf_load(__amdgpu_buffer_rsrc_t r, uint32_t lane, uint32_t uniform) {
+  const uint4_t v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)lane, (int)uniform, 0);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+// This thread's input pieces, in 16-byte units from the patch's first pixel
+// (far) or in bytes (BUF_NONE either way: outside the image), in `in`, or
+// (up = 1) in the half-resolution `up`.  They are computed once per view and
+// tile: recomputed for every channel step, places and bounds were 300 vector
+// instructions a wave and step beside 144 MFMAs.
+template <int NT, int KC, int RW, bool FAR>
+__device__ __forceinline__ void conv_places(ConvStage<NT, KC, RW>& st, int cs, int up, int y0, int x0, int H, int W) {
   using S = ConvStage<NT, KC, RW>;
-  const int tid = threadIdx.x;
-  const bool from_up = c0 < Cup;  // workgroup-uniform
 #pragma unroll
   for (int k = 0; k < S::IN_PER; ++k) {
-    const int q = tid + 256 * k;
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (q < S::IN_Q) {
-      const int piece = q % S::PQ, pix = q / S::PQ;
-      const int yy = y0 + pix / (CT_W + 2) - 1, gx = x0 + pix % (CT_W + 2) - 1;
-      if (yy >= 0 && yy < H && gx >= 0 && gx < W) {
-        const bf16* src = from_up ? up.p + ((size_t)(n * (H >> 1) + (yy >> 1)) * (W >> 1) + (gx >> 1)) * up.cs +
-                                        up.co + c0 + 8 * piece
-                                  : in.p + ((size_t)(n * H + yy) * W + gx) * in.cs + in.co + (c0 - Cup) + 8 * piece;
-        v = *reinterpret_cast<const uint4*>(src);
-      }
-    }
-    st.vin[k] = v;
+    const int q = (int)threadIdx.x + 256 * k;
+    const int piece = q % S::PQ, pix = q / S::PQ;
+    const int yy = y0 + pix / (CT_W + 2) - 1, gx = x0 + pix % (CT_W + 2) - 1;
+    // (from the patch's row y0 - 1, column x0 - 1, halved with rounding down for `up`)
+    const uint32_t dy = (uint32_t)((yy >> up) - ((y0 - 1) >> up)), dx = (uint32_t)((gx >> up) - ((x0 - 1) >> up));
+    const bool in_image = q < S::IN_Q && yy >= 0 && yy < H && gx >= 0 && gx < W;
+    const uint32_t unit = (dy * (uint32_t)(W >> up) + dx) * (uint32_t)(cs / 8) + (uint32_t)piece;
+    st.place[k] = in_image ? (FAR ? unit : 16u * unit) : BUF_NONE;
   }
+}
+
+// The loads of one channel step.  Channels [0, Cup) come from the
+// half-resolution `up` (nearest-neighbour upsampling read in place), the rest
+// from `in`; a KC step never straddles the two (Cup is a multiple of 32).
+// `src` is the patch's first pixel in the step's view, c its first channel.
+template <int NT, int KC, int RW, bool FAR>
+__device__ __forceinline__ void conv_load(ConvStage<NT, KC, RW>& st, const bf16* src, int c, const bf16* w, int c0,
+                                          int Cin, int Cout) {
+  using S = ConvStage<NT, KC, RW>;
+  // weight row = tap * 16 NT + output channel; a round of 256 threads covers
+  // whole taps
+  constexpr int ROWS = 256 / S::PQ, TAPS = ROWS / (16 * NT);
+  static_assert(TAPS * 16 * NT == ROWS, "whole taps");
+  const int row0 = (int)threadIdx.x / S::PQ, piece = (int)threadIdx.x % S::PQ;
+  if constexpr (FAR) {
+#pragma unroll
+    for (int k = 0; k < S::IN_PER; ++k) {
+      st.vin[k] = make_uint4(0u, 0u, 0u, 0u);
+      if (st.place[k] != BUF_NONE)
+        st.vin[k] = *reinterpret_cast<const uint4*>(src + 8 * (size_t)st.place[k] + c);
+    }
+#pragma unroll
+    for (int k = 0; k < S::W_PER; ++k) {
+      st.vw[k] = make_uint4(0u, 0u, 0u, 0u);
+      if ((int)threadIdx.x + 256 * k < S::W_Q)
+        st.vw[k] = *reinterpret_cast<const uint4*>(
+            w + ((size_t)(k * TAPS + row0 / (16 * NT)) * Cout + row0 % (16 * NT)) * Cin + c0 + 8 * piece);
+    }
+    return;
+  }
+  const __amdgpu_buffer_rsrc_t rin = buf_at(src), rw = buf_at(w);
+#pragma unroll
+  for (int k = 0; k < S::IN_PER; ++k) st.vin[k] = buf_load(rin, st.place[k], 2u * (uint32_t)c);
+  const uint32_t lane = 2u * (uint32_t)((row0 / (16 * NT) * Cout + row0 % (16 * NT)) * Cin + 8 * piece);
 #pragma unroll
   for (int k = 0; k < S::W_PER; ++k) {
-    const int q = tid + 256 * k;
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (q < S::W_Q) {
-      const int piece = q % S::PQ, row = q / S::PQ;  // row = tap * 16 * NT + output channel
-      const int tap = row / (16 * NT), co = row % (16 * NT);
-      v = *reinterpret_cast<const uint4*>(w + ((size_t)tap * Cout + co0 + co) * Cin + c0 + 8 * piece);
-    }
-    st.vw[k] = v;
+    const bool some = S::W_Q >= 256 * (k + 1) || (int)threadIdx.x + 256 * k < S::W_Q;
+    st.vw[k] = buf_load(rw, some ? lane : BUF_NONE, 2u * (uint32_t)(k * TAPS * Cout * Cin + c0));
   }
 }
 
@@ -298,9 +345,10 @@ __device__ __forceinline__ void conv_store_lds(const float4_t (&acc)[RW][4][NT],
 // the same input patch for different output channels run next to each other.
 // (A persistent variant, each workgroup walking tiles b, b + G, ... with the
 // next tile's first step prefetched during the last step of the current one,
-// measured slower: 16.8 ms against 14.0 ms per 7680x4320 inference, its
-// registers no longer fitting three waves per SIMD without spills.)
-template <int NT, int KC, int RW>
+// and outputs stored straight from the accumulators, took 10 % fewer cycles on
+// the wide layers but 1 % less time, the clock falling as the stalls went, and
+// 10 % more time on the 64 -> 32 layer.)
+template <int NT, int KC, int RW, bool FAR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RW == 2 ? (KC == 16 ? 3 : 2) : 1))) void k_conv3x3_lds(
     View in, const bf16* __restrict__ w, const float* __restrict__ bias, View out, int H, int W, int Cin, int Cout,
     int relu, int vec_out, ConvFuse fz, int nbx, int nbz, int n_tiles) {
@@ -308,12 +356,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RW == 2 ? (
   const int Cup = fz.Cup;
   using S = ConvStage<NT, KC, RW>;
   using F = ConvFrag<KC>;
-  constexpr int PS = S::PS, KE = KC / 4;  // fragment elements per lane
+  constexpr int PS = S::PS, WS = S::WS, KE = KC / 4;  // fragment elements per lane
   constexpr int OC = 16 * NT, OS = OC + 8;  // output tile: channels per pixel, LDS row stride
   constexpr int TR = 4 * RW;                // tile rows
   constexpr int IN_PIX = ct_in_pix(RW);
-  static_assert(TR * CT_W * OS <= IN_PIX * PS + 9 * 16 * NT * PS, "output tile fits the staging buffer");
-  __shared__ __attribute__((aligned(16))) bf16 s_buf[IN_PIX * PS + 9 * 16 * NT * PS];
+  static_assert(TR * CT_W * OS <= IN_PIX * PS + 9 * 16 * NT * WS, "output tile fits the staging buffer");
+  __shared__ __attribute__((aligned(16))) bf16 s_buf[IN_PIX * PS + 9 * 16 * NT * WS];
   bf16* const s_in = s_buf;
   bf16* const s_w = s_buf + IN_PIX * PS;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -324,6 +372,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RW == 2 ? (
   const int bz = tile % nbz, rest = tile / nbz;
   const int bx = rest % nbx, by = rest / nbx;
   const int n = by / nrb, y0 = (by % nrb) * TR, x0 = bx * CT_W, co0 = bz * 16 * NT;
+  // this lane's channels of a weight row (rows 16 t + i)
+  const int wk = KC == 32 ? 8 * S::w_piece(i, kq) : KE * kq;
   float4_t acc[RW][4][NT];
 #pragma unroll
   for (int rr = 0; rr < RW; ++rr)
@@ -332,7 +382,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RW == 2 ? (
 #pragma unroll
       for (int t = 0; t < NT; ++t) acc[rr][f][t] = float4_t{0.f, 0.f, 0.f, 0.f};
   S st;
-  conv_load<NT, KC, RW>(st, in, up, Cup, w, n, y0, x0, co0, 0, H, W, Cin, Cout);
+  // the patch's first pixel in each view (outside the image for a tile at its
+  // edge), the pieces' places in the view being read, the weights
+  auto patch = [&](const View& v, int u) {
+    return v.p + ((ptrdiff_t)(n * (H >> u) + ((y0 - 1) >> u)) * (W >> u) + ((x0 - 1) >> u)) * v.cs + v.co;
+  };
+  const bf16* const wsrc = w + (size_t)co0 * Cin;
+  const bf16* src = Cup ? patch(up, 1) : patch(in, 0);
+  conv_places<NT, KC, RW, FAR>(st, Cup ? up.cs : in.cs, Cup ? 1 : 0, y0, x0, H, W);
+  conv_load<NT, KC, RW, FAR>(st, src, 0, wsrc, 0, Cin, Cout);
   for (int c0 = 0; c0 < Cin; c0 += KC) {
     __syncthreads();  // the previous step's fragment reads are done
 #pragma unroll
@@ -343,53 +401,77 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RW == 2 ? (
 #pragma unroll
     for (int k = 0; k < S::W_PER; ++k) {
       const int q = tid + 256 * k;
-      if (q < S::W_Q) *reinterpret_cast<uint4*>(s_w + (q / S::PQ) * PS + 8 * (q % S::PQ)) = st.vw[k];
+      if (q < S::W_Q) *reinterpret_cast<uint4*>(s_w + (q / S::PQ) * WS + 8 * S::w_piece(q / S::PQ, q % S::PQ)) = st.vw[k];
     }
     __syncthreads();
-    if (c0 + KC < Cin) conv_load<NT, KC, RW>(st, in, up, Cup, w, n, y0, x0, co0, c0 + KC, H, W, Cin, Cout);
+    if (c0 + KC < Cin) {
+      if (c0 + KC == Cup) {  // on to the other view
+        src = patch(in, 0);
+        conv_places<NT, KC, RW, FAR>(st, in.cs, 0, y0, x0, H, W);
+      }
+      conv_load<NT, KC, RW, FAR>(st, src, c0 + KC < Cup ? c0 + KC : c0 + KC - Cup, wsrc, c0 + KC, Cin, Cout);
+    }
+    // A fragment's LDS read takes as long as several MFMAs: the next group's
+    // are under way while a group runs (and no more, for the registers; left
+    // to itself the compiler reads them two at a time and waits for each).
+    typedef typename F::T Frag;
     if constexpr (RW == 1) {
+      // group = tap
+      Frag a[2][4], b[2][NT];
+      auto frags = [&](int tap) {
+        const bf16* ap = s_in + ((wave + tap / 3) * (CT_W + 2) + i + tap % 3) * PS + KE * kq;
+        const bf16* bp = s_w + (tap * 16 * NT + i) * WS + wk;
 #pragma unroll
-      for (int r = 0; r < 3; ++r)
+        for (int f = 0; f < 4; ++f) a[tap & 1][f] = *reinterpret_cast<const Frag*>(ap + 16 * f * PS);
 #pragma unroll
-        for (int s = 0; s < 3; ++s) {
-          const bf16* bp = s_w + ((r * 3 + s) * 16 * NT + i) * PS + KE * kq;
-          const bf16* ap = s_in + ((wave + r) * (CT_W + 2) + i + s) * PS + KE * kq;
+        for (int t = 0; t < NT; ++t) b[tap & 1][t] = *reinterpret_cast<const Frag*>(bp + 16 * t * WS);
+      };
+      frags(0);
 #pragma unroll
-          for (int f = 0; f < 4; ++f)
+      for (int tap = 0; tap < 9; ++tap) {
+        if (tap + 1 < 9) frags(tap + 1);
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
-              acc[0][f][t] = F::mfma(*reinterpret_cast<const typename F::T*>(ap + 16 * f * PS),
-                                     *reinterpret_cast<const typename F::T*>(bp + 16 * t * PS), acc[0][f][t]);
-        }
+        for (int f = 0; f < 4; ++f)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) acc[0][f][t] = F::mfma(a[tap & 1][f], b[tap & 1][t], acc[0][f][t]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     } else {
       // Staged input row j of the wave's RW + 2 rows is tap row r = j - rr
       // of its output row rr: per tap column s, the 3 NT B fragments are
       // read once and every A fragment once, for all the rows it reaches.
+      // Group = (tap column, input row).
+      constexpr int G = 3 * (RW + 2);
+      Frag a[2][4], b[2][3][NT];
+      auto frags_a = [&](int g) {
+        const bf16* ap = s_in + ((RW * wave + g % (RW + 2)) * (CT_W + 2) + i + g / (RW + 2)) * PS + KE * kq;
 #pragma unroll
-      for (int s = 0; s < 3; ++s) {
-        typename F::T b[3][NT];
+        for (int f = 0; f < 4; ++f) a[g & 1][f] = *reinterpret_cast<const Frag*>(ap + 16 * f * PS);
+      };
+      auto frags_b = [&](int s, int r) {
 #pragma unroll
-        for (int r = 0; r < 3; ++r)
+        for (int t = 0; t < NT; ++t)
+          b[s & 1][r][t] = *reinterpret_cast<const Frag*>(s_w + ((r * 3 + s) * 16 * NT + 16 * t + i) * WS + wk);
+      };
+      frags_a(0);
 #pragma unroll
-          for (int t = 0; t < NT; ++t)
-            b[r][t] = *reinterpret_cast<const typename F::T*>(s_w + ((r * 3 + s) * 16 * NT + 16 * t + i) * PS +
-                                                              KE * kq);
+      for (int r = 0; r < 3; ++r) frags_b(0, r);
 #pragma unroll
-        for (int j = 0; j < RW + 2; ++j) {
-          const bf16* ap = s_in + ((RW * wave + j) * (CT_W + 2) + i + s) * PS + KE * kq;
+      for (int g = 0; g < G; ++g) {
+        const int s = g / (RW + 2), j = g % (RW + 2);
+        if (g + 1 < G) frags_a(g + 1);
+        if (s < 2 && j > 0) frags_b(s + 1, j - 1);
 #pragma unroll
-          for (int f = 0; f < 4; ++f) {
-            const typename F::T a = *reinterpret_cast<const typename F::T*>(ap + 16 * f * PS);
+        for (int f = 0; f < 4; ++f)
 #pragma unroll
-            for (int rr = 0; rr < RW; ++rr) {
-              const int r = j - rr;
-              if (r >= 0 && r < 3) {
+          for (int rr = 0; rr < RW; ++rr) {
+            const int r = j - rr;
+            if (r >= 0 && r < 3) {
 #pragma unroll
-                for (int t = 0; t < NT; ++t) acc[rr][f][t] = F::mfma(a, b[r][t], acc[rr][f][t]);
-              }
+              for (int t = 0; t < NT; ++t) acc[rr][f][t] = F::mfma(a[g & 1][f], b[s & 1][r][t], acc[rr][f][t]);
             }
           }
-        }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
@@ -455,7 +537,8 @@ template <int CIN, int NT, bool RELU>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_few_waves<NT>()))) void k_conv3x3_few(
     View in, const bf16* __restrict__ w, const float* __restrict__ bias, View out, int H, int W, int Cout,
     ConvFuse fz, int nbx, int nbz, int n_tiles) {
-  constexpr int PQ = CIN / 8, PS = CIN + 8, PW = CT_W + 2;
+  // (strides as in ConvStage; three workgroups of <32, 1> fit LDS at 80 bytes only)
+  constexpr int PQ = CIN / 8, PS = CIN == 16 ? 16 : NT == 2 ? 48 : 40, PW = CT_W + 2;
   constexpr int IN_Q = CF_PIX * PQ, IN_PER = (IN_Q + 255) / 256;
   constexpr int NP = 9 * CIN / 16, NQ = NP / 2;  // products of 16 channels and pairs of them per output
   __shared__ __attribute__((aligned(16))) bf16 s_in[CF_PIX * PS];
@@ -1294,9 +1377,20 @@ hipError_t conv3x3(View in, const bf16* w, const float* bias, View out, int N, i
 #undef RF_CONV_FEW
       return hipGetLastError();
     }
-#define RF_CONV_LDS(NT_, KC_, RW_)                                                                            \
-  hipLaunchKernelGGL((k_conv3x3_lds<NT_, KC_, RW_>), dim3((unsigned)n_tiles), dim3(256), 0, s, in, w, bias, out, H, \
-                     W, Cin, Cout, relu, vec_out, fz, nbx, nbz, n_tiles)
+    // Buffer loads reach 2 GiB from a tile's first pixel (of at most ten rows
+    // are read) and from the first weight; wider images and larger weights
+    // take the same kernel with 64-bit addresses.
+    const bool far = 20ll * W * std::max(in.cs, Cup ? up.cs : 0) >= (1ll << 31) - 65536 ||
+                     18ll * Cin * Cout >= (1ll << 31) - 65536;
+#define RF_CONV_LDS(NT_, KC_, RW_)                                                                                  \
+  do {                                                                                                              \
+    if (far)                                                                                                        \
+      hipLaunchKernelGGL((k_conv3x3_lds<NT_, KC_, RW_, true>), dim3((unsigned)n_tiles), dim3(256), 0, s, in, w,     \
+                         bias, out, H, W, Cin, Cout, relu, vec_out, fz, nbx, nbz, n_tiles);                         \
+    else                                                                                                            \
+      hipLaunchKernelGGL((k_conv3x3_lds<NT_, KC_, RW_, false>), dim3((unsigned)n_tiles), dim3(256), 0, s, in, w,    \
+                         bias, out, H, W, Cin, Cout, relu, vec_out, fz, nbx, nbz, n_tiles);                         \
+  } while (0)
     if (k32) {
       switch (nt) {
         case 4: RF_CONV_LDS(4, 32, 1); break;

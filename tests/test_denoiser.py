@@ -128,6 +128,33 @@ def test_conv3x3_gradients_match_torch(rf, gpu_available, Cin, Cout, W, H):
     assert (err <= 2.0 ** -8 * ref_dx.abs() + 1e-4).all(), float(err.max())
 
 
+# Pixels too far apart for 32-bit offsets (views of a few channels of wide
+# pixels): 64 and 32 outputs from whole channel steps of 32, and 16 from one of
+# 16 in two parts; a tile at each end of the row.
+@pytest.mark.parametrize("Cin,Cout", [(64, 64), (96, 32), (48, 16)])
+def test_conv3x3_of_widely_spaced_pixels(rf, gpu_available, Cin, Cout):
+    import torch
+    import torch.nn.functional as F
+    ctx = rf.Context(1 << 12, 1, 16)
+    g = torch.Generator().manual_seed(Cin)
+    W, cs, co = 130, 1 << 20, (1 << 20) - Cin
+    near = _bf16(torch.randn(1, 1, W, Cin, generator=g))
+    w = _bf16(0.1 * torch.randn(3, 3, Cout, Cin, generator=g)).cuda()
+    b = torch.randn(Cout, generator=g).cuda()
+    far = torch.empty(1, 1, W, cs, dtype=torch.bfloat16, device="cuda")
+    far[..., co:] = near.cuda()
+    out = []
+    for x, xs, xo in ((near.cuda(), Cin, 0), (far, cs, co)):
+        o = torch.zeros(1, 1, W, Cout, dtype=torch.bfloat16, device="cuda")
+        ctx.check(ctx.L.rf_nn_conv3x3(ctx.h, x.data_ptr(), xs, xo, w.data_ptr(), b.data_ptr(), o.data_ptr(), Cout, 0,
+                                      1, 1, W, Cin, Cout, 0))
+        out.append(o.cpu())
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+    ref = F.conv2d(near.float().permute(0, 3, 1, 2), w.float().cpu().permute(2, 3, 0, 1), b.cpu(), padding=1)
+    # half a bf16 ulp, and fp32 sums of 9 Cin products
+    assert ((out[0].float() - ref.permute(0, 2, 3, 1)).abs() <= 2.0 ** -8 * ref.permute(0, 2, 3, 1).abs() + 1e-4).all()
+
+
 # One pixel, tiles of exactly 8 rows x 64 pixels and one more of each, images
 # that end inside a tile, more tiles than workgroups, three channel blocks.
 @pytest.mark.parametrize("Cin,Cout,N,H,W", [(16, 32, 1, 1, 1), (32, 32, 1, 8, 64), (32, 16, 2, 9, 65),
