@@ -66,8 +66,8 @@ int ensure_shape(rf_denoiser* d, int N, int H, int W) {
   const size_t P0 = (size_t)N * H * W, P1 = P0 / 4, P2 = P0 / 16, P3 = P0 / 64;
   struct A { DevBuf* b; size_t n; };
   const A all[] = {
-      {&d->e0a, P0 * 32}, {&d->cat0, P0 * 96}, {&d->p0, P1 * 32}, {&d->e1a, P1 * 64}, {&d->cat1, P1 * 192},
-      {&d->p1, P2 * 64}, {&d->e2a, P2 * 128}, {&d->cat2, P2 * 384}, {&d->p2, P3 * 128}, {&d->b, P3 * 256},
+      {&d->e0a, P0 * 32}, {&d->cat0, P0 * 32}, {&d->p0, P1 * 32}, {&d->e1a, P1 * 64}, {&d->cat1, P1 * 64},
+      {&d->p1, P2 * 64}, {&d->e2a, P2 * 128}, {&d->cat2, P2 * 128}, {&d->p2, P3 * 128}, {&d->b, P3 * 256},
       {&d->d2, P2 * 128}, {&d->d1, P1 * 64}, {&d->d0a, P0 * 32}, {&d->d0b, P0 * 32}, {&d->o, P0 * 16},
       {&d->g_e0a, P0 * 32}, {&d->g_cat0, P0 * 96}, {&d->g_p0, P1 * 32}, {&d->g_e1a, P1 * 64},
       {&d->g_cat1, P1 * 192}, {&d->g_p1, P2 * 64}, {&d->g_e2a, P2 * 128}, {&d->g_cat2, P2 * 384},
@@ -113,14 +113,12 @@ int check_shape(rf_denoiser* d, int N, int H, int W) {
   return RF_OK;
 }
 
-// Forward pass on x (N x H x W x 16 bf16).  With y_out (inference) the
-// decoder's convolutions read the upsampled half of their concatenated input
-// straight from the lower level and the last one writes y_out = x[:4] +
-// out[:4] (fp32); training writes the upsampled halves into the
-// concatenation buffers, whose full contents the weight gradients read back,
-// and keeps the last layer's output for the loss.
+// Forward pass on x (N x H x W x 16 bf16).  The decoder's convolutions (and
+// their weight gradients) read the upsampled half of their concatenated input
+// straight from the lower level; the concatenation buffers hold the skip
+// channels only.  With y_out (inference) the last convolution writes y_out =
+// x[:4] + out[:4] (fp32); training keeps its output for the loss.
 int forward(rf_denoiser* d, const bf16* x, int N, int H, int W, float* y_out = nullptr) {
-  const bool fused_up = y_out != nullptr;
   rf_ctx* ctx = d->ctx;
   hipStream_t s = ctx->stream;
   const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4, H3 = H / 8, W3 = W / 8;
@@ -137,34 +135,23 @@ int forward(rf_denoiser* d, const bf16* x, int N, int H, int W, float* y_out = n
     f.pool = pool;
     return conv_f(l, in, out, h, w, f);
   };
-  // The skip channels of a concatenation buffer `cat` (cat_cs channels, the
-  // upsampled c_lo first): inside it for training, packed at their own
-  // channel count at inference, where no upsampled half sits beside them
-  // (whole-line writes and reads instead of a third or half of each pixel).
-  auto skip = [&](DevBuf& cat, int cat_cs, int c_lo) {
-    return fused_up ? V(cat, cat_cs - c_lo, 0) : V(cat, cat_cs, c_lo);
-  };
-  // conv l over [upsample(lo) (c_lo channels), the skip channels of `cat`]
-  auto up_conv = [&](int l, View lo, int c_lo, DevBuf& cat, int cat_cs, View out, int h, int w) -> hipError_t {
-    if (fused_up) {
-      rfn::ConvFuse f;
-      f.up = lo;
-      f.Cup = c_lo;
-      return conv_f(l, skip(cat, cat_cs, c_lo), out, h, w, f);
-    }
-    const hipError_t e = rfn::upsample2(lo, V(cat, cat_cs, 0), N, h / 2, w / 2, c_lo, s);
-    return e != hipSuccess ? e : conv(l, V(cat, cat_cs), out, h, w);
+  // conv l over [upsample(lo) (c_lo channels), skip]
+  auto up_conv = [&](int l, View lo, int c_lo, View skip, View out, int h, int w) {
+    rfn::ConvFuse f;
+    f.up = lo;
+    f.Cup = c_lo;
+    return conv_f(l, skip, out, h, w, f);
   };
   HIPCHK(ctx, conv(0, vx, V(d->e0a, 32), H, W));
-  HIPCHK(ctx, conv_pool(1, V(d->e0a, 32), skip(d->cat0, 96, 64), V(d->p0, 32), H, W));
+  HIPCHK(ctx, conv_pool(1, V(d->e0a, 32), V(d->cat0, 32), V(d->p0, 32), H, W));
   HIPCHK(ctx, conv(2, V(d->p0, 32), V(d->e1a, 64), H1, W1));
-  HIPCHK(ctx, conv_pool(3, V(d->e1a, 64), skip(d->cat1, 192, 128), V(d->p1, 64), H1, W1));
+  HIPCHK(ctx, conv_pool(3, V(d->e1a, 64), V(d->cat1, 64), V(d->p1, 64), H1, W1));
   HIPCHK(ctx, conv(4, V(d->p1, 64), V(d->e2a, 128), H2, W2));
-  HIPCHK(ctx, conv_pool(5, V(d->e2a, 128), skip(d->cat2, 384, 256), V(d->p2, 128), H2, W2));
+  HIPCHK(ctx, conv_pool(5, V(d->e2a, 128), V(d->cat2, 128), V(d->p2, 128), H2, W2));
   HIPCHK(ctx, conv(6, V(d->p2, 128), V(d->b, 256), H3, W3));
-  HIPCHK(ctx, up_conv(7, V(d->b, 256), 256, d->cat2, 384, V(d->d2, 128), H2, W2));
-  HIPCHK(ctx, up_conv(8, V(d->d2, 128), 128, d->cat1, 192, V(d->d1, 64), H1, W1));
-  HIPCHK(ctx, up_conv(9, V(d->d1, 64), 64, d->cat0, 96, V(d->d0a, 32), H, W));
+  HIPCHK(ctx, up_conv(7, V(d->b, 256), 256, V(d->cat2, 128), V(d->d2, 128), H2, W2));
+  HIPCHK(ctx, up_conv(8, V(d->d2, 128), 128, V(d->cat1, 64), V(d->d1, 64), H1, W1));
+  HIPCHK(ctx, up_conv(9, V(d->d1, 64), 64, V(d->cat0, 32), V(d->d0a, 32), H, W));
   HIPCHK(ctx, conv(10, V(d->d0a, 32), V(d->d0b, 32), H, W));
   if (y_out) {
     rfn::ConvFuse f;
@@ -184,8 +171,9 @@ int backward(rf_denoiser* d, const bf16* x, int N, int H, int W) {
   const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4, H3 = H / 8, W3 = W / 8;
   float* g = (float*)d->g.p;
   HIPCHK(ctx, rfn::zero_f32(g, d->n_params, s));
-  auto wgrad = [&](int l, View xin, View dy, int h, int w) {
-    return rfn::conv3x3_wgrad(xin, dy, g + d->L[l].w_off, g + d->L[l].b_off, N, h, w, d->L[l].cin, d->L[l].cout,
+  // up, Cup: the upsampled channels before xin's (up_conv)
+  auto wgrad = [&](int l, View xin, View dy, int h, int w, View up = View{nullptr, 0, 0}, int Cup = 0) {
+    return rfn::conv3x3_wgrad(xin, up, Cup, dy, g + d->L[l].w_off, g + d->L[l].b_off, N, h, w, d->L[l].cin, d->L[l].cout,
                               (float*)d->wg_work.p, d->wg_work.bytes / sizeof(float), s);
   };
   // with y, the gradient of the layer's input y is masked by y > 0
@@ -200,34 +188,34 @@ int backward(rf_denoiser* d, const bf16* x, int N, int H, int W) {
   HIPCHK(ctx, dgrad(11, V(d->g_o, 16), V(d->g_d0b, 32), H, W, V(d->d0b, 32)));
   HIPCHK(ctx, wgrad(10, V(d->d0a, 32), V(d->g_d0b, 32), H, W));
   HIPCHK(ctx, dgrad(10, V(d->g_d0b, 32), V(d->g_d0a, 32), H, W, V(d->d0a, 32)));
-  HIPCHK(ctx, wgrad(9, V(d->cat0, 96), V(d->g_d0a, 32), H, W));
+  HIPCHK(ctx, wgrad(9, V(d->cat0, 32), V(d->g_d0a, 32), H, W, V(d->d1, 64), 64));
   HIPCHK(ctx, dgrad(9, V(d->g_d0a, 32), V(d->g_cat0, 96), H, W));
   // dec1
   HIPCHK(ctx, rfn::upsample2_bwd(V(d->g_cat0, 96, 0), V(d->g_d1, 64), V(d->d1, 64), N, H1, W1, 64, s));
-  HIPCHK(ctx, wgrad(8, V(d->cat1, 192), V(d->g_d1, 64), H1, W1));
+  HIPCHK(ctx, wgrad(8, V(d->cat1, 64), V(d->g_d1, 64), H1, W1, V(d->d2, 128), 128));
   HIPCHK(ctx, dgrad(8, V(d->g_d1, 64), V(d->g_cat1, 192), H1, W1));
   // dec2
   HIPCHK(ctx, rfn::upsample2_bwd(V(d->g_cat1, 192, 0), V(d->g_d2, 128), V(d->d2, 128), N, H2, W2, 128, s));
-  HIPCHK(ctx, wgrad(7, V(d->cat2, 384), V(d->g_d2, 128), H2, W2));
+  HIPCHK(ctx, wgrad(7, V(d->cat2, 128), V(d->g_d2, 128), H2, W2, V(d->b, 256), 256));
   HIPCHK(ctx, dgrad(7, V(d->g_d2, 128), V(d->g_cat2, 384), H2, W2));
   // bottleneck
   HIPCHK(ctx, rfn::upsample2_bwd(V(d->g_cat2, 384, 0), V(d->g_b, 256), V(d->b, 256), N, H3, W3, 256, s));
   HIPCHK(ctx, wgrad(6, V(d->p2, 128), V(d->g_b, 256), H3, W3));
   HIPCHK(ctx, dgrad(6, V(d->g_b, 256), V(d->g_p2, 128), H3, W3));
   // enc2: skip2 gradient = concat part + pooled path
-  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p2, 128), V(d->g_cat2, 384, 256), V(d->cat2, 384, 256), N, H2, W2, 128, s));
+  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p2, 128), V(d->g_cat2, 384, 256), V(d->cat2, 128), N, H2, W2, 128, s));
   HIPCHK(ctx, wgrad(5, V(d->e2a, 128), V(d->g_cat2, 384, 256), H2, W2));
   HIPCHK(ctx, dgrad(5, V(d->g_cat2, 384, 256), V(d->g_e2a, 128), H2, W2, V(d->e2a, 128)));
   HIPCHK(ctx, wgrad(4, V(d->p1, 64), V(d->g_e2a, 128), H2, W2));
   HIPCHK(ctx, dgrad(4, V(d->g_e2a, 128), V(d->g_p1, 64), H2, W2));
   // enc1
-  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p1, 64), V(d->g_cat1, 192, 128), V(d->cat1, 192, 128), N, H1, W1, 64, s));
+  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p1, 64), V(d->g_cat1, 192, 128), V(d->cat1, 64), N, H1, W1, 64, s));
   HIPCHK(ctx, wgrad(3, V(d->e1a, 64), V(d->g_cat1, 192, 128), H1, W1));
   HIPCHK(ctx, dgrad(3, V(d->g_cat1, 192, 128), V(d->g_e1a, 64), H1, W1, V(d->e1a, 64)));
   HIPCHK(ctx, wgrad(2, V(d->p0, 32), V(d->g_e1a, 64), H1, W1));
   HIPCHK(ctx, dgrad(2, V(d->g_e1a, 64), V(d->g_p0, 32), H1, W1));
   // enc0
-  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p0, 32), V(d->g_cat0, 96, 64), V(d->cat0, 96, 64), N, H, W, 32, s));
+  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p0, 32), V(d->g_cat0, 96, 64), V(d->cat0, 32), N, H, W, 32, s));
   HIPCHK(ctx, wgrad(1, V(d->e0a, 32), V(d->g_cat0, 96, 64), H, W));
   HIPCHK(ctx, dgrad(1, V(d->g_cat0, 96, 64), V(d->g_e0a, 32), H, W, V(d->e0a, 32)));
   HIPCHK(ctx, wgrad(0, vx, V(d->g_e0a, 32), H, W));
@@ -393,7 +381,7 @@ int rf_nn_conv3x3_wgrad(rf_ctx* ctx, const void* x, int32_t x_cs, int32_t x_co, 
   DevBuf work;
   const size_t n_work = rfn::conv3x3_wgrad_work(N, H, W, Cin, Cout);
   HIPCHK(ctx, work.alloc(n_work * sizeof(float)));
-  HIPCHK(ctx, rfn::conv3x3_wgrad(View{(bf16*)x, x_cs, x_co}, View{(bf16*)dy, dy_cs, dy_co}, dw, db, N, H, W, Cin,
+  HIPCHK(ctx, rfn::conv3x3_wgrad(View{(bf16*)x, x_cs, x_co}, View{nullptr, 0, 0}, 0, View{(bf16*)dy, dy_cs, dy_co}, dw, db, N, H, W, Cin,
                                  Cout, (float*)work.p, n_work, ctx->stream));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   return RF_OK;

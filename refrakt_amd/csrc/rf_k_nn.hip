@@ -815,7 +815,8 @@ __device__ __forceinline__ bf16x8_t wgrad_frag(const bf16* p) {
 
 template <int TCO, int TCI, int SPW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TCO == 64 ? 2 : 3))) void k_wgrad_mfma(
-    View x, View dy, float* __restrict__ part, int N, int H, int W, int Cin, int Cout, int runs, int with_bias) {
+    View x, View up, int Cup, View dy, float* __restrict__ part, int N, int H, int W, int Cin, int Cout, int runs,
+    int with_bias) {
   using C = WgradCfg<TCO, TCI, SPW>;
   __shared__ __attribute__((aligned(16))) bf16 s_buf[C::LDS];
   bf16* const s_x = s_buf;                  // [row & 1][pixel][ci]
@@ -863,13 +864,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TCO == 64 ?
       if (q < C::DY_Q) *reinterpret_cast<uint4*>(s_dy + (y & 1) * C::DY_ROW + p * C::OS + 8 * pc) = vd[k];
     }
   };
+  // The input's view: half-resolution for a block of upsampled channels (TCI
+  // divides Cup).  Written out by a pass of their own they cost 33 us an 8 x
+  // 256^2 training step, and as much again in reading four copies.
+  const int us = ci0 < Cup ? 1 : 0;  // workgroup-uniform
+  const bf16* const xp = us ? up.p + up.co + ci0 : x.p + x.co + ci0 - Cup;
+  const int xcs = us ? up.cs : x.cs, Wx = W >> us, Hx = H >> us;
   auto load_x = [&](int n, int yy, int xs) {
 #pragma unroll
     for (int k = 0; k < C::X_PER; ++k) {
       const int q = tid + 256 * k, p = q / C::PQI, pc = q % C::PQI, gx = xs + p - 1;
       vx[k] = make_uint4(0u, 0u, 0u, 0u);
       if (q < C::XROW_Q && gx >= 0 && gx < W)
-        vx[k] = *reinterpret_cast<const uint4*>(x.p + ((size_t)(n * H + yy) * W + gx) * x.cs + x.co + ci0 + 8 * pc);
+        vx[k] = *reinterpret_cast<const uint4*>(xp + ((size_t)(n * Hx + (yy >> us)) * Wx + (gx >> us)) * xcs + 8 * pc);
     }
   };
   auto store_x = [&](int yy) {
@@ -1086,18 +1093,8 @@ __global__ void k_avgpool2(View in, View out, int N, int H, int W, int C) {
   out.p[po * out.cs + out.co + c] = f2bf(0.25f * s);
 }
 
-__global__ void k_upsample2(View in, View out, int N, int H, int W, int C) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int Ho = 2 * H, Wo = 2 * W;
-  if (i >= (size_t)N * Ho * Wo * C) return;
-  const int c = (int)(i % C);
-  const size_t po = i / C;
-  const int xo = (int)(po % Wo), yo = (int)((po / Wo) % Ho), n = (int)(po / ((size_t)Wo * Ho));
-  out.p[po * out.cs + out.co + c] = in.p[((size_t)(n * H + yo / 2) * W + xo / 2) * in.cs + in.co + c];
-}
-
-// 8-channel (16-byte) versions of pooling and upsampling: one thread per
-// output pixel and channel group.
+// 8-channel (16-byte) version of pooling: one thread per output pixel and
+// channel group.
 
 __global__ void k_avgpool2_v8(View in, View out, int N, int H, int W, int C) {
   const int Ho = H / 2, Wo = W / 2, G = C / 8;
@@ -1122,17 +1119,6 @@ __global__ void k_avgpool2_v8(View in, View out, int N, int H, int W, int C) {
   for (int k = 0; k < 4; ++k)
     r[k] = f2bf2(0.25f * s[2 * k], 0.25f * s[2 * k + 1]);
   *reinterpret_cast<uint4*>(out.p + po * out.cs + out.co + 8 * g) = make_uint4(r[0], r[1], r[2], r[3]);
-}
-
-__global__ void k_upsample2_v8(View in, View out, int N, int H, int W, int C) {
-  const int Ho = 2 * H, Wo = 2 * W, G = C / 8;
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)N * Ho * Wo * G) return;
-  const int g = (int)(i % G);
-  const size_t po = i / G;
-  const int xo = (int)(po % Wo), yo = (int)((po / Wo) % Ho), n = (int)(po / ((size_t)Wo * Ho));
-  *reinterpret_cast<uint4*>(out.p + po * out.cs + out.co + 8 * g) =
-      *reinterpret_cast<const uint4*>(in.p + ((size_t)(n * H + yo / 2) * W + xo / 2) * in.cs + in.co + 8 * g);
 }
 
 // Gradient of the 2x2 average added to din (8 channels per thread), then
@@ -1447,10 +1433,10 @@ int wgrad_runs(int N, int H, int W, int Cin, int Cout) {
 }
 
 template <int TCO, int TCI, int SPW>
-void launch_wgrad(dim3 grid, hipStream_t s, View x, View dy, float* work, int N, int H, int W, int Cin, int Cout,
-                  int runs, int with_bias) {
-  hipLaunchKernelGGL((k_wgrad_mfma<TCO, TCI, SPW>), grid, dim3(256), 0, s, x, dy, work, N, H, W, Cin, Cout, runs,
-                     with_bias);
+void launch_wgrad(dim3 grid, hipStream_t s, View x, View up, int Cup, View dy, float* work, int N, int H, int W,
+                  int Cin, int Cout, int runs, int with_bias) {
+  hipLaunchKernelGGL((k_wgrad_mfma<TCO, TCI, SPW>), grid, dim3(256), 0, s, x, up, Cup, dy, work, N, H, W, Cin, Cout,
+                     runs, with_bias);
 }
 }  // namespace
 
@@ -1458,19 +1444,20 @@ size_t conv3x3_wgrad_work(int N, int H, int W, int Cin, int Cout) {
   return (size_t)wgrad_runs(N, H, W, Cin, Cout) * ((size_t)9 * Cout * Cin + Cout);
 }
 
-hipError_t conv3x3_wgrad(View x, View dy, float* dw, float* db, int N, int H, int W, int Cin, int Cout, float* work,
-                         size_t work_floats, hipStream_t s) {
+hipError_t conv3x3_wgrad(View x, View up, int Cup, View dy, float* dw, float* db, int N, int H, int W, int Cin,
+                         int Cout, float* work, size_t work_floats, hipStream_t s) {
   if (Cin % 16 || Cout % 16 || N <= 0 || H <= 0 || W <= 0 || !work) return hipErrorInvalidValue;
+  if (Cup && (Cup < 0 || Cup % 32 || Cup >= Cin || H % 2 || W % 2)) return hipErrorInvalidValue;
   if (work_floats < conv3x3_wgrad_work(N, H, W, Cin, Cout)) return hipErrorInvalidValue;
   const WgradTile t = wgrad_tile(Cin, Cout);
   const int runs = wgrad_runs(N, H, W, Cin, Cout);
   const dim3 grid((unsigned)runs, (unsigned)(Cin / t.tci), (unsigned)(Cout / t.tco));
   const int wb = db ? 1 : 0;
-  if (t.tco == 64) launch_wgrad<64, 32, 2>(grid, s, x, dy, work, N, H, W, Cin, Cout, runs, wb);
-  else if (t.tco == 32 && t.tci == 32) launch_wgrad<32, 32, 1>(grid, s, x, dy, work, N, H, W, Cin, Cout, runs, wb);
-  else if (t.tco == 32) launch_wgrad<32, 16, 1>(grid, s, x, dy, work, N, H, W, Cin, Cout, runs, wb);
-  else if (t.tci == 32) launch_wgrad<16, 32, 1>(grid, s, x, dy, work, N, H, W, Cin, Cout, runs, wb);
-  else launch_wgrad<16, 16, 1>(grid, s, x, dy, work, N, H, W, Cin, Cout, runs, wb);
+  if (t.tco == 64) launch_wgrad<64, 32, 2>(grid, s, x, up, Cup, dy, work, N, H, W, Cin, Cout, runs, wb);
+  else if (t.tco == 32 && t.tci == 32) launch_wgrad<32, 32, 1>(grid, s, x, up, Cup, dy, work, N, H, W, Cin, Cout, runs, wb);
+  else if (t.tco == 32) launch_wgrad<32, 16, 1>(grid, s, x, up, Cup, dy, work, N, H, W, Cin, Cout, runs, wb);
+  else if (t.tci == 32) launch_wgrad<16, 32, 1>(grid, s, x, up, Cup, dy, work, N, H, W, Cin, Cout, runs, wb);
+  else launch_wgrad<16, 16, 1>(grid, s, x, up, Cup, dy, work, N, H, W, Cin, Cout, runs, wb);
   const int n_w = 9 * Cout * Cin, n_b = db ? Cout : 0;
   hipLaunchKernelGGL(k_wgrad_reduce, dim3((unsigned)((n_w + n_b + 63) / 64)), dim3(1024), 0, s, work, dw, db, runs,
                      n_w, n_b);
@@ -1500,14 +1487,6 @@ hipError_t avgpool2(View in, View out, int N, int H, int W, int C, hipStream_t s
 hipError_t avgpool2_bwd(View dout, View din, View y, int N, int H, int W, int C, hipStream_t s) {
   if (!v8_ok(dout, din, C) || !v8_ok(y, y, C)) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_avgpool2_bwd_v8, grid1((size_t)N * H * W * (C / 8)), dim3(256), 0, s, dout, din, y, N, H, W, C);
-  return hipGetLastError();
-}
-
-hipError_t upsample2(View in, View out, int N, int H, int W, int C, hipStream_t s) {
-  if (v8_ok(in, out, C))
-    hipLaunchKernelGGL(k_upsample2_v8, grid1((size_t)N * 4 * H * W * (C / 8)), dim3(256), 0, s, in, out, N, H, W, C);
-  else
-    hipLaunchKernelGGL(k_upsample2, grid1((size_t)N * 4 * H * W * C), dim3(256), 0, s, in, out, N, H, W, C);
   return hipGetLastError();
 }
 

@@ -48,10 +48,12 @@ hipError_t conv3x3(View in, const bf16* w, const float* bias, View out, int N, i
 // db[k] += sum_p dy[p,k] (bf16 products on the matrix cores, fp32 sums).  The
 // image rows are split over workgroups whose partial sums go to `work`
 // (conv3x3_wgrad_work(N, H, W, Cin, Cout) floats), then are added to dw/db in a
-// fixed order: deterministic, no atomics.
+// fixed order: deterministic, no atomics.  With Cup > 0 (a multiple of 32, H
+// and W even) x's first Cup channels are the 2x upsampling of `up`, read in
+// place, and x holds the others (as in ConvFuse).
 size_t conv3x3_wgrad_work(int N, int H, int W, int Cin, int Cout);
-hipError_t conv3x3_wgrad(View x, View dy, float* dw, float* db, int N, int H, int W, int Cin, int Cout, float* work,
-                         size_t work_floats, hipStream_t s);
+hipError_t conv3x3_wgrad(View x, View up, int Cup, View dy, float* dw, float* db, int N, int H, int W, int Cin,
+                         int Cout, float* work, size_t work_floats, hipStream_t s);
 // w_t[r][s][c][k] = w[2-r][2-s][k][c]: the weights of the input-gradient
 // convolution (dx = conv3x3(dy, w_t) with Cin' = Cout, Cout' = Cin).
 hipError_t flip_weights(const bf16* w, bf16* wt, int Cin, int Cout, hipStream_t s);
@@ -69,7 +71,6 @@ hipError_t avgpool2(View in, View out, int N, int H, int W, int C, hipStream_t s
 hipError_t avgpool2_bwd(View dout, View din, View y, int N, int H, int W, int C, hipStream_t s);
 // Nearest 2x upsampling (H, W are the input size) and its gradient, kept
 // where y > 0 (channel runs 16-byte aligned, C a multiple of 8).
-hipError_t upsample2(View in, View out, int N, int H, int W, int C, hipStream_t s);
 hipError_t upsample2_bwd(View dout, View din, View y, int N, int H, int W, int C, hipStream_t s);
 // y = x[:, :4] + o[:, :4] (fp32, 4 channels, when y_out != null); when t != null: loss_sum += sum (y - t)^2 and
 // do = 2 (y - t) / count in channels 0..3, 0 in the rest (16-channel do).
