@@ -175,6 +175,23 @@ __device__ __forceinline__ void conv_places(ConvStage<NT, KC, RW>& st, int cs, i
   }
 }
 
+// A 16-byte piece (the piece-th of a pixel `pixels` pixels behind the first) of
+// a row: its place, BUF_NONE for zeros, and its load.
+template <bool FAR>
+__device__ __forceinline__ uint32_t piece_place(int pixels, int cs, int piece) {
+  const uint32_t unit = (uint32_t)pixels * (uint32_t)(cs / 8) + (uint32_t)piece;
+  return FAR ? unit : 16u * unit;
+}
+template <bool FAR>
+__device__ __forceinline__ uint4 piece_load(const bf16* row, uint32_t place) {
+  if constexpr (FAR) {
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if (place != BUF_NONE) v = *reinterpret_cast<const uint4*>(row + 8 * (size_t)place);
+    return v;
+  }
+  return buf_load(buf_at(row), place, 0);
+}
+
 // The loads of one channel step.  Channels [0, Cup) come from the
 // half-resolution `up` (nearest-neighbour upsampling read in place), the rest
 // from `in`; a KC step never straddles the two (Cup is a multiple of 32).
@@ -765,8 +782,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_few_wa
 // A workgroup owns a TCO x TCI channel tile, all nine taps, and a run of
 // "units" (one 64-pixel strip of one dy row; units are strip-major, so a
 // run walks down the rows of a strip).  LDS holds pixels as they lie in
-// memory (all channels of a pixel together), two input rows of 66 pixels and
-// two dy rows, one of each being filled while the other is read.  The matrix
+// memory (all channels of a pixel together), a ring of three input rows of 66
+// pixels and two dy rows, the next being filled while the others are read.  The
+// matrix
 // operands need eight consecutive pixels of one channel per lane; gfx950's
 // transposing LDS read delivers them from that layout, so staging is one
 // 16-byte store per eight channels and a column shift is a pixel offset.
@@ -780,8 +798,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_few_wa
 // each strip's two 32-pixel K steps and add in LDS at the end.  The bias
 // gradient is the product with an all-ones B.  Each run's sums go to its own
 // slice of `part` (no atomics); k_wgrad_reduce adds the slices to dw and db
-// in a fixed order.  Per 8 x 256^2 training step the twelve layers take 0.38 ms
-// (0.62 ms before), the 192 -> 64 and 384 -> 128 layers at 640 TFLOP/s.
+// in a fixed order.  Rows are loaded two ahead: a row's products take a third
+// of a load's time, and one row ahead the waves waited two thirds of theirs.
+// Per 8 x 256^2 training step the twelve layers take 0.31 ms (0.37 ms one row
+// ahead, 0.62 ms channel-major), those of 64 outputs at 580 TFLOP/s.
 constexpr int WG_SEG = 64;  // strip width
 
 template <int TCO, int TCI, int SPW>
@@ -797,7 +817,7 @@ struct WgradCfg {
   // over the banks and keep the stores aligned
   static constexpr int OS = TCO + 8, IS = TCI + 8;
   static constexpr int X_ROW = (WG_SEG + 2) * IS, DY_ROW = WG_SEG * OS;
-  static constexpr int LDS = 2 * X_ROW + 2 * DY_ROW;  // bf16 elements
+  static constexpr int LDS = 3 * X_ROW + 2 * DY_ROW;  // bf16 elements
   static constexpr int RED_Q = 5;                     // taps per round of the K-split reduction
   static_assert(WK == 1 || GROUPS * RED_Q * SPW * 4 * 64 * 4 <= LDS * 2, "the reduction fits the staging buffers");
 };
@@ -813,14 +833,18 @@ __device__ __forceinline__ bf16x8_t wgrad_frag(const bf16* p) {
   return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-template <int TCO, int TCI, int SPW>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TCO == 64 ? 2 : 3))) void k_wgrad_mfma(
+// Waves per SIMD that the registers must allow: with three, <32, 32> spills (934
+// against 874 us for the 32-output layers of eight 8 x 256^2 training steps).
+constexpr int wgrad_waves(int TCO, int TCI) { return TCI == 16 ? 4 : TCO >= 32 ? 2 : 3; }
+
+template <int TCO, int TCI, int SPW, bool FAR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(wgrad_waves(TCO, TCI)))) void k_wgrad_mfma(
     View x, View up, int Cup, View dy, float* __restrict__ part, int N, int H, int W, int Cin, int Cout, int runs,
     int with_bias) {
   using C = WgradCfg<TCO, TCI, SPW>;
   __shared__ __attribute__((aligned(16))) bf16 s_buf[C::LDS];
-  bf16* const s_x = s_buf;                  // [row & 1][pixel][ci]
-  bf16* const s_dy = s_buf + 2 * C::X_ROW;  // [row & 1][pixel][co]
+  bf16* const s_x = s_buf;                  // [row of three][pixel][ci]
+  bf16* const s_dy = s_buf + 3 * C::X_ROW;  // [row & 1][pixel][co]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i = lane & 15, kq = lane >> 4;
   const int run = blockIdx.x, cb = blockIdx.y, kb = blockIdx.z;
@@ -845,66 +869,75 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TCO == 64 ?
   for (int t = 0; t < SPW; ++t) accb[t] = float4_t{0.f, 0.f, 0.f, 0.f};
   const uint4 one4 = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
   const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, one4);
-  uint4 vd[C::DY_PER], vx[C::X_PER];
-  // dy row y and input row yy of image n, strip at xs
-  auto load_dy = [&](int n, int y, int xs) {
-#pragma unroll
-    for (int k = 0; k < C::DY_PER; ++k) {
-      const int q = tid + 256 * k, p = q / C::PQO, pc = q % C::PQO;
-      vd[k] = make_uint4(0u, 0u, 0u, 0u);
-      if (q < C::DY_Q && xs + p < W)
-        vd[k] = *reinterpret_cast<const uint4*>(dy.p + ((size_t)(n * H + y) * W + xs + p) * dy.cs + dy.co + co0 +
-                                                8 * pc);
-    }
-  };
-  auto store_dy = [&](int y) {
-#pragma unroll
-    for (int k = 0; k < C::DY_PER; ++k) {
-      const int q = tid + 256 * k, p = q / C::PQO, pc = q % C::PQO;
-      if (q < C::DY_Q) *reinterpret_cast<uint4*>(s_dy + (y & 1) * C::DY_ROW + p * C::OS + 8 * pc) = vd[k];
-    }
-  };
   // The input's view: half-resolution for a block of upsampled channels (TCI
   // divides Cup).  Written out by a pass of their own they cost 33 us an 8 x
   // 256^2 training step, and as much again in reading four copies.
   const int us = ci0 < Cup ? 1 : 0;  // workgroup-uniform
   const bf16* const xp = us ? up.p + up.co + ci0 : x.p + x.co + ci0 - Cup;
   const int xcs = us ? up.cs : x.cs, Wx = W >> us, Hx = H >> us;
-  auto load_x = [&](int n, int yy, int xs) {
+  // Rows on their way to LDS, by the row's place in the ring of three: one
+  // being stored while the next is under way (a row's products take a third of
+  // a load's time, so one row ahead left the waves waiting).
+  uint4 vd[3][C::DY_PER], vx[3][C::X_PER];
+  uint32_t pd[C::DY_PER], px[C::X_PER];  // this thread's pieces of a strip's rows (piece_load)
+  auto places = [&](int xs) {
+#pragma unroll
+    for (int k = 0; k < C::DY_PER; ++k) {
+      const int q = tid + 256 * k, p = q / C::PQO, pc = q % C::PQO;
+      pd[k] = q < C::DY_Q && xs + p < W ? piece_place<FAR>(p, dy.cs, pc) : BUF_NONE;
+    }
 #pragma unroll
     for (int k = 0; k < C::X_PER; ++k) {
       const int q = tid + 256 * k, p = q / C::PQI, pc = q % C::PQI, gx = xs + p - 1;
-      vx[k] = make_uint4(0u, 0u, 0u, 0u);
-      if (q < C::XROW_Q && gx >= 0 && gx < W)
-        vx[k] = *reinterpret_cast<const uint4*>(xp + ((size_t)(n * Hx + (yy >> us)) * Wx + (gx >> us)) * xcs + 8 * pc);
+      px[k] = q < C::XROW_Q && gx >= 0 && gx < W ? piece_place<FAR>((gx >> us) - ((xs - 1) >> us), xcs, pc) : BUF_NONE;
     }
   };
-  auto store_x = [&](int yy) {
+  auto load_dy = [&](uint4 (&v)[C::DY_PER], int n, int y, int xs) {
+    const bf16* const src = dy.p + ((size_t)(n * H + y) * W + xs) * dy.cs + dy.co + co0;
+#pragma unroll
+    for (int k = 0; k < C::DY_PER; ++k) v[k] = piece_load<FAR>(src, pd[k]);
+  };
+  auto store_dy = [&](const uint4 (&v)[C::DY_PER], int y) {
+#pragma unroll
+    for (int k = 0; k < C::DY_PER; ++k) {
+      const int q = tid + 256 * k, p = q / C::PQO, pc = q % C::PQO;
+      if (q < C::DY_Q) *reinterpret_cast<uint4*>(s_dy + (y & 1) * C::DY_ROW + p * C::OS + 8 * pc) = v[k];
+    }
+  };
+  auto load_x = [&](uint4 (&v)[C::X_PER], int n, int yy, int xs) {
+    const bf16* const src = xp + ((ptrdiff_t)(n * Hx + (yy >> us)) * Wx + ((xs - 1) >> us)) * xcs;
+#pragma unroll
+    for (int k = 0; k < C::X_PER; ++k) v[k] = piece_load<FAR>(src, px[k]);
+  };
+  auto store_x = [&](const uint4 (&v)[C::X_PER], int slot) {
 #pragma unroll
     for (int k = 0; k < C::X_PER; ++k) {
       const int q = tid + 256 * k, p = q / C::PQI, pc = q % C::PQI;
-      if (q < C::XROW_Q) *reinterpret_cast<uint4*>(s_x + (yy & 1) * C::X_ROW + p * C::IS + 8 * pc) = vx[k];
+      if (q < C::XROW_Q) *reinterpret_cast<uint4*>(s_x + slot * C::X_ROW + p * C::IS + 8 * pc) = v[k];
     }
   };
   // fragments of the input rows around the current dy row: [row][shift][K step]
   bf16x8_t xf[3][3][C::KS];
-  auto read_x = [&](bf16x8_t (&f)[3][C::KS], int yy) {
-    const bf16* const fr = fx + (yy & 1) * C::X_ROW;
+  auto read_x = [&](bf16x8_t (&f)[3][C::KS], int slot) {
+    const bf16* const fr = fx + slot * C::X_ROW;
 #pragma unroll
     for (int sh = 0; sh < 3; ++sh)
 #pragma unroll
       for (int ks = 0; ks < C::KS; ++ks) f[sh][ks] = wgrad_frag<C::IS>(fr + (sh + 32 * ks) * C::IS);
   };
-  // One dy row; xf[R] holds input row y - 1, xf[R + 1] row y, and row y + 1
-  // is read into xf[R + 2] (indices modulo 3).  Ends with the next dy row
-  // and input row y + 2 in LDS when the strip goes on.
-  auto unit = [&](auto rot, int n, int y, int xs, bool more) {
+  // One dy row, R = its number in the strip modulo 3.  xf[R] holds input row
+  // y - 1, xf[R + 1] row y, and row y + 1 is read from ring place R + 2 into
+  // xf[R + 2] (indices modulo 3).  Ends with dy row y + 1 and input row y + 2
+  // (ring place R) in LDS and the rows behind them under way, as far as the
+  // run's `left` rows of the strip go on.
+  auto unit = [&](auto rot, int n, int y, int xs, int left) {
     constexpr int R = decltype(rot)::value;
-    const bool more_x = more && y + 2 < H;
-    if (more) load_dy(n, y + 1, xs);
-    if (more_x) load_x(n, y + 2, xs);
+    if (left > 2) {
+      load_dy(vd[(R + 2) % 3], n, y + 2, xs);
+      if (y + 3 < H) load_x(vx[(R + 1) % 3], n, y + 3, xs);
+    }
     if (active) {
-      if (y + 1 < H) read_x(xf[(R + 2) % 3], y + 1);
+      if (y + 1 < H) read_x(xf[(R + 2) % 3], (R + 2) % 3);
 #pragma unroll
       for (int ks = 0; ks < C::KS; ++ks) {
         bf16x8_t a[SPW];
@@ -928,42 +961,42 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TCO == 64 ?
         }
       }
     }
-    if (more) {
-      store_dy(y + 1);
-      if (more_x) store_x(y + 2);
-      __syncthreads();
+    if (left > 1) {
+      store_dy(vd[(R + 1) % 3], y + 1);
+      if (y + 2 < H) store_x(vx[R], R);
+      lds_barrier();
     }
   };
   for (int u = u0; u < u1;) {
     // a new strip or image
     const int row = u % rows, n = row / H, y0 = row % H, xs = (u / rows) * WG_SEG;
     const int y1 = min(H, y0 + (u1 - u));  // this run's dy rows of it: y0 .. y1 - 1
-    __syncthreads();  // the previous rows are read
-    load_dy(n, y0, xs);
-    store_dy(y0);
-    if (y0 > 0) {
-      load_x(n, y0 - 1, xs);
-      store_x(y0 - 1);
-    }
-    load_x(n, y0, xs);
-    store_x(y0);
-    __syncthreads();
+    places(xs);
+    // the first rows, all loads at once
+    load_dy(vd[0], n, y0, xs);
+    if (y0 > 0) load_x(vx[0], n, y0 - 1, xs);
+    load_x(vx[1], n, y0, xs);
+    if (y0 + 1 < H) load_x(vx[2], n, y0 + 1, xs);
+    if (y0 + 1 < y1) load_dy(vd[1], n, y0 + 1, xs);
+    lds_barrier();  // the previous rows are read
+    store_dy(vd[0], y0);
+    if (y0 > 0) store_x(vx[0], 0);
+    if (y0 + 1 < y1 && y0 + 2 < H) load_x(vx[0], n, y0 + 2, xs);
+    store_x(vx[1], 1);
+    if (y0 + 1 < H) store_x(vx[2], 2);
+    lds_barrier();
     if (active) {
-      if (y0 > 0) read_x(xf[0], y0 - 1);
-      read_x(xf[1], y0);
+      if (y0 > 0) read_x(xf[0], 0);
+      read_x(xf[1], 1);
     }
-    __syncthreads();  // row y0 - 1 makes room for row y0 + 1
-    if (y0 + 1 < H) {
-      load_x(n, y0 + 1, xs);
-      store_x(y0 + 1);
-    }
-    __syncthreads();
+    // row y0 + 2 is stored over row y0 - 1 at the end of the first unit
+    if (y0 > 0 && y0 + 1 < y1) lds_barrier();
     for (int y = y0; y < y1;) {
-      unit(std::integral_constant<int, 0>(), n, y, xs, y + 1 < y1);
+      unit(std::integral_constant<int, 0>(), n, y, xs, y1 - y);
       if (++y >= y1) break;
-      unit(std::integral_constant<int, 1>(), n, y, xs, y + 1 < y1);
+      unit(std::integral_constant<int, 1>(), n, y, xs, y1 - y);
       if (++y >= y1) break;
-      unit(std::integral_constant<int, 2>(), n, y, xs, y + 1 < y1);
+      unit(std::integral_constant<int, 2>(), n, y, xs, y1 - y);
       ++y;
     }
     u += y1 - y0;
@@ -1435,8 +1468,13 @@ int wgrad_runs(int N, int H, int W, int Cin, int Cout) {
 template <int TCO, int TCI, int SPW>
 void launch_wgrad(dim3 grid, hipStream_t s, View x, View up, int Cup, View dy, float* work, int N, int H, int W,
                   int Cin, int Cout, int runs, int with_bias) {
-  hipLaunchKernelGGL((k_wgrad_mfma<TCO, TCI, SPW>), grid, dim3(256), 0, s, x, up, Cup, dy, work, N, H, W, Cin, Cout,
-                     runs, with_bias);
+  // buffer loads reach 2 GiB from a strip's first pixel
+  if (2ll * (WG_SEG + 2) * std::max({x.cs, Cup ? up.cs : 0, dy.cs}) < (1ll << 31) - 65536)
+    hipLaunchKernelGGL((k_wgrad_mfma<TCO, TCI, SPW, false>), grid, dim3(256), 0, s, x, up, Cup, dy, work, N, H, W, Cin,
+                       Cout, runs, with_bias);
+  else
+    hipLaunchKernelGGL((k_wgrad_mfma<TCO, TCI, SPW, true>), grid, dim3(256), 0, s, x, up, Cup, dy, work, N, H, W, Cin,
+                       Cout, runs, with_bias);
 }
 }  // namespace
 

@@ -155,6 +155,23 @@ def test_conv3x3_of_widely_spaced_pixels(rf, gpu_available, Cin, Cout):
     assert ((out[0].float() - ref.permute(0, 2, 3, 1)).abs() <= 2.0 ** -8 * ref.permute(0, 2, 3, 1).abs() + 1e-4).all()
 
 
+def test_conv3x3_wgrad_of_widely_spaced_pixels(rf, gpu_available):
+    import torch
+    ctx = rf.Context(1 << 12, 1, 16)
+    g = torch.Generator().manual_seed(3)
+    N, H, W, Cin, Cout, cs = 1, 5, 3, 32, 32, 1 << 24
+    x, dy = _bf16(torch.randn(N, H, W, Cin, generator=g)).cuda(), _bf16(torch.randn(N, H, W, Cout, generator=g)).cuda()
+    far = torch.empty(N, H, W, cs, dtype=torch.bfloat16, device="cuda")
+    far[..., cs - Cin:] = x
+    out = []
+    for v, xs, xo in ((x, Cin, 0), (far, cs, cs - Cin)):
+        dw, db = torch.zeros(3, 3, Cout, Cin, device="cuda"), torch.zeros(Cout, device="cuda")
+        ctx.check(ctx.L.rf_nn_conv3x3_wgrad(ctx.h, v.data_ptr(), xs, xo, dy.data_ptr(), Cout, 0, dw.data_ptr(),
+                                            db.data_ptr(), N, H, W, Cin, Cout))
+        out.append((dw.cpu(), db.cpu()))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
 # One pixel, tiles of exactly 8 rows x 64 pixels and one more of each, images
 # that end inside a tile, more tiles than workgroups, three channel blocks.
 @pytest.mark.parametrize("Cin,Cout,N,H,W", [(16, 32, 1, 1, 1), (32, 32, 1, 8, 64), (32, 16, 2, 9, 65),
