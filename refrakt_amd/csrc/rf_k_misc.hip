@@ -178,9 +178,10 @@ __global__ __launch_bounds__(256) void k_de_radius(DEArgs g) {
   g.rad[i] = (uint8_t)v;
 }
 
-// Density estimation of a 64 x (8 V) tile of texels per workgroup of eight
-// waves, for any radius up to 100 (bound: VALU issue).  A wave owns V adjacent
-// texel rows of 64 columns, so the source row, the radius and the splat rows
+// Density estimation of a 64 x (8 V / S) tile of texels per workgroup of eight
+// waves, for any radius up to 100 (bound: VALU issue; for an image of few
+// tiles the chain of a wave's source rows, which S waves then share).  A wave
+// owns V adjacent texel rows of 64 columns and every S-th of their source rows, so the source row, the radius and the splat rows
 // it visits are uniform over the wave: the loop over them runs on the scalar
 // unit and the chord table is read with scalar loads.  LDS holds, per source
 // row, one column mask per radius (the sources whose radius is exactly r) and
@@ -224,8 +225,9 @@ __device__ __forceinline__ DEVisit<V> de_visit(CDETable* tab, int r, int i, int 
 
 // LDS words per source row of the tile: colours, masks, radii present.
 __host__ __device__ inline int dr_mask_words(int R) { return ((DR_W - 1 + 2 * R) >> 5) + 2; }
-inline uint64_t dr_tiles(uint32_t W, uint32_t H, int V) {
-  return ((uint64_t)W + DR_W - 1) / DR_W * (((uint64_t)H + DR_WAVES * V - 1) / (DR_WAVES * V));
+inline uint64_t dr_tiles(uint32_t W, uint32_t H, int V, int S = 1) {
+  const int th = DR_WAVES / S * V;
+  return ((uint64_t)W + DR_W - 1) / DR_W * (((uint64_t)H + th - 1) / th);
 }
 inline size_t dr_row_bytes(int R) {
   return (size_t)(R + 1) * dr_mask_words(R) * 4 + (R < 32 ? 4u : 16u);
@@ -281,21 +283,22 @@ __device__ __forceinline__ void de_taps(float4 (&acc)[V], const DEVisit<V>& v, i
 }
 
 // Adds a strip's sources to the wave's V texel rows.
-template <int V, int NRW, bool ALL, bool SHORT>
+template <int V, int NRW, int S, bool ALL, bool SHORT>
 __device__ __forceinline__ void de_strip(float4 (&acc)[V], CDETable* tab, const float4* src, int W, const uint32_t* s_e,
                                          const uint32_t* s_rp, int R, int K, int s0, int rows) {
   const int lane = threadIdx.x & (WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int nwd = dr_mask_words(R), mrow = (R + 1) * nwd;
-  // this wave's texel rows lie i0 - k .. i0 - k + V - 1 rows from source row k
-  const int i0 = wave * V + R - s0;
+  // this wave's texel rows lie i0 - k .. i0 - k + V - 1 rows from source row k;
+  // it takes every S-th of their source rows
+  const int i0 = wave / S * V + R - s0;
   const int k0 = max(0, i0 - R), k1 = min(rows, i0 + V + R);
 #pragma unroll
   for (int w = 0; w < NRW; ++w) {
     if (32 * w > R) break;
     // lane k holds the radii present in source row k of the strip
     const int rpv = (int)s_rp[w * K + (lane < rows ? lane : 0)];
-    for (int k = k0; k < k1; ++k) {
+    for (int k = k0 + wave % S; k < k1; k += S) {
       const int i = i0 - k;
       const int iw = i > 0 ? i : (i + V - 1 < 0 ? i + V - 1 : 0);  // the row nearest the centre
       const int low = (iw < 0 ? -iw : iw) - 32 * w;
@@ -323,9 +326,10 @@ __device__ __forceinline__ void de_strip(float4 (&acc)[V], CDETable* tab, const 
 }
 
 // SHORT: chords of at most 31 columns (radius below 16).  NRW words of 32
-// radii each.
-template <int V, int NRW, bool SHORT>
+// radii each.  S: waves that share a texel row.
+template <int V, int NRW, bool SHORT, int S>
 __global__ __launch_bounds__(64 * DR_WAVES) __attribute__((amdgpu_waves_per_eu(8))) void k_de_rows(DEArgs g, int K) {
+  constexpr int TH = DR_WAVES / S * V;  // texel rows of the tile
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ int s_odd;  // the strip holds a source that is not finite
   const int R = max(g.R, g.rmin);  // span
@@ -336,9 +340,9 @@ __global__ __launch_bounds__(64 * DR_WAVES) __attribute__((amdgpu_waves_per_eu(8
   const int lane = threadIdx.x & (WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int W = (int)g.W, H = (int)g.H;
-  const uint32_t ny = (uint32_t)(H + DR_WAVES * V - 1) / (DR_WAVES * V);
+  const uint32_t ny = (uint32_t)(H + TH - 1) / TH;
   const uint32_t tile = blockIdx.x;  // down the columns of tiles: neighbours share source rows in L2
-  const int tx0 = (int)(tile / ny) * DR_W, ty0 = (int)(tile % ny) * (DR_WAVES * V);
+  const int tx0 = (int)(tile / ny) * DR_W, ty0 = (int)(tile % ny) * TH;
   CDETable* const tab = (CDETable*)g.tab;
   float4 acc[V];
 #pragma unroll
@@ -347,7 +351,7 @@ __global__ __launch_bounds__(64 * DR_WAVES) __attribute__((amdgpu_waves_per_eu(8
   // the bin of source row 0, window column 0 (read only where a mask bit is set)
   const float4* const src = g.hist + ((ptrdiff_t)(H - 1 - ty0 + R) * W + tx0 - R + 1);
   // source row s of the tile is texel row ty0 - R + s of the image
-  const int s_begin = max(0, R - ty0), s_end = min(DR_WAVES * V + 2 * R, H - ty0 + R);
+  const int s_begin = max(0, R - ty0), s_end = min(TH + 2 * R, H - ty0 + R);
   for (int s0 = s_begin; s0 < s_end; s0 += K) {  // workgroup-uniform
     const int rows = min(K, s_end - s0);
     __syncthreads();  // the previous strip is read
@@ -395,14 +399,31 @@ __global__ __launch_bounds__(64 * DR_WAVES) __attribute__((amdgpu_waves_per_eu(8
         if (lane == 0) s_rp[w * K + k] = rp[w];
     }
     __syncthreads();
-    if (__builtin_amdgcn_readfirstlane(s_odd) == 0) de_strip<V, NRW, true, SHORT>(acc, tab, src, W, s_e, s_rp, R, K, s0, rows);
-    else de_strip<V, NRW, false, SHORT>(acc, tab, src, W, s_e, s_rp, R, K, s0, rows);
+    if (__builtin_amdgcn_readfirstlane(s_odd) == 0) de_strip<V, NRW, S, true, SHORT>(acc, tab, src, W, s_e, s_rp, R, K, s0, rows);
+    else de_strip<V, NRW, S, false, SHORT>(acc, tab, src, W, s_e, s_rp, R, K, s0, rows);
+  }
+  if constexpr (S > 1) {  // the shares of a row's waves, added in their order
+    float4* const s_part = reinterpret_cast<float4*>(smem);  // [q][wave][lane], over the masks
+    __syncthreads();  // the last strip is read
+#pragma unroll
+    for (int q = 0; q < V; ++q) s_part[(q * DR_WAVES + wave) * WAVE + lane] = acc[q];
+    __syncthreads();
+    if (wave % S == 0) {
+#pragma unroll
+      for (int q = 0; q < V; ++q)
+#pragma unroll
+        for (int p = 1; p < S; ++p) {
+          const float4 v = s_part[(q * DR_WAVES + wave + p) * WAVE + lane];
+          acc[q].x += v.x; acc[q].y += v.y; acc[q].z += v.z; acc[q].w += v.w;
+        }
+    }
   }
   const int tx = tx0 + lane;
 #pragma unroll
   for (int q = 0; q < V; ++q) {
     __builtin_amdgcn_sched_barrier(0);  // one tonemap's registers at a time
-    const int ty = ty0 + wave * V + q;
+    if (wave % S != 0) break;
+    const int ty = ty0 + wave / S * V + q;
     if (tx < W && ty < H) {
       const size_t o = (size_t)ty * W + tx;
       if (g.de_out) g.de_out[o] = acc[q];
@@ -504,16 +525,17 @@ hipError_t launch_de_chords(DETable* tab, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int V>
+template <int V, int S = 1>
 static void launch_de_rows(const DEArgs& a, int R, hipStream_t s) {
   // all source rows of the tile at once while their masks fit 32 KiB (four
   // workgroups per CU, as many as its waves allow)
   const size_t row = dr_row_bytes(R);
-  const int K = (int)std::min<size_t>({(size_t)(DR_WAVES * V + 2 * R), (size_t)WAVE, (size_t)32768 / row});
-  const dim3 grid((unsigned)dr_tiles(a.W, a.H, V));
-  if (R < 16) hipLaunchKernelGGL((k_de_rows<V, 1, true>), grid, dim3(64 * DR_WAVES), K * row, s, a, K);
-  else if (R < 32) hipLaunchKernelGGL((k_de_rows<V, 1, false>), grid, dim3(64 * DR_WAVES), K * row, s, a, K);
-  else hipLaunchKernelGGL((k_de_rows<V, 4, false>), grid, dim3(64 * DR_WAVES), K * row, s, a, K);
+  const int K = (int)std::min<size_t>({(size_t)(DR_WAVES / S * V + 2 * R), (size_t)WAVE, (size_t)32768 / row});
+  const size_t lds = std::max(K * row, S > 1 ? (size_t)V * DR_WAVES * WAVE * 16 : 0);
+  const dim3 grid((unsigned)dr_tiles(a.W, a.H, V, S));
+  if (R < 16) hipLaunchKernelGGL((k_de_rows<V, 1, true, S>), grid, dim3(64 * DR_WAVES), lds, s, a, K);
+  else if (R < 32) hipLaunchKernelGGL((k_de_rows<V, 1, false, S>), grid, dim3(64 * DR_WAVES), lds, s, a, K);
+  else hipLaunchKernelGGL((k_de_rows<V, 4, false, S>), grid, dim3(64 * DR_WAVES), lds, s, a, K);
 }
 
 hipError_t launch_de_tonemap(const DEArgs& a, hipStream_t s) {
@@ -526,17 +548,33 @@ hipError_t launch_de_tonemap(const DEArgs& a, hipStream_t s) {
     return hipGetLastError();
   }
   hipLaunchKernelGGL(k_de_radius, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
-  // Texel rows per wave.  Four share the most work per source but need many
-  // tiles to fill the chip and to even out its last round; the wider the
-  // splat, the sooner that pays.  Measured (us, 4 / 2 / 1 rows; the 32 x 32
-  // tiles in LDS they replace, and the global gather beyond radius 15):
-  // 7680x4320 radius 9: 1365 / 1720 / 2760 (1780); 2048x2048 radius 9: 240 /
-  // 236 / 329 (268), radius 24: 789 / 811 / 1252 (22258); 1920x1080 radius 9:
-  // 161 / 149 / 210 (178), radius 24: 585 / 553 / 879 (13743); 512x512 radius
-  // 9: 88 / 64 / 70 (85); 320x240 radius 9: 65 / 51 / 45 (57).
-  if (dr_tiles(a.W, a.H, 4) * (uint64_t)(R + 16) >= 65536) launch_de_rows<4>(a, R, s);
-  else if (dr_tiles(a.W, a.H, 2) >= 128) launch_de_rows<2>(a, R, s);
-  else launch_de_rows<1>(a, R, s);
+  // Texel rows per wave (V) and waves per texel row (S), by the 64 x 32 tiles
+  // of the image.  Four rows share the most work per source but leave the fewest
+  // waves; several waves a row put back the waves, and shorten the chain of
+  // source rows that bounds an image of few tiles, for a sum through LDS and
+  // masks built for fewer texels.  Measured (us, the tonemap included; V/S):
+  //               4/1   4/2   4/4   2/1   2/2   2/8
+  //   320x240  R9   64    50    42    49    39    29   (1/1, one wave a row: 45)
+  //           R24  177   108    75   140    90    52
+  //   900x480  R4   55    51    50    47    43    50
+  //            R9   89    75    64    77    63    73
+  //           R24  320   210   159   271   204   185
+  //   1900x1000 R1  53    59    66    50    55    84
+  //            R9  124   111   110   119   111   160
+  //           R24  394   299   256   403   320   389
+  //   2600x1400 R1  82    95   116    78    94   153
+  //            R7  153   154   177   157   169   280
+  //           R24  585   495   495   672   629   887
+  //   3000x1600 R9 284   287   349   325   355   578
+  //           R15  502   471   525   611   625   946
+  // and at 5000x2700 radius 15 843 with 4/1.
+  const uint64_t t = dr_tiles(a.W, a.H, 4);
+  if (t < 192) launch_de_rows<2, 8>(a, R, s);
+  else if (R < 4 && t < 2560) launch_de_rows<2, 1>(a, R, s);
+  else if (t < 1280 && R < 9) launch_de_rows<2, 2>(a, R, s);
+  else if (t < 1280) launch_de_rows<4, 4>(a, R, s);
+  else if (t < 4096 && R >= 12) launch_de_rows<4, 2>(a, R, s);
+  else launch_de_rows<4, 1>(a, R, s);
   return hipGetLastError();
 }
 

@@ -408,6 +408,15 @@ def test_density_estimation_tiles_vs_oracle(rf, orc, gpu_available, W, H, R, rmi
     assert np.abs(out.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()
 
 
+# One, two, four and eight waves per texel row: small radii, chords of 32
+# columns and more, ragged edges, rows with fewer source rows than waves.
+@pytest.mark.parametrize("W,H,R,density", [(1030, 421, 3, 0.3), (1027, 419, 1, 0.3), (1030, 421, 6, 0.3),
+                                           (1025, 422, 14, 0.1), (1025, 422, 40, 0.01), (2501, 1101, 13, 0.02),
+                                           (2501, 1101, 33, 0.004), (64, 1, 2, 1.0), (67, 3, 24, 0.5)])
+def test_density_estimation_shared_rows_vs_oracle(rf, orc, gpu_available, W, H, R, density):
+    test_density_estimation_tiles_vs_oracle(rf, orc, gpu_available, W, H, R, 0, 0.35, density)
+
+
 @pytest.mark.parametrize("W,H,R", [(97, 75, 9), (1030, 129, 20)])
 def test_density_estimation_keeps_an_infinity_in_its_splat(rf, orc, gpu_available, W, H, R):
     """A bin with an infinite colour reaches the texels of its own splat only."""
