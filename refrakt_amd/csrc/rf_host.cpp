@@ -547,6 +547,36 @@ static uint32_t sort_subdraw_passes(uint64_t P) {
   return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(64, by_samples));
 }
 
+// Records per segment of a tile of capacity cap under a plan's seg_len.
+static uint32_t tile_seg_len(uint32_t cap, uint32_t seg_len) {
+  return seg_len ? seg_len : cap > (uint32_t)rfk::SORT_SEG16 ? (uint32_t)rfk::SORT_SEG15 : (uint32_t)rfk::SORT_SEG16;
+}
+
+// A plan's seg_len (SortArgs) for S samples spread as frac.  A segment's
+// workgroup sums a record in about 0.44 ns, so in a small image the fullest
+// tile decides the pass: a 320x240 draw of 15 passes of 16384 particles has a
+// quarter of its records in one of 19 tiles, and took 36 us (12 now).  Shorter
+// segments spread it over the idle compute units, but a tile of several
+// segments adds its touched bins by quad atomics, 17 per ns over the whole
+// chip.  The length with the least of both; images of 512 tiles and more fill
+// the chip by tiles.
+static uint32_t sort_seg_len(const uint32_t* tcap, const double* frac, uint32_t nt, double S) {
+  if (nt >= 512) return 0;
+  uint32_t best = 0;
+  double least = 0.0;
+  for (const uint32_t len : {0u, 65532u, 32768u, 16384u, 8192u, 4096u}) {
+    double longest = 0.0, quads = 0.0;
+    for (uint32_t t = 0; t < nt; ++t) {
+      const double l = tile_seg_len(tcap[t], len), n = S * frac[t];
+      longest = std::max(longest, std::min(l, n));
+      if (tcap[t] > l) quads += std::ceil(n / l) * std::min(std::min(l, n), (double)(1 << rfk::SORT_TILE_SHIFT));
+    }
+    const double ns = 0.44 * longest + quads / 17.0;
+    if (len == 0u || ns < least) { least = ns; best = len; }
+  }
+  return best;
+}
+
 // Capacities of the next sort draw from the last one's distribution (20 %
 // headroom).  Without one, from the samples the histogram already holds (the
 // first draw in AUTO mode is an LDS draw into it), else 3x the mean.  Uploads
@@ -558,7 +588,7 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   const uint32_t nt = nb * rfk::SORT_TILES_PER_BUCKET;
   const uint32_t nt_used = (uint32_t)((n_bins + (1u << rfk::SORT_TILE_SHIFT) - 1) >> rfk::SORT_TILE_SHIFT);
   // Buffers that only grow, shared by the context's flames.
-  auto bind = [&](const uint32_t* dm, size_t fixed, uint32_t n_chunks, uint32_t n_segs) {
+  auto bind = [&](const uint32_t* dm, size_t fixed, uint32_t n_chunks, uint32_t n_segs, uint32_t seg_len) {
     a.cbuf = (uint32_t*)ctx->sort_cbuf.p;
     a.tbuf = (uint32_t*)ctx->sort_tbuf.p;
     a.bcur = (uint32_t*)ctx->sort_bcur.p;
@@ -573,6 +603,7 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
     a.n_tiles = nt;
     a.n_chunks = n_chunks;
     a.n_segs = n_segs;
+    a.seg_len = seg_len;
   };
   // A plan covers up to twice the draw it is made for (at most a full
   // sub-draw), so the next draw of up to that size reuses it: the same draw
@@ -583,7 +614,8 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   // capacities and work lists on the device still fit.
   if (!f->sort_meta.empty() && S <= f->sort_meta_S && 4 * S >= f->sort_meta_S && f->sort_meta_bins == n_bins &&
       f->sort_bins == n_bins && f->last_sort_overflow == 0.0) {
-    bind((const uint32_t*)f->sort_meta_dev.p, f->sort_meta_fixed, f->sort_meta_chunks, f->sort_meta_segs);
+    bind((const uint32_t*)f->sort_meta_dev.p, f->sort_meta_fixed, f->sort_meta_chunks, f->sort_meta_segs,
+         f->sort_meta_seg_len);
     return RF_OK;
   }
   if (f->sort_bins != n_bins || f->sort_bfrac.size() != nb) {
@@ -644,14 +676,12 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   const uint32_t n_chunks = (uint32_t)jobs.size();
   // tile segments, the largest first so that the long workgroups start early
   std::vector<std::pair<uint32_t, uint32_t>> segs;  // (records the segment can hold, job)
+  const uint32_t seg_len = sort_seg_len(tcap, f->sort_tfrac.data(), nt_used, (double)S);
   for (uint32_t t = 0; t < nt_used; ++t) {
-    if (tcap[t] <= (uint32_t)rfk::SORT_SEG16) {
-      segs.emplace_back(tcap[t], t << 16);
-      continue;
-    }
-    for (uint32_t k = 0; k * (uint64_t)rfk::SORT_SEG15 < tcap[t]; ++k) {
+    const uint32_t len = tile_seg_len(tcap[t], seg_len);
+    for (uint32_t k = 0; k * (uint64_t)len < tcap[t]; ++k) {
       if (k > 0xffffu) return set_err(ctx, RF_ERR_LIMIT, "sort histogram: tile too large");
-      segs.emplace_back(std::min<uint32_t>(tcap[t] - k * (uint32_t)rfk::SORT_SEG15, rfk::SORT_SEG15), (t << 16) | k);
+      segs.emplace_back(std::min<uint32_t>(tcap[t] - k * len, len), (t << 16) | k);
     }
   }
   order_segments(segs);
@@ -676,13 +706,14 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   memcpy(ctx->meta_stage.p, meta.data(), meta.size() * 4);
   HIPCHK(ctx, hipMemcpyAsync(f->sort_meta_dev.p, ctx->meta_stage.p, meta.size() * 4, hipMemcpyHostToDevice,
                              ctx->stream));
-  bind((const uint32_t*)f->sort_meta_dev.p, meta_fixed, n_chunks, n_segs);
+  bind((const uint32_t*)f->sort_meta_dev.p, meta_fixed, n_chunks, n_segs, seg_len);
   f->sort_meta.swap(meta);
   f->sort_meta_S = Sp;
   f->sort_meta_bins = n_bins;
   f->sort_meta_fixed = meta_fixed;
   f->sort_meta_chunks = n_chunks;
   f->sort_meta_segs = n_segs;
+  f->sort_meta_seg_len = seg_len;
   return RF_OK;
 }
 

@@ -218,12 +218,12 @@ __global__ __launch_bounds__(TILE_THREADS) void k_sort_tiles(SortArgs a, float4*
   const uint32_t cap = a.tcap[t];
   const uint32_t cur = a.tcur[t];
   const uint32_t count = cur < cap ? cur : cap;
-  // workgroup-uniform: a tile of at most SORT_SEG16 records is one segment
-  // summed at 2^16 - 1 per unit, a larger one segments of SORT_SEG15 at
-  // 2^15 - 1
-  const bool split = cap > (uint32_t)SORT_SEG16;
-  const uint32_t seg = split ? (uint32_t)SORT_SEG15 : (uint32_t)SORT_SEG16;
-  const float one = split ? 32767.0f : 65535.0f;
+  // workgroup-uniform: a tile of at most SORT_SEG16 records is summed at
+  // 2^16 - 1 per unit, a larger one at 2^15 - 1 in segments of SORT_SEG15 (both
+  // in shorter segments where the plan says so)
+  const bool large = cap > (uint32_t)SORT_SEG16;
+  const uint32_t seg = a.seg_len ? a.seg_len : large ? (uint32_t)SORT_SEG15 : (uint32_t)SORT_SEG16;
+  const float one = large ? 32767.0f : 65535.0f;
   const uint32_t start = (job & 0xffffu) * seg;
   if (base >= n_bins || start >= count) return;  // workgroup-uniform
   const uint32_t n = (count - start) < seg ? (count - start) : seg;
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_sort_tiles(SortArgs a, float4*
     s_t.pal[tid].b = bl;
   }
   __syncthreads();
-  // Tile offsets and both segment sizes are multiples of 4 records, so the
+  // Tile offsets and the segment sizes are multiples of 4 records, so the
   // segment starts 16-byte aligned.
   const uint32_t* src = a.tbuf + a.toff[t] + start;
   const uint4* src4 = reinterpret_cast<const uint4*>(src);

@@ -25,7 +25,8 @@ constexpr int SORT_CHUNK = 16384;                                            // 
 // records is summed by one workgroup at 2^16 - 1 per unit (a field then
 // holds at most 65532 * 65535 < 2^32, so no carry crosses into the next); a
 // larger tile is split into segments of at most SORT_SEG15 records, each
-// summed by its own workgroup at 2^15 - 1 per unit (131068 * 32767 < 2^32).
+// summed by its own workgroup at 2^15 - 1 per unit (131068 * 32767 < 2^32).  A
+// plan for a small image may cut either kind into shorter segments (seg_len).
 // Each sample's colour is rounded by at most 1 / (2 * 65535) or
 // 1 / (2 * 32767), about 2^-17 and 2^-16.
 constexpr int SORT_SEG16 = 65532;
@@ -46,6 +47,7 @@ struct SortArgs {
   uint32_t n_buckets;
   uint32_t n_tiles;        // n_buckets * SORT_TILES_PER_BUCKET
   uint32_t n_chunks, n_segs;
+  uint32_t seg_len;        // records per segment of a tile; 0: SORT_SEG16, or SORT_SEG15 of a tile that holds more
   // Batched rendering: per tile, the offset (in entries) of its frame's
   // palette in the palette array the record passes get; null when one
   // palette serves every tile.

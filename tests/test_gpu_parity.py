@@ -194,6 +194,38 @@ def test_fast_sort_stage_over_batches(rf, orc, gpu_available, waves, batches, pa
     assert np.array_equal(g_hist[..., 3].astype(np.uint32), hits)
 
 
+@pytest.mark.parametrize("P,passes,W,H", [(1 << 16, 16, 192, 160), (1 << 14, 15, 320, 240), (1 << 17, 8, 64, 64),
+                                          (1 << 15, 7, 700, 500)])
+def test_fast_sort_short_segments(rf, orc, gpu_available, P, passes, W, H):
+    """Small images: a full tile is summed in segments by several workgroups.
+    Two draws (the second planned from the first's distribution), counts and
+    positions exact, colours within the fixed point's rounding."""
+    seed, waves = 5, 8
+    fl = _linear_flame(rf, 29, W=W, H=H)
+    print(f"short segments: {W}x{H} P={P} passes={passes}", flush=True)
+    ctx = _ctx(rf, P, 1, rf.RF_ENGINE_FAST, hist_mode=rf.RF_HIST_SORT, seed=seed, waves=waves)
+    fh = ctx.flame(fl)
+    hist = ctx.histogram(W, H)
+    fh.warmup(0)
+    drawn = fh.draw_to_bins(hist, passes) + fh.draw_to_bins(hist, passes)
+    g_hist = hist.download()
+    fc = orc.flame_to_c(fl)
+    ss = orc.screen_affine(fl, W, H)
+    perms = ctx.fast_perms(waves)
+    pos = np.zeros((P, 4), np.float32)
+    orc.fast_run(fc, P, P, waves, perms, seed, 0, 1, True, False, W, H, ss, pos)
+    bins = np.zeros((H, W, 4), np.float64)
+    hits = np.zeros((H, W), np.uint32)
+    o_drawn = sum(orc.fast_run(fc, P, P, waves, perms, seed, k, passes, False, True, W, H, ss, pos, bins, hits)
+                  for k in (1, 2))
+    assert drawn == o_drawn > 0
+    assert np.array_equal(fh.particles().view(np.uint32), pos.view(np.uint32))
+    assert np.array_equal(g_hist[..., 3].astype(np.uint32), hits)
+    # a sample's colour is rounded by 1 / (2 * 32767) at most
+    tol = 1e-5 + 1e-5 * np.abs(bins[..., :3]) + hits[..., None] / 65534.0
+    assert (np.abs(g_hist[..., :3].astype(np.float64) - bins[..., :3]) <= tol).all()
+
+
 # ------------------------------------------------- non-finite particle policy
 def _nan_xform(rf, kind):
     """An xform whose output is never finite: a NaN variation weight, or an
