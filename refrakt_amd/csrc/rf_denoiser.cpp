@@ -182,6 +182,15 @@ int backward(rf_denoiser* d, const bf16* x, int N, int H, int W) {
     f.mask = y;
     return rfn::conv3x3(dy, wt_of(d, l), nullptr, dx, N, h, w, d->L[l].cout, d->L[l].cin, 0, s, f);
   };
+  // the same for a layer over [upsample(y), skip]: the gradient of the lower
+  // level's y into dlo, that of the skip channels into their place in dx
+  auto dgrad_up = [&](int l, View dy, View dx, int h, int w, View dlo, View y, int c_lo) {
+    rfn::ConvFuse f;
+    f.down = dlo;
+    f.down_mask = y;
+    f.Cdown = c_lo;
+    return rfn::conv3x3(dy, wt_of(d, l), nullptr, dx, N, h, w, d->L[l].cout, d->L[l].cin, 0, s, f);
+  };
   const View vx{(bf16*)x, 16, 0};
   // out and dec0
   HIPCHK(ctx, wgrad(11, V(d->d0b, 32), V(d->g_o, 16), H, W));
@@ -189,17 +198,14 @@ int backward(rf_denoiser* d, const bf16* x, int N, int H, int W) {
   HIPCHK(ctx, wgrad(10, V(d->d0a, 32), V(d->g_d0b, 32), H, W));
   HIPCHK(ctx, dgrad(10, V(d->g_d0b, 32), V(d->g_d0a, 32), H, W, V(d->d0a, 32)));
   HIPCHK(ctx, wgrad(9, V(d->cat0, 32), V(d->g_d0a, 32), H, W, V(d->d1, 64), 64));
-  HIPCHK(ctx, dgrad(9, V(d->g_d0a, 32), V(d->g_cat0, 96), H, W));
+  HIPCHK(ctx, dgrad_up(9, V(d->g_d0a, 32), V(d->g_cat0, 96), H, W, V(d->g_d1, 64), V(d->d1, 64), 64));
   // dec1
-  HIPCHK(ctx, rfn::upsample2_bwd(V(d->g_cat0, 96, 0), V(d->g_d1, 64), V(d->d1, 64), N, H1, W1, 64, s));
   HIPCHK(ctx, wgrad(8, V(d->cat1, 64), V(d->g_d1, 64), H1, W1, V(d->d2, 128), 128));
-  HIPCHK(ctx, dgrad(8, V(d->g_d1, 64), V(d->g_cat1, 192), H1, W1));
+  HIPCHK(ctx, dgrad_up(8, V(d->g_d1, 64), V(d->g_cat1, 192), H1, W1, V(d->g_d2, 128), V(d->d2, 128), 128));
   // dec2
-  HIPCHK(ctx, rfn::upsample2_bwd(V(d->g_cat1, 192, 0), V(d->g_d2, 128), V(d->d2, 128), N, H2, W2, 128, s));
   HIPCHK(ctx, wgrad(7, V(d->cat2, 128), V(d->g_d2, 128), H2, W2, V(d->b, 256), 256));
-  HIPCHK(ctx, dgrad(7, V(d->g_d2, 128), V(d->g_cat2, 384), H2, W2));
+  HIPCHK(ctx, dgrad_up(7, V(d->g_d2, 128), V(d->g_cat2, 384), H2, W2, V(d->g_b, 256), V(d->b, 256), 256));
   // bottleneck
-  HIPCHK(ctx, rfn::upsample2_bwd(V(d->g_cat2, 384, 0), V(d->g_b, 256), V(d->b, 256), N, H3, W3, 256, s));
   HIPCHK(ctx, wgrad(6, V(d->p2, 128), V(d->g_b, 256), H3, W3));
   HIPCHK(ctx, dgrad(6, V(d->g_b, 256), V(d->g_p2, 128), H3, W3));
   // enc2: skip2 gradient = concat part + pooled path

@@ -308,11 +308,12 @@ __device__ __forceinline__ void conv_store_lds(const float4_t (&acc)[RW][4][NT],
       }
     }
   } else {
+    const bool down = co0 < fz.Cdown;  // workgroup-uniform
 #pragma unroll
     for (int rr = 0; rr < RW; ++rr) {
       const int y = y0 + RW * wave + rr;
       const bf16* const s_o = s_buf + (RW * wave + rr) * CT_W * OS;
-      if (y < H) {
+      if (y < H && !down) {
 #pragma unroll
         for (int q = lane; q < CT_W * PQ; q += 64) {
           const int px = q / PQ, piece = q % PQ;
@@ -326,8 +327,11 @@ __device__ __forceinline__ void conv_store_lds(const float4_t (&acc)[RW][4][NT],
         }
       }
     }
-    if (fz.pool.p) {  // workgroup-uniform: the tile's 2x2 averages, summed in k_avgpool2_v8's order
-      const View& pool = fz.pool;
+    // workgroup-uniform: the tile's 2x2 averages or masked sums, added in
+    // k_avgpool2_v8's order
+    if (fz.pool.p || down) {
+      const View pool = down ? fz.down : fz.pool;
+      const float scale = down ? 1.0f : 0.25f;
       constexpr int PW = CT_W / 2, NPQ = (TR / 2) * PW * PQ;
       for (int q = tid; q < NPQ; q += 256) {
         const int piece = q % PQ, pp = (q / PQ) % PW, pr = q / (PQ * PW);
@@ -347,9 +351,13 @@ __device__ __forceinline__ void conv_store_lds(const float4_t (&acc)[RW][4][NT],
           uint32_t r[4];
 #pragma unroll
           for (int k = 0; k < 4; ++k)
-            r[k] = f2bf2(0.25f * sum[2 * k], 0.25f * sum[2 * k + 1]);
-          *reinterpret_cast<uint4*>(pool.p + ((size_t)(n * (H >> 1) + yo) * (W >> 1) + xo) * pool.cs + pool.co +
-                                    co0 + 8 * piece) = make_uint4(r[0], r[1], r[2], r[3]);
+            r[k] = f2bf2(scale * sum[2 * k], scale * sum[2 * k + 1]);
+          const size_t p = (size_t)(n * (H >> 1) + yo) * (W >> 1) + xo;
+          uint4 v = make_uint4(r[0], r[1], r[2], r[3]);
+          if (down)
+            v = relu_keep(v, *reinterpret_cast<const uint4*>(fz.down_mask.p + p * fz.down_mask.cs + fz.down_mask.co + co0 +
+                                                             8 * piece));
+          *reinterpret_cast<uint4*>(pool.p + p * pool.cs + pool.co + co0 + 8 * piece) = v;
         }
       }
     }
@@ -550,7 +558,9 @@ constexpr int CF_PIX = ct_in_pix(2);
 template <int NT>
 constexpr int conv_few_waves() { return NT == 2 ? 2 : 3; }  // workgroups per CU, by registers
 
-template <int CIN, int NT, bool RELU>
+// DOWN: the launch has fz.Cdown (and no mask or pool, whose registers it would
+// not leave).
+template <int CIN, int NT, bool RELU, bool DOWN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_few_waves<NT>()))) void k_conv3x3_few(
     View in, const bf16* __restrict__ w, const float* __restrict__ bias, View out, int H, int W, int Cout,
     ConvFuse fz, int nbx, int nbz, int n_tiles) {
@@ -725,6 +735,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_few_wa
     bf16* const orow = row(out);
     const uint32_t mlane = (uint32_t)(i * fz.mask.cs + co0 + 4 * NT * kq), olane = (uint32_t)(i * out.cs + co0 + 4 * NT * kq);
     auto inside = [&](int f, int rr) { return y0 + rr < H && x0 + 16 * f + i < W; };
+    const bool down = DOWN && co0 < fz.Cdown;  // workgroup-uniform
     // the mask of this fragment and, where registers allow, the next
     constexpr int MD = conv_few_waves<NT>() == 2 ? 2 : 1;
     Out m[MD][2];
@@ -734,11 +745,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_few_wa
         if (inside(f, rr))
           m[f % MD][rr] = *reinterpret_cast<const Out*>(mrow + (ptrdiff_t)(rr * W + 16 * f) * fz.mask.cs + mlane);
     };
-    if (MD == 2 && fz.mask.p) mask(0);  // workgroup-uniform
+    if (!DOWN && MD == 2 && fz.mask.p) mask(0);  // workgroup-uniform
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
       __builtin_amdgcn_sched_barrier(0);
-      if (fz.mask.p && f + MD - 1 < 4) mask(f + MD - 1);
+      if (!DOWN && fz.mask.p && f + MD - 1 < 4) mask(f + MD - 1);
       Out o[2];
 #pragma unroll
       for (int rr = 0; rr < 2; ++rr) {
@@ -748,12 +759,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_few_wa
         } else {
           o[rr] = out4(acc[rr][f][0], bv[0]);
         }
-        if (!inside(f, rr)) continue;
+        if (down || !inside(f, rr)) continue;
         Out v = o[rr];
-        if (fz.mask.p) v = relu_keep(v, m[f % MD][rr]);
+        if (!DOWN && fz.mask.p) v = relu_keep(v, m[f % MD][rr]);
         *reinterpret_cast<Out*>(orow + (ptrdiff_t)(rr * W + 16 * f) * out.cs + olane) = v;
       }
-      if (fz.pool.p) {  // workgroup-uniform: the 2x2 averages, summed in k_avgpool2_v8's order
+      // workgroup-uniform: the 2x2 averages or masked sums, added in
+      // k_avgpool2_v8's order
+      if (DOWN ? down : fz.pool.p != nullptr) {
+        const View pool = down ? fz.down : fz.pool;
+        const float scale = down ? 1.0f : 0.25f;
         const uint32_t* const r0 = reinterpret_cast<const uint32_t*>(&o[0]);
         const uint32_t* const r1 = reinterpret_cast<const uint32_t*>(&o[1]);
         Out pv;
@@ -765,12 +780,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_few_wa
           const uint32_t b1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)r1[h], 0xB1, 0xf, 0xf, true);
           const float lo = (((0.0f + bf_lo(r0[h])) + bf_lo(a1)) + bf_lo(r1[h])) + bf_lo(b1);
           const float hi2 = (((0.0f + bf_hi(r0[h])) + bf_hi(a1)) + bf_hi(r1[h])) + bf_hi(b1);
-          r[h] = f2bf2(0.25f * lo, 0.25f * hi2);
+          r[h] = f2bf2(scale * lo, scale * hi2);
         }
         const int yo = y0 >> 1, xo = (x0 + 16 * f + i) >> 1;
-        if ((i & 1) == 0 && yo < (H >> 1) && xo < (W >> 1))
-          *reinterpret_cast<Out*>(fz.pool.p + ((size_t)(n * (H >> 1) + yo) * (W >> 1) + xo) * fz.pool.cs + fz.pool.co +
-                                  co0 + 4 * NT * kq) = pv;
+        if ((i & 1) == 0 && yo < (H >> 1) && xo < (W >> 1)) {
+          const size_t p = (size_t)(n * (H >> 1) + yo) * (W >> 1) + xo;
+          const int c = co0 + 4 * NT * kq;
+          if (down)
+            pv = relu_keep(pv, *reinterpret_cast<const Out*>(fz.down_mask.p + p * fz.down_mask.cs + fz.down_mask.co + c));
+          *reinterpret_cast<Out*>(pool.p + p * pool.cs + pool.co + c) = pv;
+        }
       }
     }
   }
@@ -1176,32 +1195,6 @@ __global__ void k_avgpool2_bwd_v8(View dout, View din, View y, int N, int H, int
   *d = relu_keep(make_uint4(r[0], r[1], r[2], r[3]), *reinterpret_cast<const uint4*>(y.p + p * y.cs + y.co + 8 * g));
 }
 
-// Gradient of the 2x upsampling (8 channels per thread), then ReLU's mask of y.
-__global__ void k_upsample2_bwd_v8(View dout, View din, View y, int N, int H, int W, int C) {
-  const int G = C / 8;
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)N * H * W * G) return;
-  const int g = (int)(i % G);
-  const size_t p = i / G;
-  const int x = (int)(p % W), yy = (int)((p / W) % H), n = (int)(p / ((size_t)W * H));
-  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const uint4 v = *reinterpret_cast<const uint4*>(
-          dout.p + ((size_t)(n * 2 * H + 2 * yy + a) * (2 * W) + 2 * x + b) * dout.cs + dout.co + 8 * g);
-      const uint32_t q[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int k = 0; k < 4; ++k) { s[2 * k] += bf_lo(q[k]); s[2 * k + 1] += bf_hi(q[k]); }
-    }
-  uint32_t r[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) r[k] = f2bf2(s[2 * k], s[2 * k + 1]);
-  *reinterpret_cast<uint4*>(din.p + p * din.cs + din.co + 8 * g) =
-      relu_keep(make_uint4(r[0], r[1], r[2], r[3]), *reinterpret_cast<const uint4*>(y.p + p * y.cs + y.co + 8 * g));
-}
-
 inline bool v8_ok(const View& a, const View& b, int C) {
   return C % 8 == 0 && a.cs % 8 == 0 && a.co % 8 == 0 && b.cs % 8 == 0 && b.co % 8 == 0 &&
          ((uintptr_t)a.p & 15u) == 0 && ((uintptr_t)b.p & 15u) == 0;
@@ -1369,6 +1362,10 @@ hipError_t conv3x3(View in, const bf16* w, const float* bias, View out, int N, i
     if (fuse.mask.p && (!vec_out || fuse.y || fuse.mask.cs % 8 || fuse.mask.co % 8 ||
                         ((uintptr_t)fuse.mask.p & 15u) != 0))
       return hipErrorInvalidValue;
+    if (fuse.Cdown && (!vec_out || fuse.y || pool.p || fuse.Cdown % (16 * nt) || fuse.Cdown >= Cout || H % 2 || W % 2 ||
+                       fuse.down.cs % 8 || fuse.down.co % 8 || ((uintptr_t)fuse.down.p & 15u) != 0 ||
+                       fuse.down_mask.cs % 8 || fuse.down_mask.co % 8 || ((uintptr_t)fuse.down_mask.p & 15u) != 0))
+      return hipErrorInvalidValue;
     ConvFuse fz = fuse;
     if (!fuse_pool) fz.pool = View{nullptr, 0, 0};
     if (!fuse_res) { fz.res = View{nullptr, 0, 0}; fz.y = nullptr; }
@@ -1376,22 +1373,25 @@ hipError_t conv3x3(View in, const bf16* w, const float* bias, View out, int N, i
     // another path: the persistent kernel, faster at every size (32 -> 32,
     // with the call's 17 us: 2048^2 223 -> 162 us, 8 x 256^2 43 -> 33, 517 x
     // 333 28 -> 23; 16 -> 32 at 64^2 20.6 -> 17.3).
-    const bool few = (long long)10 * W * in.cs < (1ll << 31) && !k32 && nt <= 2 && Cin <= 32 && !Cup && vec_out && (!pool.p || fuse_pool) && (!fuse.y || fuse_res);
+    const bool few = (long long)10 * W * in.cs < (1ll << 31) && !k32 && nt <= 2 && Cin <= 32 && !Cup && vec_out && (!pool.p || fuse_pool) && (!fuse.y || fuse_res) &&
+                     (!fuse.Cdown || (Cin == 32 && nt == 2 && !relu && !fuse.mask.p));
     if (few) {
       int dev = 0, cus = 0;
       hipError_t e = hipGetDevice(&dev);
       if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
       if (e != hipSuccess) return e;
-#define RF_CONV_FEW(CIN_, NT_, RELU_)                                                                             \
-  hipLaunchKernelGGL((k_conv3x3_few<CIN_, NT_, RELU_>),                                                           \
+#define RF_CONV_FEW(CIN_, NT_, RELU_, DOWN_)                                                                      \
+  hipLaunchKernelGGL((k_conv3x3_few<CIN_, NT_, RELU_, DOWN_>),                                                    \
                      dim3((unsigned)(std::min(n_tiles / nbz, std::max(1, conv_few_waves<NT_>() * cus / nbz)) * nbz)), \
                      dim3(256), 0, s, in, w, bias, out, H, W, Cout, fz, nbx, nbz, n_tiles / nbz)
-      if (relu) {
-        if (Cin == 32) { if (nt == 2) RF_CONV_FEW(32, 2, true); else RF_CONV_FEW(32, 1, true); }
-        else { if (nt == 2) RF_CONV_FEW(16, 2, true); else RF_CONV_FEW(16, 1, true); }
+      if (fuse.Cdown) {
+        RF_CONV_FEW(32, 2, false, true);
+      } else if (relu) {
+        if (Cin == 32) { if (nt == 2) RF_CONV_FEW(32, 2, true, false); else RF_CONV_FEW(32, 1, true, false); }
+        else { if (nt == 2) RF_CONV_FEW(16, 2, true, false); else RF_CONV_FEW(16, 1, true, false); }
       } else {
-        if (Cin == 32) { if (nt == 2) RF_CONV_FEW(32, 2, false); else RF_CONV_FEW(32, 1, false); }
-        else { if (nt == 2) RF_CONV_FEW(16, 2, false); else RF_CONV_FEW(16, 1, false); }
+        if (Cin == 32) { if (nt == 2) RF_CONV_FEW(32, 2, false, false); else RF_CONV_FEW(32, 1, false, false); }
+        else { if (nt == 2) RF_CONV_FEW(16, 2, false, false); else RF_CONV_FEW(16, 1, false, false); }
       }
 #undef RF_CONV_FEW
       return hipGetLastError();
@@ -1430,7 +1430,7 @@ hipError_t conv3x3(View in, const bf16* w, const float* bias, View out, int N, i
       e = residual_loss(fuse.res, out, nullptr, fuse.y, nullptr, nullptr, N * H * W, 0.0f, s);
     return e;
   }
-  if (fuse.mask.p) return hipErrorInvalidValue;
+  if (fuse.mask.p || fuse.Cdown) return hipErrorInvalidValue;
   const dim3 grid((W + 63) / 64, N * H, Cout / (16 * nt));
   switch (nt) {
     case 4: hipLaunchKernelGGL(k_conv3x3<4>, grid, dim3(256), 0, s, in, w, bias, out, H, W, Cin, Cout, relu); break;
@@ -1525,12 +1525,6 @@ hipError_t avgpool2(View in, View out, int N, int H, int W, int C, hipStream_t s
 hipError_t avgpool2_bwd(View dout, View din, View y, int N, int H, int W, int C, hipStream_t s) {
   if (!v8_ok(dout, din, C) || !v8_ok(y, y, C)) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_avgpool2_bwd_v8, grid1((size_t)N * H * W * (C / 8)), dim3(256), 0, s, dout, din, y, N, H, W, C);
-  return hipGetLastError();
-}
-
-hipError_t upsample2_bwd(View dout, View din, View y, int N, int H, int W, int C, hipStream_t s) {
-  if (!v8_ok(dout, din, C) || !v8_ok(y, y, C)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_upsample2_bwd_v8, grid1((size_t)N * H * W * (C / 8)), dim3(256), 0, s, dout, din, y, N, H, W, C);
   return hipGetLastError();
 }
 

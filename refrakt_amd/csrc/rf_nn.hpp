@@ -41,6 +41,13 @@ struct ConvFuse {
   // backward; mask has the output's Cout channels, 16-byte aligned runs as
   // in the input and the output).
   View mask{nullptr, 0, 0};
+  // Cdown > 0: the first Cdown output channels (a multiple of 64 and less than
+  // Cout) are the gradient of a 2x2 upsampling: instead of being written to
+  // `out`, their 2x2 sums (of the bf16 outputs), kept where
+  // down_mask > 0, go to `down`.  H and W even, both views N x H/2 x W/2 with
+  // 16-byte aligned channel runs.
+  View down{nullptr, 0, 0}, down_mask{nullptr, 0, 0};
+  int Cdown = 0;
 };
 hipError_t conv3x3(View in, const bf16* w, const float* bias, View out, int N, int H, int W, int Cin, int Cout,
                    int relu, hipStream_t s, const ConvFuse& fuse = ConvFuse{});
@@ -69,9 +76,6 @@ hipError_t flip_weights_all(const FlipLayers& L, int n_layers, const bf16* w, bf
 // y > 0 (channel runs 16-byte aligned, C a multiple of 8).
 hipError_t avgpool2(View in, View out, int N, int H, int W, int C, hipStream_t s);
 hipError_t avgpool2_bwd(View dout, View din, View y, int N, int H, int W, int C, hipStream_t s);
-// Nearest 2x upsampling (H, W are the input size) and its gradient, kept
-// where y > 0 (channel runs 16-byte aligned, C a multiple of 8).
-hipError_t upsample2_bwd(View dout, View din, View y, int N, int H, int W, int C, hipStream_t s);
 // y = x[:, :4] + o[:, :4] (fp32, 4 channels, when y_out != null); when t != null: loss_sum += sum (y - t)^2 and
 // do = 2 (y - t) / count in channels 0..3, 0 in the rest (16-channel do).
 hipError_t residual_loss(View x, View o, const bf16* t, float* y_out, float* loss_sum, bf16* dO, int npix,
