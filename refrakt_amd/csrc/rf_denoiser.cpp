@@ -69,8 +69,8 @@ int ensure_shape(rf_denoiser* d, int N, int H, int W) {
       {&d->e0a, P0 * 32}, {&d->cat0, P0 * 32}, {&d->p0, P1 * 32}, {&d->e1a, P1 * 64}, {&d->cat1, P1 * 64},
       {&d->p1, P2 * 64}, {&d->e2a, P2 * 128}, {&d->cat2, P2 * 128}, {&d->p2, P3 * 128}, {&d->b, P3 * 256},
       {&d->d2, P2 * 128}, {&d->d1, P1 * 64}, {&d->d0a, P0 * 32}, {&d->d0b, P0 * 32}, {&d->o, P0 * 16},
-      {&d->g_e0a, P0 * 32}, {&d->g_cat0, P0 * 96}, {&d->g_p0, P1 * 32}, {&d->g_e1a, P1 * 64},
-      {&d->g_cat1, P1 * 192}, {&d->g_p1, P2 * 64}, {&d->g_e2a, P2 * 128}, {&d->g_cat2, P2 * 384},
+      {&d->g_e0a, P0 * 32}, {&d->g_cat0, P0 * 32}, {&d->g_p0, P1 * 32}, {&d->g_e1a, P1 * 64},
+      {&d->g_cat1, P1 * 64}, {&d->g_p1, P2 * 64}, {&d->g_e2a, P2 * 128}, {&d->g_cat2, P2 * 128},
       {&d->g_p2, P3 * 128}, {&d->g_b, P3 * 256}, {&d->g_d2, P2 * 128}, {&d->g_d1, P1 * 64},
       {&d->g_d0a, P0 * 32}, {&d->g_d0b, P0 * 32}, {&d->g_o, P0 * 16},
   };
@@ -183,8 +183,11 @@ int backward(rf_denoiser* d, const bf16* x, int N, int H, int W) {
     return rfn::conv3x3(dy, wt_of(d, l), nullptr, dx, N, h, w, d->L[l].cout, d->L[l].cin, 0, s, f);
   };
   // the same for a layer over [upsample(y), skip]: the gradient of the lower
-  // level's y into dlo, that of the skip channels into their place in dx
-  auto dgrad_up = [&](int l, View dy, View dx, int h, int w, View dlo, View y, int c_lo) {
+  // level's y into dlo, that of the skip channels, which follow the c_lo that
+  // are not stored, into dskip (packed: as channels of the whole gradient they
+  // took a third of each pixel's lines)
+  auto dgrad_up = [&](int l, View dy, View dskip, int h, int w, View dlo, View y, int c_lo) {
+    const View dx{dskip.p, dskip.cs, dskip.co - c_lo};
     rfn::ConvFuse f;
     f.down = dlo;
     f.down_mask = y;
@@ -198,32 +201,32 @@ int backward(rf_denoiser* d, const bf16* x, int N, int H, int W) {
   HIPCHK(ctx, wgrad(10, V(d->d0a, 32), V(d->g_d0b, 32), H, W));
   HIPCHK(ctx, dgrad(10, V(d->g_d0b, 32), V(d->g_d0a, 32), H, W, V(d->d0a, 32)));
   HIPCHK(ctx, wgrad(9, V(d->cat0, 32), V(d->g_d0a, 32), H, W, V(d->d1, 64), 64));
-  HIPCHK(ctx, dgrad_up(9, V(d->g_d0a, 32), V(d->g_cat0, 96), H, W, V(d->g_d1, 64), V(d->d1, 64), 64));
+  HIPCHK(ctx, dgrad_up(9, V(d->g_d0a, 32), V(d->g_cat0, 32), H, W, V(d->g_d1, 64), V(d->d1, 64), 64));
   // dec1
   HIPCHK(ctx, wgrad(8, V(d->cat1, 64), V(d->g_d1, 64), H1, W1, V(d->d2, 128), 128));
-  HIPCHK(ctx, dgrad_up(8, V(d->g_d1, 64), V(d->g_cat1, 192), H1, W1, V(d->g_d2, 128), V(d->d2, 128), 128));
+  HIPCHK(ctx, dgrad_up(8, V(d->g_d1, 64), V(d->g_cat1, 64), H1, W1, V(d->g_d2, 128), V(d->d2, 128), 128));
   // dec2
   HIPCHK(ctx, wgrad(7, V(d->cat2, 128), V(d->g_d2, 128), H2, W2, V(d->b, 256), 256));
-  HIPCHK(ctx, dgrad_up(7, V(d->g_d2, 128), V(d->g_cat2, 384), H2, W2, V(d->g_b, 256), V(d->b, 256), 256));
+  HIPCHK(ctx, dgrad_up(7, V(d->g_d2, 128), V(d->g_cat2, 128), H2, W2, V(d->g_b, 256), V(d->b, 256), 256));
   // bottleneck
   HIPCHK(ctx, wgrad(6, V(d->p2, 128), V(d->g_b, 256), H3, W3));
   HIPCHK(ctx, dgrad(6, V(d->g_b, 256), V(d->g_p2, 128), H3, W3));
   // enc2: skip2 gradient = concat part + pooled path
-  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p2, 128), V(d->g_cat2, 384, 256), V(d->cat2, 128), N, H2, W2, 128, s));
-  HIPCHK(ctx, wgrad(5, V(d->e2a, 128), V(d->g_cat2, 384, 256), H2, W2));
-  HIPCHK(ctx, dgrad(5, V(d->g_cat2, 384, 256), V(d->g_e2a, 128), H2, W2, V(d->e2a, 128)));
+  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p2, 128), V(d->g_cat2, 128), V(d->cat2, 128), N, H2, W2, 128, s));
+  HIPCHK(ctx, wgrad(5, V(d->e2a, 128), V(d->g_cat2, 128), H2, W2));
+  HIPCHK(ctx, dgrad(5, V(d->g_cat2, 128), V(d->g_e2a, 128), H2, W2, V(d->e2a, 128)));
   HIPCHK(ctx, wgrad(4, V(d->p1, 64), V(d->g_e2a, 128), H2, W2));
   HIPCHK(ctx, dgrad(4, V(d->g_e2a, 128), V(d->g_p1, 64), H2, W2));
   // enc1
-  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p1, 64), V(d->g_cat1, 192, 128), V(d->cat1, 64), N, H1, W1, 64, s));
-  HIPCHK(ctx, wgrad(3, V(d->e1a, 64), V(d->g_cat1, 192, 128), H1, W1));
-  HIPCHK(ctx, dgrad(3, V(d->g_cat1, 192, 128), V(d->g_e1a, 64), H1, W1, V(d->e1a, 64)));
+  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p1, 64), V(d->g_cat1, 64), V(d->cat1, 64), N, H1, W1, 64, s));
+  HIPCHK(ctx, wgrad(3, V(d->e1a, 64), V(d->g_cat1, 64), H1, W1));
+  HIPCHK(ctx, dgrad(3, V(d->g_cat1, 64), V(d->g_e1a, 64), H1, W1, V(d->e1a, 64)));
   HIPCHK(ctx, wgrad(2, V(d->p0, 32), V(d->g_e1a, 64), H1, W1));
   HIPCHK(ctx, dgrad(2, V(d->g_e1a, 64), V(d->g_p0, 32), H1, W1));
   // enc0
-  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p0, 32), V(d->g_cat0, 96, 64), V(d->cat0, 32), N, H, W, 32, s));
-  HIPCHK(ctx, wgrad(1, V(d->e0a, 32), V(d->g_cat0, 96, 64), H, W));
-  HIPCHK(ctx, dgrad(1, V(d->g_cat0, 96, 64), V(d->g_e0a, 32), H, W, V(d->e0a, 32)));
+  HIPCHK(ctx, rfn::avgpool2_bwd(V(d->g_p0, 32), V(d->g_cat0, 32), V(d->cat0, 32), N, H, W, 32, s));
+  HIPCHK(ctx, wgrad(1, V(d->e0a, 32), V(d->g_cat0, 32), H, W));
+  HIPCHK(ctx, dgrad(1, V(d->g_cat0, 32), V(d->g_e0a, 32), H, W, V(d->e0a, 32)));
   HIPCHK(ctx, wgrad(0, vx, V(d->g_e0a, 32), H, W));
   return RF_OK;
 }
