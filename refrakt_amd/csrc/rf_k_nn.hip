@@ -176,17 +176,17 @@ __device__ __forceinline__ void conv_places(ConvStage<NT, KC, RW>& st, int cs, i
 }
 
 // A 16-byte piece (the piece-th of a pixel `pixels` pixels behind the first) of
-// a row: its place, BUF_NONE for zeros, and its load.
+// a row: its place, BUF_NONE for zeros, and its load.  FAR: 64-bit addresses, at
+// any channel stride.
 template <bool FAR>
 __device__ __forceinline__ uint32_t piece_place(int pixels, int cs, int piece) {
-  const uint32_t unit = (uint32_t)pixels * (uint32_t)(cs / 8) + (uint32_t)piece;
-  return FAR ? unit : 16u * unit;
+  return FAR ? (uint32_t)(16 * pixels + piece) : 2u * (uint32_t)(pixels * cs + 8 * piece);
 }
 template <bool FAR>
-__device__ __forceinline__ uint4 piece_load(const bf16* row, uint32_t place) {
+__device__ __forceinline__ uint4 piece_load(const bf16* row, int cs, uint32_t place) {
   if constexpr (FAR) {
     uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (place != BUF_NONE) v = *reinterpret_cast<const uint4*>(row + 8 * (size_t)place);
+    if (place != BUF_NONE) v = *reinterpret_cast<const uint4*>(row + (size_t)(place / 16) * cs + 8 * (place % 16));
     return v;
   }
   return buf_load(buf_at(row), place, 0);
@@ -914,7 +914,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(wgrad_waves
   auto load_dy = [&](uint4 (&v)[C::DY_PER], int n, int y, int xs) {
     const bf16* const src = dy.p + ((size_t)(n * H + y) * W + xs) * dy.cs + dy.co + co0;
 #pragma unroll
-    for (int k = 0; k < C::DY_PER; ++k) v[k] = piece_load<FAR>(src, pd[k]);
+    for (int k = 0; k < C::DY_PER; ++k) v[k] = piece_load<FAR>(src, dy.cs, pd[k]);
   };
   auto store_dy = [&](const uint4 (&v)[C::DY_PER], int y) {
 #pragma unroll
@@ -926,7 +926,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(wgrad_waves
   auto load_x = [&](uint4 (&v)[C::X_PER], int n, int yy, int xs) {
     const bf16* const src = xp + ((ptrdiff_t)(n * Hx + (yy >> us)) * Wx + ((xs - 1) >> us)) * xcs;
 #pragma unroll
-    for (int k = 0; k < C::X_PER; ++k) v[k] = piece_load<FAR>(src, px[k]);
+    for (int k = 0; k < C::X_PER; ++k) v[k] = piece_load<FAR>(src, xcs, px[k]);
   };
   auto store_x = [&](const uint4 (&v)[C::X_PER], int slot) {
 #pragma unroll
@@ -1468,8 +1468,11 @@ int wgrad_runs(int N, int H, int W, int Cin, int Cout) {
 template <int TCO, int TCI, int SPW>
 void launch_wgrad(dim3 grid, hipStream_t s, View x, View up, int Cup, View dy, float* work, int N, int H, int W,
                   int Cin, int Cout, int runs, int with_bias) {
-  // buffer loads reach 2 GiB from a strip's first pixel
-  if (2ll * (WG_SEG + 2) * std::max({x.cs, Cup ? up.cs : 0, dy.cs}) < (1ll << 31) - 65536)
+  // buffer loads reach 2 GiB from a strip's first pixel, and take whole pieces
+  // (views at multiples of 8 channels)
+  auto whole = [](const View& v) { return ((uintptr_t)v.p & 15u) == 0 && v.cs % 8 == 0 && v.co % 8 == 0; };
+  if (2ll * (WG_SEG + 2) * std::max({x.cs, Cup ? up.cs : 0, dy.cs}) < (1ll << 31) - 65536 && whole(x) && whole(dy) &&
+      whole(up))
     hipLaunchKernelGGL((k_wgrad_mfma<TCO, TCI, SPW, false>), grid, dim3(256), 0, s, x, up, Cup, dy, work, N, H, W, Cin,
                        Cout, runs, with_bias);
   else

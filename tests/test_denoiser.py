@@ -155,16 +155,19 @@ def test_conv3x3_of_widely_spaced_pixels(rf, gpu_available, Cin, Cout):
     assert ((out[0].float() - ref.permute(0, 2, 3, 1)).abs() <= 2.0 ** -8 * ref.permute(0, 2, 3, 1).abs() + 1e-4).all()
 
 
-def test_conv3x3_wgrad_of_widely_spaced_pixels(rf, gpu_available):
+@pytest.mark.parametrize("cs,co", [(1 << 24, (1 << 24) - 32), (36, 4), (38, 2), (40, 8)])
+def test_conv3x3_wgrad_of_any_channel_stride(rf, gpu_available, cs, co):
+    """Pixels too far apart for 32-bit offsets, and views that are no multiples
+    of 8 channels, take 64-bit addresses: the same bits."""
     import torch
     ctx = rf.Context(1 << 12, 1, 16)
     g = torch.Generator().manual_seed(3)
-    N, H, W, Cin, Cout, cs = 1, 5, 3, 32, 32, 1 << 24
+    N, H, W, Cin, Cout = 1, 5, 3, 32, 32
     x, dy = _bf16(torch.randn(N, H, W, Cin, generator=g)).cuda(), _bf16(torch.randn(N, H, W, Cout, generator=g)).cuda()
     far = torch.empty(N, H, W, cs, dtype=torch.bfloat16, device="cuda")
-    far[..., cs - Cin:] = x
+    far[..., co:co + Cin] = x
     out = []
-    for v, xs, xo in ((x, Cin, 0), (far, cs, cs - Cin)):
+    for v, xs, xo in ((x, Cin, 0), (far, cs, co)):
         dw, db = torch.zeros(3, 3, Cout, Cin, device="cuda"), torch.zeros(Cout, device="cuda")
         ctx.check(ctx.L.rf_nn_conv3x3_wgrad(ctx.h, v.data_ptr(), xs, xo, dy.data_ptr(), Cout, 0, dw.data_ptr(),
                                             db.data_ptr(), N, H, W, Cin, Cout))
