@@ -588,7 +588,8 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   const uint32_t nt = nb * rfk::SORT_TILES_PER_BUCKET;
   const uint32_t nt_used = (uint32_t)((n_bins + (1u << rfk::SORT_TILE_SHIFT) - 1) >> rfk::SORT_TILE_SHIFT);
   // Buffers that only grow, shared by the context's flames.
-  auto bind = [&](const uint32_t* dm, size_t fixed, uint32_t n_chunks, uint32_t n_segs, uint32_t seg_len) {
+  auto bind = [&](const uint32_t* dm, size_t fixed, uint32_t n_chunks, uint32_t n_segs, uint32_t chunk_len,
+                  uint32_t seg_len) {
     a.cbuf = (uint32_t*)ctx->sort_cbuf.p;
     a.tbuf = (uint32_t*)ctx->sort_tbuf.p;
     a.bcur = (uint32_t*)ctx->sort_bcur.p;
@@ -603,6 +604,7 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
     a.n_tiles = nt;
     a.n_chunks = n_chunks;
     a.n_segs = n_segs;
+    a.chunk_len = chunk_len;
     a.seg_len = seg_len;
   };
   // A plan covers up to twice the draw it is made for (at most a full
@@ -615,7 +617,7 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   if (!f->sort_meta.empty() && S <= f->sort_meta_S && 4 * S >= f->sort_meta_S && f->sort_meta_bins == n_bins &&
       f->sort_bins == n_bins && f->last_sort_overflow == 0.0) {
     bind((const uint32_t*)f->sort_meta_dev.p, f->sort_meta_fixed, f->sort_meta_chunks, f->sort_meta_segs,
-         f->sort_meta_seg_len);
+         f->sort_meta_chunk_len, f->sort_meta_seg_len);
     return RF_OK;
   }
   if (f->sort_bins != n_bins || f->sort_bfrac.size() != nb) {
@@ -668,8 +670,13 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   // work lists: rebucketing chunks per bucket, summing segments per used tile
   const size_t meta_fixed = meta.size();
   std::vector<uint32_t> jobs;
+  // A draw of fewer than 96 chunks leaves most compute units idle, each chunk's
+  // workgroup taking 13 us: a quarter of the records per workgroup (one draw of
+  // 2^18 samples into 512x300 60 -> 54 us, 2^20 68 -> 64, 2^21 84 -> 86).
+  const uint32_t chunk_len = S < 96ull * rfk::SORT_CHUNK ? rfk::SORT_CHUNK_SMALL : 0;
+  const uint32_t chunk = chunk_len ? chunk_len : rfk::SORT_CHUNK;
   for (uint32_t b = 0; b < nb; ++b)
-    for (uint32_t k = 0; k * (uint64_t)rfk::SORT_CHUNK < bcap[b]; ++k) {
+    for (uint32_t k = 0; k * (uint64_t)chunk < bcap[b]; ++k) {
       if (k > 0xffffu) return set_err(ctx, RF_ERR_LIMIT, "sort histogram: bucket too large");
       jobs.push_back((b << 16) | k);
     }
@@ -706,13 +713,14 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   memcpy(ctx->meta_stage.p, meta.data(), meta.size() * 4);
   HIPCHK(ctx, hipMemcpyAsync(f->sort_meta_dev.p, ctx->meta_stage.p, meta.size() * 4, hipMemcpyHostToDevice,
                              ctx->stream));
-  bind((const uint32_t*)f->sort_meta_dev.p, meta_fixed, n_chunks, n_segs, seg_len);
+  bind((const uint32_t*)f->sort_meta_dev.p, meta_fixed, n_chunks, n_segs, chunk_len, seg_len);
   f->sort_meta.swap(meta);
   f->sort_meta_S = Sp;
   f->sort_meta_bins = n_bins;
   f->sort_meta_fixed = meta_fixed;
   f->sort_meta_chunks = n_chunks;
   f->sort_meta_segs = n_segs;
+  f->sort_meta_chunk_len = chunk_len;
   f->sort_meta_seg_len = seg_len;
   return RF_OK;
 }

@@ -38,16 +38,19 @@ __global__ void k_draw_readback(const unsigned long long* __restrict__ counter, 
 // is read back from the record itself, so the workgroup needs 69 KiB of LDS
 // and two of them (32 waves) fit on a CU.  Larger chunks pay the per-chunk
 // work (staging, reservations, scan, barriers) over more records: 8192 and
-// 4096 records per workgroup took 12 % and 30 % longer on a 7680x4320 draw.
+// 4096 records per workgroup took 12 % and 30 % longer on a 7680x4320 draw.  A
+// small draw's plan takes SORT_CHUNK_SMALL: its few chunks leave the chip idle,
+// and the pass then takes 6 us instead of 13 (2^18 records).
 constexpr int RB_THREADS = 1024;
-constexpr int RB_PER = SORT_CHUNK / RB_THREADS;  // records per thread
 
+template <int CHUNK>
 __global__ __launch_bounds__(RB_THREADS) void k_sort_rebucket(SortArgs a, float* __restrict__ bins,
                                                               const float4* __restrict__ palette) {
   static_assert(SORT_TILES_PER_BUCKET <= 4 * WAVE, "scan width");
   static_assert(SORT_TILES_PER_BUCKET <= RB_THREADS, "one thread per tile");
+  constexpr int RB_PER = CHUNK / RB_THREADS;  // records per thread
   static_assert(RB_PER % 4 == 0, "16-byte loads");
-  __shared__ uint32_t s_out[SORT_CHUNK];  // tile-ordered records
+  __shared__ uint32_t s_out[CHUNK];  // tile-ordered records
   __shared__ uint32_t s_cnt[SORT_TILES_PER_BUCKET], s_off[SORT_TILES_PER_BUCKET], s_gb[SORT_TILES_PER_BUCKET];
   __shared__ uint32_t s_total;
   __shared__ uint32_t s_toff[SORT_TILES_PER_BUCKET], s_tcap[SORT_TILES_PER_BUCKET];
@@ -57,10 +60,10 @@ __global__ __launch_bounds__(RB_THREADS) void k_sort_rebucket(SortArgs a, float*
   const uint32_t cap = a.bcap[b];
   const uint32_t cur = a.bcur[b];
   const uint32_t count = cur < cap ? cur : cap;
-  const uint32_t start = (job & 0xffffu) * (uint32_t)SORT_CHUNK;
+  const uint32_t start = (job & 0xffffu) * (uint32_t)CHUNK;
   if (start >= count) return;  // workgroup-uniform
-  const uint32_t n = (count - start) < (uint32_t)SORT_CHUNK ? (count - start) : (uint32_t)SORT_CHUNK;
-  // bucket offsets and SORT_CHUNK are multiples of 4 records: 16-byte aligned
+  const uint32_t n = (count - start) < (uint32_t)CHUNK ? (count - start) : (uint32_t)CHUNK;
+  // bucket offsets and CHUNK are multiples of 4 records: 16-byte aligned
   const uint32_t* src = a.cbuf + a.boff[b] + start;
   const uint4* src4 = reinterpret_cast<const uint4*>(src);
   if (tid < (uint32_t)SORT_TILES_PER_BUCKET) {
@@ -72,7 +75,7 @@ __global__ __launch_bounds__(RB_THREADS) void k_sort_rebucket(SortArgs a, float*
   // a full chunk (all but a bucket's last) issues its loads without per-lane
   // guards, which would otherwise make each load wait for the one before
   uint32_t rec[RB_PER];
-  if (n == (uint32_t)SORT_CHUNK) {  // workgroup-uniform
+  if (n == (uint32_t)CHUNK) {  // workgroup-uniform
 #pragma unroll
     for (int k = 0; k < RB_PER / 4; ++k) {
       const uint4 q = src4[(uint32_t)k * RB_THREADS + tid];
@@ -356,7 +359,10 @@ hipError_t launch_draw_readback(const unsigned long long* counter, uint32_t coun
 
 hipError_t launch_sort_rebucket(const SortArgs& a, float* bins, const float4* palette, hipStream_t s) {
   if (a.n_chunks == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_sort_rebucket, dim3(a.n_chunks), dim3(RB_THREADS), 0, s, a, bins, palette);
+  if (a.chunk_len == (uint32_t)SORT_CHUNK_SMALL)
+    hipLaunchKernelGGL(k_sort_rebucket<SORT_CHUNK_SMALL>, dim3(a.n_chunks), dim3(RB_THREADS), 0, s, a, bins, palette);
+  else
+    hipLaunchKernelGGL(k_sort_rebucket<SORT_CHUNK>, dim3(a.n_chunks), dim3(RB_THREADS), 0, s, a, bins, palette);
   return hipGetLastError();
 }
 

@@ -20,6 +20,7 @@ constexpr int SORT_TILES_PER_BUCKET = 1 << (SORT_COARSE_SHIFT - SORT_TILE_SHIFT)
 constexpr int SORT_MAX_BUCKETS = 256;                                        // 2^27 bins
 constexpr int SORT_STAGE_SLOTS = 4096;                                       // samples staged in LDS per flush
 constexpr int SORT_CHUNK = 16384;                                            // records per rebucketing workgroup
+constexpr int SORT_CHUNK_SMALL = 4096;                                       // the same in a small draw's plan
 // Tile sums add red | green << 32 and blue | count << 32 per record with
 // 64-bit LDS atomics, colours in fixed point.  A tile of at most SORT_SEG16
 // records is summed by one workgroup at 2^16 - 1 per unit (a field then
@@ -47,6 +48,7 @@ struct SortArgs {
   uint32_t n_buckets;
   uint32_t n_tiles;        // n_buckets * SORT_TILES_PER_BUCKET
   uint32_t n_chunks, n_segs;
+  uint32_t chunk_len;      // records per chunk: SORT_CHUNK_SMALL, or 0 for SORT_CHUNK
   uint32_t seg_len;        // records per segment of a tile; 0: SORT_SEG16, or SORT_SEG15 of a tile that holds more
   // Batched rendering: per tile, the offset (in entries) of its frame's
   // palette in the palette array the record passes get; null when one
