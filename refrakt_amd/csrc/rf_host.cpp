@@ -547,32 +547,43 @@ static uint32_t sort_subdraw_passes(uint64_t P) {
   return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(64, by_samples));
 }
 
-// Records per segment of a tile of capacity cap under a plan's seg_len.
-static uint32_t tile_seg_len(uint32_t cap, uint32_t seg_len) {
-  return seg_len ? seg_len : cap > (uint32_t)rfk::SORT_SEG16 ? (uint32_t)rfk::SORT_SEG15 : (uint32_t)rfk::SORT_SEG16;
-}
-
-// A plan's seg_len (SortArgs) for S samples spread as frac.  A segment's
-// workgroup sums a record in about 0.44 ns, so in a small image the fullest
-// tile decides the pass: a 320x240 draw of 15 passes of 16384 particles has a
-// quarter of its records in one of 19 tiles, and took 36 us (12 now).  Shorter
-// segments spread it over the idle compute units, but a tile of several
-// segments adds its touched bins by quad atomics, 17 per ns over the whole
-// chip.  The length with the least of both; images of 512 tiles and more fill
-// the chip by tiles.
-static uint32_t sort_seg_len(const uint32_t* tcap, const double* frac, uint32_t nt, double S) {
+// A plan's part_len (SortArgs) for S samples spread as frac.  A workgroup
+// sums a record in about 0.44 ns and 512 run at once, so in a small image the
+// fullest tile decides the pass: a 320x240 draw of 15 passes of 16384 particles
+// has a quarter of its records in one of 19 tiles.  Parts spread it over the
+// idle compute units, but a part adds its touched bins in device memory (about
+// 200 bins per ns over the whole chip), and the sums are read, cleared and
+// added to the histogram (55 ns a slot, 3 us at least).  The length with the
+// least of all; images of 512 tiles and more fill the chip by tiles.  Draws
+// planned without a distribution to go by, mean of three flames, in us: with
+// whole segments, by this rule, with parts of 32768, 8192 and 4096.
+//   320x240,  2^14 particles x 15   67   50    59   50   49
+//   64x64,    2^17 x 8              88   52    57   54   55
+//   512x300,  2^17 x 2              47   33    42   35   33
+//   700x500,  2^16 x 16             92   63    69   62   62
+//   1000x1000, 2^18 x 8             95   69    73   68   70
+//   900x480,  2^20 x 8             184  147   148  145  160
+//   1400x1000, 2^20 x 16           304  243   245  250  275
+//   700x500,  2^20 x 64            808  806   789  852  955
+//   1920x1080, 2^18 x 16           139  100   108   96  100
+//   1920x1080, 2^20 x 64           794  794   759  812  900
+static uint32_t sort_part_len(const uint32_t* tcap, const double* frac, uint32_t nt, double S) {
   if (nt >= 512) return 0;
   uint32_t best = 0;
   double least = 0.0;
-  for (const uint32_t len : {0u, 65532u, 32768u, 16384u, 8192u, 4096u}) {
-    double longest = 0.0, quads = 0.0;
+  for (const uint32_t len : {0u, 65536u, 32768u, 16384u, 8192u, 4096u}) {
+    double longest = S / 512.0, adds = 0.0;
+    uint32_t slots = 0;
     for (uint32_t t = 0; t < nt; ++t) {
-      const double l = tile_seg_len(tcap[t], len), n = S * frac[t];
+      const uint32_t seg = rfk::sort_seg_len(tcap[t]);
+      const double l = len ? std::min(len, seg) : seg, n = S * frac[t];
       longest = std::max(longest, std::min(l, n));
-      if (tcap[t] > l) quads += std::ceil(n / l) * std::min(std::min(l, n), (double)(1 << rfk::SORT_TILE_SHIFT));
+      if (std::min(tcap[t], seg) <= l) continue;
+      slots += (tcap[t] + seg - 1) / seg;
+      adds += std::ceil(n / l) * std::min(std::min(l, n), (double)(1 << rfk::SORT_TILE_SHIFT));
     }
-    const double ns = 0.44 * longest + quads / 17.0;
-    if (len == 0u || ns < least) { least = ns; best = len; }
+    const double ns = 0.44 * longest + adds / 200.0 + (slots ? 3000.0 + 55.0 * slots : 0.0);
+    if (slots <= rfk::SORT_MAX_SLOTS && (len == 0u || ns < least)) { least = ns; best = len; }
   }
   return best;
 }
@@ -587,9 +598,10 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   const uint32_t nb = (uint32_t)((n_bins + (1u << rfk::SORT_COARSE_SHIFT) - 1) >> rfk::SORT_COARSE_SHIFT);
   const uint32_t nt = nb * rfk::SORT_TILES_PER_BUCKET;
   const uint32_t nt_used = (uint32_t)((n_bins + (1u << rfk::SORT_TILE_SHIFT) - 1) >> rfk::SORT_TILE_SHIFT);
+  constexpr size_t MAX_TILES = (size_t)rfk::SORT_MAX_BUCKETS * rfk::SORT_TILES_PER_BUCKET;
   // Buffers that only grow, shared by the context's flames.
   auto bind = [&](const uint32_t* dm, size_t fixed, uint32_t n_chunks, uint32_t n_segs, uint32_t chunk_len,
-                  uint32_t seg_len) {
+                  uint32_t part_len, uint32_t n_slots) {
     a.cbuf = (uint32_t*)ctx->sort_cbuf.p;
     a.tbuf = (uint32_t*)ctx->sort_tbuf.p;
     a.bcur = (uint32_t*)ctx->sort_bcur.p;
@@ -605,7 +617,11 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
     a.n_chunks = n_chunks;
     a.n_segs = n_segs;
     a.chunk_len = chunk_len;
-    a.seg_len = seg_len;
+    a.part_len = part_len;
+    a.n_slots = n_slots;
+    a.slots = a.segs + n_segs;
+    a.tslot = a.slots + n_slots;
+    a.part_sum = (unsigned long long*)((uint32_t*)ctx->sort_tcur.p + MAX_TILES);
   };
   // A plan covers up to twice the draw it is made for (at most a full
   // sub-draw), so the next draw of up to that size reuses it: the same draw
@@ -615,9 +631,10 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   // mostly empty workgroups.  Same histogram and no overflow last time: the
   // capacities and work lists on the device still fit.
   if (!f->sort_meta.empty() && S <= f->sort_meta_S && 4 * S >= f->sort_meta_S && f->sort_meta_bins == n_bins &&
-      f->sort_bins == n_bins && f->last_sort_overflow == 0.0) {
+      f->sort_bins == n_bins && f->last_sort_overflow == 0.0 && ctx->sort_tcur.p &&
+      f->sort_meta_slots <= ctx->sort_part_slots) {
     bind((const uint32_t*)f->sort_meta_dev.p, f->sort_meta_fixed, f->sort_meta_chunks, f->sort_meta_segs,
-         f->sort_meta_chunk_len, f->sort_meta_seg_len);
+         f->sort_meta_chunk_len, f->sort_meta_part_len, f->sort_meta_slots);
     return RF_OK;
   }
   if (f->sort_bins != n_bins || f->sort_bfrac.size() != nb) {
@@ -683,18 +700,29 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   const uint32_t n_chunks = (uint32_t)jobs.size();
   // tile segments, the largest first so that the long workgroups start early
   std::vector<std::pair<uint32_t, uint32_t>> segs;  // (records the segment can hold, job)
-  const uint32_t seg_len = sort_seg_len(tcap, f->sort_tfrac.data(), nt_used, (double)S);
+  const uint32_t part_len = sort_part_len(tcap, f->sort_tfrac.data(), nt_used, (double)S);
+  std::vector<uint32_t> slots, tslot;
   for (uint32_t t = 0; t < nt_used; ++t) {
-    const uint32_t len = tile_seg_len(tcap[t], seg_len);
-    for (uint32_t k = 0; k * (uint64_t)len < tcap[t]; ++k) {
-      if (k > 0xffffu) return set_err(ctx, RF_ERR_LIMIT, "sort histogram: tile too large");
-      segs.emplace_back(std::min<uint32_t>(tcap[t] - k * len, len), (t << 16) | k);
-    }
+    const uint32_t seg = rfk::sort_seg_len(tcap[t]), part = part_len ? std::min(part_len, seg) : seg;
+    const uint32_t per_seg = (seg + part - 1) / part;
+    uint32_t n_seg = 0;
+    for (uint64_t s0 = 0; s0 < tcap[t]; s0 += seg, ++n_seg)
+      for (uint32_t k = 0; k < per_seg && s0 + (uint64_t)k * part < tcap[t]; ++k) {
+        if (n_seg * per_seg + k > 0xffffu) return set_err(ctx, RF_ERR_LIMIT, "sort histogram: tile too large");
+        const uint32_t len = std::min(part, seg - k * part);
+        segs.emplace_back((uint32_t)std::min<uint64_t>(tcap[t] - s0 - (uint64_t)k * part, len),
+                          (t << 16) | (n_seg * per_seg + k));
+      }
+    if (!part_len) continue;
+    tslot.push_back((uint32_t)slots.size());
+    for (uint32_t k = 0; std::min(tcap[t], seg) > part && k < n_seg; ++k) slots.push_back((t << 16) | k);
   }
   order_segments(segs);
   for (const auto& sg : segs) jobs.push_back(sg.second);
   const uint32_t n_segs = (uint32_t)segs.size();
   meta.insert(meta.end(), jobs.begin(), jobs.end());
+  meta.insert(meta.end(), slots.begin(), slots.end());
+  meta.insert(meta.end(), tslot.begin(), tslot.end());
   // grow to at least what a full sub-draw with measured fractions needs (1.2 S
   // plus the per-bucket and per-tile minimums), so the buffers are allocated
   // once per context rather than at every longer draw
@@ -703,8 +731,15 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   if (ctx->sort_cbuf.bytes < cb * 4) HIPCHK(ctx, ctx->sort_cbuf.alloc(std::max(cb, cb_min) * 4));
   if (ctx->sort_tbuf.bytes < ct * 4) HIPCHK(ctx, ctx->sort_tbuf.alloc(std::max(ct, ct_min) * 4));
   if (ctx->sort_bcur.bytes < (size_t)nb * 4) HIPCHK(ctx, ctx->sort_bcur.alloc((size_t)rfk::SORT_MAX_BUCKETS * 4));
-  if (ctx->sort_tcur.bytes < (size_t)nt * 4)
-    HIPCHK(ctx, ctx->sort_tcur.alloc((size_t)rfk::SORT_MAX_BUCKETS * rfk::SORT_TILES_PER_BUCKET * 4));
+  const uint32_t n_slots = (uint32_t)slots.size();
+  if (!ctx->sort_tcur.p || n_slots > ctx->sort_part_slots) {
+    uint32_t n = n_slots ? 32 : 0;
+    while (n < n_slots) n *= 2;
+    ctx->sort_part_slots = 0;
+    HIPCHK(ctx, ctx->sort_tcur.alloc(MAX_TILES * 4 + (size_t)n * rfk::SORT_SLOT_WORDS * 8));
+    ctx->sort_part_slots = n;
+    ctx->sort_part_clear = false;
+  }
   if (f->sort_meta_dev.bytes < meta.size() * 4) HIPCHK(ctx, f->sort_meta_dev.alloc(meta.size() * 4 * 2));
   // every draw ends with a stream synchronisation, so the stage is free here;
   // sized once for any plan up to 1 MiB (pinned allocations are slow, and a
@@ -713,7 +748,7 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   memcpy(ctx->meta_stage.p, meta.data(), meta.size() * 4);
   HIPCHK(ctx, hipMemcpyAsync(f->sort_meta_dev.p, ctx->meta_stage.p, meta.size() * 4, hipMemcpyHostToDevice,
                              ctx->stream));
-  bind((const uint32_t*)f->sort_meta_dev.p, meta_fixed, n_chunks, n_segs, chunk_len, seg_len);
+  bind((const uint32_t*)f->sort_meta_dev.p, meta_fixed, n_chunks, n_segs, chunk_len, part_len, n_slots);
   f->sort_meta.swap(meta);
   f->sort_meta_S = Sp;
   f->sort_meta_bins = n_bins;
@@ -721,7 +756,8 @@ static int sort_prepare(rf_ctx* ctx, rf_flame* f, const float4* hist, uint32_t n
   f->sort_meta_chunks = n_chunks;
   f->sort_meta_segs = n_segs;
   f->sort_meta_chunk_len = chunk_len;
-  f->sort_meta_seg_len = seg_len;
+  f->sort_meta_part_len = part_len;
+  f->sort_meta_slots = n_slots;
   return RF_OK;
 }
 
@@ -846,21 +882,31 @@ static int do_draw(rf_ctx* ctx, rf_flame* f, rf_hist* h, uint32_t num_iter, cons
       a.n_iter = last;
       if (hm_run == RF_HIST_SORT) {
         HIPCHK(ctx, rfk::launch_sort_reset(a.sort, ctx->stream, (unsigned long long*)ctx->counter.p,
-                                           counter_cleared ? 0u : counter_words));
+                                           counter_cleared ? 0u : counter_words,
+                                           a.sort.n_slots && !ctx->sort_part_clear
+                                               ? ctx->sort_part_slots * rfk::SORT_SLOT_WORDS : 0u));
         counter_cleared = true;
       }
       const int rc3 = fast_launch(ctx, f, a, P, hm_run);
       if (rc3) return rc3;
       if (hm_run == RF_HIST_SORT) {
         HIPCHK(ctx, rfk::launch_sort_rebucket(a.sort, a.bins, a.palette, ctx->stream));
+        // cleared by the reset, and again behind the tile pass by the one that
+        // adds them to the histogram, the last time with the readback
+        if (a.sort.n_slots) ctx->sort_part_clear = false;
         HIPCHK(ctx, rfk::launch_sort_tiles(a.sort, a.bins, h->w * h->h, a.palette, ctx->stream));
+        if (a.sort.n_slots && done + last < num_iter) {
+          HIPCHK(ctx, rfk::launch_sort_parts(a.sort, a.bins, h->w * h->h, ctx->stream));
+          ctx->sort_part_clear = true;
+        }
       }
     }
     sort_used = hm_run == RF_HIST_SORT && num_iter;
     sort_args = a.sort;
     sort_S = P * (uint64_t)last;
   }
-  HIPCHK(ctx, hipEventRecord(ctx->ev[3], ctx->stream));
+  const bool parts = sort_used && sort_args.n_slots;
+  if (!parts) HIPCHK(ctx, hipEventRecord(ctx->ev[3], ctx->stream));
   // counter slots, then the sort cursors, read back by one kernel into pinned
   // memory behind one synchronisation
   const size_t cur_words = sort_used ? (size_t)sort_args.n_buckets + sort_args.n_tiles : 0;
@@ -871,9 +917,12 @@ static int do_draw(rf_ctx* ctx, rf_flame* f, rf_hist* h, uint32_t num_iter, cons
   const uint64_t* slots = static_cast<const uint64_t*>(ctx->readback.p);
   uint32_t* cur_host = reinterpret_cast<uint32_t*>(static_cast<char*>(ctx->readback.p) + counter_bytes);
   HIPCHK(ctx, rfk::launch_draw_readback((const unsigned long long*)ctx->counter.p, counter_words,
-                                        sort_used ? sort_args.bcur : nullptr, sort_args.n_buckets,
-                                        sort_used ? sort_args.tcur : nullptr, sort_args.n_tiles,
-                                        (uint32_t*)ctx->readback.dev, ctx->stream));
+                                        sort_used ? &sort_args : nullptr, (uint32_t*)ctx->readback.dev, ctx->stream,
+                                        parts ? (float*)h->ptr : nullptr, h->w * h->h));
+  if (parts) {
+    ctx->sort_part_clear = true;
+    HIPCHK(ctx, hipEventRecord(ctx->ev[3], ctx->stream));
+  }
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   uint64_t cnt[2] = {0, 0};
   for (int k = 0; k < rfk::COUNTER_SLOTS; ++k) {

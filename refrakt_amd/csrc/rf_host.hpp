@@ -104,6 +104,9 @@ struct rf_ctx {
   rfh::DevBuf counter;         // u64 [drawn, samples added in the LDS bin cache]
   // RF_HIST_SORT buffers: bucket and tile records, cursors, offsets, capacities
   rfh::DevBuf sort_cbuf, sort_tbuf, sort_bcur, sort_tcur, sort_mass;
+  // sort_tcur ends with the sums of the tile segments cut into parts
+  uint32_t sort_part_slots = 0;
+  bool sort_part_clear = false;  // they are zero
   // a draw's readbacks: counter slots, then (sort draws) bucket and tile
   // cursors, written by one kernel
   rfh::HostBuf readback;
@@ -153,7 +156,7 @@ struct rf_flame {
   rfh::DevBuf sort_meta_dev;
   uint64_t sort_meta_S = 0;
   uint32_t sort_meta_bins = 0, sort_meta_chunks = 0, sort_meta_segs = 0, sort_meta_chunk_len = 0,
-           sort_meta_seg_len = 0;
+           sort_meta_part_len = 0, sort_meta_slots = 0;
   size_t sort_meta_fixed = 0;
   // Flame program: the host copy of the Block (its structure selects the
   // program), whether the last fast-engine launch ran one.

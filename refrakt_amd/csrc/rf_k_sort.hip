@@ -10,24 +10,15 @@ namespace {
 using namespace detail;
 
 // Clears the cursors of a sort draw and, on a call's first sub-draw, the
-// draw counters (one launch instead of a cursor reset plus a memset).
-__global__ void k_sort_reset(SortArgs a, unsigned long long* __restrict__ counter, uint32_t counter_words) {
+// draw counters (one launch instead of a cursor reset plus a memset) and new
+// part sums.
+__global__ void k_sort_reset(SortArgs a, unsigned long long* __restrict__ counter, uint32_t counter_words,
+                             uint32_t part_words) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < a.n_buckets) a.bcur[i] = 0u;
   if (i < a.n_tiles) a.tcur[i] = 0u;
   if (i < counter_words) counter[i] = 0ull;
-}
-
-// A draw's readback in one launch: the counter words, then the bucket and
-// tile cursors, stored straight into pinned host memory (out is its device
-// address), instead of one copy command per array.
-__global__ void k_draw_readback(const unsigned long long* __restrict__ counter, uint32_t counter_words,
-                                const uint32_t* __restrict__ bcur, uint32_t nb, const uint32_t* __restrict__ tcur,
-                                uint32_t nt, uint32_t* __restrict__ out) {
-  const uint32_t cw = 2u * counter_words, n = cw + nb + nt;
-  const uint32_t* c32 = reinterpret_cast<const uint32_t*>(counter);
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    out[i] = i < cw ? c32[i] : (i < cw + nb ? bcur[i - cw] : tcur[i - cw - nb]);
+  if (i < part_words) a.part_sum[i] = 0ull;
 }
 
 // One workgroup per chunk of SORT_CHUNK records of a bucket (the host lists
@@ -162,7 +153,9 @@ __global__ __launch_bounds__(RB_THREADS) void k_sort_rebucket(SortArgs a, float*
 // touched bins are added to the histogram:
 // with a plain read-modify-write when the tile is one segment (tiles are
 // disjoint, and every overflow was added by earlier kernels), with quad
-// atomics when several segments share the tile.  68 KiB of LDS: two
+// atomics when several segments share the tile.  A workgroup that has only a
+// part of a segment adds its integers to the segment's in device memory
+// instead (sort_parts).  68 KiB of LDS: two
 // workgroups of 16 waves per CU (tiles of 2^11 bins, 36 KiB and four
 // workgroups of 8 waves, took 30 % longer on a 1024x1024 draw: the per-tile
 // clearing, palette and write-back are paid over half the records).  Each
@@ -211,6 +204,84 @@ __device__ __forceinline__ void tile_add_batch(TileSums& t, const uint32_t* r) {
   }
 }
 
+// A tile's fixed point: 2^16 - 1 per unit for one of at most SORT_SEG16
+// records of room, else 2^15 - 1.
+__device__ __forceinline__ float tile_one(uint32_t cap) { return cap > (uint32_t)SORT_SEG16 ? 32767.0f : 65535.0f; }
+
+// A bin's sums as float colours and count.
+__device__ __forceinline__ float4 tile_value(uint64_t rg, uint64_t bc, float inv) {
+  return make_float4((float)(uint32_t)rg * inv, (float)(uint32_t)(rg >> 32) * inv, (float)(uint32_t)bc * inv,
+                     (float)(uint32_t)(bc >> 32));
+}
+
+// Records of segment si of a tile that holds count, and their parts.
+__device__ __forceinline__ uint32_t seg_parts(uint32_t count, uint32_t si, uint32_t seg, uint32_t part) {
+  return (min(count - si * seg, seg) + part - 1) / part;
+}
+
+// Segments summed in parts: their integers to float and into the histogram,
+// with plain read-modify-writes where the tile has no other segment.  A quarter
+// of a tile per workgroup.  The sums are left zero.  (Done by the workgroup
+// that adds a segment's last part, behind a fence and a counter, it took 3 to
+// 9 us longer a draw than as a launch of its own, which a draw's readback
+// saves.)
+constexpr int PARTS_THREADS = 256, PARTS_BPT = 4;
+constexpr uint32_t PARTS_BLOCKS = TILE_BINS / (PARTS_THREADS * PARTS_BPT);  // per slot
+__device__ __forceinline__ void sort_parts(const SortArgs& a, float4* __restrict__ hist, uint32_t n_bins,
+                                           uint32_t block) {
+  const uint32_t slot = block / PARTS_BLOCKS;
+  const uint32_t t = a.slots[slot] >> 16, si = a.slots[slot] & 0xffffu;
+  const uint32_t cap = a.tcap[t], count = min(a.tcur[t], cap), seg = sort_seg_len(cap);
+  if (si * seg >= count || seg_parts(count, si, seg, a.part_len) < 2u) return;  // workgroup-uniform
+  const bool shared = cap > seg;
+  const float inv = 1.0f / tile_one(cap);
+  const uint32_t i0 = block % PARTS_BLOCKS * (PARTS_THREADS * PARTS_BPT) + threadIdx.x;
+  unsigned long long* const p = a.part_sum + (size_t)slot * 2 * TILE_BINS + i0;
+  const uint32_t base = (t << SORT_TILE_SHIFT) + i0;
+  uint64_t rg[PARTS_BPT], bc[PARTS_BPT];
+#pragma unroll
+  for (int k = 0; k < PARTS_BPT; ++k) {
+    rg[k] = p[k * PARTS_THREADS];
+    bc[k] = p[TILE_BINS + k * PARTS_THREADS];
+  }
+#pragma unroll
+  for (int k = 0; k < PARTS_BPT; ++k) {
+    const uint32_t b = base + k * PARTS_THREADS;
+    const bool add = bc[k] != 0ull && b < n_bins;
+    const float4 v = tile_value(rg[k], bc[k], inv);
+    if (shared) {  // workgroup-uniform
+      bin_quad_vals(reinterpret_cast<float*>(hist), b, add, v);
+    } else if (add) {
+      float4 h = hist[b];
+      h.x += v.x; h.y += v.y; h.z += v.z; h.w += v.w;
+      hist[b] = h;
+    }
+    if (add) { p[k * PARTS_THREADS] = 0ull; p[TILE_BINS + k * PARTS_THREADS] = 0ull; }
+  }
+}
+
+__global__ __launch_bounds__(PARTS_THREADS) void k_sort_parts(SortArgs a, float4* __restrict__ hist, uint32_t n_bins) {
+  sort_parts(a, hist, n_bins, blockIdx.x);
+}
+
+// A draw's end in one launch: `copiers` workgroups store the counter words,
+// then the bucket and tile cursors, straight into pinned host memory (out is
+// its device address), instead of one copy command per array; the workgroups
+// behind them add the segments in parts.
+__global__ __launch_bounds__(PARTS_THREADS) void k_draw_readback(const unsigned long long* __restrict__ counter,
+                                                                uint32_t counter_words, SortArgs a,
+                                                                uint32_t* __restrict__ out, uint32_t copiers,
+                                                                float4* __restrict__ hist, uint32_t n_bins) {
+  if (blockIdx.x >= copiers) {
+    sort_parts(a, hist, n_bins, blockIdx.x - copiers);
+    return;
+  }
+  const uint32_t nb = a.n_buckets, cw = 2u * counter_words, n = cw + nb + a.n_tiles;
+  const uint32_t* c32 = reinterpret_cast<const uint32_t*>(counter);
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += copiers * blockDim.x)
+    out[i] = i < cw ? c32[i] : (i < cw + nb ? a.bcur[i - cw] : a.tcur[i - cw - nb]);
+}
+
 __global__ __launch_bounds__(TILE_THREADS) void k_sort_tiles(SortArgs a, float4* __restrict__ hist, uint32_t n_bins,
                                                             const float4* __restrict__ palette) {
   __shared__ TileSums s_t;
@@ -223,13 +294,14 @@ __global__ __launch_bounds__(TILE_THREADS) void k_sort_tiles(SortArgs a, float4*
   const uint32_t count = cur < cap ? cur : cap;
   // workgroup-uniform: a tile of at most SORT_SEG16 records is summed at
   // 2^16 - 1 per unit, a larger one at 2^15 - 1 in segments of SORT_SEG15 (both
-  // in shorter segments where the plan says so)
-  const bool large = cap > (uint32_t)SORT_SEG16;
-  const uint32_t seg = a.seg_len ? a.seg_len : large ? (uint32_t)SORT_SEG15 : (uint32_t)SORT_SEG16;
-  const float one = large ? 32767.0f : 65535.0f;
-  const uint32_t start = (job & 0xffffu) * seg;
+  // in parts, a workgroup each, where the plan says so)
+  const uint32_t seg = sort_seg_len(cap);
+  const float one = tile_one(cap);
+  const uint32_t part = a.part_len ? a.part_len : seg, per_seg = (seg + part - 1) / part;
+  const uint32_t si = (job & 0xffffu) / per_seg, in_seg = (job & 0xffffu) % per_seg * part;
+  const uint32_t start = si * seg + in_seg;
   if (base >= n_bins || start >= count) return;  // workgroup-uniform
-  const uint32_t n = (count - start) < seg ? (count - start) : seg;
+  const uint32_t n = min(count - start, min(part, seg - in_seg));
   for (uint32_t i = tid; i < (uint32_t)TILE_BINS; i += TILE_THREADS) {
     s_t.rg[i] = 0ull;
     s_t.bc[i] = 0ull;
@@ -244,8 +316,8 @@ __global__ __launch_bounds__(TILE_THREADS) void k_sort_tiles(SortArgs a, float4*
     s_t.pal[tid].b = bl;
   }
   __syncthreads();
-  // Tile offsets and the segment sizes are multiples of 4 records, so the
-  // segment starts 16-byte aligned.
+  // Tile offsets, segments and parts are multiples of 4 records, so the
+  // records start 16-byte aligned.
   const uint32_t* src = a.tbuf + a.toff[t] + start;
   const uint4* src4 = reinterpret_cast<const uint4*>(src);
   const uint32_t n4 = n / 4;
@@ -278,17 +350,26 @@ __global__ __launch_bounds__(TILE_THREADS) void k_sort_tiles(SortArgs a, float4*
   const float inv = 1.0f / one;
   constexpr int BPT = TILE_BINS / TILE_THREADS;  // bins per thread
   static_assert(BPT * TILE_THREADS == TILE_BINS, "bins per thread");
+  if (a.part_len && seg_parts(count, si, seg, part) > 1u) {  // workgroup-uniform: sort_parts goes on
+    unsigned long long* const p = a.part_sum + (size_t)(a.tslot[t] + si) * 2 * TILE_BINS;
+#pragma unroll
+    for (int k = 0; k < BPT; ++k) {
+      const uint32_t i = (uint32_t)k * TILE_THREADS + tid;
+      const uint64_t bc = s_t.bc[i];
+      if (bc == 0ull) continue;  // no record, no colour
+      __hip_atomic_fetch_add(p + i, s_t.rg[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_fetch_add(p + TILE_BINS + i, bc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return;
+  }
   float4 v[BPT];
   bool add[BPT];
 #pragma unroll
   for (int k = 0; k < BPT; ++k) {
     const uint32_t i = (uint32_t)k * TILE_THREADS + tid;
     const uint64_t bc = s_t.bc[i];
-    const uint64_t rg = s_t.rg[i];
-    const uint32_t c = (uint32_t)(bc >> 32);
-    v[k] = make_float4((float)(uint32_t)rg * inv, (float)(uint32_t)(rg >> 32) * inv, (float)(uint32_t)bc * inv,
-                       (float)c);
-    add[k] = base + i < n_bins && c != 0u;
+    v[k] = tile_value(s_t.rg[i], bc, inv);
+    add[k] = base + i < n_bins && bc != 0ull;
   }
   if (shared) {  // workgroup-uniform
 #pragma unroll
@@ -338,22 +419,26 @@ hipError_t launch_sort_tile_mass(const float4* bins, uint32_t n_bins, uint32_t n
   return hipGetLastError();
 }
 
-hipError_t launch_sort_reset(const SortArgs& a, hipStream_t s, unsigned long long* counter, uint32_t counter_words) {
+hipError_t launch_sort_reset(const SortArgs& a, hipStream_t s, unsigned long long* counter, uint32_t counter_words,
+                             uint32_t part_words) {
   uint32_t n = a.n_tiles > a.n_buckets ? a.n_tiles : a.n_buckets;
   if (!counter) counter_words = 0;
   if (counter_words > n) n = counter_words;
+  if (part_words > n) n = part_words;
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_sort_reset, dim3((n + 255) / 256), dim3(256), 0, s, a, counter, counter_words);
+  hipLaunchKernelGGL(k_sort_reset, dim3((n + 255) / 256), dim3(256), 0, s, a, counter, counter_words, part_words);
   return hipGetLastError();
 }
 
-hipError_t launch_draw_readback(const unsigned long long* counter, uint32_t counter_words, const uint32_t* bcur,
-                                uint32_t nb, const uint32_t* tcur, uint32_t nt, uint32_t* out, hipStream_t s) {
-  const uint32_t n = 2u * counter_words + (bcur ? nb : 0u) + (tcur ? nt : 0u);
-  if (n == 0) return hipSuccess;
-  const uint32_t blocks = (n + 255) / 256 < 64u ? (n + 255) / 256 : 64u;
-  hipLaunchKernelGGL(k_draw_readback, dim3(blocks), dim3(256), 0, s, counter, counter_words, bcur, bcur ? nb : 0u,
-                     tcur, tcur ? nt : 0u, out);
+hipError_t launch_draw_readback(const unsigned long long* counter, uint32_t counter_words, const SortArgs* a,
+                                uint32_t* out, hipStream_t s, float* bins, uint32_t n_bins) {
+  const SortArgs g = a ? *a : SortArgs{};
+  const uint32_t n = 2u * counter_words + g.n_buckets + g.n_tiles;
+  const uint32_t copiers = (n + PARTS_THREADS - 1) / PARTS_THREADS < 64u ? (n + PARTS_THREADS - 1) / PARTS_THREADS : 64u;
+  const uint32_t grid = copiers + (bins ? g.n_slots * PARTS_BLOCKS : 0u);
+  if (grid == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_draw_readback, dim3(grid), dim3(PARTS_THREADS), 0, s, counter, counter_words, g, out, copiers,
+                     reinterpret_cast<float4*>(bins), n_bins);
   return hipGetLastError();
 }
 
@@ -370,6 +455,13 @@ hipError_t launch_sort_tiles(const SortArgs& a, float* bins, uint32_t n_bins, co
   if (a.n_segs == 0) return hipSuccess;
   hipLaunchKernelGGL(k_sort_tiles, dim3(a.n_segs), dim3(TILE_THREADS), 0, s, a, reinterpret_cast<float4*>(bins),
                      n_bins, palette);
+  return hipGetLastError();
+}
+
+hipError_t launch_sort_parts(const SortArgs& a, float* bins, uint32_t n_bins, hipStream_t s) {
+  if (a.n_slots == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_sort_parts, dim3(a.n_slots * PARTS_BLOCKS), dim3(PARTS_THREADS), 0, s, a,
+                     reinterpret_cast<float4*>(bins), n_bins);
   return hipGetLastError();
 }
 

@@ -4,7 +4,7 @@
 // 4-byte records into coarse buckets of 2^19 bins, a second kernel splits
 // each bucket into 128 tiles of 2^12 bins, and a third accumulates every tile
 // in LDS and adds it to the histogram with one plain read-modify-write per
-// touched bin.  Records carry no weight, so the mode needs unit opacities;
+// touched bin (a tile of many records in segments and parts, below).  Records carry no weight, so the mode needs unit opacities;
 // the LDS sums are fixed point, so palette values must lie in [0, 1].
 #pragma once
 #ifndef __HIPCC_RTC__
@@ -27,11 +27,17 @@ constexpr int SORT_CHUNK_SMALL = 4096;                                       // 
 // holds at most 65532 * 65535 < 2^32, so no carry crosses into the next); a
 // larger tile is split into segments of at most SORT_SEG15 records, each
 // summed by its own workgroup at 2^15 - 1 per unit (131068 * 32767 < 2^32).  A
-// plan for a small image may cut either kind into shorter segments (seg_len).
+// plan for a small image may have several workgroups sum a segment in parts
+// (part_len): their integers are added in device memory, so a segment's sums
+// are the same, and rounded to float once, however it is cut.
 // Each sample's colour is rounded by at most 1 / (2 * 65535) or
 // 1 / (2 * 32767), about 2^-17 and 2^-16.
 constexpr int SORT_SEG16 = 65532;
 constexpr int SORT_SEG15 = 131068;
+// Records per segment of a tile of capacity cap.
+constexpr uint32_t sort_seg_len(uint32_t cap) { return cap > (uint32_t)SORT_SEG16 ? SORT_SEG15 : SORT_SEG16; }
+constexpr uint32_t SORT_MAX_SLOTS = 1024;  // segments a plan may cut into parts
+constexpr uint32_t SORT_SLOT_WORDS = 2u << SORT_TILE_SHIFT;  // u64 sums of one (64 KiB)
 constexpr uint32_t SORT_NONE = 0xffffffffu;
 
 struct SortArgs {
@@ -44,12 +50,19 @@ struct SortArgs {
   const uint32_t* toff;    // per tile: first record in tbuf
   const uint32_t* tcap;    // per tile: capacity
   const uint32_t* chunks;  // rebucketing work: (bucket << 16) | chunk index, one per workgroup
-  const uint32_t* segs;    // tile work: (tile << 16) | segment index, one per workgroup
+  const uint32_t* segs;    // tile work: (tile << 16) | part index over the tile's segments, one per workgroup
   uint32_t n_buckets;
   uint32_t n_tiles;        // n_buckets * SORT_TILES_PER_BUCKET
   uint32_t n_chunks, n_segs;
   uint32_t chunk_len;      // records per chunk: SORT_CHUNK_SMALL, or 0 for SORT_CHUNK
-  uint32_t seg_len;        // records per segment of a tile; 0: SORT_SEG16, or SORT_SEG15 of a tile that holds more
+  uint32_t part_len;       // records per part of a segment; 0: whole segments
+  // With parts: per slot (tile << 16) | segment of a segment that may have
+  // several parts, per tile the slot of its first segment, and per slot
+  // SORT_SLOT_WORDS integer sums, zero between draws.
+  uint32_t n_slots;
+  const uint32_t* slots;
+  const uint32_t* tslot;
+  unsigned long long* part_sum;
   // Batched rendering: per tile, the offset (in entries) of its frame's
   // palette in the palette array the record passes get; null when one
   // palette serves every tile.
@@ -86,16 +99,21 @@ inline uint32_t sort_grid(uint32_t n_batches, uint32_t n_iter, uint32_t n_bucket
   return grid > least ? grid : least;
 }
 
-// Clears the cursors and, when counter is given, counter_words words of it.
+// Clears the cursors, counter_words words of counter and part_words of the
+// parts' sums.
 hipError_t launch_sort_reset(const SortArgs& a, hipStream_t s, unsigned long long* counter = nullptr,
-                             uint32_t counter_words = 0);
-// Copies counter_words 64-bit counters, then nb bucket and nt tile cursors
-// (either array may be null) into out, 32-bit words, in one launch; out may
-// be the device address of pinned host memory.
-hipError_t launch_draw_readback(const unsigned long long* counter, uint32_t counter_words, const uint32_t* bcur,
-                                uint32_t nb, const uint32_t* tcur, uint32_t nt, uint32_t* out, hipStream_t s);
+                             uint32_t counter_words = 0, uint32_t part_words = 0);
+// Copies counter_words 64-bit counters, then (a given) its bucket and tile
+// cursors into out, 32-bit words, in one launch; out may be the device address
+// of pinned host memory.  With bins the same launch ends a draw whose segments
+// were summed in parts (launch_sort_parts).
+hipError_t launch_draw_readback(const unsigned long long* counter, uint32_t counter_words, const SortArgs* a,
+                                uint32_t* out, hipStream_t s, float* bins = nullptr, uint32_t n_bins = 0);
 hipError_t launch_sort_rebucket(const SortArgs& a, float* bins, const float4* palette, hipStream_t s);
+// Sums the tiles' records.  With n_slots > 0 the segments in parts are still to
+// be added to bins, by launch_sort_parts or launch_draw_readback.
 hipError_t launch_sort_tiles(const SortArgs& a, float* bins, uint32_t n_bins, const float4* palette, hipStream_t s);
+hipError_t launch_sort_parts(const SortArgs& a, float* bins, uint32_t n_bins, hipStream_t s);
 // mass[t] = sum of the count channel over tile t of a histogram (t < n_tiles).
 hipError_t launch_sort_tile_mass(const float4* bins, uint32_t n_bins, uint32_t n_tiles, float* mass, hipStream_t s);
 #endif

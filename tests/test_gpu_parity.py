@@ -226,6 +226,49 @@ def test_fast_sort_short_segments(rf, orc, gpu_available, P, passes, W, H):
     assert (np.abs(g_hist[..., :3].astype(np.float64) - bins[..., :3]) <= tol).all()
 
 
+@pytest.mark.parametrize("P,passes,W,H", [(1 << 12, 6, 64, 64), (1 << 14, 8, 320, 240), (1 << 14, 15, 320, 240),
+                                          (1 << 16, 16, 700, 500), (1 << 18, 8, 1000, 1000)])
+def test_fast_sort_small_images_round_once(rf, gpu_available, P, passes, W, H):
+    """A tile of one segment (131068 records of room) is summed in integers,
+    however many workgroups sum it, and rounded to float once: with one colour
+    every bin holds exactly its count's multiple of it, and the same draw twice
+    has the same bits."""
+    print(f"small images round once: {W}x{H} P={P} passes={passes}", flush=True)
+
+    def draw(fl):
+        ctx = _ctx(rf, P, 1, rf.RF_ENGINE_FAST, hist_mode=rf.RF_HIST_SORT, seed=5, waves=8)
+        fh = ctx.flame(fl)
+        fh.warmup(19)  # both draws on the attractor
+        fh.draw_to_bins(ctx.histogram(W, H), 1)
+        hist = ctx.histogram(W, H)
+        fh.draw_to_bins(hist, passes)  # more than twice the first: planned from its distribution
+        assert fh.sort_overflow() == 0.0
+        return hist.download().reshape(-1, 4)
+
+    fl = _linear_flame(rf, 29, W=W, H=H)
+    colour = np.array([0.3, 0.7123, 0.951], np.float32)
+    fl.palette[:, :3] = colour
+    h = draw(fl)
+    n = h[:, 3].astype(np.uint64)
+    tile = np.arange(W * H) >> 12
+    # a plan's room for a tile: 1.2 times the records of twice this draw, and 512
+    room = (2.4 * np.bincount(tile, weights=n) + 512)[tile]
+    checked = 0
+    for one, of_tile in ((65535, room < 60000), (32767, (room > 70000) & (room < 125000))):
+        sel = of_tile & (n > 0)
+        checked += int(sel.sum())
+        q = np.floor(colour * np.float32(one) + np.float32(0.5)).astype(np.uint64)
+        total = (n[sel, None] * q).astype(np.float32)
+        inv = np.float32(1.0) / np.float32(one)
+        # the reciprocal within one ulp, the same for every bin
+        assert any(np.array_equal(total * i, h[sel, :3])
+                   for i in (inv, np.nextafter(inv, np.float32(0)), np.nextafter(inv, np.float32(1))))
+    assert checked > 0
+    fl = _linear_flame(rf, 29, W=W, H=H)
+    a, b = draw(fl), draw(fl)
+    assert np.array_equal(a[room < 125000].view(np.uint32), b[room < 125000].view(np.uint32))
+
+
 # ------------------------------------------------- non-finite particle policy
 def _nan_xform(rf, kind):
     """An xform whose output is never finite: a NaN variation weight, or an
