@@ -199,6 +199,25 @@ void give(std::unique_ptr<Stage> s) {
   if (p.holders > 0 && p.idle.size() < kIdle) p.idle.push_back(std::move(s));
 }  // else freed
 
+// Makes a device current for its lifetime: events and pinned memory belong to
+// the current device, and a slot's event is recorded on the copy's stream.
+class OnDevice {
+ public:
+  explicit OnDevice(int device) {
+    if (hipGetDevice(&before_) != hipSuccess) before_ = device;
+    if (before_ != device) (void)hipSetDevice(device);
+    device_ = device;
+  }
+  ~OnDevice() {
+    if (before_ != device_) (void)hipSetDevice(before_);
+  }
+  OnDevice(const OnDevice&) = delete;
+  OnDevice& operator=(const OnDevice&) = delete;
+
+ private:
+  int before_ = 0, device_ = 0;
+};
+
 hipError_t plain(void* host, const void* device, size_t n, hipStream_t s) {
   const hipError_t e = hipMemcpyAsync(host, device, n, hipMemcpyDeviceToHost, s);
   return e == hipSuccess ? hipStreamSynchronize(s) : e;
@@ -212,10 +231,14 @@ hipError_t download(void* host, const void* device, size_t n, hipStream_t s) {
   if (hipPointerGetAttributes(&at, host) == hipSuccess && at.type == hipMemoryTypeHost)
     return plain(host, device, n, s);  // pinned already: one transfer at full rate
   (void)hipGetLastError();             // not a pointer the runtime knows: the usual case
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
+  hipDevice_t dev = 0;
+  hipError_t e = hipStreamGetDevice(s, &dev);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return plain(host, device, n, s);
+  }
   try {
+    const OnDevice on(dev);
     std::unique_ptr<Stage> st = take(dev);
     if (!st->ready(n > chunk_bytes(n))) {
       (void)hipGetLastError();

@@ -1,0 +1,41 @@
+// Runs one scenario of device-to-host copies on the fake runtime
+// (fake_hip/hip/hip_runtime.h); exits with 0 where it went as it should.
+#include "../refrakt_amd/csrc/rf_stage.cpp"
+
+#include <stdio.h>
+
+#include <string>
+
+static int fail(const char* what, size_t n) {
+  printf("%s at %zu bytes\n", what, n);
+  return 1;
+}
+
+static int copies(FakeStream s, size_t n) {
+  std::vector<unsigned char> src(n), dst(n, 0);
+  for (size_t i = 0; i < n; ++i) src[i] = (unsigned char)(i * 2654435761u >> 13);
+  if (rfh::download(dst.data(), src.data(), n, &s) != hipSuccess) return fail("error", n);
+  if (src != dst) return fail("wrong bytes", n);
+  return 0;
+}
+
+// The stream's device is not the calling thread's.
+static int other_device() {
+  rfh::stage_hold();
+  for (const size_t n : {(size_t)1 << 10, (size_t)1 << 20, (size_t)5 << 20, ((size_t)40 << 20) + 3}) {
+    for (const int current : {0, 1, 0})
+      for (const int stream : {1, 0}) {
+        fake::device = current;
+        if (int rc = copies(FakeStream{stream}, n)) return rc;
+        if (fake::device != current) return fail("current device changed", n);
+      }
+  }
+  rfh::stage_release();
+  return fake::live_events || !fake::pinned.empty() ? fail("left over", 0) : 0;
+}
+
+int main(int argc, char** argv) {
+  const std::string which = argc > 1 ? argv[1] : "";
+  if (which == "other_device") return other_device();
+  return 2;
+}

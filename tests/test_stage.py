@@ -1,0 +1,23 @@
+"""Device-to-host copies (rf_stage.cpp) on a fake runtime of two devices, on
+the CPU: what one GPU cannot show."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def stage(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("stage") / "stage")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", "-I", os.path.join(HERE, "fake_hip"),
+                    os.path.join(HERE, "stage_driver.cpp"), "-o", exe], check=True)
+    return lambda which: subprocess.run([exe, which], capture_output=True, text=True, timeout=60)
+
+
+def test_copies_on_another_devices_stream(stage):
+    """A context of one device, a thread whose current device is another: copies
+    of every length work and leave the current device alone."""
+    r = stage("other_device")
+    assert r.returncode == 0, r.stdout
