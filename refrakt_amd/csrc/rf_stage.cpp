@@ -232,8 +232,7 @@ hipError_t download(void* host, const void* device, size_t n, hipStream_t s) {
     return plain(host, device, n, s);  // pinned already: one transfer at full rate
   (void)hipGetLastError();             // not a pointer the runtime knows: the usual case
   hipDevice_t dev = 0;
-  hipError_t e = hipStreamGetDevice(s, &dev);
-  if (e != hipSuccess) {
+  if (hipStreamGetDevice(s, &dev) != hipSuccess) {
     (void)hipGetLastError();
     return plain(host, device, n, s);
   }
@@ -244,9 +243,12 @@ hipError_t download(void* host, const void* device, size_t n, hipStream_t s) {
       (void)hipGetLastError();
       return plain(host, device, n, s);
     }
-    e = st->copy((char*)host, (const char*)device, n, s);
-    give(std::move(st));
-    return e;
+    if (st->copy((char*)host, (const char*)device, n, s) == hipSuccess) {
+      give(std::move(st));
+      return hipSuccess;
+    }
+    (void)hipGetLastError();  // of the stage, which goes; the copy's own error shows again
+    return plain(host, device, n, s);
   } catch (...) {  // out of host memory before or after the copy, never during it
     return plain(host, device, n, s);
   }

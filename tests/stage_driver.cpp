@@ -34,8 +34,23 @@ static int other_device() {
   return fake::live_events || !fake::pinned.empty() ? fail("left over", 0) : 0;
 }
 
+// Staging that fails on its way is not the caller's error.
+static int failing_stage() {
+  rfh::stage_hold();
+  const size_t n = ((size_t)40 << 20) + 3;
+  for (const int records : {0, 1, 5}) {
+    fake::records_left = records;
+    if (int rc = copies(FakeStream{0}, n)) return rc;
+    fake::records_left = -1;
+    if (int rc = copies(FakeStream{0}, n)) return rc;
+  }
+  rfh::stage_release();
+  return fake::live_events || !fake::pinned.empty() ? fail("left over", 0) : 0;
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   if (which == "other_device") return other_device();
+  if (which == "failing_stage") return failing_stage();
   return 2;
 }

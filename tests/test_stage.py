@@ -21,3 +21,10 @@ def test_copies_on_another_devices_stream(stage):
     of every length work and leave the current device alone."""
     r = stage("other_device")
     assert r.returncode == 0, r.stdout
+
+
+def test_copies_while_staging_fails(stage):
+    """An event that cannot be recorded, at once or after some transfers: the
+    bytes arrive by the plain copy, and the next copy is staged again."""
+    r = stage("failing_stage")
+    assert r.returncode == 0, r.stdout
