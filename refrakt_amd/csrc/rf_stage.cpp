@@ -228,8 +228,8 @@ hipError_t plain(void* host, const void* device, size_t n, hipStream_t s) {
 hipError_t download(void* host, const void* device, size_t n, hipStream_t s) {
   if (n < kDirect) return plain(host, device, n, s);
   hipPointerAttribute_t at;
-  if (hipPointerGetAttributes(&at, host) == hipSuccess && at.type == hipMemoryTypeHost)
-    return plain(host, device, n, s);  // pinned already: one transfer at full rate
+  if (hipPointerGetAttributes(&at, host) == hipSuccess && at.type != hipMemoryTypeUnregistered)
+    return plain(host, device, n, s);  // pinned (one transfer at full rate), or not the host's to write
   (void)hipGetLastError();             // not a pointer the runtime knows: the usual case
   hipDevice_t dev = 0;
   if (hipStreamGetDevice(s, &dev) != hipSuccess) {

@@ -48,9 +48,29 @@ static int failing_stage() {
   return fake::live_events || !fake::pinned.empty() ? fail("left over", 0) : 0;
 }
 
+// A destination that the runtime knows is not written by the host: one
+// transfer straight into it.
+static int known_destination(hipMemoryType type, bool straight) {
+  rfh::stage_hold();
+  const size_t n = (size_t)5 << 20;
+  std::vector<unsigned char> src(n, 7), dst(n, 0);
+  FakeStream s{0};
+  fake::known = dst.data();
+  fake::known_type = type;
+  if (rfh::download(dst.data(), src.data(), n, &s) != hipSuccess) return fail("error", n);
+  if (src != dst) return fail("wrong bytes", n);
+  if ((fake::last.dst == dst.data() && fake::last.n == n) != straight) return fail("other way", n);
+  rfh::stage_release();
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   if (which == "other_device") return other_device();
   if (which == "failing_stage") return failing_stage();
+  if (which == "pinned") return known_destination(hipMemoryTypeHost, true);
+  if (which == "device") return known_destination(hipMemoryTypeDevice, true);
+  if (which == "managed") return known_destination(hipMemoryTypeManaged, true);
+  if (which == "unregistered") return known_destination(hipMemoryTypeUnregistered, false);
   return 2;
 }

@@ -1,6 +1,7 @@
 """Device-to-host copies: histograms come back byte for byte at the sizes where
 the path changes (plain copy, one pinned slot, several half or whole slots, a
 last partial one), into pinned memory too, and from two threads at once."""
+import ctypes
 import threading
 
 import numpy as np
@@ -29,6 +30,20 @@ def test_download_at_slot_edges(rf, gpu_available, n):
     pinned = torch.empty((n, 4), dtype=torch.float32, pin_memory=True)
     ctx.check(ctx.L.rf_hist_download(h.h, pinned.numpy().ctypes.data_as(ctx.L.rf_hist_download.argtypes[1])))
     assert np.array_equal(pinned.numpy(), want[0])
+
+
+@pytest.mark.parametrize("n", [4095, 4097, 131073, 1048577])
+def test_download_into_device_memory(rf, gpu_available, n):
+    """A device pointer as the destination, as hipMemcpy takes one."""
+    import torch
+    ctx = rf.Context(1 << 12, 1, 16)
+    b = _bins(torch, n, n)
+    h = ctx.histogram(n, 1, b.data_ptr())
+    out = torch.zeros_like(b)
+    torch.cuda.synchronize()
+    fp = ctx.L.rf_hist_download.argtypes[1]
+    ctx.check(ctx.L.rf_hist_download(h.h, ctypes.cast(out.data_ptr(), fp)))
+    assert torch.equal(out, b)
 
 
 def test_download_from_two_threads(rf, gpu_available):

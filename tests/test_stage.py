@@ -28,3 +28,11 @@ def test_copies_while_staging_fails(stage):
     bytes arrive by the plain copy, and the next copy is staged again."""
     r = stage("failing_stage")
     assert r.returncode == 0, r.stdout
+
+
+@pytest.mark.parametrize("kind", ["pinned", "device", "managed", "unregistered"])
+def test_destinations_the_runtime_knows(stage, kind):
+    """Pinned, device and managed memory take one transfer; only memory that the
+    runtime does not know is written by the host's threads."""
+    r = stage(kind)
+    assert r.returncode == 0, r.stdout
