@@ -963,10 +963,9 @@ static int de_args(rf_ctx* ctx, rf_hist* h, const rf_de_params* de, rfk::DEArgs&
   }
   const size_t nb = (size_t)h->w * h->h;
   if (h->de_rad.bytes < nb) HIPCHK(ctx, h->de_rad.alloc(nb));
-  if (!ctx->de_tab.p) {
-    HIPCHK(ctx, ctx->de_tab.alloc(sizeof(rfk::DETable)));
-    HIPCHK(ctx, rfk::launch_de_chords((rfk::DETable*)ctx->de_tab.p, ctx->stream));
-  }
+  HIPCHK(ctx, rfh::fill_once(ctx->de_tab, sizeof(rfk::DETable), [&](void* p) {
+    return rfk::launch_de_chords((rfk::DETable*)p, ctx->stream);
+  }));
   a.rad = (uint8_t*)h->de_rad.p;
   a.tab = (const rfk::DETable*)ctx->de_tab.p;
   return RF_OK;

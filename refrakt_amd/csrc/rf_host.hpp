@@ -8,6 +8,7 @@
 
 #include "../../include/refrakt_amd.h"
 #include "rf_device.hpp"
+#include "rf_once.hpp"
 #include "rf_stage.hpp"
 
 struct rf_ctx;
