@@ -154,9 +154,9 @@ __device__ __forceinline__ uint4 buf_load(__amdgpu_buffer_rsrc_t r, uint32_t lan
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 
-// This thread's input pieces, in 16-byte units from the patch's first pixel
-// (far) or in bytes (BUF_NONE either way: outside the image), in `in`, or
-// (up = 1) in the half-resolution `up`.  They are computed once per view and
+// This thread's input pieces in `in`, or (up = 1) in the half-resolution `up`:
+// bytes from the patch's first pixel or (FAR, where 32 bits need not hold them)
+// row, column and piece; BUF_NONE outside the image.  They are computed once per view and
 // tile: recomputed for every channel step, places and bounds were 300 vector
 // instructions a wave and step beside 144 MFMAs.
 template <int NT, int KC, int RW, bool FAR>
@@ -170,8 +170,9 @@ __device__ __forceinline__ void conv_places(ConvStage<NT, KC, RW>& st, int cs, i
     // (from the patch's row y0 - 1, column x0 - 1, halved with rounding down for `up`)
     const uint32_t dy = (uint32_t)((yy >> up) - ((y0 - 1) >> up)), dx = (uint32_t)((gx >> up) - ((x0 - 1) >> up));
     const bool in_image = q < S::IN_Q && yy >= 0 && yy < H && gx >= 0 && gx < W;
-    const uint32_t unit = (dy * (uint32_t)(W >> up) + dx) * (uint32_t)(cs / 8) + (uint32_t)piece;
-    st.place[k] = in_image ? (FAR ? unit : 16u * unit) : BUF_NONE;
+    const uint32_t at = FAR ? dy << 10 | dx << 3 | (uint32_t)piece
+                            : 16u * ((dy * (uint32_t)(W >> up) + dx) * (uint32_t)(cs / 8) + (uint32_t)piece);
+    st.place[k] = in_image ? at : BUF_NONE;
   }
 }
 
@@ -195,10 +196,11 @@ __device__ __forceinline__ uint4 piece_load(const bf16* row, int cs, uint32_t pl
 // The loads of one channel step.  Channels [0, Cup) come from the
 // half-resolution `up` (nearest-neighbour upsampling read in place), the rest
 // from `in`; a KC step never straddles the two (Cup is a multiple of 32).
-// `src` is the patch's first pixel in the step's view, c its first channel.
+// `src` is the patch's first pixel in the step's view of `width` columns and
+// channel stride cs, c its first channel.
 template <int NT, int KC, int RW, bool FAR>
-__device__ __forceinline__ void conv_load(ConvStage<NT, KC, RW>& st, const bf16* src, int c, const bf16* w, int c0,
-                                          int Cin, int Cout) {
+__device__ __forceinline__ void conv_load(ConvStage<NT, KC, RW>& st, const bf16* src, int width, int cs, int c,
+                                          const bf16* w, int c0, int Cin, int Cout) {
   using S = ConvStage<NT, KC, RW>;
   // weight row = tap * 16 NT + output channel; a round of 256 threads covers
   // whole taps
@@ -210,7 +212,8 @@ __device__ __forceinline__ void conv_load(ConvStage<NT, KC, RW>& st, const bf16*
     for (int k = 0; k < S::IN_PER; ++k) {
       st.vin[k] = make_uint4(0u, 0u, 0u, 0u);
       if (st.place[k] != BUF_NONE)
-        st.vin[k] = *reinterpret_cast<const uint4*>(src + 8 * (size_t)st.place[k] + c);
+        st.vin[k] = *reinterpret_cast<const uint4*>(
+            src + ((size_t)(st.place[k] >> 10) * width + (st.place[k] >> 3 & 127u)) * cs + 8 * (st.place[k] & 7u) + c);
     }
 #pragma unroll
     for (int k = 0; k < S::W_PER; ++k) {
@@ -415,7 +418,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RW == 2 ? (
   const bf16* const wsrc = w + (size_t)co0 * Cin;
   const bf16* src = Cup ? patch(up, 1) : patch(in, 0);
   conv_places<NT, KC, RW, FAR>(st, Cup ? up.cs : in.cs, Cup ? 1 : 0, y0, x0, H, W);
-  conv_load<NT, KC, RW, FAR>(st, src, 0, wsrc, 0, Cin, Cout);
+  conv_load<NT, KC, RW, FAR>(st, src, Cup ? W >> 1 : W, Cup ? up.cs : in.cs, 0, wsrc, 0, Cin, Cout);
   for (int c0 = 0; c0 < Cin; c0 += KC) {
     __syncthreads();  // the previous step's fragment reads are done
 #pragma unroll
@@ -434,7 +437,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RW == 2 ? (
         src = patch(in, 0);
         conv_places<NT, KC, RW, FAR>(st, in.cs, 0, y0, x0, H, W);
       }
-      conv_load<NT, KC, RW, FAR>(st, src, c0 + KC < Cup ? c0 + KC : c0 + KC - Cup, wsrc, c0 + KC, Cin, Cout);
+      const bool of_up = c0 + KC < Cup;
+      conv_load<NT, KC, RW, FAR>(st, src, of_up ? W >> 1 : W, of_up ? up.cs : in.cs, of_up ? c0 + KC : c0 + KC - Cup,
+                                 wsrc, c0 + KC, Cin, Cout);
     }
     // A fragment's LDS read takes as long as several MFMAs: the next group's
     // are under way while a group runs (and no more, for the registers; left

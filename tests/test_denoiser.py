@@ -155,6 +155,29 @@ def test_conv3x3_of_widely_spaced_pixels(rf, gpu_available, Cin, Cout):
     assert ((out[0].float() - ref.permute(0, 2, 3, 1)).abs() <= 2.0 ** -8 * ref.permute(0, 2, 3, 1).abs() + 1e-4).all()
 
 
+def test_conv3x3_of_pixels_gigabytes_apart(rf, gpu_available):
+    """A row of 33 GiB: its pixels' places from the tile's first exceed 32 bits
+    of 16-byte units."""
+    import torch
+    ctx = rf.Context(1 << 12, 1, 16)
+    g = torch.Generator().manual_seed(1)
+    W, cs, Cin, Cout = 66, 1 << 28, 64, 64
+    near = _bf16(torch.randn(1, 1, W, Cin, generator=g)).cuda()
+    w = _bf16(0.1 * torch.randn(3, 3, Cout, Cin, generator=g)).cuda()
+    b = torch.randn(Cout, generator=g).cuda()
+    far = torch.empty(1, 1, W, cs, dtype=torch.bfloat16, device="cuda")
+    far[..., cs - Cin:] = near
+    out = []
+    for x, xs, xo in ((near, Cin, 0), (far, cs, cs - Cin)):
+        o = torch.zeros(1, 1, W, Cout, dtype=torch.bfloat16, device="cuda")
+        ctx.check(ctx.L.rf_nn_conv3x3(ctx.h, x.data_ptr(), xs, xo, w.data_ptr(), b.data_ptr(), o.data_ptr(), Cout, 0,
+                                      1, 1, W, Cin, Cout, 0))
+        out.append(o.cpu())
+    del far
+    torch.cuda.empty_cache()
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+
+
 @pytest.mark.parametrize("cs,co", [(1 << 24, (1 << 24) - 32), (36, 4), (38, 2), (40, 8)])
 def test_conv3x3_wgrad_of_any_channel_stride(rf, gpu_available, cs, co):
     """Pixels too far apart for 32-bit offsets, and views that are no multiples
