@@ -1378,7 +1378,10 @@ hipError_t conv3x3(View in, const bf16* w, const float* bias, View out, int N, i
     // another path: the persistent kernel, faster at every size (32 -> 32,
     // with the call's 17 us: 2048^2 223 -> 162 us, 8 x 256^2 43 -> 33, 517 x
     // 333 28 -> 23; 16 -> 32 at 64^2 20.6 -> 17.3).
-    const bool few = (long long)10 * W * in.cs < (1ll << 31) && !k32 && nt <= 2 && Cin <= 32 && !Cup && vec_out && (!pool.p || fuse_pool) && (!fuse.y || fuse_res) &&
+    // (Its 32-bit offsets reach ten rows of the input, and of the other views a
+    // tile's 64 pixels.)
+    const bool few = (long long)10 * W * in.cs < (1ll << 31) &&
+                     std::max({out.cs, fuse.mask.cs, fuse.res.cs}) < (1 << 24) && !k32 && nt <= 2 && Cin <= 32 && !Cup && vec_out && (!pool.p || fuse_pool) && (!fuse.y || fuse_res) &&
                      (!fuse.Cdown || (Cin == 32 && nt == 2 && !relu && !fuse.mask.p));
     if (few) {
       int dev = 0, cus = 0;

@@ -155,6 +155,28 @@ def test_conv3x3_of_widely_spaced_pixels(rf, gpu_available, Cin, Cout):
     assert ((out[0].float() - ref.permute(0, 2, 3, 1)).abs() <= 2.0 ** -8 * ref.permute(0, 2, 3, 1).abs() + 1e-4).all()
 
 
+@pytest.mark.parametrize("Cout,cs", [(32, 1 << 29), (16, 1 << 29), (32, (1 << 24) + 8), (32, (1 << 24) - 8)])
+def test_conv3x3_into_pixels_gigabytes_apart(rf, gpu_available, Cout, cs):
+    """Narrow layers into a row of 16 GiB: its pixels' places exceed 32 bits."""
+    import torch
+    ctx = rf.Context(1 << 12, 1, 16)
+    g = torch.Generator().manual_seed(Cout)
+    W, Cin = 16, 32
+    x = _bf16(torch.randn(1, 1, W, Cin, generator=g)).cuda()
+    w = _bf16(0.1 * torch.randn(3, 3, Cout, Cin, generator=g)).cuda()
+    b = torch.randn(Cout, generator=g).cuda()
+    near = torch.zeros(1, 1, W, Cout, dtype=torch.bfloat16, device="cuda")
+    far = torch.empty(1, 1, W, cs, dtype=torch.bfloat16, device="cuda")
+    far[..., cs - Cout:] = 0
+    for o, os_, oo in ((near, Cout, 0), (far, cs, cs - Cout)):
+        ctx.check(ctx.L.rf_nn_conv3x3(ctx.h, x.data_ptr(), Cin, 0, w.data_ptr(), b.data_ptr(), o.data_ptr(), os_, oo,
+                                      1, 1, W, Cin, Cout, 1))
+    got = far[..., cs - Cout:].cpu()
+    del far
+    torch.cuda.empty_cache()
+    assert torch.equal(near.cpu().view(torch.int16), got.view(torch.int16))
+
+
 def test_conv3x3_of_pixels_gigabytes_apart(rf, gpu_available):
     """A row of 33 GiB: its pixels' places from the tile's first exceed 32 bits
     of 16-byte units."""
