@@ -223,7 +223,8 @@ __device__ __forceinline__ DEVisit<V> de_visit(CDETable* tab, int r, int i, int 
   return v;
 }
 
-// LDS words per source row of the tile: colours, masks, radii present.
+// LDS of a source row of the tile: the masks' words per radius, then (in bytes,
+// dr_row_bytes) those of all radii and the radii present.
 __host__ __device__ inline int dr_mask_words(int R) { return ((DR_W - 1 + 2 * R) >> 5) + 2; }
 inline uint64_t dr_tiles(uint32_t W, uint32_t H, int V, int S = 1) {
   const int th = DR_WAVES / S * V;
@@ -525,7 +526,8 @@ hipError_t launch_de_chords(DETable* tab, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int V, int S = 1>
+// RMAX: the largest radius that is launched with this V and S.
+template <int V, int S, int RMAX>
 static void launch_de_rows(const DEArgs& a, int R, hipStream_t s) {
   // all source rows of the tile at once while their masks fit 32 KiB (four
   // workgroups per CU, as many as its waves allow)
@@ -533,9 +535,12 @@ static void launch_de_rows(const DEArgs& a, int R, hipStream_t s) {
   const int K = (int)std::min<size_t>({(size_t)(DR_WAVES / S * V + 2 * R), (size_t)WAVE, (size_t)32768 / row});
   const size_t lds = std::max(K * row, S > 1 ? (size_t)V * DR_WAVES * WAVE * 16 : 0);
   const dim3 grid((unsigned)dr_tiles(a.W, a.H, V, S));
-  if (R < 16) hipLaunchKernelGGL((k_de_rows<V, 1, true, S>), grid, dim3(64 * DR_WAVES), lds, s, a, K);
-  else if (R < 32) hipLaunchKernelGGL((k_de_rows<V, 1, false, S>), grid, dim3(64 * DR_WAVES), lds, s, a, K);
-  else hipLaunchKernelGGL((k_de_rows<V, 4, false, S>), grid, dim3(64 * DR_WAVES), lds, s, a, K);
+  if (R < 16) {
+    hipLaunchKernelGGL((k_de_rows<V, 1, true, S>), grid, dim3(64 * DR_WAVES), lds, s, a, K);
+  } else if constexpr (RMAX >= 16) {
+    if (R < 32) hipLaunchKernelGGL((k_de_rows<V, 1, false, S>), grid, dim3(64 * DR_WAVES), lds, s, a, K);
+    else hipLaunchKernelGGL((k_de_rows<V, 4, false, S>), grid, dim3(64 * DR_WAVES), lds, s, a, K);
+  }
 }
 
 hipError_t launch_de_tonemap(const DEArgs& a, hipStream_t s) {
@@ -569,12 +574,12 @@ hipError_t launch_de_tonemap(const DEArgs& a, hipStream_t s) {
   //           R15  502   471   525   611   625   946
   // and at 5000x2700 radius 15 843 with 4/1.
   const uint64_t t = dr_tiles(a.W, a.H, 4);
-  if (t < 192) launch_de_rows<2, 8>(a, R, s);
-  else if (R < 4 && t < 2560) launch_de_rows<2, 1>(a, R, s);
-  else if (t < 1280 && R < 9) launch_de_rows<2, 2>(a, R, s);
-  else if (t < 1280) launch_de_rows<4, 4>(a, R, s);
-  else if (t < 4096 && R >= 12) launch_de_rows<4, 2>(a, R, s);
-  else launch_de_rows<4, 1>(a, R, s);
+  if (t < 192) launch_de_rows<2, 8, DE_MAX_R>(a, R, s);
+  else if (R < 4 && t < 2560) launch_de_rows<2, 1, 3>(a, R, s);
+  else if (t < 1280 && R < 9) launch_de_rows<2, 2, 8>(a, R, s);
+  else if (t < 1280) launch_de_rows<4, 4, DE_MAX_R>(a, R, s);
+  else if (t < 4096 && R >= 12) launch_de_rows<4, 2, DE_MAX_R>(a, R, s);
+  else launch_de_rows<4, 1, DE_MAX_R>(a, R, s);
   return hipGetLastError();
 }
 

@@ -483,6 +483,12 @@ def test_density_estimation_tiles_vs_oracle(rf, orc, gpu_available, W, H, R, rmi
     assert np.abs(out.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()
 
 
+# 4096 tiles of 64 x 32 and more, one wave a row, at every class of radius.
+@pytest.mark.parametrize("R,density", [(3, 0.01), (13, 0.006), (20, 0.004), (50, 0.001)])
+def test_density_estimation_of_many_tiles_vs_oracle(rf, orc, gpu_available, R, density):
+    test_density_estimation_tiles_vs_oracle(rf, orc, gpu_available, 4097, 2017, R, 0, 0.3, density)
+
+
 # One, two, four and eight waves per texel row: small radii, chords of 32
 # columns and more, ragged edges, rows with fewer source rows than waves.
 @pytest.mark.parametrize("W,H,R,density", [(1030, 421, 3, 0.3), (1027, 419, 1, 0.3), (1030, 421, 6, 0.3),
