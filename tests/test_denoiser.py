@@ -415,6 +415,128 @@ def test_unet_gradients_at_tile_edges(rf, gpu_available, N, H, W):
         assert cos > 0.99 and rel < 0.1, (i, cos, rel)
 
 
+class _Steps:
+    """The training step's gradients in separate steps: whole convolutions and
+    weight gradients of tensors that are written out (concatenations and
+    upsampled channels among them), and masks, pooling and 2x2 sums in torch."""
+
+    def __init__(self, rf, p):
+        import torch
+        self.t, self.ctx, off = torch, rf.Context(1 << 12, 1, 16), 0
+        self.layers = []
+        for cin, cout, relu in SPEC:
+            n = 9 * cin * cout
+            w = torch.from_numpy(p[off:off + n].copy()).cuda().to(torch.bfloat16).contiguous()
+            b = torch.from_numpy(p[off + n:off + n + cout].copy()).cuda()
+            wt = torch.empty_like(w)
+            self.ctx.check(self.ctx.L.rf_nn_flip_weights(self.ctx.h, w.data_ptr(), wt.data_ptr(), cin, cout))
+            self.layers.append((w, b, wt, cin, cout, relu))
+            off += n + cout
+        self.grads = [None] * len(SPEC)
+
+    def _conv(self, x, w, b, cin, cout, relu):
+        t, L = self.t, self.ctx.L
+        x = x.contiguous()
+        N, H, W, _ = x.shape
+        o = t.empty(N, H, W, cout, dtype=t.bfloat16, device="cuda")
+        self.ctx.check(L.rf_nn_conv3x3(self.ctx.h, x.data_ptr(), cin, 0, w.data_ptr(), b.data_ptr() if b is not None else None,
+                                       o.data_ptr(), cout, 0, N, H, W, cin, cout, relu))
+        return o
+
+    def conv(self, i, x):
+        w, b, _, cin, cout, relu = self.layers[i]
+        return self._conv(x, w, b, cin, cout, relu)
+
+    def dgrad(self, i, dy):
+        _, _, wt, cin, cout, _ = self.layers[i]
+        return self._conv(dy, wt, None, cout, cin, 0)
+
+    def wgrad(self, i, x, dy):
+        t, (_, _, _, cin, cout, _) = self.t, self.layers[i]
+        x, dy = x.contiguous(), dy.contiguous()
+        N, H, W, _ = x.shape
+        dw, db = t.zeros(9 * cin * cout, device="cuda"), t.zeros(cout, device="cuda")
+        self.ctx.check(self.ctx.L.rf_nn_conv3x3_wgrad(self.ctx.h, x.data_ptr(), cin, 0, dy.data_ptr(), cout, 0,
+                                                      dw.data_ptr(), db.data_ptr(), N, H, W, cin, cout))
+        self.grads[i] = t.cat([dw, db])
+
+    def sum4(self, x):
+        """2x2 sums in float, left to right and top to bottom."""
+        f = x.float()
+        return ((f[:, ::2, ::2] + f[:, ::2, 1::2]) + f[:, 1::2, ::2]) + f[:, 1::2, 1::2]
+
+    def run(self, x, target):
+        t = self.t
+        bf = lambda v: v.to(t.bfloat16)
+        keep = lambda v, y: t.where(y > 0, v, t.zeros_like(v))
+        up = lambda v: v.repeat_interleave(2, 1).repeat_interleave(2, 2)
+        pool = lambda v: bf(0.25 * self.sum4(v))
+        e0a = self.conv(0, x)
+        e0 = self.conv(1, e0a)
+        p0 = pool(e0)
+        e1a = self.conv(2, p0)
+        e1 = self.conv(3, e1a)
+        p1 = pool(e1)
+        e2a = self.conv(4, p1)
+        e2 = self.conv(5, e2a)
+        p2 = pool(e2)
+        b = self.conv(6, p2)
+        c2 = t.cat([up(b), e2], 3)
+        d2 = self.conv(7, c2)
+        c1 = t.cat([up(d2), e1], 3)
+        d1 = self.conv(8, c1)
+        c0 = t.cat([up(d1), e0], 3)
+        d0a = self.conv(9, c0)
+        d0b = self.conv(10, d0a)
+        o = self.conv(11, d0b)
+        npix = x.shape[0] * x.shape[1] * x.shape[2]
+        inv = float(np.float32(1.0) / (np.float32(4.0) * np.float32(npix)))
+        g = t.zeros_like(o)
+        g[..., :4] = bf(2.0 * ((x[..., :4].float() + o[..., :4].float()) - target[..., :4].float()) * inv)
+        for i, xin, y in ((11, d0b, d0b), (10, d0a, d0a)):
+            self.wgrad(i, xin, g)
+            g = keep(self.dgrad(i, g), y)
+        skips = []
+        for i, cat, lo in ((9, c0, d1), (8, c1, d2), (7, c2, b)):
+            self.wgrad(i, cat, g)
+            d = self.dgrad(i, g)
+            skips.append(d[..., lo.shape[3]:])
+            g = keep(bf(self.sum4(d[..., :lo.shape[3]])), lo)
+        for i, xin, skip, a, y, gs in ((6, p2, e2, 5, e2a, skips[2]), (4, p1, e1, 3, e1a, skips[1]),
+                                       (2, p0, e0, 1, e0a, skips[0])):
+            self.wgrad(i, xin, g)
+            pooled = up(self.dgrad(i, g)).float()
+            g = keep(bf(gs.float() + 0.25 * pooled), skip)
+            self.wgrad(a, y, g)
+            g = keep(self.dgrad(a, g), y)
+        self.wgrad(0, x, g)
+        return t.cat(self.grads).cpu().numpy()
+
+
+# Every level one pixel, tiles and strips that end inside an image at each
+# level, in each direction, and batches.
+@pytest.mark.parametrize("N,H,W", [(1, 8, 8), (2, 24, 72), (1, 16, 136), (1, 16, 528), (1, 264, 16), (3, 40, 200),
+                                   (1, 72, 264)])
+def test_unet_gradients_have_the_separate_steps_bits(rf, gpu_available, N, H, W):
+    """Masks, pooling, 2x2 sums and upsampled reads fused into the convolutions
+    and weight gradients change no bit of the gradient."""
+    print(f"gradients in separate steps: {N}x{H}x{W}", flush=True)
+    ctx = rf.Context(1 << 12, 1, 16)
+    dn = ctx.denoiser(seed=4)
+    p = dn.params()
+    p[-(9 * 32 * 16 + 16):] *= 10.0
+    dn.set_params(p)
+    x, t = (v.permute(0, 2, 3, 1).contiguous().cuda() for v in _inputs(N + W, N, H, W))
+    g, _ = dn.grads(x.data_ptr(), t.data_ptr(), N, H, W)
+    ref = _Steps(rf, p).run(x, t)
+    off = 0
+    for i, (cin, cout, _) in enumerate(SPEC):
+        n = 9 * cin * cout + cout
+        assert np.abs(ref[off:off + n]).max() > 0
+        assert np.array_equal(g[off:off + n], ref[off:off + n]), i
+        off += n
+
+
 def _unet_ref_autograd(pt, x):
     import torch
     import torch.nn.functional as F
