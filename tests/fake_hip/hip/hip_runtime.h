@@ -5,6 +5,7 @@
 #include <stddef.h>
 #include <string.h>
 
+#include <condition_variable>
 #include <mutex>
 #include <set>
 
@@ -23,6 +24,9 @@ namespace fake {
 inline thread_local int device = 0;
 inline std::mutex mu;
 inline std::set<void*> pinned;             // from hipHostMalloc
+inline size_t pinned_peak = 0;             // the most of them at once
+inline int meet = 0, met = 0;              // copies wait until `meet` have begun (0: none waits)
+inline std::condition_variable all_met;
 inline void* known = nullptr;              // a pointer the runtime knows
 inline hipMemoryType known_type = hipMemoryTypeDevice;
 inline int records_left = -1;              // event records before they fail (-1: never)
@@ -39,6 +43,7 @@ inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
   std::lock_guard<std::mutex> lk(fake::mu);
   *p = ::operator new(n);
   fake::pinned.insert(*p);
+  if (fake::pinned.size() > fake::pinned_peak) fake::pinned_peak = fake::pinned.size();
   return hipSuccess;
 }
 inline hipError_t hipHostFree(void* p) {
@@ -62,7 +67,10 @@ inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t) {
   memcpy(dst, src, n);
+  std::unique_lock<std::mutex> lk(fake::mu);
   fake::last = {dst, n};
+  if (fake::met < fake::meet && ++fake::met == fake::meet) fake::all_met.notify_all();
+  fake::all_met.wait(lk, [] { return fake::met >= fake::meet; });
   return hipSuccess;
 }
 inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {

@@ -64,10 +64,33 @@ static int known_destination(hipMemoryType type, bool straight) {
   return 0;
 }
 
+// More threads than stages: no stage is made for one copy.
+static int many_threads() {
+  rfh::stage_hold();
+  fake::meet = 6;
+  std::vector<int> rc(6, 0);
+  std::vector<std::thread> ts;
+  for (int t = 0; t < 6; ++t)
+    ts.emplace_back([&rc, t] { rc[t] = copies(FakeStream{0}, ((size_t)5 << 20) + t); });
+  for (auto& t : ts) t.join();
+  for (int r : rc)
+    if (r) return r;
+  // two stages of two allocations each
+  if (fake::pinned_peak > 4) return fail("too many stages", 5u << 20);
+  // both idle, and for another device one of them gives way
+  const size_t n = (size_t)5 << 20;
+  if (int r = copies(FakeStream{1}, n)) return r;
+  if (fake::last.n == n) return fail("not staged", n);
+  if (fake::pinned_peak > 4) return fail("a third stage", n);
+  rfh::stage_release();
+  return fake::live_events || !fake::pinned.empty() ? fail("left over", 0) : 0;
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   if (which == "other_device") return other_device();
   if (which == "failing_stage") return failing_stage();
+  if (which == "many_threads") return many_threads();
   if (which == "pinned") return known_destination(hipMemoryTypeHost, true);
   if (which == "device") return known_destination(hipMemoryTypeDevice, true);
   if (which == "managed") return known_destination(hipMemoryTypeManaged, true);

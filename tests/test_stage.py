@@ -36,3 +36,10 @@ def test_destinations_the_runtime_knows(stage, kind):
     runtime does not know is written by the host's threads."""
     r = stage(kind)
     assert r.returncode == 0, r.stdout
+
+
+def test_more_threads_than_stages(stage):
+    """Pinned memory and threads stay those of two stages; the other copies are
+    plain ones instead of waiting for a stage made for them."""
+    r = stage("many_threads")
+    assert r.returncode == 0, r.stdout
