@@ -309,6 +309,20 @@ __device__ __forceinline__ void de_strip(float4 (&acc)[V], CDETable* tab, const 
       if (!radii) continue;
       const uint32_t* const er = s_e + k * mrow;
       const float4* const cr = src - (ptrdiff_t)(s0 + k) * W;  // bins run bottom-up
+      if (SHORT && (radii & 1u)) {
+        // radius 0 (iw is 0): the source is its own texel, in one of the rows
+        // (above 15 radii are many and this saves less than it costs)
+        const int col = lane + R;
+        float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (er[col >> 5] >> (col & 31) & 1u) c = de_source(cr, col);
+#pragma unroll
+        for (int q = 0; q < V; ++q)
+          if (q == -i) {  // wave-uniform
+            acc[q].x += c.x; acc[q].y += c.y; acc[q].z += c.z; acc[q].w += c.w;
+          }
+        radii &= ~1u;
+        if (!radii) continue;
+      }
       int r = 32 * w + __builtin_ctz(radii);
       DEVisit<V> next = de_visit<V>(tab, r, i, iw);
       for (;;) {
@@ -363,42 +377,87 @@ __global__ __launch_bounds__(64 * DR_WAVES) __attribute__((amdgpu_waves_per_eu(8
       if (k >= rows || x >= SW || px < 1 || px >= W) return DE_EMPTY;
       return g.rad[(size_t)(H - 1 - (ty0 - R + s0 + k)) * W + px];
     };
-    uint32_t v0 = radius_at(wave, lane), v1 = radius_at(wave, WAVE + lane);
-    for (int k = wave; k < rows; k += DR_WAVES) {
-      uint32_t* const er = s_e + k * mrow;
-      for (int q = lane; q < mrow; q += WAVE) er[q] = 0u;
-      uint32_t rp[NRW];
+    // this row's masks of 64 columns from x0, one round per radius among them
+    auto put_masks = [&](uint32_t* er, uint32_t v, int x0, uint32_t (&rp)[NRW]) {
+      const int r = v == DE_EMPTY ? -1 : (int)(v & (DE_ODD - 1u));
+      uint64_t left = __builtin_amdgcn_ballot_w64(r >= 0);
+      uint32_t* const ex = er + (x0 >> 5);
+      const bool put = lane < 2 && (x0 >> 5) + lane < nwd;
+      while (left) {
+        const int rr = __builtin_amdgcn_readlane(r, __builtin_ctzll(left));
+        const uint64_t m = __builtin_amdgcn_ballot_w64(r == rr);
+        left &= ~m;
+        if (put) ex[rr * nwd + lane] = (uint32_t)(m >> (32 * lane));
+        if constexpr (NRW == 1) {
+          rp[0] |= 1u << rr;
+        } else {
 #pragma unroll
-      for (int w = 0; w < NRW; ++w) rp[w] = 0u;
-      bool odd = false;
-      for (int x0 = 0; x0 < SW; x0 += WAVE) {
-        // this row's first 128 columns were loaded during the previous row
-        const uint32_t v = x0 == 0 ? v0 : (x0 == WAVE ? v1 : radius_at(k, x0 + lane));
-        if (x0 == 0) v0 = radius_at(k + DR_WAVES, lane);
-        if (x0 == WAVE) v1 = radius_at(k + DR_WAVES, WAVE + lane);
-        const int r = v == DE_EMPTY ? -1 : (int)(v & (DE_ODD - 1u));
-        odd = odd || (v != DE_EMPTY && v >= DE_ODD);
+          for (int w = 0; w < NRW; ++w) rp[w] |= (rr >> 5) == w ? 1u << (rr & 31) : 0u;
+        }
+      }
+    };
+    bool odd = false;
+    auto is_odd = [](uint32_t v) { return v != DE_EMPTY && v >= DE_ODD; };
+    if constexpr (SHORT) {
+      // The 2 R columns beyond the first 64 of several rows in one go: `tw`
+      // lanes for each of G rows, a round per radius for all of them.  A pass
+      // of its own for each row took nearly half of the masks' time, which at
+      // small radii is a third of the kernel's: with this and the shorter way
+      // of radius 0 (de_strip) 7680x4320 at 0.3 samples a texel takes 585 us
+      // instead of 635 at radius 1, 1130 instead of 1185 at radius 9.
+      const int ts = R <= 4 ? 3 : R <= 8 ? 4 : 5, tw = 1 << ts, G = WAVE >> ts;
+      uint32_t v0 = radius_at(wave, lane);
+      for (int k0 = wave; k0 < rows; k0 += DR_WAVES * G) {
+        const int tk = k0 + DR_WAVES * (lane >> ts);
+        const uint32_t vt = radius_at(tk, WAVE + (lane & (tw - 1)));
+        for (int k = k0; k < min(rows, k0 + DR_WAVES * G); k += DR_WAVES) {
+          uint32_t* const er = s_e + k * mrow;
+          for (int q = lane; q < mrow; q += WAVE) er[q] = 0u;
+          uint32_t rp[NRW] = {0u};
+          const uint32_t v = v0;
+          v0 = radius_at(k + DR_WAVES, lane);  // the next row's, under way
+          odd = odd || is_odd(v);
+          put_masks(er, v, 0, rp);
+          if (lane == 0) s_rp[k] = rp[0];
+        }
+        odd = odd || is_odd(vt);
+        const int r = vt == DE_EMPTY ? -1 : (int)(vt & (DE_ODD - 1u));
+        uint32_t rpt = 0u;
         uint64_t left = __builtin_amdgcn_ballot_w64(r >= 0);
-        uint32_t* const ex = er + (x0 >> 5);
-        const bool put = lane < 2 && (x0 >> 5) + lane < nwd;
-        while (left) {  // one round per radius among these 64 columns
+        while (left) {
           const int rr = __builtin_amdgcn_readlane(r, __builtin_ctzll(left));
           const uint64_t m = __builtin_amdgcn_ballot_w64(r == rr);
           left &= ~m;
-          if (put) ex[rr * nwd + lane] = (uint32_t)(m >> (32 * lane));
-          if constexpr (NRW == 1) {
-            rp[0] |= 1u << rr;
-          } else {
-#pragma unroll
-            for (int w = 0; w < NRW; ++w) rp[w] |= (rr >> 5) == w ? 1u << (rr & 31) : 0u;
+          const uint32_t bits = (uint32_t)(m >> lane) & (uint32_t)((1ull << tw) - 1ull);
+          if ((lane & (tw - 1)) == 0 && bits != 0u) {
+            s_e[tk * mrow + rr * nwd + WAVE / 32] = bits;
+            rpt |= 1u << rr;
           }
         }
+        if (rpt != 0u) s_rp[tk] |= rpt;
       }
-      if (odd) s_odd = 1;
+    } else {
+      uint32_t v0 = radius_at(wave, lane), v1 = radius_at(wave, WAVE + lane);
+      for (int k = wave; k < rows; k += DR_WAVES) {
+        uint32_t* const er = s_e + k * mrow;
+        for (int q = lane; q < mrow; q += WAVE) er[q] = 0u;
+        uint32_t rp[NRW];
 #pragma unroll
-      for (int w = 0; w < NRW; ++w)
-        if (lane == 0) s_rp[w * K + k] = rp[w];
+        for (int w = 0; w < NRW; ++w) rp[w] = 0u;
+        for (int x0 = 0; x0 < SW; x0 += WAVE) {
+          // this row's first 128 columns were loaded during the previous row
+          const uint32_t v = x0 == 0 ? v0 : (x0 == WAVE ? v1 : radius_at(k, x0 + lane));
+          if (x0 == 0) v0 = radius_at(k + DR_WAVES, lane);
+          if (x0 == WAVE) v1 = radius_at(k + DR_WAVES, WAVE + lane);
+          odd = odd || is_odd(v);
+          put_masks(er, v, x0, rp);
+        }
+#pragma unroll
+        for (int w = 0; w < NRW; ++w)
+          if (lane == 0) s_rp[w * K + k] = rp[w];
+      }
     }
+    if (odd) s_odd = 1;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(s_odd) == 0) de_strip<V, NRW, S, true, SHORT>(acc, tab, src, W, s_e, s_rp, R, K, s0, rows);
     else de_strip<V, NRW, S, false, SHORT>(acc, tab, src, W, s_e, s_rp, R, K, s0, rows);
@@ -559,20 +618,20 @@ hipError_t launch_de_tonemap(const DEArgs& a, hipStream_t s) {
   // source rows that bounds an image of few tiles, for a sum through LDS and
   // masks built for fewer texels.  Measured (us, the tonemap included; V/S):
   //               4/1   4/2   4/4   2/1   2/2   2/8
-  //   320x240  R9   64    50    42    49    39    29   (1/1, one wave a row: 45)
-  //           R24  177   108    75   140    90    52
-  //   900x480  R4   55    51    50    47    43    50
-  //            R9   89    75    64    77    63    73
-  //           R24  320   210   159   271   204   185
-  //   1900x1000 R1  53    59    66    50    55    84
-  //            R9  124   111   110   119   111   160
-  //           R24  394   299   256   403   320   389
-  //   2600x1400 R1  82    95   116    78    94   153
-  //            R7  153   154   177   157   169   280
-  //           R24  585   495   495   672   629   887
-  //   3000x1600 R9 284   287   349   325   355   578
-  //           R15  502   471   525   611   625   946
-  // and at 5000x2700 radius 15 843 with 4/1.
+  //   320x240  R9   63    49    41    49    39    28   (1/1, one wave a row: 44)
+  //           R24  180   108    77   141    91    54
+  //   900x480  R4   52    50    48    48    43    50
+  //            R9   86    74    64    79    66    72
+  //           R24  334   215   175   282   225   189
+  //   1900x1000 R1  50    56    64    50    57    85
+  //            R9  122   109   107   120   111   149
+  //           R24  414   316   271   431   338   407
+  //   2600x1400 R1  76    93   113    78    98   157
+  //            R7  150   151   174   162   171   265
+  //           R24  620   522   522   739   677   945
+  //   3000x1600 R9 277   284   334   330   356   542
+  //           R15  469   443   490   597   603   847
+  // and at 5000x2700 radius 15 857 with 4/1.
   const uint64_t t = dr_tiles(a.W, a.H, 4);
   if (t < 192) launch_de_rows<2, 8, DE_MAX_R>(a, R, s);
   else if (R < 4 && t < 2560) launch_de_rows<2, 1, 3>(a, R, s);

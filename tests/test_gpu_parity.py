@@ -498,6 +498,33 @@ def test_density_estimation_shared_rows_vs_oracle(rf, orc, gpu_available, W, H, 
     test_density_estimation_tiles_vs_oracle(rf, orc, gpu_available, W, H, R, 0, 0.35, density)
 
 
+# The columns beyond a tile's first 64 in groups of 8, 16 and 32 lanes, full and
+# ragged rows, and an infinity among them.
+@pytest.mark.parametrize("W,H,R,rmin,density", [(130, 70, 4, 0, 0.9), (130, 71, 5, 5, 0.5), (129, 37, 8, 0, 0.9),
+                                                (191, 33, 15, 0, 0.6), (1030, 421, 4, 0, 0.4), (1030, 421, 8, 1, 0.4),
+                                                (2501, 2150, 2, 0, 0.1)])
+def test_density_estimation_tile_tails_vs_oracle(rf, orc, gpu_available, W, H, R, rmin, density):
+    test_density_estimation_tiles_vs_oracle(rf, orc, gpu_available, W, H, R, rmin, 0.35, density)
+
+
+@pytest.mark.parametrize("px", [61, 64, 65, 72, 73])
+def test_density_estimation_keeps_an_infinity_of_a_tile_tail(rf, orc, gpu_available, px):
+    import torch
+    W, H, R = 130, 41, 9
+    h = _sparse_hist(np.random.default_rng(px), W, H)
+    h[H // 2, px] = [0.5, np.inf, 0.5, 1.0]
+    ctx = _ctx(rf, 1 << 10, 1, rf.RF_ENGINE_FAST)
+    hist = ctx.histogram(W, H)
+    hist.upload(h)
+    out = torch.zeros((H, W, 4), dtype=torch.float32, device="cuda")
+    ctx.density_estimate(hist, rf.DEParams(R, 0, 0.4), out.data_ptr())
+    g = out.cpu().numpy()
+    ref = orc.density(h, R, 0, 0.4, fp32=True)
+    fin = np.isfinite(ref)
+    assert (~fin).sum() > R * R and np.array_equal(np.isfinite(g), fin) and not np.isnan(g).any()
+    assert np.abs(g[fin] - ref[fin]).max() <= 2e-5 * np.abs(ref[fin]).max()
+
+
 @pytest.mark.parametrize("W,H,R", [(97, 75, 9), (1030, 129, 20)])
 def test_density_estimation_keeps_an_infinity_in_its_splat(rf, orc, gpu_available, W, H, R):
     """A bin with an infinite colour reaches the texels of its own splat only."""
