@@ -269,6 +269,45 @@ def test_fast_sort_small_images_round_once(rf, gpu_available, P, passes, W, H):
     assert np.array_equal(a[room < 125000].view(np.uint32), b[room < 125000].view(np.uint32))
 
 
+def test_fast_sort_parts_over_subdraws(rf, orc, gpu_available):
+    """A call of several sub-draws into a small image, twice: the parts' sums are
+    added and cleared behind each, counts as the replica's and the same bits."""
+    P, passes, W, H, seed, waves = 1 << 12, 150, 64, 64, 5, 8
+    fl = _linear_flame(rf, 29, W=W, H=H)
+
+    def draw():
+        ctx = _ctx(rf, P, 1, rf.RF_ENGINE_FAST, hist_mode=rf.RF_HIST_SORT, seed=seed, waves=waves)
+        fh = ctx.flame(fl)
+        fh.warmup(19)
+        fh.draw_to_bins(ctx.histogram(W, H), 1)  # the distribution
+        hist = ctx.histogram(W, H)
+        a = fh.draw_to_bins(hist, passes)
+        first = hist.download()
+        b = fh.draw_to_bins(hist, 64)  # the same plan, added to the first
+        assert fh.sort_overflow() == 0.0
+        return ctx, a, b, first, hist.download()
+
+    ctx, a, b, first, both = draw()
+    fc = orc.flame_to_c(fl)
+    ss = orc.screen_affine(fl, W, H)
+    perms = ctx.fast_perms(waves)
+    pos = np.zeros((P, 4), np.float32)
+    orc.fast_run(fc, P, P, waves, perms, seed, 0, 20, True, False, W, H, ss, pos)
+    hits = np.zeros((H, W), np.uint32)
+    orc.fast_run(fc, P, P, waves, perms, seed, 1, 1, False, True, W, H, ss, pos, None, np.zeros((H, W), np.uint32))
+    n = sum(orc.fast_run(fc, P, P, waves, perms, seed, 2 + k, m, False, True, W, H, ss, pos, None, hits)
+            for k, m in enumerate((64, 64, 22)))
+    assert a == n and np.array_equal(first[..., 3].astype(np.uint32), hits)
+    n = orc.fast_run(fc, P, P, waves, perms, seed, 5, 64, False, True, W, H, ss, pos, None, hits)
+    assert b == n and np.array_equal(both[..., 3].astype(np.uint32), hits)
+    # 262144 samples a sub-draw in one tile: segments of 131068, so the order of
+    # their sums is free; each sample's colour is off by 1 / (2 * 32767) at most
+    again = draw()[4]
+    assert np.array_equal(again[..., 3], both[..., 3])
+    tol = 1e-5 * np.abs(both[..., :3]) + 2 * hits[..., None] / 65534.0
+    assert (np.abs(again[..., :3] - both[..., :3]) <= tol).all()
+
+
 # ------------------------------------------------- non-finite particle policy
 def _nan_xform(rf, kind):
     """An xform whose output is never finite: a NaN variation weight, or an
