@@ -296,7 +296,8 @@ typedef struct rf_batch_config {
   int32_t block_waves;         /* 4 or 8: a work item is 64 * block_waves particles */
   int32_t hist_mode;           /* RF_HIST_QUAD, RF_HIST_LDS or RF_HIST_SORT (sort needs unit
                                   opacities and palettes in [0, 1], else LDS or quad run;
-                                  its record capacities come from the last finished replay) */
+                                  its record capacities are planned when the graph is
+                                  captured, from the last replay finished by then) */
   uint32_t iters;              /* binned iterations per particle */
   uint32_t fuse;               /* unbinned iterations per particle before those */
 } rf_batch_config;

@@ -1,9 +1,8 @@
 // Denoiser network kernels: interface between rf_denoiser.cpp and rf_k_nn.hip.
 //
 // Activations are NHWC bf16.  A "view" (ptr, cs, co) addresses channels
-// [co, co + C) of a tensor whose pixels are cs channels apart, so skip
-// connections are written straight into the channel range of the
-// concatenated tensor that consumes them.
+// [co, co + C) of a tensor whose pixels are cs channels apart.  A convolution
+// over a concatenation reads its two parts from two views (ConvFuse::up).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -41,8 +40,8 @@ struct ConvFuse {
   // backward; mask has the output's Cout channels, 16-byte aligned runs as
   // in the input and the output).
   View mask{nullptr, 0, 0};
-  // Cdown > 0: the first Cdown output channels (a multiple of 64 and less than
-  // Cout) are the gradient of a 2x2 upsampling: instead of being written to
+  // Cdown > 0: the first Cdown output channels (a multiple of the channels of a
+  // workgroup, 64, 32 or 16 by what divides Cout, and less than Cout) are the gradient of a 2x2 upsampling: instead of being written to
   // `out`, their 2x2 sums (of the bf16 outputs), kept where
   // down_mask > 0, go to `down`.  H and W even, both views N x H/2 x W/2 with
   // 16-byte aligned channel runs.

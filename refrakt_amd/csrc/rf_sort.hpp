@@ -83,10 +83,12 @@ struct SortArgs {
 //   64 buckets           277 / 171  308 / 205  334 / 254  384 / 326  605 / 500
 // Where more than half a stage is filled anyway, up to 32 buckets (one line of
 // cursors) hide the flushes behind the other workgroups' iterations and the
-// coarser grid costs more than it saves (*: not done).  More batches than four
-// fill no stage better than 7/8 of what four do, and a grid below the resident
-// workgroups leaves compute units idle: 262144 particles, 5 iterations, 68 us
-// with one batch, 79 with three.
+// coarser grid costs more than it saves (*: not done).  Up to eight batches
+// gain nothing over four: 1 and 3 iterations 105 and 195 us instead of 102 and
+// 184 into 2048^2, 125 and 205 instead of 122 and 194 into 4096^2, and with
+// four times the particles 294 and 560 instead of 296 and 570.  A grid below
+// the resident workgroups leaves compute units idle: 262144 particles, 5
+// iterations, 68 us with one batch, 79 with three.
 inline uint32_t sort_grid(uint32_t n_batches, uint32_t n_iter, uint32_t n_buckets, uint32_t stage,
                           uint32_t resident) {
   if (n_iter == 0 || (n_buckets <= 32 && n_iter > stage / 2)) return n_batches;
