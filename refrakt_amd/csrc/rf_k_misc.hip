@@ -396,7 +396,6 @@ __global__ __launch_bounds__(64 * DR_WAVES) __attribute__((amdgpu_waves_per_eu(8
         }
       }
     };
-    bool odd = false;
     auto is_odd = [](uint32_t v) { return v != DE_EMPTY && v >= DE_ODD; };
     if constexpr (SHORT) {
       // The 2 R columns beyond the first 64 of several rows in one go: `tw`
@@ -406,6 +405,7 @@ __global__ __launch_bounds__(64 * DR_WAVES) __attribute__((amdgpu_waves_per_eu(8
       // of radius 0 (de_strip) 7680x4320 at 0.3 samples a texel takes 585 us
       // instead of 635 at radius 1, 1130 instead of 1185 at radius 9.
       const int ts = R <= 4 ? 3 : R <= 8 ? 4 : 5, tw = 1 << ts, G = WAVE >> ts;
+      bool odd = false;
       uint32_t v0 = radius_at(wave, lane);
       for (int k0 = wave; k0 < rows; k0 += DR_WAVES * G) {
         const int tk = k0 + DR_WAVES * (lane >> ts);
@@ -436,6 +436,7 @@ __global__ __launch_bounds__(64 * DR_WAVES) __attribute__((amdgpu_waves_per_eu(8
         }
         if (rpt != 0u) s_rp[tk] |= rpt;
       }
+      if (odd) s_odd = 1;
     } else {
       uint32_t v0 = radius_at(wave, lane), v1 = radius_at(wave, WAVE + lane);
       for (int k = wave; k < rows; k += DR_WAVES) {
@@ -444,6 +445,7 @@ __global__ __launch_bounds__(64 * DR_WAVES) __attribute__((amdgpu_waves_per_eu(8
         uint32_t rp[NRW];
 #pragma unroll
         for (int w = 0; w < NRW; ++w) rp[w] = 0u;
+        bool odd = false;
         for (int x0 = 0; x0 < SW; x0 += WAVE) {
           // this row's first 128 columns were loaded during the previous row
           const uint32_t v = x0 == 0 ? v0 : (x0 == WAVE ? v1 : radius_at(k, x0 + lane));
@@ -452,12 +454,12 @@ __global__ __launch_bounds__(64 * DR_WAVES) __attribute__((amdgpu_waves_per_eu(8
           odd = odd || is_odd(v);
           put_masks(er, v, x0, rp);
         }
+        if (odd) s_odd = 1;
 #pragma unroll
         for (int w = 0; w < NRW; ++w)
           if (lane == 0) s_rp[w * K + k] = rp[w];
       }
     }
-    if (odd) s_odd = 1;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(s_odd) == 0) de_strip<V, NRW, S, true, SHORT>(acc, tab, src, W, s_e, s_rp, R, K, s0, rows);
     else de_strip<V, NRW, S, false, SHORT>(acc, tab, src, W, s_e, s_rp, R, K, s0, rows);
