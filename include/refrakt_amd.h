@@ -218,7 +218,10 @@ int rf_hist_create(rf_ctx* ctx, uint32_t width, uint32_t height, rf_hist** out);
 int rf_hist_wrap(rf_ctx* ctx, void* device_ptr, uint32_t width, uint32_t height, rf_hist** out);
 void rf_hist_destroy(rf_hist* hist);
 int rf_hist_zero(rf_hist* hist);                    /* ≙ bins.zero_out() */
-int rf_hist_download(rf_hist* hist, float* host);   /* W*H*4 floats */
+/* W*H*4 floats.  Downloads of 64 KB and more into ordinary memory (histograms,
+ * images, particles, gradients) go through pinned memory of the process, at most
+ * 64 MB, and up to sixteen threads, which are freed with the last context. */
+int rf_hist_download(rf_hist* hist, float* host);
 int rf_hist_upload(rf_hist* hist, const float* host);
 void* rf_hist_device_ptr(rf_hist* hist);
 
